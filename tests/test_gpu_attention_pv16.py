@@ -121,6 +121,28 @@ def test_accuracy_mode_on_rows_that_one_key_dominates(dev):
         assert e16 <= 2e-2, e16
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal,blocks", [(False, 16), (True, 16), (False, 2), (False, 1)])
+def test_accuracy_mode_maximum_recovery(dev, D, causal, blocks):
+    """The weights are computed with the running maximum as it is; a score more than eleven octaves above it becomes
+    an infinite float16 weight, seen in the row sums, and the block is computed again.  Scores that climb by 4.3
+    octaves a block force that every third block, in every row (a last block of 45 keys; also one and two blocks,
+    the shortest runs of the two-stage ring)."""
+    import paroatten_amd as P
+    from test_gpu_attention import _ramp_case
+    B, H, N = 1, 2, 64 * blocks - 19
+    q, k, v = _ramp_case(B, H, N, D, torch.float16, 7 + D, "ramp")
+    mask = torch.ones(H, blocks, blocks, dtype=torch.bool)
+    o_ref, lse_ref = _oracle(q, k, v, mask, D, causal, False)
+    args = (q.to(dev), k.to(dev), v.to(dev), mask.to(dev))
+    o, lse = P.paroattn_qk_int8_pv_fp16_cuda(*args, is_causal=causal, pv_f16=True, return_lse=True)
+    # weights and outputs rounded to 2^-11 each of at most max|v| < 5
+    assert (o.cpu().float() - o_ref).abs().max().item() <= 2 * 2.0 ** -11 * float(v.abs().max())
+    # an exponent is formed as score * scale + bias in fp32, both about 10680707 * scale: half an ulp of that each
+    assert (lse.cpu() - lse_ref).abs().max().item() <= 2e-3
+    assert torch.equal(o, P.paroattn_qk_int8_pv_fp16_cuda(*args, is_causal=causal, pv_f16=True))
+
+
 def test_prepacked_tiles_and_the_unpermuting_store(dev):
     """The kernel on operands packed beforehand (paro_v_f16_pack + paro_attn_sparse_fwd with the flag) gives the
     bits of the one-call entry point; with the unpermuting store, the rows land where permute_attn_out would put

@@ -177,7 +177,6 @@ __global__ void __launch_bounds__(256) rope_permute_quant_kernel(const PrepParam
       vov[i] = (int)(((int64_t)src[i] * p.vs_n + c) * 2);
     }
   }
-  const int n_chunks = (p.N + V_CHUNK - 1) / V_CHUNK;
   const int q_bytes = (int)((((int64_t)p.N - 1) * p.qs_n + D) * 2);
   const int k_bytes = (int)((((int64_t)p.N - 1) * p.ks_n + D) * 2);
   const int v_bytes = (int)((((int64_t)p.N - 1) * p.vs_n + D) * 2);
@@ -209,7 +208,7 @@ __global__ void __launch_bounds__(256) rope_permute_quant_kernel(const PrepParam
     const __amdgpu_buffer_rsrc_t rm = raw_buffer(km ? p.k_mean + b * p.ms_b + head * p.ms_h : p.k, km ? D * 2 : 0);
     buffer_load4_lds(rm, smem + L::KM_OFF + par * 256, lane * 4);
     const __amdgpu_buffer_rsrc_t rs =
-        raw_buffer(bh < 0 ? p.v_stats : p.v_stats + v_recp_offset(bh, n_chunks, D), bh < 0 ? 0 : 2 * D * 4);
+        raw_buffer(bh < 0 ? p.v_stats : p.v_stats + v_recp_offset(bh, p.N, D), bh < 0 ? 0 : 2 * D * 4);
     buffer_load16_lds(rs, smem + L::ST_OFF + par * 1024, lane * 16);
   };
   auto load_v = [&](int slot) {
@@ -366,7 +365,7 @@ static inline int k_sum_blocks(int n_chunks, int BH) { return ceil_div(n_chunks,
 struct KvStatsParams {
   const unsigned short* k; const unsigned short* v;
   const float* cos_t; const float* sin_t;
-  float* k_partial; float* v_partial;
+  float* k_partial; float* v_work;
   unsigned short* k_mean; float* v_scale; float* v_mean;
   int B, H, N, n_text, k_chunks, v_chunks, k_blocks, smooth_v;
   int64_t ks_b, ks_h, ks_n, vs_b, vs_h, vs_n, ms_b, ms_h;
@@ -380,7 +379,7 @@ __global__ void __launch_bounds__(256) kv_stats_kernel(const KvStatsParams p) {
   } else {
     const int i = blockIdx.x - p.k_blocks;
     const int chunk = i % p.v_chunks, bh = i / p.v_chunks;
-    v_stats_body<DT, D>(p.v, p.v_partial, p.N, p.v_chunks, p.vs_b, p.vs_h, p.vs_n, chunk, bh % p.H, bh / p.H, p.H);
+    v_stats_body<DT, D>(p.v, p.v_work + v_stats_offset((int64_t)p.B * p.H, p.N, D), p.N, p.v_chunks, p.vs_b, p.vs_h, p.vs_n, chunk, bh % p.H, bh / p.H, p.H);
   }
 }
 
@@ -390,7 +389,7 @@ __global__ void __launch_bounds__(1024) kv_finalize_kernel(const KvStatsParams p
   if ((int)blockIdx.x < BH)
     k_mean_finalize_body<DT, D>(p.k_partial, p.k_mean, p.N, p.k_chunks, p.ms_b, p.ms_h, p.H, blockIdx.x);
   else
-    v_finalize_body<D>(p.v_partial, p.v_scale, p.v_mean, p.N, p.v_chunks, p.smooth_v, (int64_t)blockIdx.x - BH);
+    v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.N, p.v_chunks, p.smooth_v, (int64_t)blockIdx.x - BH, BH);
 }
 
 template <int DT, int D>
@@ -535,10 +534,10 @@ static int prep_impl(bool compute_k_mean, const void* q, const void* k, const vo
   } else {
     KvStatsParams sp;
     sp.k = (const unsigned short*)k; sp.v = (const unsigned short*)v; sp.cos_t = cos; sp.sin_t = sin;
-    sp.v_partial = (float*)workspace;
+    sp.v_work = (float*)workspace;
     sp.k_partial = (float*)workspace + paro_v_fp8_partial_floats(B, H, N, D);   // behind the V partials
     sp.k_mean = (unsigned short*)k_mean; sp.v_scale = v_scale; sp.v_mean = v_mean;
-    sp.B = B; sp.H = H; sp.N = N; sp.n_text = n_text; sp.k_chunks = ceil_div(N, K_CHUNK); sp.v_chunks = ceil_div(N, V_CHUNK);
+    sp.B = B; sp.H = H; sp.N = N; sp.n_text = n_text; sp.k_chunks = ceil_div(N, K_CHUNK); sp.v_chunks = ceil_div(N, v_chunk(N));
     sp.k_blocks = k_sum_blocks(sp.k_chunks, B * H); sp.smooth_v = smooth_v;
     sp.ks_b = k_stride_b; sp.ks_h = k_stride_h; sp.ks_n = k_stride_n;
     sp.vs_b = v_stride_b; sp.vs_h = v_stride_h; sp.vs_n = v_stride_n; sp.ms_b = mean_stride_b; sp.ms_h = mean_stride_h;
@@ -567,7 +566,7 @@ static int prep_impl(bool compute_k_mean, const void* q, const void* k, const vo
   p.q = (const unsigned short*)q; p.k = (const unsigned short*)k; p.v = (const unsigned short*)v;
   p.cos_t = cos; p.sin_t = sin; p.orders = (const int*)orders; p.k_mean = (const unsigned short*)k_mean;
   p.q8 = q8; p.q_scale = q_scale; p.k8 = k8; p.k_scale = k_scale; p.v8 = v8; p.v_stats = (const float*)workspace;
-  p.v_resid = smooth_v ? (float*)workspace + v_resid_offset((int64_t)B * H, ceil_div(N, V_CHUNK), D) : nullptr;
+  p.v_resid = smooth_v ? (float*)workspace + v_resid_offset((int64_t)B * H, N, D) : nullptr;
   p.BH = B * H; p.H = H; p.N = N; p.nb = nb; p.n_text = n_text; p.F = F; p.Hh = Hh; p.W = W; p.head_split = head_split;
   p.qs_b = q_stride_b; p.qs_h = q_stride_h; p.qs_n = q_stride_n;
   p.ks_b = k_stride_b; p.ks_h = k_stride_h; p.ks_n = k_stride_n;

@@ -4,11 +4,13 @@
 
 namespace paro {
 
-// tokens per workgroup of the two statistics passes.  Measured: the V statistics (three values per
-// channel to reduce and write) want long chunks, 1024 beats 256 by 7 %; the K mean, launched per group
-// of heads, runs out of workgroups beyond 256.
+// tokens per workgroup of the two statistics passes.  Measured: over long sequences the V statistics (three values
+// per channel to reduce and write) want long chunks, 1024 beats 256 by 7 % at 17776 tokens; up to 8192 tokens there
+// are then too few workgroups, and the pass takes as long as one workgroup needs for its chunk (see v_stats_body).
+// The K mean, launched per group of heads, runs out of workgroups beyond 256.
 constexpr int V_CHUNK = 1024;  // per-channel V statistics
 constexpr int K_CHUNK = 256;   // rotated K mean
+__host__ __device__ constexpr int v_chunk(int N) { return N > 256 && N <= 8192 ? 256 : V_CHUNK; }
 
 // strides of the (f,h,w) coordinates in the permuted order `order`
 // (0 FHW, 1 FWH, 2 HWF, 3 HFW, 4 WHF, 5 WFH).  Written as selects: a switch that assigns through the
@@ -170,11 +172,15 @@ __device__ __forceinline__ void pack_v_tile(const unsigned short* tile, uint8_t*
   }
 }
 
-// residual sums of pack_v_tile: [B*Hkv][nb][2 row tiles][D] floats behind the statistics partials
-__host__ __device__ inline int64_t v_resid_offset(int64_t BH, int n_chunks, int D) { return BH * n_chunks * 3 * D; }
+// The work buffer of the V conversion: [BH][ceil(N / V_CHUNK)][3][D] floats, then the residual sums of pack_v_tile,
+// [BH][nb][2 row tiles][D].  The statistics partials, [BH][ceil(N / v_chunk(N))][3][D], are in the first part with long
+// chunks and in the second with short ones (3 ceil(N / 256) <= 2 ceil(N / 64) beyond 64 tokens): the residuals are
+// written after the partials have been read.
+__host__ __device__ inline int64_t v_resid_offset(int64_t BH, int N, int D) { return BH * ((N + V_CHUNK - 1) / V_CHUNK) * 3 * D; }
+__host__ __device__ inline int64_t v_stats_offset(int64_t BH, int N, int D) { return v_chunk(N) == V_CHUNK ? 0 : v_resid_offset(BH, N, D); }
 
-// where v_fp8_stats leaves recp[b,h,:] inside the partial-sum workspace
-__host__ __device__ inline int64_t v_recp_offset(int64_t bh, int n_chunks, int D) { return bh * n_chunks * 3 * D; }
+// where the second step of the statistics leaves recp[b,h,:] and behind it mean[b,h,:]: in the first part
+__host__ __device__ inline int64_t v_recp_offset(int64_t bh, int N, int D) { return bh * ((N + V_CHUNK - 1) / V_CHUNK) * 3 * D; }
 
 // per-(batch, head, channel) statistics of V: v_scale = max|v - mean| / 448, v_mean = mean over the
 // N tokens (0 if !smooth), and recp = 448 / max|v - mean| at partial[v_recp_offset(bh, ...) + ch];

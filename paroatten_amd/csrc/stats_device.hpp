@@ -3,10 +3,13 @@
 // The launches that use them: v_fp8.hip (V alone), fused_prep.hip (K alone, or K and V in one launch).
 #pragma once
 #include "paro_device.hpp"
+#include <type_traits>
 
 namespace paro {
 
-// Per-channel sum, minimum and maximum of one V_CHUNK-token chunk of one (batch, head): 256 threads.
+// Per-channel sum, minimum and maximum of one v_chunk(N)-token chunk of one (batch, head): 256 threads.  Rows are
+// requested in batches of eight, in the last chunk too (rows past the end re-read the last one and are not taken): a
+// row at a time, the 738 rows of the last of two chunks took 15.7 us at N = 1762, B = 2, H = 4, D = 64.
 template <int DT, int D>
 __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ v, float* __restrict__ partial, int N,
                                              int n_chunks, int64_t vs_b, int64_t vs_h, int64_t vs_n, int chunk, int h,
@@ -32,26 +35,27 @@ __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ 
       mx[j] = fmaxf(mx[j], f);
     }
   };
-  const int tok0 = chunk * V_CHUNK + t / LPR;
-  if (chunk * V_CHUNK + V_CHUNK <= N) {
-    // full chunk (uniform): batches of VS_BATCH independent loads, then the arithmetic
-    constexpr int VS_BATCH = 8;
-    for (int r = 0; r < V_CHUNK; r += ROWS * VS_BATCH) {
+  const int len = v_chunk(N), first = chunk * len, tok0 = first + t / LPR;
+  constexpr int VS_BATCH = 8;
+  auto walk = [&](auto whole) {
+    for (int r = 0; r < len; r += ROWS * VS_BATCH) {
+      if (!decltype(whole)::value && first + r >= N) break;
       v4i raw[VS_BATCH];
 #pragma unroll
-      for (int u = 0; u < VS_BATCH; u++)
+      for (int u = 0; u < VS_BATCH; u++) {
         // (non-temporal: measured 3-5 us faster per launch of the entry point and of the per-layer sequence
         // than ordinary loads, although the packing pass reads the same tensor right afterwards)
-        raw[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(vb + (int64_t)(tok0 + r + u * ROWS) * vs_n));
+        const int tok = tok0 + r + u * ROWS;
+        raw[u] = __builtin_nontemporal_load(
+            reinterpret_cast<const v4i*>(vb + (int64_t)(decltype(whole)::value ? tok : min(tok, N - 1)) * vs_n));
+      }
 #pragma unroll
-      for (int u = 0; u < VS_BATCH; u++) take(raw[u]);
+      for (int u = 0; u < VS_BATCH; u++)
+        if (decltype(whole)::value || tok0 + r + u * ROWS < N) take(raw[u]);
     }
-  } else {
-    for (int r = 0; r < V_CHUNK; r += ROWS) {
-      const int tok = tok0 + r;
-      if (tok < N) take(*reinterpret_cast<const v4i*>(vb + (int64_t)tok * vs_n));
-    }
-  }
+  };
+  if (first + len <= N) walk(std::true_type{});
+  else walk(std::false_type{});
   // lanes that share a column sit LPR apart: 8 lanes round the row (D = 64 only), then lane ^ 16, ^ 32
 #pragma unroll
   for (int j = 0; j < 8; j++) {
@@ -90,15 +94,16 @@ __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ 
 }
 
 
-// mean, scale and reciprocal scale of one (batch, head) from its chunk statistics: 1024 threads.
+// mean, scale and reciprocal scale of one (batch, head) from its chunk statistics: 1024 threads.  `work`: the work
+// buffer of the V conversion (v_stats_offset, v_recp_offset).
 template <int D>
-__device__ __forceinline__ void v_finalize_body(float* partial, float* __restrict__ v_scale, float* __restrict__ v_mean,
-                                                int N, int n_chunks, int smooth, int64_t bh) {
+__device__ __forceinline__ void v_finalize_body(float* work, float* __restrict__ v_scale, float* __restrict__ v_mean,
+                                                int N, int n_chunks, int smooth, int64_t bh, int64_t BH) {
   // 1024 / D slices of the chunk range per channel, combined through LDS in a fixed order
   constexpr int SL = 1024 / D;
   __shared__ float red[3][SL][D];
   const int ch = threadIdx.x % D, sl = threadIdx.x / D;
-  const float* p = partial + bh * n_chunks * 3 * D;
+  const float* p = work + v_stats_offset(BH, N, D) + bh * n_chunks * 3 * D;
   float s = 0.f, mn = INFINITY, mx = -INFINITY;
   for (int c = sl; c < n_chunks; c += SL) {
     s += p[(c * 3 + 0) * D + ch];
@@ -119,10 +124,10 @@ __device__ __forceinline__ void v_finalize_body(float* partial, float* __restric
     const float amax = fmaxf(mx - mean, mean - mn);
     v_scale[bh * D + ch] = amax / 448.0f;
     if (v_mean) v_mean[bh * D + ch] = mean;
-    // every thread of this workgroup has read its partials before the barrier above: the head of the
-    // region is free to carry the reciprocal, and behind it the mean, to the pack kernel
-    partial[v_recp_offset(bh, n_chunks, D) + ch] = amax > 0.f ? 448.0f / amax : 0.f;
-    partial[v_recp_offset(bh, n_chunks, D) + D + ch] = mean;
+    // (long chunks: the partials of this (batch, head) are in the same place; every thread of the workgroup has read
+    // its own before the barrier above)
+    work[v_recp_offset(bh, N, D) + ch] = amax > 0.f ? 448.0f / amax : 0.f;
+    work[v_recp_offset(bh, N, D) + D + ch] = mean;
   }
 }
 
@@ -170,26 +175,28 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
     }
   };
   const int tok_first = chunk * K_CHUNK;
-  const bool full = tok_first + K_CHUNK <= N && bh0 + KM_GROUP <= BH &&
-                    (cos_t == nullptr || tok_first >= n_text);   // uniform: every row there, every row rotated alike
-  if (full) {
-    // batches of KB tokens per thread: their table pieces and K rows are all requested before the first is used
-    // (ordinary loads for K: it was just written by the projection and is read again by the preparation pass)
-    const bool rot = cos_t != nullptr;
-    const unsigned short* kp[KM_GROUP];
+  // batches of KB tokens per thread: their table pieces and K rows are all requested before the first is used
+  // (ordinary loads for K: it was just written by the projection and is read again by the preparation pass).
+  // `whole`: every row and head is there and every row rotated alike; otherwise rows and heads past the end re-read
+  // the last one, such rows are not added and such heads not stored, and a row says for itself whether it is rotated
+  const bool tables = cos_t != nullptr;
+  const unsigned short* kp[KM_GROUP];
 #pragma unroll
-    for (int g = 0; g < KM_GROUP; g++) {
-      const int bh = bh0 + g, b = bh / H, h = bh - b * H;
-      kp[g] = k + b * ks_b + h * ks_h + col;
-    }
+  for (int g = 0; g < KM_GROUP; g++) {
+    const int bh = min(bh0 + g, BH - 1), b = bh / H, h = bh - b * H;
+    kp[g] = k + b * ks_b + h * ks_h + col;
+  }
+  auto walk = [&](auto whole_c) {
+    constexpr bool whole = decltype(whole_c)::value;
     for (int r = t / LPR; r < K_CHUNK; r += ROWS * KB) {
+      if (!whole && tok_first + (r - t / LPR) >= N) break;
       v4f c0[KB], c1[KB], s0[KB], s1[KB];
       v4i raw[KB][KM_GROUP];
 #pragma unroll
       for (int u = 0; u < KB; u++) {
-        const int tok = tok_first + r + u * ROWS;
-        if (rot) {
-          const int64_t o = (int64_t)(tok - n_text) * D + col;
+        const int tok = whole ? tok_first + r + u * ROWS : min(tok_first + r + u * ROWS, N - 1);
+        if (tables) {
+          const int64_t o = (int64_t)(whole ? tok - n_text : max(tok - n_text, 0)) * D + col;
           c0[u] = *reinterpret_cast<const v4f*>(cos_t + o); c1[u] = *reinterpret_cast<const v4f*>(cos_t + o + 4);
           s0[u] = *reinterpret_cast<const v4f*>(sin_t + o); s1[u] = *reinterpret_cast<const v4f*>(sin_t + o + 4);
         }
@@ -197,29 +204,14 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
         for (int g = 0; g < KM_GROUP; g++) raw[u][g] = *reinterpret_cast<const v4i*>(kp[g] + (int64_t)tok * ks_n);
       }
 #pragma unroll
-      for (int u = 0; u < KB; u++) add_rows(raw[u], rot, c0[u], c1[u], s0[u], s1[u]);
-    }
-  } else {
-    for (int r = t / LPR; r < K_CHUNK; r += ROWS) {
-      const int tok = tok_first + r;
-      if (tok >= N) break;
-      const bool rot = cos_t != nullptr && tok >= n_text;
-      v4f c0 = {}, c1 = {}, s0 = {}, s1 = {};
-      if (rot) {
-        const int64_t o = (int64_t)(tok - n_text) * D + col;
-        c0 = *reinterpret_cast<const v4f*>(cos_t + o); c1 = *reinterpret_cast<const v4f*>(cos_t + o + 4);
-        s0 = *reinterpret_cast<const v4f*>(sin_t + o); s1 = *reinterpret_cast<const v4f*>(sin_t + o + 4);
+      for (int u = 0; u < KB; u++) {
+        const int tok = tok_first + r + u * ROWS;
+        if (whole || tok < N) add_rows(raw[u], tables && (whole || tok >= n_text), c0[u], c1[u], s0[u], s1[u]);
       }
-      v4i raw[KM_GROUP];
-#pragma unroll
-      for (int g = 0; g < KM_GROUP; g++) {
-        const int bh = min(bh0 + g, BH - 1);   // (a group past the last head re-reads it; its sums are not stored)
-        const int b = bh / H, h = bh - b * H;
-        raw[g] = *reinterpret_cast<const v4i*>(k + b * ks_b + h * ks_h + (int64_t)tok * ks_n + col);
-      }
-      add_rows(raw, rot, c0, c1, s0, s1);
     }
-  }
+  };
+  if (tok_first + K_CHUNK <= N && bh0 + KM_GROUP <= BH && (!tables || tok_first >= n_text)) walk(std::true_type{});
+  else walk(std::false_type{});
   __shared__ float red[4][KM_GROUP][D];
 #pragma unroll
   for (int g = 0; g < KM_GROUP; g++) {

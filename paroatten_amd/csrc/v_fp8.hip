@@ -3,7 +3,7 @@
 // tiles straight from HBM to LDS and reads each A operand as one contiguous 16-byte piece per lane.
 //
 // Three launches, all HBM-bound and deterministic (no float atomics):
-//   v_stats    : per V_CHUNK-token chunk, per channel: sum, min, max      (reads V once)
+//   v_stats    : per v_chunk(N)-token chunk, per channel: sum, min, max      (reads V once)
 //   v_finalize : per (b,h,channel): mean = sum/N, amax = max(max-mean, mean-min), scale = amax/448,
 //                recp = 448/amax
 //   v_pack     : per 64-token tile: (v-mean)*recp -> e4m3, fragment order  (reads V once more), and the
@@ -29,10 +29,10 @@ __global__ void __launch_bounds__(256) v_stats_kernel(const unsigned short* __re
 }
 
 template <int D>
-__global__ void __launch_bounds__(1024) v_finalize_kernel(float* partial, float* __restrict__ v_scale,
+__global__ void __launch_bounds__(1024) v_finalize_kernel(float* work, float* __restrict__ v_scale,
                                                           float* __restrict__ v_mean, int N, int n_chunks,
                                                           int smooth) {
-  v_finalize_body<D>(partial, v_scale, v_mean, N, n_chunks, smooth, blockIdx.x);
+  v_finalize_body<D>(work, v_scale, v_mean, N, n_chunks, smooth, blockIdx.x, gridDim.x);
 }
 
 template <int DT, int D>
@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __res
                                                      uint8_t* __restrict__ v8,
                                                      const float* __restrict__ v_recp,
                                                      const float* __restrict__ v_mean, float* __restrict__ resid,
-                                                     int N, int nb, int n_chunks,
+                                                     int N, int nb,
                                                      int64_t vs_b, int64_t vs_h, int64_t vs_n) {
   constexpr int LPR = D / 8;
   constexpr int ROWS = 256 / LPR;
@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __res
   }
   __syncthreads();
   float rs[D / 64];
-  pack_v_tile<DT, D, PITCH>(tile, v8 + (bh * nb + kb) * (int64_t)(64 * D), v_recp + v_recp_offset(bh, n_chunks, D),
+  pack_v_tile<DT, D, PITCH>(tile, v8 + (bh * nb + kb) * (int64_t)(64 * D), v_recp + v_recp_offset(bh, N, D),
                             v_mean ? v_mean + bh * D : nullptr, kb * 64, N, t, rs);
   if (resid != nullptr && (t & 63) < 32) {
     const int wave = t >> 6;
@@ -110,9 +110,9 @@ int v_fp8_add_residual(const float* resid, const float* v_scale, float* v_mean, 
 template <int DT, int D>
 static int run_v_stats(const void* v, float* v_scale, float* v_mean, float* partial, int B, int Hkv, int N,
                        int64_t vs_b, int64_t vs_h, int64_t vs_n, int smooth, hipStream_t st) {
-  const int n_chunks = ceil_div(N, V_CHUNK);
+  const int n_chunks = ceil_div(N, v_chunk(N));
   hipLaunchKernelGGL((v_stats_kernel<DT, D>), dim3(n_chunks, Hkv, B), dim3(256), 0, st, (const unsigned short*)v,
-                     partial, N, n_chunks, vs_b, vs_h, vs_n);
+                     partial + v_stats_offset((int64_t)B * Hkv, N, D), N, n_chunks, vs_b, vs_h, vs_n);
   PARO_HIP(hipGetLastError());
   hipLaunchKernelGGL((v_finalize_kernel<D>), dim3(B * Hkv), dim3(1024), 0, st, partial, v_scale, v_mean, N,
                      n_chunks, smooth);
@@ -133,11 +133,11 @@ int v_fp8_stats(const void* v, int dtype, float* v_scale, float* v_mean, float* 
 template <int DT, int D>
 static int run_v_pack(const void* v, uint8_t* v8, float* partial, float* v_scale, float* v_mean, int B, int Hkv,
                       int N, int64_t vs_b, int64_t vs_h, int64_t vs_n, hipStream_t st) {
-  const int nb = ceil_div(N, 64), n_chunks = ceil_div(N, V_CHUNK);
+  const int nb = ceil_div(N, 64);
   // without smoothing there is no mean to correct
-  float* resid = v_mean ? partial + v_resid_offset((int64_t)B * Hkv, n_chunks, D) : nullptr;
+  float* resid = v_mean ? partial + v_resid_offset((int64_t)B * Hkv, N, D) : nullptr;
   hipLaunchKernelGGL((v_pack_kernel<DT, D>), dim3(nb, Hkv, B), dim3(256), 0, st, (const unsigned short*)v, v8,
-                     partial, v_mean, resid, N, nb, n_chunks, vs_b, vs_h, vs_n);
+                     partial, v_mean, resid, N, nb, vs_b, vs_h, vs_n);
   PARO_HIP(hipGetLastError());
   if (resid) return v_fp8_add_residual(resid, v_scale, v_mean, B, Hkv, N, D, st);
   return PARO_OK;
@@ -181,7 +181,7 @@ extern "C" int64_t paro_v_fp8_bytes(int B, int Hkv, int N, int D) {
   return (int64_t)B * Hkv * paro::ceil_div(N, 64) * 64 * D;
 }
 extern "C" int64_t paro_v_fp8_partial_floats(int B, int Hkv, int N, int D) {
-  // statistics partials (sum, min, max per chunk and channel), then the residual sums per row tile
+  // see v_resid_offset: statistics (sum, min, max per chunk and channel), residual sums per row tile
   return (int64_t)B * Hkv * ((int64_t)paro::ceil_div(N, paro::V_CHUNK) * 3 + (int64_t)paro::ceil_div(N, 64) * 2) * D;
 }
 

@@ -127,3 +127,25 @@ def test_per_channel_fp8_reference_order(dev):
     assert int(diff.max()) <= 1 and float((diff != 0).float().mean()) <= 1e-3
     v8n, vsn, none = _q().per_channel_fp8(v.to(dev), smooth_v=False, tile_order=False, scale_max=224.0)
     assert none is None and torch.allclose(vsn.cpu(), v.float().abs().amax(dim=2) / 224.0, rtol=2e-6)
+
+
+@pytest.mark.parametrize("N", [1, 64, 255, 256, 257, 1025, 8191, 8192, 8193])
+def test_v_statistics_at_the_edges_of_the_chunks(dev, N):
+    """Scale and offset of the V codes over one chunk, ragged last chunks, and either side of the lengths where the
+    chunk changes (256 and 8192 tokens), D = 64 with three heads and D = 128 with one."""
+    from conftest import untile_v8, v8_offset_expected
+    Q = _q()
+    for B, H, D, dtype in ((2, 3, 64, torch.float16), (1, 1, 128, torch.bfloat16)):
+        g = torch.Generator().manual_seed(N + D)
+        v = (torch.randn(B, H, N, D, generator=g) + torch.randn(1, H, 1, D, generator=g)).to(dtype)
+        v8, scale, offset = Q.per_channel_fp8(v.to(dev))
+        mean = v.double().mean(dim=2, keepdim=True)
+        amax = (v.double() - mean).abs().amax(dim=2)
+        # fp32 sums of N values: at most N half-ulps of the largest partial sum, divided by N; then amax / 448 in fp32
+        err = v.double().abs().sum(dim=2) * 2.0 ** -24 + 1e-30
+        assert ((scale.cpu().double() * 448 - amax).abs() <= err + 2.0 ** -22 * amax).all()
+        tokens = untile_v8(v8, B, H, N, D)
+        want = v8_offset_expected(v, tokens, scale)
+        # the offset: the same mean, plus the residuals summed in fp32 (each below 16 codes times the scale)
+        assert ((offset.cpu().double() - want).abs() <= 2 * err + N * 16 * scale.cpu().double() * 2.0 ** -24 + 1e-6).all()
+        assert int(tokens[:, :, N:].max() if tokens.shape[2] > N else 0) == 0

@@ -229,6 +229,31 @@ int paro_qk_int8_sv_f16_attn(const int8_t* q8, const int8_t* k8, const void* v, 
                              float sm_scale, int smooth_v, int flags, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
+ * (2d) The operator above the extension in one call: INT8 quantisation of q and k (per-warp scales, groups of 32 and 64
+ * tokens, or per-thread ones), then (2c).  Stands in for paroattn_qk_int8_pv_fp16_cuda below its argument checks
+ * (paroattention/core.py:86-216).  q [B,H,Nq,D], k, v [B,Hkv,Nk,D], out [B,H,Nq,D], all in the 16-bit `dtype`, through
+ * element strides (either layout), last dim contiguous; q, k, v 16-byte aligned, strides multiples of 8.
+ * smooth_k: the token mean of K (rounded to the input dtype) is subtracted before quantisation.
+ * lse (may be NULL): fp32 [B,H,Nq], the NATURAL log-sum-exp of the scores of q and k as given: with smooth_k it includes
+ * sm_scale * q . mean, which the quantised scores lack.
+ * qk_quant_gran 2 or 3 as in (2c); flags as in (2b).
+ * workspace: paro_attn_operator_workspace_bytes() bytes of device memory (256-byte aligned); nothing of it has to be
+ * initialised, and nothing in it is of use after the call.
+ * ------------------------------------------------------------------------------------------- */
+int64_t paro_attn_operator_workspace_bytes(int B, int H, int Hkv, int Nq, int Nk, int D, int smooth_k, int with_lse,
+                                           int qk_quant_gran, int flags);
+int paro_attn_operator(const void* q, const void* k, const void* v, int dtype, void* out,
+                       const uint8_t* sparse, int64_t sparse_batch_stride, float* lse,
+                       void* workspace, int64_t workspace_bytes,
+                       int B, int H, int Hkv, int Nq, int Nk, int D,
+                       int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                       int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                       int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
+                       int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
+                       int is_causal, int qk_quant_gran, float sm_scale, int smooth_k, int smooth_v, int flags,
+                       void* stream);
+
+/* ---------------------------------------------------------------------------------------------
  * (3) Fused 3-D RoPE + per-head F/H/W token permutation, and the inverse permutation.
  * Stands in for the Python head loops permute_qk / permute_attn_out
  * (paroattention/cogvideox.py:22-62, 64-110; paroattention/wan.py:25-63, 65-111), the RoPE that

@@ -59,6 +59,9 @@ SIGNATURES = {
                                          _I, _I, _I, _I, _I, _I,
                                          _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L,
                                          _I, _I, _I, _F, _I, _I, _P]),
+    "paro_attn_operator_workspace_bytes": (c_int64, [_I, _I, _I, _I, _I, _I, _I, _I, _I, _I]),
+    "paro_attn_operator": (c_int, [_P, _P, _P, _I, _P, _P, _L, _P, _P, _L, _I, _I, _I, _I, _I, _I,
+                                   _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _I, _I, _F, _I, _I, _I, _P]),
     "paro_rope_permute_fwd": (c_int, [_P, _P, _P, _P, _P, _P, _I, _P, _P, _P,
                                       _I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _P]),
     "paro_permute_inv": (c_int, [_P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _P]),
@@ -105,6 +108,23 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_ops = None
+
+
+def ops():
+    """The `_ops` submodule of the compiled extension (csrc/torch_binding.cpp -> _ext.so): the package's own entry points
+    with their argument checks, allocations and launches in native code.  Raises ImportError if it is not built."""
+    global _ops
+    if _ops is None:
+        load()
+        try:
+            from . import _ext
+        except ImportError as e:
+            raise ImportError(f"paroatten_amd/_ext.so is not built: run `python paroatten_amd/build.py` ({e})") from e
+        _ops = _ext._ops
+    return _ops
 
 
 def check(rc: int):

@@ -11,9 +11,9 @@ from typing import Any, Optional
 
 import torch
 
+from . import _lib
 from . import _qattn_sm80 as qattn
-from .quant import per_thread_int8
-from .quant import per_warp_int8 as per_warp_int8_cuda
+from .quant import per_warp_int8 as per_warp_int8_cuda  # noqa: F401  (the reference's module-level name)
 
 
 def paroattn(q, k, v, tensor_layout: str = "HND", is_causal: bool = False, sm_scale: Optional[float] = None,
@@ -58,55 +58,30 @@ def paroattn_qk_int8_pv_fp16_cuda(q, k, v, sparse, tensor_layout: str = "HND", i
     if qk_quant_gran == "per_thread" and pv_f16:
         raise NotImplementedError("qk_quant_gran='per_thread' is not available with pv_f16")
 
-    # launch on the tensors' device, as the reference's set_device workaround does (core.py:168-174)
-    with torch.cuda.device(v.device):
-        layout_flag = 0 if tensor_layout == "NHD" else 1
-        head_dim_og = q.size(-1)
-        if head_dim_og < 64:
-            pad = 64 - head_dim_og
-        elif 64 < head_dim_og < 128:
-            pad = 128 - head_dim_og
-        elif head_dim_og > 128:
-            raise ValueError(f"Unsupported head_dim: {head_dim_og}")
-        else:
-            pad = 0
-        if pad:
-            q = torch.nn.functional.pad(q, (0, pad))
-            k = torch.nn.functional.pad(k, (0, pad))
-            v = torch.nn.functional.pad(v, (0, pad))
-        assert q.stride(-1) == 1 and k.stride(-1) == 1 and v.stride(-1) == 1, "Last dim of qkv must be contiguous."
-        if sm_scale is None:
-            sm_scale = head_dim_og ** -0.5
-        seq_dim = 1 if layout_flag == 0 else 2
-        km = k.mean(dim=seq_dim, keepdim=True) if smooth_k else None
-        if qk_quant_gran == "per_thread":
-            # (core.py:204-205 of the reference pairs per-block scales, softmax scale folded in, with the kernel's
-            # per-thread path, whose shape check rejects them; here the scales are made at that granularity)
-            q_int8, q_scale, k_int8, k_scale = per_thread_int8(q, k, km, tensor_layout=tensor_layout)
-        else:
-            q_int8, q_scale, k_int8, k_scale = per_warp_int8_cuda(q, k, km, BLKQ=64, WARPQ=32, BLKK=64,
-                                                                  tensor_layout=tensor_layout)
-        o = torch.empty(q.size(), dtype=dtype, device=q.device)
-        lse = qattn.qk_int8_sv_f16_accum_f16_attn(q_int8, k_int8, v, o, q_scale, k_scale, layout_flag,
-                                                  1 if is_causal else 0, 3 if qk_quant_gran == "per_thread" else 2,
-                                                  sm_scale, 1 if return_lse else 0,
-                                                  sparse, smooth_v=smooth_v, exact_exp=exact_exp,
-                                                  two_waves=two_waves, pv_f16=pv_f16)
-        o = o[..., :head_dim_og]
-        if return_lse:
-            lse = lse / 1.44269504
-            if km is not None:
-                # the kernel saw K - km: every score of row i is lower by sm_scale * q_i . km, which the softmax
-                # does not notice but the log-sum-exp does; put it back, so that lse is that of the scores of q
-                # and k as given (what a caller that merges partial results over key ranges needs)
-                groups = q.size(2 if layout_flag == 0 else 1) // km.size(2 if layout_flag == 0 else 1)
-                if layout_flag == 0:   # q [B,N,H,D], km [B,1,Hkv,D]
-                    kmh = km.float().repeat_interleave(groups, dim=2)
-                    corr = torch.stack([(q[b].float() * kmh[b]).sum(-1).transpose(0, 1) for b in range(q.size(0))])
-                else:                  # q [B,H,N,D], km [B,Hkv,1,D]
-                    kmh = km.float().repeat_interleave(groups, dim=1)
-                    corr = torch.stack([torch.bmm(q[b].float(), kmh[b].transpose(1, 2)).squeeze(-1)
-                                        for b in range(q.size(0))])
-                lse = lse + corr * sm_scale
-            return o, lse
-        return o
+    layout_flag = 0 if tensor_layout == "NHD" else 1
+    head_dim_og = q.size(-1)
+    if head_dim_og < 64:
+        pad = 64 - head_dim_og
+    elif 64 < head_dim_og < 128:
+        pad = 128 - head_dim_og
+    elif head_dim_og > 128:
+        raise ValueError(f"Unsupported head_dim: {head_dim_og}")
+    else:
+        pad = 0
+    if pad:
+        q = torch.nn.functional.pad(q, (0, pad))
+        k = torch.nn.functional.pad(k, (0, pad))
+        v = torch.nn.functional.pad(v, (0, pad))
+    assert q.stride(-1) == 1 and k.stride(-1) == 1 and v.stride(-1) == 1, "Last dim of qkv must be contiguous."
+    if tensor_layout not in ("HND", "NHD"):
+        raise ValueError(f"Unknown tensor layout: {tensor_layout}")
+    if sm_scale is None:
+        sm_scale = head_dim_og ** -0.5
+    # (core.py:204-205 of the reference pairs per-block scales, softmax scale folded in, with the kernel's per-thread path,
+    # whose shape check rejects them; here the scales are made at the granularity asked for)
+    result = _lib.ops().attn_operator(q, k, v, sparse, layout_flag, bool(is_causal), 3 if qk_quant_gran == "per_thread" else 2,
+                                      sm_scale, bool(return_lse), bool(smooth_k), bool(smooth_v),
+                                      qattn._flags(exact_exp, None, two_waves, pv_f16))
+    if pad:
+        return (result[0][..., :head_dim_og], result[1]) if return_lse else result[..., :head_dim_og]
+    return result

@@ -17,7 +17,9 @@ struct AttnParams {
   const float* v_mean;
   const uint8_t* sparse;
   void* out;
-  float* lse;
+  float* lse;            // what is stored: base-2 log-sum-exp * lse_scale (+ lse_add[row], if given)
+  float lse_scale;
+  const float* lse_add;
   int32_t* s_dump;
   int64_t sparse_bs;
   int64_t qs_b, qs_h, qs_n;
@@ -45,6 +47,10 @@ constexpr float FAST_EXP_SHIFT = -0.35f;  // centres the linear-mantissa error o
 // fast path: the real-valued byte b becomes the 16-bit field round((b + 0.5) * 256), whose HIGH byte is
 // round(b); the field is bounded by 0x7FFF, so the byte is bounded by 0x7F
 constexpr float FAST_FIELD_SCALE = 256.0f / 32767.0f;
+
+__device__ __forceinline__ void store_lse(const AttnParams& p, int64_t row, float lse2) {
+  p.lse[row] = p.lse_add != nullptr ? fmaf(lse2, p.lse_scale, p.lse_add[row]) : lse2 * p.lse_scale;
+}
 
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
@@ -103,5 +109,14 @@ int launch_attn_w64(const AttnParams& p, int out_dtype, bool causal, bool exact,
 // The kernel with a float16 P.V product (attn_sparse_pv16.hip): p.v8 points at paro_v_f16_pack's tiles, p.v_scale
 // and p.v_mean may be null.  Either head size, with or without lse, plain launch.
 int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hipStream_t st);
+
+// paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip) with the two values that go into a stored log-sum-exp.
+int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
+                     const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
+                     void* out, int out_dtype, float* lse, float lse_scale, const float* lse_add, int32_t* s_dump, int B,
+                     int H, int Hkv, int Nq, int Nk, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                     int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
+                     int64_t o_stride_n, float sm_scale, int is_causal, int flags, const int32_t* orders, int n_text, int F,
+                     int Hh, int W, void* stream);
 
 }  // namespace paro

@@ -190,7 +190,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
-      if (p.lse && lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = -INFINITY;
+      if (p.lse && lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, -INFINITY);
     }
     return;
   }
@@ -658,7 +658,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     // the log-sum-exp uses the exact fp32 row sum, not the sum of the FP8-rounded weights
     const float d_full = d_exact + __shfl_xor(d_exact, 32, 64);
     if (p.lse && qrow < p.Nq && lh == 0)
-      p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET;
+      store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET);
   }
 }
 
@@ -846,14 +846,13 @@ static int dispatch_attn(const AttnParams& p, int is_causal, bool dump, bool exa
 }  // namespace paro
 
 namespace paro {
-static int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale,
-                            const float* k_scale, const float* v_scale, const float* v_mean,
-                            const uint8_t* sparse, int64_t sparse_batch_stride, void* out, int out_dtype,
-                            float* lse, int32_t* s_dump, int B, int H, int Hkv, int Nq, int Nk, int D,
-                            int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_b,
-                            int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
-                            int64_t o_stride_n, float sm_scale, int is_causal, int flags, const int32_t* orders,
-                            int n_text, int F, int Hh, int W, void* stream) {
+int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
+                     const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
+                     void* out, int out_dtype, float* lse, float lse_scale, const float* lse_add, int32_t* s_dump, int B,
+                     int H, int Hkv, int Nq, int Nk, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                     int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
+                     int64_t o_stride_n, float sm_scale, int is_causal, int flags, const int32_t* orders, int n_text, int F,
+                     int Hh, int W, void* stream) {
   PARO_CHECK((flags & ~(PARO_ATTN_EXACT_EXP | PARO_ATTN_PACED | PARO_ATTN_UNPACED | PARO_ATTN_TWO_WAVES |
                         PARO_ATTN_PV_F16 | PARO_ATTN_QK_PER_THREAD)) == 0 &&
                  (flags & (PARO_ATTN_PACED | PARO_ATTN_UNPACED)) != (PARO_ATTN_PACED | PARO_ATTN_UNPACED),
@@ -898,7 +897,7 @@ static int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v
   }
   AttnParams p;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.v_mean = v_mean;
-  p.sparse = sparse; p.out = out; p.lse = lse; p.s_dump = s_dump; p.sparse_bs = sparse_batch_stride;
+  p.sparse = sparse; p.out = out; p.lse = lse; p.lse_scale = lse_scale; p.lse_add = lse_add; p.s_dump = s_dump; p.sparse_bs = sparse_batch_stride;
   p.qs_b = q_stride_b; p.qs_h = q_stride_h; p.qs_n = q_stride_n;
   p.ks_b = k_stride_b; p.ks_h = k_stride_h; p.ks_n = k_stride_n;
   p.os_b = o_stride_b; p.os_h = o_stride_h; p.os_n = o_stride_n;
@@ -940,7 +939,7 @@ extern "C" int paro_attn_sparse_fwd(const int8_t* q8, const int8_t* k8, const ui
                                     int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
                                     int64_t o_stride_n, float sm_scale, int is_causal, int flags, void* stream) {
   return paro::attn_sparse_impl(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out,
-                                out_dtype, lse, s_dump, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n,
+                                out_dtype, lse, 1.0f, nullptr, s_dump, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n,
                                 k_stride_b, k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale,
                                 is_causal, flags, nullptr, 0, 0, 0, 0, stream);
 }
@@ -961,7 +960,7 @@ extern "C" int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8
              "paro_attn_sparse_unpermute_fwd: n_text + F*H*W = %d + %d*%d*%d does not equal the token count %d",
              n_text, F, Hh, W, Nq);
   return attn_sparse_impl(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out, out_dtype,
-                          lse, nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
+                          lse, 1.0f, nullptr, nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
                           k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale, is_causal, flags,
                           orders, n_text, F, Hh, W, stream);
 }

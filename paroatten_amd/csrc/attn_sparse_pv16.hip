@@ -29,6 +29,7 @@
 // fragment imposes on the B operand (a lane's weights 8*(s%2) .. 8*(s%2)+7 of row tile s/2 are its B fragment of
 // step s), so that no data moves between lanes from one product to the next.  Tokens past the end are 0.
 #include "attn_common.hpp"
+#include "v_pack_device.hpp"
 
 namespace paro {
 
@@ -146,7 +147,7 @@ __global__ void __launch_bounds__(128, (D == 64 && !LSE ? 3 : 2)) attn_sparse_pv
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
-      if (LSE && lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = -INFINITY;
+      if (LSE && lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, -INFINITY);
     }
     return;
   }
@@ -397,7 +398,7 @@ __global__ void __launch_bounds__(128, (D == 64 && !LSE ? 3 : 2)) attn_sparse_pv
   if constexpr (LSE) {   // (the exact sum of the weights before their rounding)
     const float d_full = d_exact + __shfl_xor(d_exact, 32, 64);
     if (qrow < p.Nq && lh == 0)
-      p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET;
+      store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET);
   }
 }
 
@@ -426,41 +427,12 @@ int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hip
   return out_dtype == PARO_DTYPE_F16 ? dispatch_pv16<128, PARO_DTYPE_F16>(p, causal, st) : dispatch_pv16<128, PARO_DTYPE_BF16>(p, causal, st);
 }
 
-// ---- V -> float16 tiles in fragment order ---------------------------------------------------------------
-// One workgroup per (batch, kv-head, 64-token block): the block goes through LDS row by row (16-byte loads) and
-// leaves as D/32 x 4 pieces of 1 KB (16 bytes per lane).
+// ---- V -> float16 tiles in fragment order: one workgroup per (batch, kv-head, 64-token block) ----
 template <int DT, int D>
 __global__ void __launch_bounds__(256) v_f16_pack_kernel(const unsigned short* __restrict__ v, unsigned short* __restrict__ out,
                                                          int Hkv, int N, int nb, int64_t sb, int64_t sh, int64_t sn) {
-  __shared__ __attribute__((aligned(16))) unsigned short tile[64 * (D + 8)];   // rows padded by 16 bytes
   const int kb = blockIdx.x % nb, bh = blockIdx.x / nb;
-  const int b = bh / Hkv, hk = bh % Hkv;
-  const unsigned short* src = v + b * sb + hk * sh;
-  constexpr int CPR = D / 8;   // 16-byte chunks per row
-  for (int c = threadIdx.x; c < 64 * CPR; c += 256) {
-    const int row = c / CPR, ch = c % CPR;
-    const int tok = kb * 64 + row;
-    v4i x = {0, 0, 0, 0};
-    if (tok < N) x = *reinterpret_cast<const v4i*>(src + (int64_t)tok * sn + ch * 8);
-    *reinterpret_cast<v4i*>(tile + row * (D + 8) + ch * 8) = x;
-  }
-  __syncthreads();
-  unsigned short* dst = out + ((int64_t)bh * nb + kb) * (64 * D);
-  for (int pl = threadIdx.x; pl < (D / 32) * 4 * 64; pl += 256) {
-    const int lane = pl & 63, piece = pl >> 6;
-    const int dt = piece >> 2, s = piece & 3;
-    const int chn = 32 * dt + (lane & 31);
-    unsigned short r[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int row = 32 * (s >> 1) + 16 * (s & 1) + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      const unsigned short raw = tile[row * (D + 8) + chn];
-      r[e] = DT == PARO_DTYPE_F16 ? raw : F16x<PARO_DTYPE_F16>::from_f32(F16x<PARO_DTYPE_BF16>::to_f32(raw));
-    }
-    *reinterpret_cast<v4i*>(dst + (int64_t)pl * 8) =
-        v4i{(int)(r[0] | ((unsigned)r[1] << 16)), (int)(r[2] | ((unsigned)r[3] << 16)),
-            (int)(r[4] | ((unsigned)r[5] << 16)), (int)(r[6] | ((unsigned)r[7] << 16))};
-  }
+  v_f16_pack_body<DT, D>(v + bh / Hkv * sb + bh % Hkv * sh, out, N, nb, sn, kb, bh);
 }
 
 }  // namespace paro

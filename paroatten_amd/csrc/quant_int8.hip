@@ -1,11 +1,5 @@
-// Per-group symmetric INT8 quantisation of Q / K (HBM-bound).
-//
-// One 64-lane wave owns one group of G tokens x D channels: every lane holds G*D/64 values in
-// registers (16-byte loads, consecutive lanes on consecutive addresses), the group maximum is a
-// wave reduction, and the int8 result leaves as 8-byte stores.  Nothing goes through LDS.
-// Arithmetic follows QuantInt8Kernel of the reference (csrc/fused/fused.cu:64-198) in IEEE fp32:
-// this file is compiled without fast-math and with fp contraction off.
-#include "paro_device.hpp"
+// Per-group symmetric INT8 quantisation of Q / K (HBM-bound): the launches; the bodies are in quant_device.hpp.
+#include "quant_device.hpp"
 
 namespace paro {
 
@@ -15,152 +9,24 @@ __global__ void __launch_bounds__(256) quant_int8_kernel(
     int8_t* __restrict__ out, float* __restrict__ scale, int N, int n_groups,
     int64_t xs_b, int64_t xs_h, int64_t xs_n, int64_t ms_b, int64_t ms_h,
     int64_t os_b, int64_t os_h, int64_t os_n, int64_t ss_b, int64_t ss_h, float sm_scale) {
-  constexpr int LPR = D / 8;          // lanes per token row (16-byte chunks)
-  constexpr int CH = G * D / 512;     // 16-byte chunks per lane
-  constexpr int ROWS_PER_IT = 64 / LPR;
-  const int lane = threadIdx.x & 63;
   const int g = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (g >= n_groups) return;
   const int h = blockIdx.y, b = blockIdx.z;
-  const int col = (lane % LPR) * 8;
-  const int row0 = lane / LPR;
-
-  float mv[8];
-  if constexpr (MEAN) {
-    const v4i m = *reinterpret_cast<const v4i*>(mean + b * ms_b + h * ms_h + col);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      mv[2 * j] = F16x<DT>::to_f32((unsigned short)(m[j] & 0xffff));
-      mv[2 * j + 1] = F16x<DT>::to_f32((unsigned short)((unsigned)m[j] >> 16));
-    }
-  }
-
-  const unsigned short* xb = x + b * xs_b + h * xs_h + col;
-  v4i raw[CH];
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = g * G + i * ROWS_PER_IT + row0;
-    raw[i] = (tok < N) ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(xb + (int64_t)tok * xs_n))
-                       : v4i{0, 0, 0, 0};
-  }
-
-  // value of element (chunk i, slot j) after mean subtraction / scaling; recomputed in the
-  // second pass instead of being kept, so that only the packed input stays in registers
-  auto value = [&](int i, int j) -> float {
-    float f = elem16_to_f32<DT>(raw[i], j);
-    if constexpr (MEAN) f -= mv[j];
-    if constexpr (SMS) f *= sm_scale;
-    return f;
-  };
-
-  float amax = 0.0000001f;
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = g * G + i * ROWS_PER_IT + row0;
-    if (tok < N) {  // rows past the end read as zero, whatever the mean
-#pragma unroll
-      for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(value(i, j)));
-    }
-  }
-  amax = wave_max(amax);
-  if (lane == 0) scale[b * ss_b + h * ss_h + g] = amax / 127.0f;
-  const float inv = 127.0f / amax;
-
-  int8_t* ob = out + b * os_b + h * os_h + col;
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = g * G + i * ROWS_PER_IT + row0;
-    // |value * (127/amax)| <= 127 up to rounding: the reference's clamp to [-128,127] never acts
-    float y[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) y[j] = value(i, j) * inv;
-    if (tok < N)
-      __builtin_nontemporal_store(
-          v2i{(int)pack4_rint_i8(y[0], y[1], y[2], y[3]), (int)pack4_rint_i8(y[4], y[5], y[6], y[7])},
-          reinterpret_cast<v2i*>(ob + (int64_t)tok * os_n));
-  }
+  quant_group_body<DT, D, G, MEAN, SMS>(x + b * xs_b + h * xs_h, MEAN ? mean + b * ms_b + h * ms_h : nullptr,
+                                        out + b * os_b + h * os_h, scale + b * ss_b + h * ss_h, N, g, xs_n, os_n, sm_scale);
 }
 
-// The same arithmetic on the per-thread groups of qk_quant_gran 3: a wave owns 64 tokens and their 16 (Q: two
-// 32-token groups of 8) or 4 (K) scales.  Token row r of the 64 belongs to group
-//   Q: (r / 32) * 8 + r % 8        K: (r % 8) / 2
-// A lane's chunks sit in rows row0 + i * ROWS_PER_IT; every group maximum is a full wave reduction of the
-// lanes' contributions to that group (the kernel is bound by HBM, not by these).
 template <int DT, int D, bool KEY, bool MEAN>
 __global__ void __launch_bounds__(256) quant_int8_per_thread_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ mean, int8_t* __restrict__ out,
     float* __restrict__ scale, int N, int n_blocks, int64_t xs_b, int64_t xs_h, int64_t xs_n, int64_t ms_b,
     int64_t ms_h, int64_t os_b, int64_t os_h, int64_t os_n) {
-  constexpr int LPR = D / 8;
-  constexpr int CH = 64 * D / 512;
-  constexpr int ROWS_PER_IT = 64 / LPR;
-  constexpr int NG = KEY ? 4 : 16;
-  const int lane = threadIdx.x & 63;
   const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (w >= n_blocks) return;
   const int h = blockIdx.y, b = blockIdx.z, H = gridDim.y;
-  const int col = (lane % LPR) * 8;
-  const int row0 = lane / LPR;
-  auto group_of = [](int r) { return KEY ? (r % 8) / 2 : (r / 32) * 8 + r % 8; };
-
-  float mv[8];
-  if constexpr (MEAN) {
-    const v4i m = *reinterpret_cast<const v4i*>(mean + b * ms_b + h * ms_h + col);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      mv[2 * j] = F16x<DT>::to_f32((unsigned short)(m[j] & 0xffff));
-      mv[2 * j + 1] = F16x<DT>::to_f32((unsigned short)((unsigned)m[j] >> 16));
-    }
-  }
-  const unsigned short* xb = x + b * xs_b + h * xs_h + col;
-  v4i raw[CH];
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = w * 64 + i * ROWS_PER_IT + row0;
-    raw[i] = (tok < N) ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(xb + (int64_t)tok * xs_n))
-                       : v4i{0, 0, 0, 0};
-  }
-  auto value = [&](int i, int j) -> float {
-    float f = elem16_to_f32<DT>(raw[i], j);
-    if constexpr (MEAN) f -= mv[j];
-    return f;
-  };
-  // this lane's maximum per chunk, then per group over the wave
-  float cmax[CH];
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = w * 64 + i * ROWS_PER_IT + row0;
-    cmax[i] = 0.f;
-    if (tok < N) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) cmax[i] = fmaxf(cmax[i], fabsf(value(i, j)));
-    }
-  }
-  float inv[CH];
-#pragma unroll
-  for (int g = 0; g < NG; g++) {
-    float a = 0.0000001f;
-#pragma unroll
-    for (int i = 0; i < CH; i++)
-      if (group_of(i * ROWS_PER_IT + row0) == g) a = fmaxf(a, cmax[i]);
-    a = wave_max(a);
-    if (lane == 0) scale[((int64_t)b * H + h) * ((int64_t)n_blocks * NG) + (int64_t)w * NG + g] = a / 127.0f;
-#pragma unroll
-    for (int i = 0; i < CH; i++)
-      if (group_of(i * ROWS_PER_IT + row0) == g) inv[i] = 127.0f / a;
-  }
-  int8_t* ob = out + b * os_b + h * os_h + col;
-#pragma unroll
-  for (int i = 0; i < CH; i++) {
-    const int tok = w * 64 + i * ROWS_PER_IT + row0;
-    float y[8];
-#pragma unroll
-    for (int j = 0; j < 8; j++) y[j] = value(i, j) * inv[i];
-    if (tok < N)
-      __builtin_nontemporal_store(
-          v2i{(int)pack4_rint_i8(y[0], y[1], y[2], y[3]), (int)pack4_rint_i8(y[4], y[5], y[6], y[7])},
-          reinterpret_cast<v2i*>(ob + (int64_t)tok * os_n));
-  }
+  quant_per_thread_body<DT, D, KEY, MEAN>(x + b * xs_b + h * xs_h, MEAN ? mean + b * ms_b + h * ms_h : nullptr,
+                                          out + b * os_b + h * os_h,
+                                          scale + ((int64_t)b * H + h) * ((int64_t)n_blocks * (KEY ? 4 : 16)), N, w, xs_n, os_n);
 }
 
 template <int DT, int D, int G>

@@ -10,7 +10,8 @@ namespace paro {
 // Per-channel sum, minimum and maximum of one v_chunk(N)-token chunk of one (batch, head): 256 threads.  Rows are
 // requested in batches of eight, in the last chunk too (rows past the end re-read the last one and are not taken): a
 // row at a time, the 738 rows of the last of two chunks took 15.7 us at N = 1762, B = 2, H = 4, D = 64.
-template <int DT, int D>
+// SUM_ONLY: only the sums, [chunk][D] (the mean of an unrotated K).
+template <int DT, int D, bool SUM_ONLY = false>
 __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ v, float* __restrict__ partial, int N,
                                              int n_chunks, int64_t vs_b, int64_t vs_h, int64_t vs_n, int chunk, int h,
                                              int b, int H) {
@@ -31,8 +32,10 @@ __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ 
     for (int j = 0; j < 8; j++) {
       const float f = elem16_to_f32<DT>(raw, j);
       s[j] += f;
-      mn[j] = fminf(mn[j], f);
-      mx[j] = fmaxf(mx[j], f);
+      if constexpr (!SUM_ONLY) {
+        mn[j] = fminf(mn[j], f);
+        mx[j] = fmaxf(mx[j], f);
+      }
     }
   };
   const int len = v_chunk(N), first = chunk * len, tok0 = first + t / LPR;
@@ -46,8 +49,8 @@ __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ 
         // (non-temporal: measured 3-5 us faster per launch of the entry point and of the per-layer sequence
         // than ordinary loads, although the packing pass reads the same tensor right afterwards)
         const int tok = tok0 + r + u * ROWS;
-        raw[u] = __builtin_nontemporal_load(
-            reinterpret_cast<const v4i*>(vb + (int64_t)(decltype(whole)::value ? tok : min(tok, N - 1)) * vs_n));
+        const v4i* src = reinterpret_cast<const v4i*>(vb + (int64_t)(decltype(whole)::value ? tok : min(tok, N - 1)) * vs_n);
+        raw[u] = SUM_ONLY ? *src : __builtin_nontemporal_load(src);
       }
 #pragma unroll
       for (int u = 0; u < VS_BATCH; u++)
@@ -62,30 +65,43 @@ __device__ __forceinline__ void v_stats_body(const unsigned short* __restrict__ 
     float a, b;
     if constexpr (LPR == 8) {
       s[j] += row_dpp<0x128>(s[j]);
-      mn[j] = fminf(mn[j], row_dpp<0x128>(mn[j]));
-      mx[j] = fmaxf(mx[j], row_dpp<0x128>(mx[j]));
+      if constexpr (!SUM_ONLY) {
+        mn[j] = fminf(mn[j], row_dpp<0x128>(mn[j]));
+        mx[j] = fmaxf(mx[j], row_dpp<0x128>(mx[j]));
+      }
     }
     with_lane_xor16(s[j], a, b);  s[j] = a + b;
+    if constexpr (SUM_ONLY) {
+      with_lane_xor32(s[j], a, b);  s[j] = a + b;
+      continue;
+    }
     with_lane_xor16(mn[j], a, b); mn[j] = fminf(a, b);
     with_lane_xor16(mx[j], a, b); mx[j] = fmaxf(a, b);
     with_lane_xor32(s[j], a, b);  s[j] = a + b;
     with_lane_xor32(mn[j], a, b); mn[j] = fminf(a, b);
     with_lane_xor32(mx[j], a, b); mx[j] = fmaxf(a, b);
   }
-  __shared__ float red[4][3][D];
+  __shared__ float red[4][SUM_ONLY ? 1 : 3][D];
   if (lane < LPR) {
 #pragma unroll
     for (int j = 0; j < 8; j++) {
       red[wave][0][col + j] = s[j];
-      red[wave][1][col + j] = mn[j];
-      red[wave][2][col + j] = mx[j];
+      if constexpr (!SUM_ONLY) {
+        red[wave][1][col + j] = mn[j];
+        red[wave][2][col + j] = mx[j];
+      }
     }
   }
   __syncthreads();
   if (t < D) {
     const float ss = (red[0][0][t] + red[1][0][t]) + (red[2][0][t] + red[3][0][t]);
-    const float mm = fminf(fminf(red[0][1][t], red[1][1][t]), fminf(red[2][1][t], red[3][1][t]));
-    const float xx = fmaxf(fmaxf(red[0][2][t], red[1][2][t]), fmaxf(red[2][2][t], red[3][2][t]));
+    if constexpr (SUM_ONLY) {
+      partial[((int64_t)(b * H + h) * n_chunks + chunk) * D + t] = ss;
+      return;
+    }
+    constexpr int MN = SUM_ONLY ? 0 : 1, MX = SUM_ONLY ? 0 : 2;
+    const float mm = fminf(fminf(red[0][MN][t], red[1][MN][t]), fminf(red[2][MN][t], red[3][MN][t]));
+    const float xx = fmaxf(fmaxf(red[0][MX][t], red[1][MX][t]), fmaxf(red[2][MX][t], red[3][MX][t]));
     float* p = partial + (((int64_t)(b * H + h) * n_chunks + chunk) * 3) * D;
     p[t] = ss;
     p[D + t] = mm;

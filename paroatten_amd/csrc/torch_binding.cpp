@@ -6,6 +6,9 @@
 //   _qattn_sm80  csrc/qattn/pybind_sm80.cpp:21-27, csrc/qattn/attn_cuda_sm80.h:19-69
 //   _fused       csrc/fused/pybind.cpp:21-33,      csrc/fused/fused.h:19-76
 //   _rope        csrc/rope/pybind.cpp:5-8,         csrc/rope/rope.h:6
+// and a fourth, _ops, which the package's own Python layer calls: whole operators with their argument checks,
+// allocations and launches (a call of a few hundred tokens is bound by this host work: 85 us a call at 416 tokens from
+// Python over eight launches).
 // Checks fail as the reference's do: TORCH_CHECK -> RuntimeError with the texts of csrc/utils.cuh:20-38,
 // std::invalid_argument -> ValueError for unsupported layouts, head dims and flags
 // (csrc/dispatch_utils.h:23-112).  Unlike the reference's launches (legacy default stream, no device
@@ -315,6 +318,55 @@ std::vector<torch::Tensor> rope_permutation(torch::Tensor Q, torch::Tensor K, to
   return {QO, KO};
 }
 
+// ---- _ops ---------------------------------------------------------------------------------------------
+// the block mask: bool or byte [B,H,nbq,nbk], or [H,nbq,nbk] shared by the batch; returns its batch stride
+int64_t check_mask(const torch::Tensor& sparse, int64_t B, int64_t H, int64_t nbq, int64_t nbk) {
+  on_gpu(sparse, "sparse");
+  TORCH_CHECK(sparse.scalar_type() == at::kBool || sparse.scalar_type() == at::kByte,
+              "Tensor sparse must have dtype (torch::kBool)");
+  contiguous(sparse, "sparse");
+  if (sparse.dim() == 4) {
+    TORCH_CHECK(sparse.sizes() == at::IntArrayRef({B, H, nbq, nbk}), "Tensor sparse must have shape (batch_size, num_qo_heads, ",
+                nbq, ", ", nbk, "), got ", sparse.sizes());
+    return sparse.stride(0);
+  }
+  TORCH_CHECK(sparse.dim() == 3 && sparse.sizes() == at::IntArrayRef({H, nbq, nbk}),
+              "Tensor sparse must have shape ([batch_size,] num_qo_heads, ", nbq, ", ", nbk, "), got ", sparse.sizes());
+  return 0;
+}
+
+// core.paroattn_qk_int8_pv_fp16_cuda behind its assertions: q, k, v of one 16-bit dtype on one GPU, head size 64 or 128.
+// Returns the output, or (output, log-sum-exp).
+py::object attn_operator(torch::Tensor q, torch::Tensor k, torch::Tensor v, torch::Tensor sparse, int tensor_layout,
+                         bool is_causal, int qk_quant_gran, double sm_scale, bool return_lse, bool smooth_k, bool smooth_v,
+                         int flags) {
+  dims(q, "query", 4); dims(k, "key", 4); dims(v, "value", 4);
+  const int sn = tensor_layout == 0 ? 1 : 2, sh = tensor_layout == 0 ? 2 : 1;
+  const int64_t B = q.size(0), D = q.size(3), H = q.size(sh), Hkv = k.size(sh), Nq = q.size(sn), Nk = k.size(sn);
+  if (D != 64 && D != 128) throw std::invalid_argument("Unsupported head dim: " + std::to_string(D));
+  TORCH_CHECK(k.size(0) == B && k.size(3) == D, "Tensor key must have the batch size and head dim of query");
+  TORCH_CHECK(v.sizes() == k.sizes(), "Tensor value must have the shape of key");
+  if (Hkv == 0 || H % Hkv != 0)
+    throw std::invalid_argument("num_qo_heads (" + std::to_string(H) + ") must be divisible by num_kv_heads (" +
+                                std::to_string(Hkv) + ")");
+  const int64_t sparse_bs = check_mask(sparse, B, H, (Nq + 63) / 64, (Nk + 63) / 64);
+  const c10::DeviceGuard guard(q.device());
+  torch::Tensor out = torch::empty(q.sizes(), q.options()), lse;
+  if (return_lse) lse = torch::empty({B, H, Nq}, q.options().dtype(at::kFloat));
+  const int64_t ws_bytes = paro_attn_operator_workspace_bytes((int)B, (int)H, (int)Hkv, (int)Nq, (int)Nk, (int)D, smooth_k,
+                                                              return_lse, qk_quant_gran, flags);
+  torch::Tensor ws = torch::empty({ws_bytes}, q.options().dtype(at::kByte));
+  check_rc(paro_attn_operator(q.data_ptr(), k.data_ptr(), v.data_ptr(), half_code(q, "paroattn"), out.data_ptr(),
+                              static_cast<const uint8_t*>(sparse.data_ptr()), sparse_bs,
+                              return_lse ? lse.data_ptr<float>() : nullptr, ws.data_ptr(), ws_bytes, (int)B, (int)H, (int)Hkv,
+                              (int)Nq, (int)Nk, (int)D, q.stride(0), q.stride(sh), q.stride(sn), k.stride(0), k.stride(sh),
+                              k.stride(sn), v.stride(0), v.stride(sh), v.stride(sn), out.stride(0), out.stride(sh),
+                              out.stride(sn), is_causal, qk_quant_gran, (float)sm_scale, smooth_k, smooth_v, flags,
+                              stream_of(q)));
+  if (return_lse) return py::make_tuple(out, lse);
+  return py::cast(out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -338,5 +390,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   fused.def("scale_fuse_quant_cuda", &scale_fuse_quant_cuda);
   fused.def("mean_scale_fuse_quant_cuda", &mean_scale_fuse_quant_cuda);
   auto rope = m.def_submodule("_rope");
+  auto ops = m.def_submodule("_ops");
+  ops.def("attn_operator", &attn_operator);
   rope.def("rope_permutation", &rope_permutation, "RoPE op with permutation.");
 }

@@ -18,6 +18,7 @@
 // Arithmetic follows MeanScaleKernel of the reference (csrc/fused/fused.cu:316-427) except that the
 // mean divides by the true token count.
 #include "stats_device.hpp"
+#include "v_pack_device.hpp"
 
 namespace paro {
 
@@ -36,38 +37,12 @@ __global__ void __launch_bounds__(1024) v_finalize_kernel(float* work, float* __
 }
 
 template <int DT, int D>
-__global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __restrict__ v,
-                                                     uint8_t* __restrict__ v8,
-                                                     const float* __restrict__ v_recp,
-                                                     const float* __restrict__ v_mean, float* __restrict__ resid,
-                                                     int N, int nb,
-                                                     int64_t vs_b, int64_t vs_h, int64_t vs_n) {
-  constexpr int LPR = D / 8;
-  constexpr int ROWS = 256 / LPR;
-  constexpr int PITCH = D + 8;  // 16-bit elements; +16 bytes keeps rows on different banks
-  __shared__ unsigned short tile[64 * PITCH];
-  const int t = threadIdx.x;
-  const int kb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int64_t bh = (int64_t)b * gridDim.y + h;
-  const int col = (t % LPR) * 8;
-  const unsigned short* vb = v + b * vs_b + h * vs_h + col;
-#pragma unroll
-  for (int r = t / LPR; r < 64; r += ROWS) {
-    const int tok = kb * 64 + r;
-    const v4i raw = (tok < N) ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(vb + (int64_t)tok * vs_n))
-                              : v4i{0, 0, 0, 0};
-    *reinterpret_cast<v4i*>(&tile[r * PITCH + col]) = raw;
-  }
-  __syncthreads();
-  float rs[D / 64];
-  pack_v_tile<DT, D, PITCH>(tile, v8 + (bh * nb + kb) * (int64_t)(64 * D), v_recp + v_recp_offset(bh, N, D),
-                            v_mean ? v_mean + bh * D : nullptr, kb * 64, N, t, rs);
-  if (resid != nullptr && (t & 63) < 32) {
-    const int wave = t >> 6;
-#pragma unroll
-    for (int n = 0; n < D / 64; n++)
-      resid[((bh * nb + kb) * 2 + (wave & 1)) * D + 32 * ((wave >> 1) + 2 * n) + (t & 31)] = rs[n];
-  }
+__global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __restrict__ v, uint8_t* __restrict__ v8,
+                                                     const float* __restrict__ work, const float* __restrict__ v_mean,
+                                                     float* __restrict__ resid, int N, int nb, int64_t vs_b,
+                                                     int64_t vs_h, int64_t vs_n) {
+  const int h = blockIdx.y, b = blockIdx.z;
+  v_pack_body<DT, D>(v + b * vs_b + h * vs_h, v8, work, v_mean, resid, N, nb, vs_n, blockIdx.x, (int64_t)b * gridDim.y + h);
 }
 
 // v_mean += v_scale * (sum over tiles and row tiles of the residual sums) / N.  A thread takes four

@@ -1,0 +1,55 @@
+"""GPU test of the operator in one native call (paro_attn_operator) against the chain of its parts: the quantisers and the
+extension entry point, each of which has its own parity tests against the oracle."""
+import pytest
+import torch
+
+from paroatten_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,D,layout,groups,mode", [
+    (1, 64, "HND", 1, "fp8"), (63, 64, "NHD", 2, "fp8"), (64, 128, "HND", 1, "fp8"), (65, 64, "HND", 1, "f16"),
+    (129, 128, "NHD", 1, "f16"), (257, 64, "HND", 2, "thread"), (300, 128, "NHD", 1, "thread"), (1000, 64, "HND", 1, "fp8"),
+])
+@pytest.mark.parametrize("smooth_k", [False, True])
+def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode, smooth_k):
+    """Edges of the groups of 32 and 64 tokens, of four groups per workgroup and of the statistics chunks; both layouts,
+    grouped heads, every product and granularity, with and without the mean and the log-sum-exp."""
+    import paroatten_amd as P
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    B, Hkv, dtype = 2, 2, torch.float16 if D == 64 else torch.bfloat16
+    H, nb, sd = Hkv * groups, (N + 63) // 64, 2 if layout == "HND" else 1
+    g = torch.Generator().manual_seed(N + D)
+
+    def make(h):   # multiples of 1/8 below 8: sums of up to 1000 of them are exact in fp32, whatever their order
+        shape = (B, h, N, D) if layout == "HND" else (B, N, h, D)
+        return (torch.randint(-63, 64, shape, generator=g) / 8).to(dtype).to(dev)
+    q, k, v = make(H), make(Hkv), make(Hkv)
+    mask = synth.make_block_mask(H, nb, 0.6, seed=N, device=dev)
+    km = k.double().mean(dim=sd, keepdim=True).float().to(dtype) if smooth_k else None
+    if mode == "thread":
+        q8, qs, k8, ks = Q.per_thread_int8(q, k, km, tensor_layout=layout)
+    else:
+        q8, qs, k8, ks = Q.per_warp_int8(q, k, km, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout=layout)
+    kw = dict(pv_f16=mode == "f16")
+    args = (0 if layout == "NHD" else 1, 0, 3 if mode == "thread" else 2, D ** -0.5)
+    o_ref = torch.empty_like(q)
+    qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, *args, 0, mask, **kw)
+    o_lse_ref = torch.empty_like(q)
+    lse2 = qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_lse_ref, qs, ks, *args, 1, mask, **kw)
+    call = dict(tensor_layout=layout, smooth_k=smooth_k, qk_quant_gran="per_thread" if mode == "thread" else "per_warp", **kw)
+    assert torch.equal(P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, **call), o_ref)
+    o, lse = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, return_lse=True, **call)
+    assert torch.equal(o, o_lse_ref)
+    want = lse2.double() * 0.6931471805599453
+    scale = want.abs()
+    if smooth_k:
+        qh = q if layout == "HND" else q.transpose(1, 2)
+        kh = (km if layout == "HND" else km.transpose(1, 2)).repeat_interleave(groups, dim=1).double()
+        corr = (qh.double() * kh).sum(-1) * D ** -0.5
+        want = want + corr
+        scale = scale + (qh.double() * kh).abs().sum(-1) * D ** -0.5
+    # one product and one sum in fp32, and an fp32 dot product of D terms
+    assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()

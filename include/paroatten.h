@@ -39,7 +39,7 @@ extern "C" {
 /* flags of the attention entry points */
 #define PARO_ATTN_EXACT_EXP 1 /* P = e4m3(2^x) by hardware exponential + FP8 conversion instead of the fast
                                  direct construction of the e4m3 byte (see paro_attn_sparse_fwd) */
-#define PARO_ATTN_PACED 2     /* launch form, results are bit-identical either way: a resident set of workgroups per
+#define PARO_ATTN_PACED 2     /* launch form, results are bit-identical to the plain one: a resident set of workgroups per
                                  XCD takes the q-blocks generation by generation, so that workgroups running
                                  together walk the key sequence together and share K8 / V8 tiles in the XCD's L2 */
 #define PARO_ATTN_UNPACED 4   /* one workgroup per q-block, started as the hardware pleases.  With neither flag the
@@ -49,9 +49,11 @@ extern "C" {
                                  masks made of one contiguous run per row lose a few per cent.  A generation waits for
                                  all but a share of its workgroups (PARO_ATTN_PACE_SLACK; default half the L2's share
                                  of a head, at most a quarter of them) and at most PARO_ATTN_PACE_SPINS rounds. */
-#define PARO_ATTN_TWO_WAVES 8 /* kernel form, results are bit-identical either way: two waves per 64-row q-block
-                                 (32 q-rows each) also where the library would pick the one-wave-per-q-block
-                                 kernel (head size 64, no lse, plain launch), which is the faster of the two there */
+#define PARO_ATTN_TWO_WAVES 8 /* kernel form: two waves per 64-row q-block (32 q-rows each) also where the
+                                 library would pick one wave per q-block (head size 64, no lse, plain launch, more
+                                 than 1024 q-blocks; bit-identical results) or several key blocks of a q-block at a
+                                 time (without any of the form flags, up to 256 q-blocks and at least 20 key blocks;
+                                 the same weights, summed in another order) */
 #define PARO_ATTN_PV_F16 16   /* accuracy mode: the P.V product in float16 with fp32 accumulation, as the reference's
                                  qk_int8_sv_f16_accum_f16_attn computes it (csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:263-391),
                                  instead of FP8 e4m3 P and V.  True exponentials; V as given (no per-channel scale, no

@@ -18,7 +18,8 @@ Differences, all relaxations or added checks:
     csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:112-116, 129-133) runs the two-wave kernel;
     quant.per_thread_int8 makes such scales (the reference has no quantiser for them);
   * keyword `pacing=True/False` picks the launch form of the attention kernel (see PARO_ATTN_PACED in
-    include/paroatten.h; bit-identical results), None leaves it to the library;
+    include/paroatten.h; bit-identical results), None leaves it to the library (which takes several key blocks of a
+    q-block at a time where there are few q-blocks: the same weights, summed in another order);
   * `sparse` IS validated (the reference reads it through a raw pointer unchecked): bool or uint8,
     on the GPU, contiguous, shape [B,H,nbq,nbk] or [H,nbq,nbk] (shared by the batch);
   * the INT4 and INT8-P.V variants registered by the reference are experimental prototypes with
@@ -39,7 +40,7 @@ def _chk(cond, msg):
 
 def _flags(exact_exp, pacing, two_waves=False, pv_f16=False):
     """pacing: None (the library chooses), True (PARO_ATTN_PACED) or False (PARO_ATTN_UNPACED); two_waves:
-    PARO_ATTN_TWO_WAVES.  Launch and kernel form only: results are bit-identical.  pv_f16: PARO_ATTN_PV_F16, the
+    PARO_ATTN_TWO_WAVES.  Launch and kernel form only.  pv_f16: PARO_ATTN_PV_F16, the
     float16 P.V product."""
     f = _lib.PARO_ATTN_EXACT_EXP if exact_exp else 0
     if pv_f16:

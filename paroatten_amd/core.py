@@ -44,7 +44,7 @@ def paroattn_qk_int8_pv_fp16_cuda(q, k, v, sparse, tensor_layout: str = "HND", i
     smooth_k subtracts the per-(batch,head) token mean of K before quantisation (softmax is
     invariant to it; the returned lse is corrected by sm_scale * q . mean, so it is that of the given q and k); smooth_v does the same for V inside the FP8 conversion and adds the mean back;
     exact_exp trades speed for fp32-evaluated softmax exponentials (see _qattn_sm80); two_waves picks the
-    two-waves-per-q-block kernel where the library would take the one-wave one (bit-identical results);
+    two-waves-per-q-block kernel also where the library would take another form (PARO_ATTN_TWO_WAVES);
     pv_f16 is the accuracy mode: the P.V product in float16 with fp32 accumulation, as the reference computes
     it (qk_int8_sv_f16_accum_f16_attn), instead of FP8 e4m3: about half the speed, float16 instead of e4m3 error
     on rows that a few keys dominate.

@@ -110,6 +110,11 @@ int launch_attn_w64(const AttnParams& p, int out_dtype, bool causal, bool exact,
 // and p.v_mean may be null.  Either head size, with or without lse, plain launch.
 int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hipStream_t st);
 
+// The kernel that takes several kept blocks of a q-block at a time (attn_sparse_split.hip): either head size, with or
+// without lse, plain launch.  split_width: how many, or 0 where another kernel is the faster one.
+int split_width(const AttnParams& p, int D);
+int launch_attn_split(const AttnParams& p, int D, int out_dtype, bool causal, bool exact, hipStream_t st);
+
 // paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip) with the two values that go into a stored log-sum-exp.
 int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
                      const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,

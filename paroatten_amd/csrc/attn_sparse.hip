@@ -918,9 +918,14 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
     return out_dtype == PARO_DTYPE_F16 ? dispatch_attn_per_thread<128, PARO_DTYPE_F16>(p, is_causal, exact, st)
                                        : dispatch_attn_per_thread<128, PARO_DTYPE_BF16>(p, is_causal, exact, st);
   }
+  // too few q-blocks to fill the card: several kept blocks of each at a time (attn_sparse_split.hip)
+  if (!dump && p.pacing == 0 && (flags & PARO_ATTN_TWO_WAVES) == 0 && split_width(p, D) != 0)
+    return launch_attn_split(p, D, out_dtype, is_causal != 0, exact, st);
   // D = 64 without lse or score dump: one wave per q-block (attn_sparse_w64.hip), unless the caller asks for the
-  // two-wave kernel or the launch is to be paced (only the two-wave kernel has the paced form)
-  if (D == 64 && lse == nullptr && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && !want_pacing(p, D))
+  // two-wave kernel, the launch is to be paced (only the two-wave kernel has the paced form), or there is no more than one
+  // q-block per SIMD: the latency of a q-block's walk is what counts then, and two waves halve the work of each (N = 4096:
+  // 22.3 instead of 28.1 us with 512 q-blocks, 28.3 instead of 29.5 us with 1024; 51.7 instead of 47.0 us with 2048)
+  if (D == 64 && lse == nullptr && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && p.total > 1024 && !want_pacing(p, D))
     return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
   if (D == 64) {
     if (out_dtype == PARO_DTYPE_F16) return dispatch_attn<64, PARO_DTYPE_F16>(p, is_causal, dump, exact, st);

@@ -1,0 +1,84 @@
+"""The attention kernel for few q-blocks (several kept key blocks of a q-block at a time) against the two-wave kernel, which
+is held to the oracle elsewhere: the same weights, code for code, so that outputs differ by the order of fp32 sums and the
+rounding to 16 bits only."""
+import pytest
+import torch
+
+from paroatten_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(a, b, v):
+    """One unit in the last place of the 16-bit output, and 2^-18 of max|v| for the fp32 sums (a few dozen partial sums,
+    each off by 2^-24 of sums of |p v| <= max|v|)."""
+    ulp = 2.0 ** -10 if a.dtype == torch.float16 else 2.0 ** -7
+    a, b = a.double(), b.double()
+    assert torch.isfinite(a).all()
+    assert ((a - b).abs() <= ulp * b.abs() + 2.0 ** -18 * float(v.abs().max())).all()
+
+
+# (B, H, blocks of 64 tokens): four blocks at a time up to 128 q-blocks, two up to 256; 20 blocks is the shortest list
+@pytest.mark.parametrize("B,H,nb", [(1, 1, 20), (1, 6, 21), (2, 4, 32), (1, 1, 129), (1, 4, 64)])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("causal,mode", [(False, "fast"), (True, "fast"), (False, "exact"), (True, "lse")])
+def test_same_result_as_two_waves(dev, B, H, nb, D, dtype, causal, mode):
+    """Rows of 0, 1, 2 ... kept blocks (so that a round is full, ragged or empty), a last block of 45 tokens."""
+    import paroatten_amd as P
+    N = nb * 64 - 19
+    q, k, v = (t.to(dev) for t in synth.make_qkv(B, H, N, D, dtype, seed=nb))
+    mask = synth.make_block_mask(H, nb, 0.4, seed=nb, device=dev)
+    for i in range(min(nb, 12)):   # the first rows of head 0 keep i blocks from the diagonal down
+        mask[0, i] = False
+        for j in range(i):
+            mask[0, i, (i - j) % nb] = True
+    kw = dict(is_causal=causal, smooth_k=True, exact_exp=mode == "exact", return_lse=mode == "lse")
+    a = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, **kw)
+    b = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, two_waves=True, **kw)
+    if mode == "lse":
+        finite = torch.isfinite(b[1])
+        assert torch.equal(torch.isfinite(a[1]), finite)
+        assert ((a[1] - b[1])[finite].abs() <= 1e-5).all()   # log of a sum whose terms are added in another order
+        a, b = a[0], b[0]
+    _close(a, b, v)
+    assert torch.count_nonzero(a[:, 0, :64]) == 0   # the q-block without a kept block
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H", [4, 8])
+@pytest.mark.parametrize("pattern,causal,density", [("ramp", False, 1.0), ("ramp", True, 1.0), ("ramp", False, 0.5), ("spike", False, 0.5)])
+def test_maximum_settled_in_list_order(dev, D, H, pattern, causal, density):
+    """Scores that climb by 4.3 octaves a block move the maximum in every block of a round (each wave in turn, the later
+    ones after computing their weights again), spikes in single ones; four and two blocks a round."""
+    import paroatten_amd as P
+    from test_gpu_attention import _ramp_case
+    B, nb = 1, 24
+    q, k, v = (t.to(dev) for t in _ramp_case(B, H, 64 * nb - 19, D, torch.float16, 7 + D, pattern))
+    mask = synth.make_block_mask(H, nb, density, seed=5, device=dev)
+    if density == 1.0:
+        mask[:] = True
+    for exact in (False, True):
+        a = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, is_causal=causal, exact_exp=exact)
+        b = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, is_causal=causal, exact_exp=exact, two_waves=True)
+        _close(a, b, v)
+
+
+def test_grouped_heads_and_unpermuting_store(dev):
+    """Grouped heads, keys of another length than the queries, token-major output through the inverse permutation."""
+    from paroatten_amd import _qattn_sm80 as qattn, quant as Q
+    H, Hkv, D, grid, n_text = 4, 2, 64, (4, 12, 27), 32
+    N, Nk = n_text + grid[0] * grid[1] * grid[2], 1500
+    q, _, _ = (t.to(dev) for t in synth.make_qkv(1, H, N, D, torch.float16, seed=1))
+    _, k, v = (t.to(dev) for t in synth.make_qkv(1, Hkv, Nk, D, torch.float16, seed=2))
+    mask = torch.rand(H, (N + 63) // 64, (Nk + 63) // 64, device=dev) < 0.4
+    q8, qs, _, _ = Q.per_warp_int8(q, q, None, BLKQ=64, WARPQ=32, BLKK=64)
+    _, _, k8, ks = Q.per_warp_int8(k, k, None, BLKQ=64, WARPQ=32, BLKK=64)
+    v8, vsc, vm = Q.per_channel_fp8(v)
+    orders = torch.tensor([0, 2, 3, 5], dtype=torch.int32, device=dev)
+    outs = []
+    for two in (False, True):
+        o = torch.zeros(1, N, H, D, dtype=torch.float16, device=dev).transpose(1, 2)
+        qattn.attn_sparse_prepacked(q8, k8, v8, vsc, vm, o, qs, ks, D ** -0.5, mask, unpermute=(orders, grid, n_text),
+                                    two_waves=two)
+        outs.append(o)
+    _close(outs[0], outs[1], v)

@@ -36,10 +36,9 @@ struct AttnParams {
 };
 
 // P~ = 2^(S*c - m + P_EXP_OFFSET).  m is the running row maximum, refreshed lazily: only when a
-// block's maximum exceeds it by more than P_HEADROOM are m, O and the row sums rescaled, so that
-// P~ <= 2^(P_EXP_OFFSET + P_HEADROOM) = 2^8.75 < 448, the largest e4m3 value.
+// weight would round to more than 448, the largest e4m3 value (a score about 3.8 octaves above m), are m, O and the
+// row sums rescaled.
 constexpr float P_EXP_OFFSET = 5.0f;
-constexpr float P_HEADROOM = 3.75f;
 constexpr int S_MAGIC_BITS = 0x4B400000;  // float 1.5 * 2^23
 constexpr float S_MAGIC_F = 12582912.0f;
 constexpr int FP8_ONES = 0x38383838;  // four e4m3 1.0

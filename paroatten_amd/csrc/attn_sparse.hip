@@ -56,8 +56,9 @@ template <int D> struct AttnLds {
   }
 };
 
-// Waves per SIMD the register budget is set for: the D = 64 production variants fit 168 registers.
-#define PARO_ATTN_WAVES_PER_SIMD ((D == 64 && !CAUSAL && !DUMP && !LSE) ? 3 : 2)
+// Waves per SIMD the register budget is set for: the D = 64 variants fit 168 registers (but for the score dump, and the fast
+// path with the causal diagonal).
+#define PARO_ATTN_WAVES_PER_SIMD ((D == 64 && !DUMP && (!CAUSAL || EXACT)) ? 3 : 2)
 
 // One 64-row q-block `vid` (numbered over batch, head, q-block) by one workgroup of two waves.
 //
@@ -302,7 +303,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   v8i ones = {sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word};
   asm volatile("" : "+v"(ones));  // same: resident constant operand
   float m_i = -1e30f;
-  float m_thr = -1e30f, m_off = 0.f, m_off8 = 0.f;  // m + headroom and the m-dependent offsets (see step)
+  float m_off = 0.f, m_off8 = 0.f;  // the m-dependent offsets (see step)
   float d_exact = 0.f;  // LSE only: sum of the unrounded P~ of this lane's 32 kv-columns per block
 
   // ---- prologue ------------------------------------------------------------------------------
@@ -344,17 +345,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
 
-  // the product O^T += V8^T . P~^T, plus the row sums of the ROUNDED P~ from one more MFMA against the
-  // selector operand; idx 0..DT_TILES-1 = output tiles, DT_TILES = row sums
+  // the product O^T += V8^T . P~^T
   v4i vfrag[DT_TILES][2];
   auto pv_one = [&](const v8i& pf, int idx) {
-    if (idx < DT_TILES) {
-      const v8i a = {vfrag[idx][0][0], vfrag[idx][0][1], vfrag[idx][0][2], vfrag[idx][0][3],
-                     vfrag[idx][1][0], vfrag[idx][1][1], vfrag[idx][1][2], vfrag[idx][1][3]};
-      o_acc[idx] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, pf, o_acc[idx], 0, 0, 0, 0, 0, 0);
-    } else {
-      d_acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
-    }
+    const v8i a = {vfrag[idx][0][0], vfrag[idx][0][1], vfrag[idx][0][2], vfrag[idx][0][3],
+                   vfrag[idx][1][0], vfrag[idx][1][1], vfrag[idx][1][2], vfrag[idx][1][3]};
+    o_acc[idx] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, pf, o_acc[idx], 0, 0, 0, 0, 0, 0);
   };
   auto read_v_frags = [&](int ST) {
 #pragma unroll
@@ -364,7 +360,6 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
         vfrag[dt][mt] = *reinterpret_cast<const v4i*>(smem + ST * Lds::VTILE + vr_base + (dt * 2 + mt) * 1024);
   };
 
-  constexpr int N_PV = DT_TILES + 1;     // MFMAs of one P.V (+ row sums)
   // One block.  `acc` holds its S^T on entry and that of the next block on exit.  sk1: K stage of block
   // it+1; sv: V stage of block it; skn / svn: the stages this iteration's DMA refills.
   auto step = [&](int it, int sk1, int sv, int skn, int svn) {
@@ -456,7 +451,6 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       const float m_new = fmaxf(m_i, m_blk);
       const float alpha = __builtin_amdgcn_exp2f(m_i - m_new);
       m_i = m_new;
-      m_thr = m_new + P_HEADROOM;
       m_off = P_EXP_OFFSET - m_new;
       m_off8 = (8.0f * (P_EXP_OFFSET + 7.0f - m_new) + FAST_EXP_SHIFT + 0.5f) * FAST_FIELD_SCALE;
       bias = fmaf(-S_MAGIC_F, c, m_off);
@@ -474,25 +468,49 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 
     // -- VALU phase: the softmax weights of this block as 8 words of four e4m3 values each
     v8i pf;
-    constexpr bool OPTIMISTIC = !EXACT;
-    if constexpr (OPTIMISTIC) {
-      // Fast path: the e4m3 byte of 2^t is built directly: byte = round(8*(t + 7) + FAST_EXP_SHIFT), i.e.
-      // exponent field floor(t)+7 and a mantissa that interpolates 2^frac(t) linearly between powers of
-      // two (at most 6 % off, shifted to be centred).  Per word of four weights: four fmas (the affine
-      // map scaled so that the byte lands in the HIGH half of a 16-bit field, result clamped to [0,1], which
-      // sends masked and underflowing elements to 0 and bounds the field by 0x7FFF, the byte by 0x7F), two
-      // v_cvt_pknorm_i16_f32 (each rounds two values to 16-bit fields) and one v_perm_b32 that gathers the
-      // four high bytes.  Instead of fma + v_exp_f32 + half a packed FP8 conversion per weight.
-      // Word r = word r%4 of row tile r/4.
-      //
-      // It is optimistic about the maximum: the weights are computed with the running maximum as it is.
-      // A weight above 448, the largest e4m3 value (a score more than 3.8 octaves above the running
-      // maximum), comes out as the byte 0x7F, which is the e4m3 NaN: the row sums, taken by the matrix pipe
-      // from the same bytes BEFORE anything else uses them, turn NaN in that column, and only then is the
-      // block maximum searched (17 v_max3 otherwise spent on every block), the maximum refreshed and the
-      // eight words computed again (the scores are still in `acc`: the next block's S^T is issued below).
-      // Nothing is spent on tracking in the common case, and O never sees a NaN.
-      auto fast_words = [&]() {
+    float rs = 0.f;   // LSE: the sum of the unrounded weights
+    // Fast path: the e4m3 byte of 2^t is built directly: byte = round(8*(t + 7) + FAST_EXP_SHIFT), i.e.
+    // exponent field floor(t)+7 and a mantissa that interpolates 2^frac(t) linearly between powers of
+    // two (at most 6 % off, shifted to be centred).  Per word of four weights: four fmas (the affine
+    // map scaled so that the byte lands in the HIGH half of a 16-bit field, result clamped to [0,1], which
+    // sends masked and underflowing elements to 0 and bounds the field by 0x7FFF, the byte by 0x7F), two
+    // v_cvt_pknorm_i16_f32 (each rounds two values to 16-bit fields) and one v_perm_b32 that gathers the
+    // four high bytes.  Exact path: fma, hardware exponential and half a packed FP8 conversion per weight.
+    // Word r = word r%4 of row tile r/4.
+    //
+    // Both are optimistic about the maximum: the weights are computed with the running maximum as it is.
+    // A weight that would round to more than 448, the largest e4m3 value, comes out as the byte 0x7F, which is the
+    // e4m3 NaN (the conversion instruction gives it too): the row sums, taken by the matrix pipe
+    // from the same bytes BEFORE anything else uses them, turn NaN in that column, and only then is the
+    // block maximum searched (17 v_max3 otherwise spent on every block: with exact exponentials, 117 vector
+    // instructions and bound by them, 1.78 -> 1.65 ms at B = 2, H = 48, N = 17776, D = 64, density 0.3, 2.00 -> 1.91 ms
+    // with the log-sum-exp; 1.04 -> 1.00 ms at D = 128, H = 40, N = 16384), the maximum refreshed and the
+    // eight words computed again (the scores are still in `acc`: the next block's S^T is issued below).
+    // Nothing is spent on tracking in the common case, and O never sees a NaN.
+    auto words = [&]() {
+      if constexpr (EXACT) {
+        rs = 0.f;
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+          const int mt = r >> 2, i0 = 4 * (r & 3);
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 0], c, bias));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 1], c, bias));
+          const float p2 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 2], PT ? cb : c, PT ? biasb : bias));
+          const float p3 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 3], PT ? cb : c, PT ? biasb : bias));
+          if constexpr (LSE) {
+            rs += p0;
+            rs += p1;
+            rs += p2;
+            rs += p3;
+            asm volatile("" : "+v"(rs));   // (taken here: deferred to the weights' acceptance, the sum would keep all of them)
+          }
+          int w;
+          cvt_pk_fp8<false>(w, p0, p1);
+          cvt_pk_fp8<true>(w, p2, p3);
+          pf[r] = w;
+          __builtin_amdgcn_sched_barrier(0);   // (word by word: the registers of a third wave per SIMD)
+        }
+      } else {
         float u_cur[4], u_nxt[4];
 #pragma unroll
         for (int q = 0; q < 4; q++)
@@ -521,54 +539,30 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
           for (int q = 0; q < 4; q++) u_cur[q] = u_nxt[q];
           __builtin_amdgcn_sched_barrier(0);
         }
-      };
-      fast_words();
-      v4f d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
-      // the fragment reads of the matrix phase are issued here: they cover the latency of the product above
-      __builtin_amdgcn_sched_barrier(0);
-      read_k_frags(sk1);
-      if constexpr (D == 64) read_v_frags(sv);
-      __builtin_amdgcn_sched_barrier(0);
-      // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
-      // and d_new[1]; a NaN byte of either row makes its own sum NaN whatever the hardware makes of 0 x NaN)
-      if (it == 0 || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
-        apply_refresh(block_max());
-        fast_words();
-        d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
-      }
-      d_acc = d_new;
-    } else {
-      // Exact path: lazy refresh decided up front from the block maximum (P~ <= 2^(OFFSET + HEADROOM)),
-      // then P~ = e4m3_rne(2^(S*c - m + OFFSET)): hardware exponential and the packed FP8 conversion
-      const float m_blk = block_max();
-      if (__ballot(m_blk > m_thr) != 0ull) apply_refresh(m_blk);
-      float rs = 0.f;
-#pragma unroll
-      for (int r = 0; r < 8; r++) {
-        const int mt = r >> 2, i0 = 4 * (r & 3);
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 0], c, bias));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 1], c, bias));
-        const float p2 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 2], PT ? cb : c, PT ? biasb : bias));
-        const float p3 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 3], PT ? cb : c, PT ? biasb : bias));
-        if constexpr (LSE) rs += (p0 + p1) + (p2 + p3);
-        int w;
-        cvt_pk_fp8<false>(w, p0, p1);
-        cvt_pk_fp8<true>(w, p2, p3);
-        pf[r] = w;
-      }
-      if constexpr (LSE) d_exact += rs;
+            }
+    };
+    words();
+    v4f d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
+    // the fragment reads of the matrix phase are issued here: they cover the latency of the product above
+    // (fetching the K fragments at the head of the iteration instead, so that they arrive under the VALU
+    // phase, measured 2 % slower at D = 128, 7 % with the dense mask)
+    __builtin_amdgcn_sched_barrier(0);
+    read_k_frags(sk1);
+    if constexpr (D == 64) read_v_frags(sv);
+    __builtin_amdgcn_sched_barrier(0);
+    // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
+    // and d_new[1]; a NaN byte of either row makes its own sum NaN whatever the hardware makes of 0 x NaN)
+    if (it == 0 || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
+      apply_refresh(block_max());
+      words();
+      d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
     }
+    d_acc = d_new;
+    if constexpr (LSE) d_exact += rs;
     __builtin_amdgcn_sched_barrier(0);
 
     // -- matrix phase: S^T of the next block first (the next VALU phase waits for it alone), then this
     //    block's P.V and row sums, which run on under that VALU phase
-    // (fetching the K fragments at the head of the iteration instead, so that they arrive under the VALU
-    // phase, measured 2 % slower at D = 128, 7 % with the dense mask)
-    if constexpr (EXACT) {   // (the fast path has issued these reads already)
-      read_k_frags(sk1);
-      if constexpr (D == 64) read_v_frags(sv);
-    }
-    __builtin_amdgcn_sched_barrier(0);
     if constexpr (D == 128) {
       // the V fragments are fetched while the S^T products issue: after the two products of k-step ks the K
       // fragments of that step are dead, and two V pieces take their place (+1-2 % against fetching all
@@ -587,9 +581,9 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       qk_mfma();
       __builtin_amdgcn_sched_barrier(0);
     }
-    // (fast path: the row sums have been taken above)
+    // (the row sums have been taken above)
 #pragma unroll
-    for (int i = 0; i < (EXACT ? N_PV : DT_TILES); i++) pv_one(pf, i);
+    for (int i = 0; i < DT_TILES; i++) pv_one(pf, i);
     __builtin_amdgcn_sched_barrier(0);
     if (it + 1 < cnt) dump_s(kb_1);
 

@@ -58,7 +58,7 @@ constexpr float S_INV2PI_F = 10680707.0f / 67108864.0f;
 constexpr float S_INV2PI_SCALE = 67108864.0f;
 
 template <int D, int OUT_DT, bool LSE>
-__global__ void __launch_bounds__(128, (D == 64 && !LSE ? 3 : 2)) attn_sparse_pv16_kernel(const AttnParams p, const int causal) {
+__global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kernel(const AttnParams p, const int causal) {
   using Lds = Pv16Lds<D>;
   constexpr int KS = D / 32;         // k-steps of the QK MFMA
   constexpr int DT_TILES = D / 32;   // 32-channel tiles of O^T
@@ -300,7 +300,10 @@ __global__ void __launch_bounds__(128, (D == 64 && !LSE ? 3 : 2)) attn_sparse_pv
           v2f w;
           w[0] = __builtin_amdgcn_exp2f(fmaf(s[mt][i], c, bias));
           w[1] = __builtin_amdgcn_exp2f(fmaf(s[mt][i + 1], c, bias));
-          if constexpr (LSE) rs += w[0] + w[1];
+          if constexpr (LSE) {
+            rs += w[0] + w[1];
+            asm volatile("" : "+v"(rs));   // (taken here: deferred to the weights' acceptance, the sum would keep all of them)
+          }
           const v2h hw = __builtin_convertvector(w, v2h);
           pf[k][2 * j] = hw[0];
           pf[k][2 * j + 1] = hw[1];

@@ -198,8 +198,8 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
 #pragma unroll
       for (int i = 0; i < 16; i++) o_acc[dt][i] *= alpha;
   };
-  // the weights of the scores in acc against the maximum as it is, and their row sums; true where one left e4m3
-  // (attn_sparse.hip describes the two forms; the exact one decides from the block's maximum)
+  // the weights of the scores in acc against the maximum as it is, and their row sums, NaN where a weight left e4m3
+  // (attn_sparse.hip describes the two forms)
   auto block_max = [&](const v16i (&acc)[2], float c) __attribute__((always_inline)) {
     float mx = max3(__int_as_float(acc[0][0]), __int_as_float(acc[0][1]), __int_as_float(acc[1][0]));
     mx = max3(mx, __int_as_float(acc[1][1]), __int_as_float(acc[1][1]));
@@ -221,7 +221,10 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
         float u[4];
 #pragma unroll
         for (int q = 0; q < 4; q++) u[q] = __builtin_amdgcn_exp2f(fmaf(__int_as_float(acc[r >> 2][4 * (r & 3) + q]), c, bias));
-        if constexpr (LSE) rs += (u[0] + u[1]) + (u[2] + u[3]);
+        if constexpr (LSE) {
+          rs += (u[0] + u[1]) + (u[2] + u[3]);
+          asm volatile("" : "+v"(rs));   // (taken here: deferred, the sum would keep all the weights)
+        }
         int w;
         cvt_pk_fp8<false>(w, u[0], u[1]);
         cvt_pk_fp8<true>(w, u[2], u[3]);
@@ -240,9 +243,8 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     }
     d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
   };
-  auto left_range = [&](const v16i (&acc)[2], float c) __attribute__((always_inline)) {   // wave-uniform
-    if constexpr (EXACT) return __ballot(block_max(acc, c) > m_i + P_HEADROOM) != 0ull;
-    else return __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull;
+  auto left_range = [&]() __attribute__((always_inline)) {   // wave-uniform
+    return __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull;
   };
   // A round in which a weight left e4m3 (and the first): the waves settle the maximum in list order.  i: the first wave
   // that said so, flag: the round's flags.  Returns by what this wave's accumulators have to be multiplied after its product.
@@ -270,7 +272,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
           rescale(alpha);
           if (active) {
             words(acc, c);
-            left = left_range(acc, c);
+            left = left_range();
           }
         }
       }
@@ -332,7 +334,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     bool left = r == 0 && wave == 0;
     if (active && r > 0) {
       words(cur, c);
-      left = left_range(cur, c);
+      left = left_range();
     }
     if (lane == 0) flag[wave] = left;
     qk(nxt, kfrag[K_LDS ? 0 : par ^ 1]);

@@ -232,7 +232,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   v8i ones = {sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word};
   asm volatile("" : "+v"(ones));
   float m_i[2] = {-1e30f, -1e30f};
-  float m_thr[2] = {-1e30f, -1e30f}, m_off[2] = {0.f, 0.f}, m_off8[2] = {0.f, 0.f};
+  float m_off[2] = {0.f, 0.f}, m_off8[2] = {0.f, 0.f};
   v8i pf[2];   // the weights of the newest block of each half, eight words of four e4m3 values
 
   auto pv_one = [&](auto hfc, int dt) {
@@ -292,7 +292,6 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     const float m_new = fmaxf(m_i[hf], m_blk);
     const float alpha = __builtin_amdgcn_exp2f(m_i[hf] - m_new);
     m_i[hf] = m_new;
-    m_thr[hf] = m_new + P_HEADROOM;
     m_off[hf] = P_EXP_OFFSET - m_new;
     m_off8[hf] = (8.0f * (P_EXP_OFFSET + 7.0f - m_new) + FAST_EXP_SHIFT + 0.5f) * FAST_FIELD_SCALE;
     d_acc[hf][0] *= alpha;                                    // lanes 0..15: q-row lane
@@ -377,24 +376,18 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     if constexpr (WEIGHTS) {
       const float c = qsc[Y] * clist[yi];
       mask_edge(yc, kb_y);
-      if constexpr (EXACT) {
-        const float m_blk = block_max(yc, c);
-        if (__ballot(m_blk > m_thr[Y]) != 0ull) apply_refresh(yc, m_blk);
-      }
       affine(yc, c, cs, bs);
       word_fma(yc, ub, 0, cs, bs);
       word_fma(yc, ub, 1, cs, bs);
       word_pack(yc, ub, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // accept the weights of half X (fast path: unless one of them overflowed e4m3, seen as a NaN row sum; then
-    // the maximum is refreshed and the words are computed again: the scores are still in acc[X])
-    if constexpr (!EXACT) {
-      if (__ballot(__builtin_isunordered(d_new[X][0], d_new[X][1])) != 0ull) {
-        const float cx = qsc[X] * clist[xi];
-        apply_refresh(xc, block_max(xc, cx));
-        all_words(xc, cx);
-      }
+    // accept the weights of half X, unless one of them overflowed e4m3, seen as a NaN row sum; then
+    // the maximum is refreshed and the words are computed again: the scores are still in acc[X]
+    if (__ballot(__builtin_isunordered(d_new[X][0], d_new[X][1])) != 0ull) {
+      const float cx = qsc[X] * clist[xi];
+      apply_refresh(xc, block_max(xc, cx));
+      all_words(xc, cx);
     }
     d_acc[X] = d_new[X];
     __builtin_amdgcn_sched_barrier(0);
@@ -474,13 +467,13 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   read_k_frags(1);
   read_v_frags(0);
   {
-    // the first block gives both halves their first maximum (the fast path does not search one again unless a
+    // the first block gives both halves their first maximum (one is not searched again unless a
     // weight overflows); half A's weights of it are due before the loop
     const float ks0 = clist[0];
     mask_edge(IC<0>{}, kb_c);
     mask_edge(IC<1>{}, kb_c);
     apply_refresh(IC<0>{}, block_max(IC<0>{}, qsc[0] * ks0));
-    if constexpr (!EXACT) apply_refresh(IC<1>{}, block_max(IC<1>{}, qsc[1] * ks0));
+    apply_refresh(IC<1>{}, block_max(IC<1>{}, qsc[1] * ks0));
     all_words(IC<0>{}, qsc[0] * ks0);
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

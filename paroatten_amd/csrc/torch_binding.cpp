@@ -367,6 +367,195 @@ py::object attn_operator(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
   return py::cast(out);
 }
 
+using OptTensor = c10::optional<torch::Tensor>;
+
+void hnd(const torch::Tensor& x, const char* name) {
+  TORCH_CHECK(x.is_cuda(), "Tensor ", name, " must be a CUDA tensor");
+  dims(x, name, 4);
+  TORCH_CHECK(x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16, "Tensor ", name, " must be float16 or bfloat16");
+  lastdim_contiguous(x, name);
+}
+int code_of(const torch::Tensor& x) { return x.scalar_type() == at::kHalf ? PARO_DTYPE_F16 : PARO_DTYPE_BF16; }
+
+void check_orders(const torch::Tensor& orders, int64_t H) {
+  TORCH_CHECK(orders.is_cuda(), "Tensor orders must be a CUDA tensor");
+  TORCH_CHECK(orders.scalar_type() == at::kInt && orders.dim() == 1 && orders.numel() == H && orders.is_contiguous(),
+              "orders must be a contiguous int32 tensor of ", H, " entries (one per head)");
+}
+
+struct Tables { const float *cos, *sin; };
+Tables check_tables(const OptTensor& cos, const OptTensor& sin, int64_t n_img, int64_t D) {
+  if (!cos) return {nullptr, nullptr};
+  TORCH_CHECK(sin, "cos and sin must be given together");
+  auto one = [&](const torch::Tensor& t, const char* name) {
+    TORCH_CHECK(t.is_cuda(), "Tensor ", name, " must be a CUDA tensor");
+    TORCH_CHECK(t.scalar_type() == at::kFloat && t.dim() == 2 && t.size(0) == n_img && t.size(1) == D && t.is_contiguous(),
+                "Tensor ", name, " must be contiguous float32 of shape (", n_img, ", ", D, ")");
+    return t.data_ptr<float>();
+  };
+  return {one(*cos, "cos"), one(*sin, "sin")};
+}
+
+// permute.rope_permute
+std::vector<OptTensor> rope_permute(const OptTensor& q, const OptTensor& k, const OptTensor& v, const torch::Tensor& orders,
+                                    int F, int Hh, int W, int n_text, const OptTensor& cos, const OptTensor& sin) {
+  const OptTensor* in[3] = {&q, &k, &v};
+  const torch::Tensor* ref = nullptr;
+  for (auto* t : in)
+    if (*t) {
+      hnd(**t, "input");
+      if (!ref) ref = &**t;
+      TORCH_CHECK((*t)->sizes() == ref->sizes() && (*t)->strides() == ref->strides() && (*t)->scalar_type() == ref->scalar_type(),
+                  "q, k, v must share shape, strides and dtype");
+    }
+  TORCH_CHECK(ref, "one of q, k, v must be given");
+  const int64_t B = ref->size(0), H = ref->size(1), N = ref->size(2), D = ref->size(3);
+  check_orders(orders, H);
+  const Tables tab = check_tables(cos, sin, (int64_t)F * Hh * W, D);
+  const c10::DeviceGuard guard(ref->device());
+  std::vector<OptTensor> out(3);
+  void *src[3] = {}, *dst[3] = {};
+  for (int i = 0; i < 3; i++)
+    if (*in[i]) {
+      out[i] = torch::empty({B, H, N, D}, ref->options());
+      src[i] = (*in[i])->data_ptr();
+      dst[i] = out[i]->data_ptr();
+    }
+  check_rc(paro_rope_permute_fwd(src[0], src[1], src[2], dst[0], dst[1], dst[2], code_of(*ref), tab.cos, tab.sin,
+                                 orders.data_ptr<int32_t>(), (int)B, (int)H, (int)N, (int)D, n_text, F, Hh, W, ref->stride(0),
+                                 ref->stride(1), ref->stride(2), H * N * D, N * D, D, stream_of(*ref)));
+  return out;
+}
+
+// permute.permute_inverse
+torch::Tensor permute_inverse(const torch::Tensor& o, const torch::Tensor& orders, int F, int Hh, int W, int n_text,
+                              const OptTensor& out_) {
+  hnd(o, "attn_out");
+  const int64_t B = o.size(0), H = o.size(1), N = o.size(2), D = o.size(3);
+  check_orders(orders, H);
+  const c10::DeviceGuard guard(o.device());
+  torch::Tensor out;
+  if (out_) {
+    out = *out_;
+    hnd(out, "out");
+    TORCH_CHECK(out.sizes() == o.sizes() && out.scalar_type() == o.scalar_type() && out.device() == o.device(),
+                "out must have attn_out's shape, dtype and device");
+  } else {
+    out = torch::empty({B, H, N, D}, o.options());
+  }
+  check_rc(paro_permute_inv(o.data_ptr(), out.data_ptr(), code_of(o), orders.data_ptr<int32_t>(), (int)B, (int)H, (int)N, (int)D,
+                            n_text, F, Hh, W, o.stride(0), o.stride(1), o.stride(2), out.stride(0), out.stride(1),
+                            out.stride(2), stream_of(o)));
+  return out;
+}
+
+// permute.rope_permute_quant: (q8, q_scale, k8, k_scale, v8, v_scale, v_mean or None, k_mean or None).  km: a K mean that is
+// subtracted; compute_km: it is taken in the call.
+std::vector<OptTensor> rope_permute_quant(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v,
+                                          const torch::Tensor& orders, int F, int Hh, int W, int n_text, const OptTensor& cos,
+                                          const OptTensor& sin, OptTensor km, bool compute_km, bool smooth_v) {
+  hnd(q, "query");
+  hnd(k, "key");
+  hnd(v, "value");
+  TORCH_CHECK(k.sizes() == q.sizes() && v.sizes() == q.sizes() && k.scalar_type() == q.scalar_type() &&
+                  v.scalar_type() == q.scalar_type(),
+              "q, k, v must share shape and dtype");
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), nb = (N + 63) / 64;
+  check_orders(orders, H);
+  const Tables tab = check_tables(cos, sin, (int64_t)F * Hh * W, D);
+  const c10::DeviceGuard guard(q.device());
+  if (compute_km) km = torch::empty({B, H, 1, D}, q.options());
+  if (km) {
+    TORCH_CHECK(km->is_cuda(), "Tensor km must be a CUDA tensor");
+    TORCH_CHECK(km->scalar_type() == q.scalar_type() && km->sizes() == at::IntArrayRef({B, H, 1, D}) && km->stride(-1) == 1,
+                "Tensor km must have shape (", B, ", ", H, ", 1, ", D, ") and the dtype of key");
+  }
+  const auto i8 = q.options().dtype(at::kChar), u8 = q.options().dtype(at::kByte), f32 = q.options().dtype(at::kFloat);
+  torch::Tensor q8 = torch::empty({B, H, N, D}, i8), k8 = torch::empty({B, H, N, D}, i8);
+  torch::Tensor q_scale = torch::empty({B, H, nb * 2}, f32), k_scale = torch::empty({B, H, nb}, f32);
+  torch::Tensor v8 = torch::empty({paro_v_fp8_bytes((int)B, (int)H, (int)N, (int)D)}, u8);
+  torch::Tensor v_scale = torch::empty({B, H, D}, f32), v_mean = torch::empty({B, H, D}, f32);
+  const int64_t ws_bytes = compute_km ? paro_prep_smooth_workspace_bytes((int)B, (int)H, (int)N, (int)D)
+                                      : paro_prep_workspace_bytes((int)B, (int)H, (int)N, (int)D);
+  torch::Tensor ws = torch::empty({ws_bytes}, u8);
+  auto call = [&](auto entry) {
+    check_rc(entry(q.data_ptr(), k.data_ptr(), v.data_ptr(), code_of(q), tab.cos, tab.sin, orders.data_ptr<int32_t>(),
+                   km ? km->data_ptr() : nullptr, q8.data_ptr<int8_t>(), q_scale.data_ptr<float>(), k8.data_ptr<int8_t>(),
+                   k_scale.data_ptr<float>(), v8.data_ptr<uint8_t>(), v_scale.data_ptr<float>(), v_mean.data_ptr<float>(),
+                   ws.data_ptr(), ws_bytes, (int)B, (int)H, (int)N, (int)D, n_text, F, Hh, W, q.stride(0), q.stride(1),
+                   q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+                   km ? km->stride(0) : 0, km ? km->stride(1) : 0, smooth_v ? 1 : 0, stream_of(q)));
+  };
+  if (compute_km) call(&paro_rope_k_mean_permute_quant_fwd);
+  else call(&paro_rope_permute_quant_fwd);
+  return {q8, q_scale, k8, k_scale, v8, v_scale, smooth_v ? OptTensor(v_mean) : c10::nullopt, compute_km ? km : c10::nullopt};
+}
+
+// _qattn_sm80.attn_sparse_prepacked; unpermute: orders with (F, Hh, W) and n_text, or none
+torch::Tensor attn_sparse_prepacked(const torch::Tensor& q8, const torch::Tensor& k8, const torch::Tensor& v8,
+                                    const OptTensor& v_scale, const OptTensor& v_mean, const torch::Tensor& output,
+                                    const torch::Tensor& q_scale, const torch::Tensor& k_scale, double sm_scale,
+                                    const torch::Tensor& sparse, int is_causal, bool return_lse, int flags,
+                                    const OptTensor& orders, int F, int Hh, int W, int n_text) {
+  const bool pv16 = (flags & PARO_ATTN_PV_F16) != 0;
+  auto gpu = [](const torch::Tensor& x, const char* name, bool contig) {
+    on_gpu(x, name);
+    if (contig) contiguous(x, name);
+  };
+  gpu(q8, "query", true); gpu(k8, "key", true); gpu(v8, "value", true); gpu(output, "output", false);
+  gpu(q_scale, "query_scale", true); gpu(k_scale, "key_scale", true);
+  TORCH_CHECK(v_scale || pv16, "Tensor v_scale must be given");
+  if (v_scale) gpu(*v_scale, "v_scale", true);
+  gpu(sparse, "sparse", true);
+  TORCH_CHECK(q8.scalar_type() == at::kChar && k8.scalar_type() == at::kChar, "Tensor query/key must have dtype (torch::kInt8)");
+  TORCH_CHECK(q8.dim() == 4 && k8.dim() == 4, "Tensor query/key must have dimension number (4)");
+  const int64_t B = q8.size(0), H = q8.size(1), Nq = q8.size(2), D = q8.size(3), Hkv = k8.size(1), Nk = k8.size(2);
+  if (D != 64 && D != 128) throw std::invalid_argument("Unsupported head dim: " + std::to_string(D));
+  TORCH_CHECK(k8.size(0) == B && k8.size(3) == D, "Tensor key must have the batch size and head dim of query");
+  if (Hkv == 0 || H % Hkv != 0)
+    throw std::invalid_argument("num_qo_heads (" + std::to_string(H) + ") must be divisible by num_kv_heads (" +
+                                std::to_string(Hkv) + ")");
+  const int64_t nbq = (Nq + 63) / 64, nbk = (Nk + 63) / 64;
+  TORCH_CHECK((int64_t)v8.nbytes() == (pv16 ? paro_v_f16_bytes((int)B, (int)Hkv, (int)Nk, (int)D)
+                                            : paro_v_fp8_bytes((int)B, (int)Hkv, (int)Nk, (int)D)),
+              "Tensor value has the wrong size for ", pv16 ? "float16" : "FP8", " tiles");
+  TORCH_CHECK(q_scale.scalar_type() == at::kFloat && k_scale.scalar_type() == at::kFloat &&
+                  q_scale.sizes() == at::IntArrayRef({B, H, nbq * 2}) && k_scale.sizes() == at::IntArrayRef({B, Hkv, nbk}),
+              "Tensor query_scale / key_scale must have shapes (B, H, 2*nbq) / (B, Hkv, nbk)");
+  const std::vector<int64_t> vs = {B, Hkv, D};
+  TORCH_CHECK((!v_scale || (v_scale->sizes() == at::IntArrayRef(vs) && v_scale->scalar_type() == at::kFloat)) &&
+                  (!v_mean || (v_mean->sizes() == at::IntArrayRef(vs) && v_mean->scalar_type() == at::kFloat && v_mean->is_cuda())),
+              "Tensor v_scale / v_mean must have shape (B, Hkv, head_dim)");
+  TORCH_CHECK(output.sizes() == at::IntArrayRef({B, H, Nq, D}) && output.stride(-1) == 1 &&
+                  (output.scalar_type() == at::kHalf || output.scalar_type() == at::kBFloat16),
+              "Tensor output must be float16/bfloat16 [B,H,N,D] with a contiguous last dimension");
+  const int64_t sparse_bs = check_mask(sparse, B, H, nbq, nbk);
+  const c10::DeviceGuard guard(q8.device());
+  torch::Tensor lse = return_lse ? torch::empty({B, H, Nq}, q8.options().dtype(at::kFloat)) : torch::empty({0});
+  float* lse_p = return_lse ? lse.data_ptr<float>() : nullptr;
+  const float* vsp = v_scale ? v_scale->data_ptr<float>() : nullptr;
+  const float* vmp = v_mean ? v_mean->data_ptr<float>() : nullptr;
+  const uint8_t* mask = static_cast<const uint8_t*>(sparse.data_ptr());
+  if (orders) {
+    TORCH_CHECK(orders->is_cuda() && orders->scalar_type() == at::kInt && orders->dim() == 1 && orders->numel() == H &&
+                    orders->is_contiguous(),
+                "orders must be a contiguous int32 GPU tensor of ", H, " entries");
+    check_rc(paro_attn_sparse_unpermute_fwd(
+        q8.data_ptr<int8_t>(), k8.data_ptr<int8_t>(), static_cast<const uint8_t*>(v8.data_ptr()), q_scale.data_ptr<float>(),
+        k_scale.data_ptr<float>(), vsp, vmp, mask, sparse_bs, output.data_ptr(), code_of(output), lse_p, (int)B, (int)H, (int)Hkv,
+        (int)Nq, (int)Nk, (int)D, q8.stride(0), q8.stride(1), q8.stride(2), k8.stride(0), k8.stride(1), k8.stride(2),
+        output.stride(0), output.stride(1), output.stride(2), (float)sm_scale, is_causal, flags, orders->data_ptr<int32_t>(),
+        n_text, F, Hh, W, stream_of(q8)));
+  } else {
+    check_rc(paro_attn_sparse_fwd(
+        q8.data_ptr<int8_t>(), k8.data_ptr<int8_t>(), static_cast<const uint8_t*>(v8.data_ptr()), q_scale.data_ptr<float>(),
+        k_scale.data_ptr<float>(), vsp, vmp, mask, sparse_bs, output.data_ptr(), code_of(output), lse_p, nullptr, (int)B, (int)H,
+        (int)Hkv, (int)Nq, (int)Nk, (int)D, q8.stride(0), q8.stride(1), q8.stride(2), k8.stride(0), k8.stride(1), k8.stride(2),
+        output.stride(0), output.stride(1), output.stride(2), (float)sm_scale, is_causal, flags, stream_of(q8)));
+  }
+  return lse;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -392,5 +581,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   auto rope = m.def_submodule("_rope");
   auto ops = m.def_submodule("_ops");
   ops.def("attn_operator", &attn_operator);
+  ops.def("attn_sparse_prepacked", &attn_sparse_prepacked);
+  ops.def("rope_permute", &rope_permute);
+  ops.def("rope_permute_quant", &rope_permute_quant);
+  ops.def("permute_inverse", &permute_inverse);
   rope.def("rope_permutation", &rope_permutation, "RoPE op with permutation.");
 }

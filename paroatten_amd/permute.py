@@ -50,29 +50,8 @@ def rope_permute(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Option
     """out[b,h,perm_h(t)] = rope(in[b,h,t]) for q and k, permutation only for v; text tokens
     [0,n_text) are copied through.  cos/sin: fp32 [F*H*W, D] (full-width tables, every frequency
     may be repeated over its channel pair as diffusers does); None = no rotation."""
-    ref = next(t for t in (q, k, v) if t is not None)
-    _check_hnd(ref, "input")
-    B, H, N, D = ref.shape
-    for t in (q, k, v):
-        if t is not None:
-            _check_hnd(t, "input")
-            if t.shape != ref.shape or t.stride() != ref.stride() or t.dtype != ref.dtype:
-                raise RuntimeError("q, k, v must share shape, strides and dtype")
-    _check_orders(orders, H)
     F, Hh, W = (int(x) for x in grid)
-    if cos is not None:
-        for t, n in ((cos, "cos"), (sin, "sin")):
-            _lib.require_gpu(t, n)
-            if t.dtype != torch.float32 or tuple(t.shape) != (F * Hh * W, D) or not t.is_contiguous():
-                raise RuntimeError(f"Tensor {n} must be contiguous float32 of shape ({F * Hh * W}, {D})")
-    outs = [None if t is None else torch.empty((B, H, N, D), dtype=t.dtype, device=t.device) for t in (q, k, v)]
-    o_ref = next(o for o in outs if o is not None)
-    _lib.on(ref).paro_rope_permute_fwd(
-        ptr(q), ptr(k), ptr(v), ptr(outs[0]), ptr(outs[1]), ptr(outs[2]), _lib.DTYPE_CODE[ref.dtype],
-        ptr(cos), ptr(sin), ptr(orders), B, H, N, D, int(n_text), F, Hh, W,
-        ref.stride(0), ref.stride(1), ref.stride(2), o_ref.stride(0), o_ref.stride(1), o_ref.stride(2),
-        stream_of(ref))
-    return tuple(outs)
+    return tuple(_lib.ops().rope_permute(q, k, v, orders, F, Hh, W, int(n_text), cos, sin))
 
 
 class PreparedOperands(NamedTuple):
@@ -123,45 +102,14 @@ def rope_permute_quant(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, orders
     [B,H,1,D] in the input dtype (see rope_k_mean), or the string "mean": the mean of the rotated K is taken
     inside the same call (its pass over K shares a launch with the V statistics) and returned as the `k_mean`
     field of the result."""
-    _check_hnd(q, "query")
-    B, H, N, D = q.shape
-    for t, n in ((k, "key"), (v, "value")):
-        _check_hnd(t, n)
-        if t.shape != q.shape or t.dtype != q.dtype:
-            raise RuntimeError("q, k, v must share shape and dtype")
-    _check_orders(orders, H)
-    F, Hh, W = (int(x) for x in grid)
-    _tables_ok(cos, sin, F * Hh * W, D)
-    ms_b = ms_h = 0
     compute_km = isinstance(km, str)
     if compute_km:
         if km != "mean":
             raise ValueError("km must be None, a tensor, or the string 'mean'")
-        km = torch.empty((B, H, 1, D), dtype=q.dtype, device=q.device)
-    if km is not None:
-        _lib.require_gpu(km, "km")
-        if km.dtype != q.dtype or tuple(km.shape) != (B, H, 1, D) or km.stride(-1) != 1:
-            raise RuntimeError(f"Tensor km must have shape ({B}, {H}, 1, {D}) and the dtype of key")
-        ms_b, ms_h = km.stride(0), km.stride(1)
-    lib = load()
-    dev = q.device
-    nb = (N + 63) // 64
-    q8 = torch.empty((B, H, N, D), dtype=torch.int8, device=dev)
-    k8 = torch.empty((B, H, N, D), dtype=torch.int8, device=dev)
-    q_scale = torch.empty((B, H, nb * 2), dtype=torch.float32, device=dev)
-    k_scale = torch.empty((B, H, nb), dtype=torch.float32, device=dev)
-    v8 = torch.empty(int(lib.paro_v_fp8_bytes(B, H, N, D)), dtype=torch.uint8, device=dev)
-    v_scale = torch.empty((B, H, D), dtype=torch.float32, device=dev)
-    v_mean = torch.empty((B, H, D), dtype=torch.float32, device=dev)
-    ws_bytes = lib.paro_prep_smooth_workspace_bytes(B, H, N, D) if compute_km else lib.paro_prep_workspace_bytes(B, H, N, D)
-    ws = torch.empty(int(ws_bytes), dtype=torch.uint8, device=dev)
-    entry = _lib.on(q).paro_rope_k_mean_permute_quant_fwd if compute_km else _lib.on(q).paro_rope_permute_quant_fwd
-    entry(
-        ptr(q), ptr(k), ptr(v), _lib.DTYPE_CODE[q.dtype], ptr(cos), ptr(sin), ptr(orders), ptr(km),
-        ptr(q8), ptr(q_scale), ptr(k8), ptr(k_scale), ptr(v8), ptr(v_scale), ptr(v_mean), ptr(ws), ws.numel(),
-        B, H, N, D, int(n_text), F, Hh, W, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
-        k.stride(2), v.stride(0), v.stride(1), v.stride(2), ms_b, ms_h, 1 if smooth_v else 0, stream_of(q))
-    return PreparedOperands(q8, q_scale, k8, k_scale, v8, v_scale, v_mean if smooth_v else None, km if compute_km else None)
+        km = None
+    F, Hh, W = (int(x) for x in grid)
+    return PreparedOperands(*_lib.ops().rope_permute_quant(q, k, v, orders, F, Hh, W, int(n_text), cos, sin, km, compute_km,
+                                                           bool(smooth_v)))
 
 
 def permute_inverse(o: torch.Tensor, orders: torch.Tensor, grid: Sequence[int], n_text: int,
@@ -170,20 +118,8 @@ def permute_inverse(o: torch.Tensor, orders: torch.Tensor, grid: Sequence[int], 
     `out`, if given, is any [B,H,N,D] view with a contiguous last dimension that does not overlap `o`
     (e.g. the transpose of an [B,N,H,D] buffer, which makes the result token-major for the output
     projection without another pass)."""
-    _check_hnd(o, "attn_out")
-    B, H, N, D = o.shape
-    _check_orders(orders, H)
     F, Hh, W = (int(x) for x in grid)
-    if out is None:
-        out = torch.empty((B, H, N, D), dtype=o.dtype, device=o.device)
-    else:
-        _check_hnd(out, "out")
-        if out.shape != o.shape or out.dtype != o.dtype or out.device != o.device:
-            raise RuntimeError("out must have attn_out's shape, dtype and device")
-    _lib.on(o).paro_permute_inv(ptr(o), ptr(out), _lib.DTYPE_CODE[o.dtype], ptr(orders), B, H, N, D, int(n_text),
-                                  F, Hh, W, o.stride(0), o.stride(1), o.stride(2),
-                                  out.stride(0), out.stride(1), out.stride(2), stream_of(o))
-    return out
+    return _lib.ops().permute_inverse(o, orders, F, Hh, W, int(n_text), out)
 
 
 def permute_index_map(orders: torch.Tensor, grid: Sequence[int]) -> torch.Tensor:

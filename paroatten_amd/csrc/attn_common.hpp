@@ -47,6 +47,21 @@ constexpr float FAST_EXP_SHIFT = -0.35f;  // centres the linear-mantissa error o
 // round(b); the field is bounded by 0x7FFF, so the byte is bounded by 0x7F
 constexpr float FAST_FIELD_SCALE = 256.0f / 32767.0f;
 
+// The q-block (numbered over batch, head, q-block) that is the slot-th of XCD xcd, per = ceil(total / 8) to each;
+// p.total or more: none.  Each XCD walks a contiguous range of them, so that the K8 / V8 of the head it is working on
+// stay in its own L2.  Causal: a q-block's work grows with its index.  The longest of a head go first, so that short ones
+// fill the card at the end, and heads that do not come out even are dealt out q-block by q-block, since the two halves of
+// a head are 1 : 3 in work.  B = 2, H = 32, N = 8192, D = 128, every block below the diagonal, kernel alone: 609 -> 592 us;
+// B = 1, H = 48, D = 64: 273 -> 257 us.
+template <bool CAUSAL>
+__device__ __forceinline__ int qblock_of(const AttnParams& p, int xcd, int slot, int per) {
+  if constexpr (!CAUSAL) return xcd * per + slot;
+  const int heads = p.total / p.nbq, own = (heads >> 3) * p.nbq;   // q-blocks of the heads that an XCD has to itself
+  const int i = slot < own ? xcd * own + slot : 8 * own + (slot - own) * 8 + xcd;
+  const int head = i / p.nbq;
+  return head < heads ? head * p.nbq + (p.nbq - 1 - (i - head * p.nbq)) : p.total;
+}
+
 __device__ __forceinline__ void store_lse(const AttnParams& p, int64_t row, float lse2) {
   p.lse[row] = p.lse_add != nullptr ? fmaf(lse2, p.lse_scale, p.lse_add[row]) : lse2 * p.lse_scale;
 }

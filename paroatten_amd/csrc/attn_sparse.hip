@@ -658,9 +658,8 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
 __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_kernel(const AttnParams p) {
-  // XCD-aware renumbering: hardware deals workgroup ids round-robin to the 8 XCDs
-  const int per = gridDim.x >> 3;
-  const int vid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  // hardware deals workgroup ids round-robin to the 8 XCDs
+  const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
   attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>(p, vid);
 }
@@ -690,13 +689,12 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
     attn_sparse_paced_kernel(const AttnParams p, unsigned* __restrict__ counters, const int per, const int spin_limit,
                              const int slack) {
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, G = gridDim.x >> 3;
-  const int first = xcd * per, last = min(first + per, p.total);
   unsigned arrivals = 0;
   bool waiting = true;   // a workgroup that has once waited in vain goes on without waiting for the rest of the launch
-  for (int base = first; base < last; base += G) {
-    const int vid = base + slot;
-    if (vid < last) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>(p, vid);
-    if (base + G >= last) break;
+  for (int base = 0; base < per; base += G) {
+    const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
+    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>(p, vid);
+    if (base + G >= per) break;
     // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
     __syncthreads();   // also: both waves are done with this q-block's lists in LDS
     if (threadIdx.x == 0) {

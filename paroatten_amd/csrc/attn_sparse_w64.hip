@@ -537,10 +537,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
 
 template <int OUT_DT, bool CAUSAL, bool EXACT>
 __global__ void __launch_bounds__(64, 2) attn_sparse_w64_kernel(const AttnParams p) {
-  // XCD-aware renumbering: hardware deals workgroup ids round-robin to the 8 XCDs; each XCD walks a contiguous
-  // range of (batch, head, q-block), so the K8 / V8 of the head it is working on stay in its own L2
-  const int per = gridDim.x >> 3;
-  const int vid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  // hardware deals workgroup ids round-robin to the 8 XCDs
+  const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
   attn_qblock_w64<OUT_DT, CAUSAL, EXACT>(p, vid);
 }

@@ -50,8 +50,8 @@ extern "C" {
                                  all but a share of its workgroups (PARO_ATTN_PACE_SLACK; default half the L2's share
                                  of a head, at most a quarter of them) and at most PARO_ATTN_PACE_SPINS rounds. */
 #define PARO_ATTN_TWO_WAVES 8 /* kernel form: two waves per 64-row q-block (32 q-rows each) also where the
-                                 library would pick one wave per q-block (head size 64, no lse, plain launch, more
-                                 than 1024 q-blocks; bit-identical results) or several key blocks of a q-block at a
+                                 library would pick one wave per q-block (head size 64, plain launch, more than
+                                 1024 q-blocks; bit-identical results) or several key blocks of a q-block at a
                                  time (without any of the form flags, up to 256 q-blocks and at least 20 key blocks;
                                  the same weights, summed in another order) */
 #define PARO_ATTN_PV_F16 16   /* accuracy mode: the P.V product in float16 with fp32 accumulation, as the reference's

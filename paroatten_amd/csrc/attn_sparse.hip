@@ -835,6 +835,23 @@ static int dispatch_attn(const AttnParams& p, int is_causal, bool dump, bool exa
                    : launch_attn<D, OUT_DT, false, false, false, false>(p, st);
 }
 
+// Whether the two-wave kernel is the faster one for so few q-blocks at D = 64.  Up to one q-block per SIMD the latency of a
+// q-block's walk is what counts, and two waves halve the work of each (N = 4096: 22.3 instead of 28.1 us with 512 q-blocks,
+// 28.3 instead of 29.5 us with 1024).  Beyond, the card holds 2048 q-blocks of one wave or 1536 of two waves at a time, and
+// the kernel whose last round is the fuller one wins until rounds no longer count: N = 8192, density 0.3, one wave / two
+// waves, fast exponentials 51.0 / 45.5 us and log-sum-exp 81.0 / 67.0 us with 1536 q-blocks, 54.5 / 61.0 and 80.7 / 91.2
+// with 2048, 70.1 / 66.5 and 104.2 / 93.9 with 2304, 86.8 / 83.9 and 121.3 / 118.6 with 3072, 93.8 / 96.7 and 139.4 / 138.1
+// with 3584, 151.3 / 156.6 and 218.8 / 221.5 with 6144.  (With more than 340 key blocks the lists leave the LDS of a
+// compute unit five workgroups of two waves instead of six.)  Causal q-blocks differ too much in length for rounds; there the
+// longest ones set the time of a launch of few heads, the more so with true exponentials: N = 8192, every block below the
+// diagonal, 112.4 / 86.3 us and log-sum-exp 191.5 / 152.7 us with 2048 q-blocks, 250.8 / 254.4 and 386.9 / 366.9 with 6144,
+// 480.1 / 508.6 and 694.0 / 701.2 with 12288; N = 17920, log-sum-exp, 2000.8 / 1963.8 with 16240.
+static bool two_waves_fill_better(const AttnParams& p, bool causal, bool exact) {
+  if (p.total <= 1024) return true;
+  if (causal) return p.total <= 2048 || (exact && (p.total <= 4096 || p.total <= 64 * p.nbk));
+  return p.nbk <= 340 && (p.total <= 1536 || (p.total > 2048 && p.total <= 3072));
+}
+
 }  // namespace paro
 
 namespace paro {
@@ -913,11 +930,10 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   // too few q-blocks to fill the card: several kept blocks of each at a time (attn_sparse_split.hip)
   if (!dump && p.pacing == 0 && (flags & PARO_ATTN_TWO_WAVES) == 0 && split_width(p, D) != 0)
     return launch_attn_split(p, D, out_dtype, is_causal != 0, exact, st);
-  // D = 64 without lse or score dump: one wave per q-block (attn_sparse_w64.hip), unless the caller asks for the
-  // two-wave kernel, the launch is to be paced (only the two-wave kernel has the paced form), or there is no more than one
-  // q-block per SIMD: the latency of a q-block's walk is what counts then, and two waves halve the work of each (N = 4096:
-  // 22.3 instead of 28.1 us with 512 q-blocks, 28.3 instead of 29.5 us with 1024; 51.7 instead of 47.0 us with 2048)
-  if (D == 64 && lse == nullptr && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && p.total > 1024 && !want_pacing(p, D))
+  // D = 64 without score dump: one wave per q-block (attn_sparse_w64.hip), unless the caller asks for the two-wave
+  // kernel, the launch is to be paced (only the two-wave kernel has the paced form), or two waves fill the card better
+  if (D == 64 && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && !want_pacing(p, D) &&
+      !two_waves_fill_better(p, is_causal != 0, exact || lse != nullptr))
     return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
   if (D == 64) {
     if (out_dtype == PARO_DTYPE_F16) return dispatch_attn<64, PARO_DTYPE_F16>(p, is_causal, dump, exact, st);

@@ -16,6 +16,10 @@
 // K8 and V8 tiles come in by LDS-DMA through two stages each (the wave moves whole tiles, two blocks ahead);
 // their fragments are read once per block, right after the last product that used the previous ones.
 //
+// With the log-sum-exp 253 of 256 registers are taken (the sums of the unrounded weights are two per half, of the accepted
+// blocks and of the newest): B = 1, H = 48, N = 8960, density 0.5, 421 us by two waves per q-block, 414 us here; N = 17664,
+// 1523 and 1481 us.
+//
 // Semantics: qk_int_sv_f16_attn_kernel of the reference (csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:44-726) as its
 // host instantiates it (:1022-1048); see attn_sparse.hip for the line-by-line correspondence.
 #include "attn_common.hpp"
@@ -46,10 +50,11 @@ __device__ __forceinline__ int lane_here() {
   return x;
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
 __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int vid) {
   using Lds = W64Lds;
   constexpr int D = 64;
+  static_assert(EXACT || !LSE, "the log-sum-exp needs true exponentials");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* clist = reinterpret_cast<float*>(smem + Lds::LIST_OFF);  // [nbk + LIST_PAD + 1] k_scale of kept blocks
   unsigned short* klist = reinterpret_cast<unsigned short*>(clist + p.nbk + Lds::LIST_PAD + 1);  // their indices
@@ -140,6 +145,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
         unsigned short* outp = out_row_ptr(qrow[hf]);
 #pragma unroll
         for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
+        if constexpr (LSE)
+          if (lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow[hf], -INFINITY);
       }
     return;
   }
@@ -233,6 +240,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   asm volatile("" : "+v"(ones));
   float m_i[2] = {-1e30f, -1e30f};
   float m_off[2] = {0.f, 0.f}, m_off8[2] = {0.f, 0.f};
+  // LSE: sums of the unrounded weights of this lane's 32 columns per block, accepted and of the newest block
+  float d_exact[2] = {0.f, 0.f}, rs[2] = {0.f, 0.f};
   v8i pf[2];   // the weights of the newest block of each half, eight words of four e4m3 values
 
   auto pv_one = [&](auto hfc, int dt) {
@@ -294,6 +303,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     m_i[hf] = m_new;
     m_off[hf] = P_EXP_OFFSET - m_new;
     m_off8[hf] = (8.0f * (P_EXP_OFFSET + 7.0f - m_new) + FAST_EXP_SHIFT + 0.5f) * FAST_FIELD_SCALE;
+    if constexpr (LSE) d_exact[hf] *= alpha;
     d_acc[hf][0] *= alpha;                                    // lanes 0..15: q-row lane
     d_acc[hf][1] *= __shfl(alpha, (lane_here() & 15) + 16, 64);   // and q-row lane + 16
 #pragma unroll
@@ -317,6 +327,15 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     constexpr int hf = decltype(hfc)::value;
     const float* u = ub[r & 1];
     if constexpr (EXACT) {
+      if constexpr (LSE) {
+        float sum = r == 0 ? 0.f : rs[hf];
+        sum += u[0];
+        sum += u[1];
+        sum += u[2];
+        sum += u[3];
+        rs[hf] = sum;
+        asm volatile("" : "+v"(rs[hf]));   // (taken here: deferred to the acceptance it would keep all the weights)
+      }
       int w;
       cvt_pk_fp8<false>(w, u[0], u[1]);
       cvt_pk_fp8<true>(w, u[2], u[3]);
@@ -390,6 +409,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
       all_words(xc, cx);
     }
     d_acc[X] = d_new[X];
+    if constexpr (LSE) d_exact[X] += rs[X];
     __builtin_amdgcn_sched_barrier(0);
     // matrix and vector instructions alternate: a word is 7 instructions (9.5 with true exponentials)
     if constexpr (!LAST) {
@@ -515,6 +535,12 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     const float d_lo = __shfl(d_acc[hf][0], e32 & 15, 64), d_hi = __shfl(d_acc[hf][1], e32 & 15, 64);
     const float inv = 1.0f / (e32 < 16 ? d_lo : d_hi);
     const int row = qb * 64 + hf * 32 + e32;
+    if constexpr (LSE) {
+      // from the exact fp32 row sum, not the sum of the rounded weights
+      const float d_full = d_exact[hf] + __shfl_xor(d_exact[hf], 32, 64);
+      if (row < p.Nq && eh == 0)
+        store_lse(p, ((int64_t)b * p.H + h) * p.Nq + row, m_i[hf] + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET);
+    }
     if (row < p.Nq) {
       unsigned short* outp = out_row_ptr(row);
 #pragma unroll
@@ -535,19 +561,19 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   }
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
 __global__ void __launch_bounds__(64, 2) attn_sparse_w64_kernel(const AttnParams p) {
   // hardware deals workgroup ids round-robin to the 8 XCDs
   const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
-  attn_qblock_w64<OUT_DT, CAUSAL, EXACT>(p, vid);
+  attn_qblock_w64<OUT_DT, CAUSAL, EXACT, LSE>(p, vid);
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
 static int launch_w64(const AttnParams& p, hipStream_t st) {
   const size_t smem = W64Lds::LIST_OFF + (((size_t)(p.nbk + W64Lds::LIST_PAD + 1) * 6 + 15) & ~(size_t)15);
   const int grid = ((p.total + 7) / 8) * 8;
-  auto kern = attn_sparse_w64_kernel<OUT_DT, CAUSAL, EXACT>;
+  auto kern = attn_sparse_w64_kernel<OUT_DT, CAUSAL, EXACT, LSE>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64), smem, st, p);
@@ -555,13 +581,16 @@ static int launch_w64(const AttnParams& p, hipStream_t st) {
   return PARO_OK;
 }
 
+template <int OUT_DT>
+static int dispatch_w64(const AttnParams& p, bool causal, bool exact, hipStream_t st) {
+  if (p.lse != nullptr) return causal ? launch_w64<OUT_DT, true, true, true>(p, st) : launch_w64<OUT_DT, false, true, true>(p, st);
+  if (exact) return causal ? launch_w64<OUT_DT, true, true, false>(p, st) : launch_w64<OUT_DT, false, true, false>(p, st);
+  return causal ? launch_w64<OUT_DT, true, false, false>(p, st) : launch_w64<OUT_DT, false, false, false>(p, st);
+}
+
 int launch_attn_w64(const AttnParams& p, int out_dtype, bool causal, bool exact, hipStream_t st) {
-  if (out_dtype == PARO_DTYPE_F16) {
-    if (causal) return exact ? launch_w64<PARO_DTYPE_F16, true, true>(p, st) : launch_w64<PARO_DTYPE_F16, true, false>(p, st);
-    return exact ? launch_w64<PARO_DTYPE_F16, false, true>(p, st) : launch_w64<PARO_DTYPE_F16, false, false>(p, st);
-  }
-  if (causal) return exact ? launch_w64<PARO_DTYPE_BF16, true, true>(p, st) : launch_w64<PARO_DTYPE_BF16, true, false>(p, st);
-  return exact ? launch_w64<PARO_DTYPE_BF16, false, true>(p, st) : launch_w64<PARO_DTYPE_BF16, false, false>(p, st);
+  return out_dtype == PARO_DTYPE_F16 ? dispatch_w64<PARO_DTYPE_F16>(p, causal, exact, st)
+                                     : dispatch_w64<PARO_DTYPE_BF16>(p, causal, exact, st);
 }
 
 }  // namespace paro

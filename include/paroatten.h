@@ -43,8 +43,8 @@ extern "C" {
                                  XCD takes the q-blocks generation by generation, so that workgroups running
                                  together walk the key sequence together and share K8 / V8 tiles in the XCD's L2 */
 #define PARO_ATTN_UNPACED 4   /* one workgroup per q-block, started as the hardware pleases.  With neither flag the
-                                 library paces when one head's K8 + V8 exceed an XCD's 4 MB L2 (environment variable
-                                 PARO_ATTN_PACING=0/1 overrides that default).  Scattered masks on long sequences gain
+                                 library paces when one head's K8 + V8 exceed 7 MB at head size 128 (causal 16 MB) or
+                                 12 MB at 64 (environment variable PARO_ATTN_PACING=0/1 overrides that default).  Scattered masks on long sequences gain
                                  (Wan 720p, uniformly random blocks: 26 -> 39 % of the MFMA peak, 4x fewer L2 fills);
                                  masks made of one contiguous run per row lose a few per cent.  A generation waits for
                                  all but a share of its workgroups (PARO_ATTN_PACE_SLACK; default half the L2's share

@@ -749,14 +749,21 @@ static int pace_device(PaceDevice* out) {
 
 // The caller's flags decide (PARO_ATTN_PACED / PARO_ATTN_UNPACED); without either, the environment
 // variable PARO_ATTN_PACING (0: never, 1: always) does, and without that the launch is paced when one
-// head's K8 + V8 exceed the 4 MB L2 of an XCD.  PARO_ATTN_PACE_SPINS: rounds (about 1 us each) a workgroup
+// head's K8 + V8 exceed what the plain launch still gets out of the 4 MB L2 of an XCD and the memory-side cache.  A layer
+// (preparation included) with rotary embedding at density 0.3, paced / plain, scattered masks: D = 128, 4.5 MB 893 / 820 us,
+// 5 MB 1061 / 979, 6 MB 1403 / 1362, 6.9 MB 1803 / 1782, 8 MB 3744 / 3903 (40 heads), 18 MB 13131 / 18596; rows of one run,
+// 6.9 MB 1798 / 1689.  D = 64, where plain means the one-wave kernel: 4.6 MB 1915 / 1628, 6.9 MB 2638 / 2430, 8.8 MB 3049 /
+// 3099, 12.3 MB 4503 / 4434, runs 4476 / 3635.  Causal q-blocks differ in length, and a generation lasts as long as its
+// longest: D = 128, density 0.2, the kernel alone, 8 MB 797 / 704, 11 MB 734 / 665, 18 MB 1864 / 1849, density 0.5 there
+// 4238 / 4282.
+// PARO_ATTN_PACE_SPINS: rounds (about 1 us each) a workgroup
 // waits for its generation at most (default: half the number of key blocks, between 64 and 4096).
 // PARO_ATTN_PACE_SLACK: how many of an XCD's resident workgroups a generation does not wait for (default: half
 // the share of the head's K8 + V8 that the L2 holds, at most a quarter of them).
-static bool want_pacing(const AttnParams& p, int D) {
+static bool want_pacing(const AttnParams& p, int D, bool causal) {
   if (p.pacing != 0) return p.pacing > 0;
   if (const char* e = getenv("PARO_ATTN_PACING")) return e[0] == '1';
-  return (int64_t)p.nbk * 64 * D * 2 > (int64_t)4 << 20;
+  return (int64_t)p.nbk * 64 * D * 2 > (int64_t)(D == 64 ? 12 : causal ? 16 : 7) << 20;
 }
 
 // bytes of the kept-block list in LDS: per key block a 16-bit index and its k scale (four with per-thread scales)
@@ -769,7 +776,7 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
   const size_t smem = AttnLds<D>::LIST_OFF + attn_list_bytes(p.nbk, AttnLds<D>::LIST_PAD, PT);
   // (per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup,
   // Wan 720p, the paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms)
-  if (!DUMP && want_pacing(p, D) && (!PT || smem <= 40 * 1024)) {
+  if (!DUMP && want_pacing(p, D, CAUSAL) && (!PT || smem <= 40 * 1024)) {
     auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>;
     if (smem > 48 * 1024)
       PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
@@ -932,7 +939,7 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
     return launch_attn_split(p, D, out_dtype, is_causal != 0, exact, st);
   // D = 64 without score dump: one wave per q-block (attn_sparse_w64.hip), unless the caller asks for the two-wave
   // kernel, the launch is to be paced (only the two-wave kernel has the paced form), or two waves fill the card better
-  if (D == 64 && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && !want_pacing(p, D) &&
+  if (D == 64 && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && !want_pacing(p, D, is_causal != 0) &&
       !two_waves_fill_better(p, is_causal != 0, exact || lse != nullptr))
     return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
   if (D == 64) {

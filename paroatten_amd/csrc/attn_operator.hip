@@ -38,13 +38,14 @@ struct OpParams {
 
 template <int DT, int D>
 __global__ void __launch_bounds__(256) op_stats_kernel(const OpParams p) {
-  const int both = p.stats_k + p.stats_v;   // K and V of a head one after the other
-  const int h = blockIdx.y / both, b = blockIdx.z;
-  if (p.stats_k && blockIdx.y % both == 0)
+  // K and V of a head one after the other, in x: y and z keep the whole range of head and batch counts
+  const int h = blockIdx.y, b = blockIdx.z;
+  const int k_chunks = p.stats_k ? p.chunks : 0;
+  if ((int)blockIdx.x < k_chunks)
     v_stats_body<DT, D, true>(p.k, p.k_partial, p.Nk, p.chunks, p.ks_b, p.ks_h, p.ks_n, blockIdx.x, h, b, p.Hkv);
   else
     v_stats_body<DT, D>(p.v, p.v_work + v_stats_offset((int64_t)p.B * p.Hkv, p.Nk, D), p.Nk, p.chunks, p.vs_b, p.vs_h,
-                        p.vs_n, blockIdx.x, h, b, p.Hkv);
+                        p.vs_n, (int)blockIdx.x - k_chunks, h, b, p.Hkv);
 }
 
 template <int DT, int D>
@@ -133,7 +134,7 @@ struct OpLayout {
 template <int DT, int D>
 static int launch_op_prep(const OpParams& p, bool per_thread, bool f16v, hipStream_t st) {
   if (p.stats_k + p.stats_v > 0) {
-    hipLaunchKernelGGL((op_stats_kernel<DT, D>), dim3(p.chunks, p.Hkv * (p.stats_k + p.stats_v), p.B), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((op_stats_kernel<DT, D>), dim3(p.chunks * (p.stats_k + p.stats_v), p.Hkv, p.B), dim3(256), 0, st, p);
     hipLaunchKernelGGL((op_finalize_kernel<DT, D>), dim3(p.B * p.Hkv * (p.stats_k + p.stats_v)), dim3(1024), 0, st, p);
   }
   const int q_blocks = p.B * p.H * ceil_div(per_thread ? p.nbq : 2 * p.nbq, 4);
@@ -172,8 +173,8 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
              qk_quant_gran);
   const bool per_thread = qk_quant_gran == 3, f16v = (flags & PARO_ATTN_PV_F16) != 0;
   PARO_CHECK(!(per_thread && f16v), PARO_ERR_UNSUPPORTED, "per-thread scales do not go with PARO_ATTN_PV_F16");
-  PARO_CHECK((int64_t)B * 2 <= MAX_GRID_YZ && H <= MAX_GRID_YZ, PARO_ERR_RUNTIME,
-             "paro_attn_operator: batch or head count too large (limits %d and %d)", MAX_GRID_YZ / 2, MAX_GRID_YZ);
+  PARO_CHECK(B <= MAX_GRID_YZ && H <= MAX_GRID_YZ, PARO_ERR_RUNTIME,
+             "paro_attn_operator: batch or head count exceeds %d", MAX_GRID_YZ);
   PARO_CHECK((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16) == 0 &&
                  ((q_stride_b | q_stride_h | q_stride_n | k_stride_b | k_stride_h | k_stride_n | v_stride_b | v_stride_h |
                    v_stride_n) % 8) == 0,

@@ -53,3 +53,19 @@ def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode,
         scale = scale + (qh.double() * kh).abs().sum(-1) * D ** -0.5
     # one product and one sum in fp32, and an fp32 dot product of D terms
     assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()
+
+
+@pytest.mark.parametrize("B,H,smooth_k", [(32769, 1, True), (1, 32769, False)])
+def test_operator_batch_and_head_counts_of_16_bits(dev, B, H, smooth_k):
+    """Batch and head counts above half a grid dimension, as the quantisers and the V conversion take them: the same as the
+    last 1100 batch entries or heads by themselves (both calls have more than the 1024 q-blocks of the split kernels)."""
+    import paroatten_amd as P
+    g = torch.Generator(device=dev).manual_seed(3)
+    q, k, v = (torch.randn(B, H, 17, 64, generator=g, device=dev).half() for _ in range(3))
+    mask = torch.ones(H, 1, 1, dtype=torch.bool, device=dev)
+    kw = dict(tensor_layout="HND", smooth_k=smooth_k)
+    o = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, **kw)
+    tail = (slice(-1100, None),) if B > 1 else (slice(None), slice(-1100, None))
+    part = P.paroattn_qk_int8_pv_fp16_cuda(q[tail].contiguous(), k[tail].contiguous(), v[tail].contiguous(),
+                                           mask if B > 1 else mask[-1100:], **kw)
+    assert torch.equal(o[tail], part)

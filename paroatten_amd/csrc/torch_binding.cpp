@@ -350,19 +350,23 @@ py::object attn_operator(torch::Tensor q, torch::Tensor k, torch::Tensor v, torc
     throw std::invalid_argument("num_qo_heads (" + std::to_string(H) + ") must be divisible by num_kv_heads (" +
                                 std::to_string(Hkv) + ")");
   const int64_t sparse_bs = check_mask(sparse, B, H, (Nq + 63) / 64, (Nk + 63) / 64);
-  const c10::DeviceGuard guard(q.device());
-  torch::Tensor out = torch::empty(q.sizes(), q.options()), lse;
-  if (return_lse) lse = torch::empty({B, H, Nq}, q.options().dtype(at::kFloat));
-  const int64_t ws_bytes = paro_attn_operator_workspace_bytes((int)B, (int)H, (int)Hkv, (int)Nq, (int)Nk, (int)D, smooth_k,
-                                                              return_lse, qk_quant_gran, flags);
-  torch::Tensor ws = torch::empty({ws_bytes}, q.options().dtype(at::kByte));
-  check_rc(paro_attn_operator(q.data_ptr(), k.data_ptr(), v.data_ptr(), half_code(q, "paroattn"), out.data_ptr(),
-                              static_cast<const uint8_t*>(sparse.data_ptr()), sparse_bs,
-                              return_lse ? lse.data_ptr<float>() : nullptr, ws.data_ptr(), ws_bytes, (int)B, (int)H, (int)Hkv,
-                              (int)Nq, (int)Nk, (int)D, q.stride(0), q.stride(sh), q.stride(sn), k.stride(0), k.stride(sh),
-                              k.stride(sn), v.stride(0), v.stride(sh), v.stride(sn), out.stride(0), out.stride(sh),
-                              out.stride(sn), is_causal, qk_quant_gran, (float)sm_scale, smooth_k, smooth_v, flags,
-                              stream_of(q)));
+  torch::Tensor out, lse;
+  {
+    const py::gil_scoped_release unlocked;   // the launches wait while the queue is full: not with the interpreter lock
+    const c10::DeviceGuard guard(q.device());
+    out = torch::empty(q.sizes(), q.options());
+    if (return_lse) lse = torch::empty({B, H, Nq}, q.options().dtype(at::kFloat));
+    const int64_t ws_bytes = paro_attn_operator_workspace_bytes((int)B, (int)H, (int)Hkv, (int)Nq, (int)Nk, (int)D, smooth_k,
+                                                                return_lse, qk_quant_gran, flags);
+    torch::Tensor ws = torch::empty({ws_bytes}, q.options().dtype(at::kByte));
+    check_rc(paro_attn_operator(q.data_ptr(), k.data_ptr(), v.data_ptr(), half_code(q, "paroattn"), out.data_ptr(),
+                                static_cast<const uint8_t*>(sparse.data_ptr()), sparse_bs,
+                                return_lse ? lse.data_ptr<float>() : nullptr, ws.data_ptr(), ws_bytes, (int)B, (int)H, (int)Hkv,
+                                (int)Nq, (int)Nk, (int)D, q.stride(0), q.stride(sh), q.stride(sn), k.stride(0), k.stride(sh),
+                                k.stride(sn), v.stride(0), v.stride(sh), v.stride(sn), out.stride(0), out.stride(sh),
+                                out.stride(sn), is_causal, qk_quant_gran, (float)sm_scale, smooth_k, smooth_v, flags,
+                                stream_of(q)));
+  }
   if (return_lse) return py::make_tuple(out, lse);
   return py::cast(out);
 }
@@ -580,10 +584,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   fused.def("mean_scale_fuse_quant_cuda", &mean_scale_fuse_quant_cuda);
   auto rope = m.def_submodule("_rope");
   auto ops = m.def_submodule("_ops");
-  ops.def("attn_operator", &attn_operator);
-  ops.def("attn_sparse_prepacked", &attn_sparse_prepacked);
-  ops.def("rope_permute", &rope_permute);
-  ops.def("rope_permute_quant", &rope_permute_quant);
-  ops.def("permute_inverse", &permute_inverse);
+  const py::call_guard<py::gil_scoped_release> unlocked;
+  ops.def("attn_operator", &attn_operator);   // releases the lock itself: its result is a Python object
+  ops.def("attn_sparse_prepacked", &attn_sparse_prepacked, unlocked);
+  ops.def("rope_permute", &rope_permute, unlocked);
+  ops.def("rope_permute_quant", &rope_permute_quant, unlocked);
+  ops.def("permute_inverse", &permute_inverse, unlocked);
   rope.def("rope_permutation", &rope_permutation, "RoPE op with permutation.");
 }

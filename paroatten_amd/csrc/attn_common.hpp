@@ -36,9 +36,12 @@ struct AttnParams {
 };
 
 // P~ = 2^(S*c - m + P_EXP_OFFSET).  m is the running row maximum, refreshed lazily: only when a
-// weight would round to more than 448, the largest e4m3 value (a score about 3.8 octaves above m), are m, O and the
-// row sums rescaled.
+// weight leaves the range of e4m3 are m, O and the row sums rescaled.  Fast exponentials: a weight that would round to
+// more than 448, the largest e4m3 value (a score about 3.8 octaves above m).  True exponentials: a block maximum more than
+// P_HEADROOM above m.  (The weight of a fresh maximum is 2^5, which e4m3 holds exactly: letting it grow to the last code
+// cost up to 0.2 % in the error against 64 bits.)
 constexpr float P_EXP_OFFSET = 5.0f;
+constexpr float P_HEADROOM = 3.75f;
 constexpr int S_MAGIC_BITS = 0x4B400000;  // float 1.5 * 2^23
 constexpr float S_MAGIC_F = 12582912.0f;
 constexpr int FP8_ONES = 0x38383838;  // four e4m3 1.0
@@ -78,6 +81,20 @@ template <bool HI>
 __device__ __forceinline__ void cvt_pk_fp8(int& w, float a, float b) {
   if constexpr (HI) asm("v_cvt_pk_fp8_f32 %0, %1, %2 op_sel:[0,0,1]" : "+v"(w) : "v"(a), "v"(b));
   else asm("v_cvt_pk_fp8_f32 %0, %1, %2" : "=v"(w) : "v"(a), "v"(b));  // upper half: don't care, overwritten next
+}
+
+// Whether one of a block's weights (true exponentials, 64 columns of 32 q-rows as e4m3 bytes) can be above
+// 2^(P_EXP_OFFSET + P_HEADROOM) = 420.4, without a search: as e5m2 the bytes from 0x7C on (384 and up, e4m3's NaN among
+// them) are infinite or NaN and all others finite, so that a product against the selector operand of the row sums tells,
+// on the matrix pipe, of which a kernel with true exponentials leaves most idle (it is bound by its 117 vector instructions
+// a block).  B = 2, H = 48, N = 17776, D = 64, density 0.3, with the V conversion: 1.89 ms with a search of the block maximum,
+// 17 v_max3, on every block, 1.82 ms this way, 1.81 ms when only a weight beyond the last code moved the maximum; with the
+// log-sum-exp, two waves per q-block, 2.14, 2.12 and 2.07 ms.
+__device__ __forceinline__ v4f headroom_probe(const v8i& selector, const v8i& weights) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(selector, weights, v4f{0.f, 0.f, 0.f, 0.f}, 0, 1, 0, 0, 0, 0);
+}
+__device__ __forceinline__ bool headroom_suspect(const v4f& probe) {   // wave-uniform
+  return __ballot(!(probe[0] + probe[1] < INFINITY)) != 0ull;
 }
 
 // a*b + c clamped to [0,1] (the clamp is an output modifier: no extra instruction)

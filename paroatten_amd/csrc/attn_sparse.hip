@@ -479,13 +479,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     // Word r = word r%4 of row tile r/4.
     //
     // Both are optimistic about the maximum: the weights are computed with the running maximum as it is.
-    // A weight that would round to more than 448, the largest e4m3 value, comes out as the byte 0x7F, which is the
-    // e4m3 NaN (the conversion instruction gives it too): the row sums, taken by the matrix pipe
-    // from the same bytes BEFORE anything else uses them, turn NaN in that column, and only then is the
-    // block maximum searched (17 v_max3 otherwise spent on every block: with exact exponentials, 117 vector
-    // instructions and bound by them, 1.78 -> 1.65 ms at B = 2, H = 48, N = 17776, D = 64, density 0.3, 2.00 -> 1.91 ms
-    // with the log-sum-exp; 1.04 -> 1.00 ms at D = 128, H = 40, N = 16384), the maximum refreshed and the
+    // Fast path: a weight that would round to more than 448, the largest e4m3 value, comes out as the byte 0x7F, which is
+    // the e4m3 NaN: the row sums, taken by the matrix pipe from the same bytes BEFORE anything else uses them, turn NaN
+    // in that column, and only then is the block maximum searched (17 v_max3), the maximum refreshed and the
     // eight words computed again (the scores are still in `acc`: the next block's S^T is issued below).
+    // Exact path: headroom_probe says whether a weight can have passed the headroom, and only then is the block
+    // maximum searched and compared with it; the row sums are taken once the weights stand.
     // Nothing is spent on tracking in the common case, and O never sees a NaN.
     auto words = [&]() {
       if constexpr (EXACT) {
@@ -495,18 +494,17 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
           const int mt = r >> 2, i0 = 4 * (r & 3);
           const float p0 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 0], c, bias));
           const float p1 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 1], c, bias));
-          const float p2 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 2], PT ? cb : c, PT ? biasb : bias));
-          const float p3 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 3], PT ? cb : c, PT ? biasb : bias));
-          if constexpr (LSE) {
-            rs += p0;
-            rs += p1;
-            rs += p2;
-            rs += p3;
-            asm volatile("" : "+v"(rs));   // (taken here: deferred to the weights' acceptance, the sum would keep all of them)
-          }
           int w;
           cvt_pk_fp8<false>(w, p0, p1);
+          float p01 = p0 + p1;
+          if constexpr (LSE) asm volatile("" : "+v"(p01));
+          const float p2 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 2], PT ? cb : c, PT ? biasb : bias));
+          const float p3 = __builtin_amdgcn_exp2f(fmaf(s[mt][i0 + 3], PT ? cb : c, PT ? biasb : bias));
           cvt_pk_fp8<true>(w, p2, p3);
+          if constexpr (LSE) {
+            rs += p01 + (p2 + p3);
+            asm volatile("" : "+v"(rs));   // (taken here: deferred to the weights' acceptance, the sum would keep all of them)
+          }
           pf[r] = w;
           __builtin_amdgcn_sched_barrier(0);   // (word by word: the registers of a third wave per SIMD)
         }
@@ -539,26 +537,40 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
           for (int q = 0; q < 4; q++) u_cur[q] = u_nxt[q];
           __builtin_amdgcn_sched_barrier(0);
         }
-            }
+      }
     };
+    auto row_sums = [&]() { return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0); };
     words();
-    v4f d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
+    v4f d_new;   // EXACT: the probe
+    if constexpr (EXACT) d_new = headroom_probe(ones, pf);
+    else d_new = row_sums();
     // the fragment reads of the matrix phase are issued here: they cover the latency of the product above
     // (fetching the K fragments at the head of the iteration instead, so that they arrive under the VALU
     // phase, measured 2 % slower at D = 128, 7 % with the dense mask)
     __builtin_amdgcn_sched_barrier(0);
-    read_k_frags(sk1);
-    if constexpr (D == 64) read_v_frags(sv);
+    if constexpr (!(D == 64 && EXACT && PT)) read_k_frags(sk1);
+    if constexpr (D == 64 && !EXACT) read_v_frags(sv);
     __builtin_amdgcn_sched_barrier(0);
     // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
     // and d_new[1]; a NaN byte of either row makes its own sum NaN whatever the hardware makes of 0 x NaN)
-    if (it == 0 || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
+    if constexpr (EXACT) {
+      if (it == 0 || headroom_suspect(d_new)) {
+        const float m_blk = block_max();
+        if (__ballot(m_blk > m_i + P_HEADROOM) != 0ull) {
+          apply_refresh(m_blk);
+          words();
+        }
+      }
+      d_new = row_sums();
+    } else if (it == 0 || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
       apply_refresh(block_max());
       words();
-      d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
+      d_new = row_sums();
     }
     d_acc = d_new;
     if constexpr (LSE) d_exact += rs;
+    if constexpr (D == 64 && EXACT && PT) read_k_frags(sk1);
+    if constexpr (D == 64 && EXACT) read_v_frags(sv);   // (behind the search: its registers)
     __builtin_amdgcn_sched_barrier(0);
 
     // -- matrix phase: S^T of the next block first (the next VALU phase waits for it alone), then this

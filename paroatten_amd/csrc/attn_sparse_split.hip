@@ -9,7 +9,7 @@
 // wave adds the shares up at the end.
 //
 // The weights of a block are rounded against the running maximum, so all waves keep the maximum that the walk in list
-// order would have: it changes only when a weight leaves e4m3 (rarely, and in the first block), each wave says so in LDS
+// order would have: it changes only when a weight leaves its range (rarely, and in the first block), each wave says so in LDS
 // before the round's barrier, and the waves of such a round settle it in list order.  A wave before the block that
 // moved the maximum keeps its weights and is rescaled after its product, one behind it computes its own again.
 #include "attn_common.hpp"
@@ -179,7 +179,8 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   for (int dt = 0; dt < DT; dt++)
 #pragma unroll
     for (int i = 0; i < 16; i++) o_acc[dt][i] = 0.f;
-  v4f d_acc = {0.f, 0.f, 0.f, 0.f}, d_new = {0.f, 0.f, 0.f, 0.f};   // lanes 0..15: rows lane and lane + 16 in [0], [1]
+  v4f d_acc = {0.f, 0.f, 0.f, 0.f};   // lanes 0..15: rows lane and lane + 16 in [0], [1]
+  v4f d_new = {0.f, 0.f, 0.f, 0.f};   // with the newest block, not yet accepted; EXACT: its headroom_probe
   const int sel_word = ((lane & 15) == ((lane >> 4) & 1)) ? FP8_ONES : 0;
   const v8i ones = {sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word};
   float m_i = -1e30f, m_off = 0.f, m_off8 = 0.f, d_exact = 0.f, rs = 0.f;
@@ -198,8 +199,8 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
 #pragma unroll
       for (int i = 0; i < 16; i++) o_acc[dt][i] *= alpha;
   };
-  // the weights of the scores in acc against the maximum as it is, and their row sums, NaN where a weight left e4m3
-  // (attn_sparse.hip describes the two forms)
+  // the weights of the scores in acc against the maximum as it is, and their row sums, NaN where a weight left e4m3;
+  // EXACT: the probe for a weight beyond the headroom (attn_sparse.hip describes the two forms)
   auto block_max = [&](const v16i (&acc)[2], float c) __attribute__((always_inline)) {
     float mx = max3(__int_as_float(acc[0][0]), __int_as_float(acc[0][1]), __int_as_float(acc[1][0]));
     mx = max3(mx, __int_as_float(acc[1][1]), __int_as_float(acc[1][1]));
@@ -241,12 +242,14 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
         pf[r] = (int)__builtin_amdgcn_perm((unsigned)cvt_pknorm_i16(u[1], u[3]), (unsigned)cvt_pknorm_i16(u[0], u[2]), 0x07030501u);
       }
     }
-    d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
+    if constexpr (EXACT) d_new = headroom_probe(ones, pf);
+    else d_new = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
   };
-  auto left_range = [&]() __attribute__((always_inline)) {   // wave-uniform
-    return __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull;
+  auto left_range = [&](const v16i (&acc)[2], float c) __attribute__((always_inline)) {   // wave-uniform
+    if constexpr (EXACT) return headroom_suspect(d_new) && __ballot(block_max(acc, c) > m_i + P_HEADROOM) != 0ull;
+    else return __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull;
   };
-  // A round in which a weight left e4m3 (and the first): the waves settle the maximum in list order.  i: the first wave
+  // A round in which a weight left its range (and the first): the waves settle the maximum in list order.  i: the first wave
   // that said so, flag: the round's flags.  Returns by what this wave's accumulators have to be multiplied after its product.
   using Flags = std::conditional_t<W == 4, unsigned, unsigned short>;   // a byte per wave
   auto settle = [&](const v16i (&acc)[2], float c, bool active, int i, uint8_t* flag) __attribute__((always_inline)) {
@@ -272,7 +275,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
           rescale(alpha);
           if (active) {
             words(acc, c);
-            left = left_range();
+            left = left_range(acc, c);
           }
         }
       }
@@ -334,7 +337,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     bool left = r == 0 && wave == 0;
     if (active && r > 0) {
       words(cur, c);
-      left = left_range();
+      left = left_range(cur, c);
     }
     if (lane == 0) flag[wave] = left;
     qk(nxt, kfrag[K_LDS ? 0 : par ^ 1]);
@@ -350,7 +353,8 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
                        vfrag[par][dt][1][0], vfrag[par][dt][1][1], vfrag[par][dt][1][2], vfrag[par][dt][1][3]};
         o_acc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, pf, o_acc[dt], 0, 0, 0, 0, 0, 0);
       }
-      d_acc = d_new;
+      if constexpr (EXACT) d_acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, d_acc, 0, 0, 0, 0, 0, 0);
+      else d_acc = d_new;
       if constexpr (LSE) d_exact += rs;
     }
     if (f != 0) rescale(post);

@@ -16,9 +16,9 @@
 // K8 and V8 tiles come in by LDS-DMA through two stages each (the wave moves whole tiles, two blocks ahead);
 // their fragments are read once per block, right after the last product that used the previous ones.
 //
-// With the log-sum-exp 253 of 256 registers are taken (the sums of the unrounded weights are two per half, of the accepted
-// blocks and of the newest): B = 1, H = 48, N = 8960, density 0.5, 421 us by two waves per q-block, 414 us here; N = 17664,
-// 1523 and 1481 us.
+// With the log-sum-exp 254 of 256 registers are taken (the sums of the unrounded weights are two per half, of the accepted
+// blocks and of the newest): B = 1, H = 48, N = 8960, density 0.5, with the V conversion 483 us by two waves per q-block,
+// 460 us here; N = 17664, 1.66 and 1.58 ms.
 //
 // Semantics: qk_int_sv_f16_attn_kernel of the reference (csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:44-726) as its
 // host instantiates it (:1022-1048); see attn_sparse.hip for the line-by-line correspondence.
@@ -234,7 +234,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   // row sums of the rounded weights: selector operand as in attn_sparse.hip (lanes 0..15 get the sums of
   // q-rows lane and lane + 16 of the half in [0] and [1])
   v4f d_acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  v4f d_new[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};   // sums including the newest block, not yet accepted
+  // sums including the newest block, not yet accepted; EXACT: its headroom_probe (sums are taken when it is accepted)
+  v4f d_new[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   const int sel_word = ((lane & 15) == ((lane >> 4) & 1)) ? FP8_ONES : 0;
   v8i ones = {sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word};
   asm volatile("" : "+v"(ones));
@@ -252,7 +253,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   };
   auto row_sums = [&](auto hfc) {
     constexpr int hf = decltype(hfc)::value;
-    d_new[hf] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf[hf], d_acc[hf], 0, 0, 0, 0, 0, 0);
+    if constexpr (EXACT) d_new[hf] = headroom_probe(ones, pf[hf]);
+    else d_new[hf] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf[hf], d_acc[hf], 0, 0, 0, 0, 0, 0);
   };
 
   // columns past the end of K (last block) or above the diagonal (causal) leave the softmax: their scores
@@ -328,12 +330,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
     const float* u = ub[r & 1];
     if constexpr (EXACT) {
       if constexpr (LSE) {
-        float sum = r == 0 ? 0.f : rs[hf];
-        sum += u[0];
-        sum += u[1];
-        sum += u[2];
-        sum += u[3];
-        rs[hf] = sum;
+        rs[hf] = (r == 0 ? 0.f : rs[hf]) + ((u[0] + u[1]) + (u[2] + u[3]));
         asm volatile("" : "+v"(rs[hf]));   // (taken here: deferred to the acceptance it would keep all the weights)
       }
       int w;
@@ -401,14 +398,26 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
       word_pack(yc, ub, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // accept the weights of half X, unless one of them overflowed e4m3, seen as a NaN row sum; then
-    // the maximum is refreshed and the words are computed again: the scores are still in acc[X]
-    if (__ballot(__builtin_isunordered(d_new[X][0], d_new[X][1])) != 0ull) {
-      const float cx = qsc[X] * clist[xi];
-      apply_refresh(xc, block_max(xc, cx));
-      all_words(xc, cx);
+    // accept the weights of half X, unless one of them overflowed e4m3, seen as a NaN row sum (EXACT: passed the
+    // headroom); then the maximum is refreshed and the words are computed again: the scores are still in acc[X]
+    if constexpr (EXACT) {
+      if (headroom_suspect(d_new[X])) {
+        const float cx = qsc[X] * clist[xi];
+        const float m_blk = block_max(xc, cx);
+        if (__ballot(m_blk > m_i[X] + P_HEADROOM) != 0ull) {
+          apply_refresh(xc, m_blk);
+          all_words(xc, cx);
+        }
+      }
+      d_acc[X] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf[X], d_acc[X], 0, 0, 0, 0, 0, 0);
+    } else {
+      if (__ballot(__builtin_isunordered(d_new[X][0], d_new[X][1])) != 0ull) {
+        const float cx = qsc[X] * clist[xi];
+        apply_refresh(xc, block_max(xc, cx));
+        all_words(xc, cx);
+      }
+      d_acc[X] = d_new[X];
     }
-    d_acc[X] = d_new[X];
     if constexpr (LSE) d_exact[X] += rs[X];
     __builtin_amdgcn_sched_barrier(0);
     // matrix and vector instructions alternate: a word is 7 instructions (9.5 with true exponentials)
@@ -488,7 +497,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   read_v_frags(0);
   {
     // the first block gives both halves their first maximum (one is not searched again unless a
-    // weight overflows); half A's weights of it are due before the loop
+    // weight leaves its range); half A's weights of it are due before the loop
     const float ks0 = clist[0];
     mask_edge(IC<0>{}, kb_c);
     mask_edge(IC<1>{}, kb_c);

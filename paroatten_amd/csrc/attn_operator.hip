@@ -52,7 +52,7 @@ template <int DT, int D>
 __global__ void __launch_bounds__(1024) op_finalize_kernel(const OpParams p) {
   const int BH = p.B * p.Hkv;
   if ((int)blockIdx.x < BH * p.stats_k)
-    k_mean_finalize_body<DT, D>(p.k_partial, p.k_mean, p.Nk, p.chunks, (int64_t)p.Hkv * D, D, p.Hkv, blockIdx.x);
+    k_mean_finalize_body<DT, D, double>(p.k_partial, p.k_mean, p.Nk, p.chunks, (int64_t)p.Hkv * D, D, p.Hkv, blockIdx.x);
   else
     v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.Nk, p.chunks, p.smooth_v, (int64_t)blockIdx.x - BH * p.stats_k, BH);
 }

@@ -55,6 +55,25 @@ def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode,
     assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()
 
 
+@pytest.mark.parametrize("N,D,dtype", [(416, 64, torch.float16), (2000, 128, torch.bfloat16), (32760, 128, torch.float16)])
+def test_k_mean_is_the_rounded_mean(dev, N, D, dtype):
+    """The K mean that the operator takes is the one that 64-bit sums round to, on inputs of which sums in one fp32
+    accumulator per thread give a few channels the neighbouring value."""
+    import paroatten_amd as P
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    H, nb = 64, (N + 63) // 64
+    g = torch.Generator(device=dev).manual_seed(N)
+    k = (torch.randn(H, N, D, generator=g, device=dev) + 3 * torch.randn(H, 1, D, generator=g, device=dev)).to(dtype)[None]
+    q, v = k[..., :64, :].contiguous(), k.flip(2).contiguous()
+    mask = torch.ones(H, 1, nb, dtype=torch.bool, device=dev)
+    km = k.double().mean(dim=2, keepdim=True).to(dtype)
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, km, BLKQ=64, WARPQ=32, BLKK=64)
+    o_ref = torch.empty_like(q)
+    qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, 1, 0, 2, D ** -0.5, 0, mask, two_waves=True)
+    assert torch.equal(P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, smooth_k=True, two_waves=True), o_ref)
+
+
 @pytest.mark.parametrize("B,H,smooth_k", [(32769, 1, True), (1, 32769, False)])
 def test_operator_batch_and_head_counts_of_16_bits(dev, B, H, smooth_k):
     """Batch and head counts above half a grid dimension, as the quantisers and the V conversion take them: the same as the

@@ -149,3 +149,21 @@ def test_v_statistics_at_the_edges_of_the_chunks(dev, N):
         # the offset: the same mean, plus the residuals summed in fp32 (each below 16 codes times the scale)
         assert ((offset.cpu().double() - want).abs() <= 2 * err + N * 16 * scale.cpu().double() * 2.0 ** -24 + 1e-6).all()
         assert int(tokens[:, :, N:].max() if tokens.shape[2] > N else 0) == 0
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_v_mean_as_near_to_64_bits_as_the_library_reduction(dev, D):
+    """The mean of 8192 tokens (32 chunks), seen in v_scale = max |v - mean| / 448 where it is the larger part: no
+    further from 64 bits, over many channels, than with torch's fp32 mean."""
+    Q = _q()
+    N, H = 8192, 24
+    g = torch.Generator().manual_seed(N)
+    v = (torch.randn(1, H, N, D, generator=g) + 8 * torch.randn(1, H, 1, D, generator=g)).half().to(dev)
+    _, scale, _ = Q.per_channel_fp8(v)
+    lo, hi = v.float().amin(2), v.float().amax(2)
+
+    def scale_with(mean):
+        return torch.maximum(hi.to(mean.dtype) - mean, mean - lo.to(mean.dtype)) / 448.0
+    exact = scale_with(v.double().mean(2))
+    rms = [float((s.double() / exact - 1).pow(2).mean().sqrt()) for s in (scale.view_as(exact), scale_with(v.float().mean(2)))]
+    assert rms[0] <= rms[1], rms

@@ -26,14 +26,17 @@
 
 namespace {
 
+// NotImplementedError in Python.  An exception of C++, translated once the call has the interpreter lock again: the entry
+// points of _ops run without it.
+struct Unsupported : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
 void check_rc(int rc) {
   if (rc == PARO_OK) return;
   const std::string msg = paro_last_error();
   if (rc == PARO_ERR_INVALID_VALUE) throw std::invalid_argument(msg);
-  if (rc == PARO_ERR_UNSUPPORTED) {
-    PyErr_SetString(PyExc_NotImplementedError, msg.c_str());
-    throw py::error_already_set();
-  }
+  if (rc == PARO_ERR_UNSUPPORTED) throw Unsupported(msg);
   TORCH_CHECK(false, msg);
 }
 
@@ -152,10 +155,8 @@ torch::Tensor qk_int8_sv_f16_accum_f16_attn(torch::Tensor query, torch::Tensor k
 
 torch::Tensor prototype_variant(torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                                 int, int, int, float, int, torch::Tensor) {
-  PyErr_SetString(PyExc_NotImplementedError,
-                  "experimental variant of the reference (INT4 Q/K or INT8 P.V) without a working caller; "
-                  "use qk_int8_sv_f16_accum_f16_attn");
-  throw py::error_already_set();
+  throw Unsupported("experimental variant of the reference (INT4 Q/K or INT8 P.V) without a working caller; "
+                    "use qk_int8_sv_f16_accum_f16_attn");
 }
 
 // ---- _fused -----------------------------------------------------------------------------------------
@@ -564,6 +565,13 @@ torch::Tensor attn_sparse_prepacked(const torch::Tensor& q8, const torch::Tensor
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "paroattention's extension modules (_qattn_sm80, _fused, _rope) over libparoatten_hip.so (gfx950)";
+  py::register_local_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const Unsupported& e) {
+      PyErr_SetString(PyExc_NotImplementedError, e.what());
+    }
+  });
   m.def("abi_version", &paro_abi_version);
   auto qattn = m.def_submodule("_qattn_sm80");
   qattn.def("qk_int8_sv_f16_accum_f16_attn", &qk_int8_sv_f16_accum_f16_attn, "QK int8 sv f16 accum f16 attn");

@@ -129,3 +129,23 @@ def test_extension_matches_ctypes_mirrors_bit_for_bit(ext, dev):
     side.synchronize()
     b = _rope.rope_permutation(Q, K, freq, True)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.gpu
+def test_unsupported_combinations_raise_without_the_interpreter_lock(ext, dev):
+    """The package's own entry points run without the interpreter lock: a combination that the library does not have comes
+    back as NotImplementedError from there too, and the call after it works."""
+    import paroatten_amd as P
+    from paroatten_amd import _lib, _qattn_sm80 as qattn, quant as Q
+    N, D = 200, 64
+    q, k, v = (t.to(dev) for t in synth.make_qkv(1, 2, N, D, torch.float16, seed=4))
+    mask = torch.ones(2, 4, 4, dtype=torch.bool, device=dev)
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, None, BLKQ=64, WARPQ=32, BLKK=64)
+    flags = _lib.PARO_ATTN_PV_F16
+    for _ in range(3):
+        with pytest.raises(NotImplementedError, match="per-thread"):
+            ext._ops.attn_operator(q, k, v, mask, 1, False, 3, D ** -0.5, False, False, True, flags)
+        with pytest.raises(NotImplementedError, match="PARO_ATTN_QK_PER_THREAD"):
+            ext._ops.attn_sparse_prepacked(q8, k8, qattn.v_f16_tiles(v), None, None, torch.empty_like(q), qs, ks, D ** -0.5, mask,
+                                           0, False, flags | _lib.PARO_ATTN_QK_PER_THREAD, None, 0, 0, 0, 0)
+    assert torch.isfinite(P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask).float()).all()

@@ -292,9 +292,12 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   auto block_of = [&](int r) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)klist[r * W + wave]); };
   int kb_c = block_of(0), kb_1 = block_of(1), kb_2 = block_of(2);
   if constexpr (K_LDS) {
+    // (issued in this order: the count below leaves in flight what comes after the first tile)
     dma_k(kb_c, 0);
+    __builtin_amdgcn_sched_barrier(0);
     dma_k(kb_1, 1);
     load_v(kb_c, vfrag[0]);
+    __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D / 16 + 2 * DT) : "memory");
     read_k(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -101,7 +101,8 @@ def build(force: bool = True, verbose: bool = False) -> Path:
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + len(DIAG_SOURCES))) as ex:
         objs = list(ex.map(lambda s: _compile(s, verbose), SOURCES + DIAG_SOURCES))
     for lib, members in ((LIB, objs[:len(SOURCES)]), (DIAG_LIB, objs[len(SOURCES):])):
-        cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, members), "-o", str(lib)]
+        # (with its name inside, a copy that is loaded first is also the one that _ext.so binds: _lib.load, PAROATTEN_LIB)
+        cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", f"-Wl,-soname,{lib.name}", *map(str, members), "-o", str(lib)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")

@@ -4,6 +4,9 @@ reference's exception types before anything touches a GPU."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -145,6 +148,22 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         L.load()
     monkeypatch.delenv("PAROATTEN_LIB")
     L.load()
+
+
+def test_chosen_library_is_the_only_one_mapped(tmp_path):
+    """PAROATTEN_LIB chooses the library for the compiled extension's calls too: one copy in the process."""
+    import paroatten_amd._lib as L
+    copy = tmp_path / "elsewhere" / L.LIB_PATH.name
+    copy.parent.mkdir()
+    shutil.copy(L.LIB_PATH, copy)
+    code = ("import paroatten_amd._lib as L; L.ops(); "
+            "print(sorted({l.split()[-1] for l in open('/proc/self/maps') if 'libparoatten_hip' in l}))")
+    for chosen in (copy, L.LIB_PATH):
+        r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PAROATTEN_LIB=str(chosen)), text=True,
+                           capture_output=True, timeout=300, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+        if "_ext.so is not built" in r.stderr:
+            pytest.skip("compiled extension unavailable")
+        assert r.stdout.strip() == str([str(chosen)]), r.stdout + r.stderr
 
 
 def test_mask_generator_contract():

@@ -29,6 +29,7 @@ PARO_ATTN_QK_PER_THREAD = 32
 DTYPE_CODE = {torch.float16: 0, torch.bfloat16: 1}
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libparoatten_hip.so"
+EXT_PATH = Path(__file__).resolve().parent / "_ext.so"
 
 _I, _L, _F, _P = c_int, c_int64, c_float, c_void_p
 
@@ -115,14 +116,19 @@ _ops = None
 
 def ops():
     """The `_ops` submodule of the compiled extension (csrc/torch_binding.cpp -> _ext.so): the package's own entry points
-    with their argument checks, allocations and launches in native code.  Raises ImportError if it is not built."""
+    with their argument checks, allocations and launches in native code; without a built extension (build.py --no-ext) the
+    same calls through ctypes.  Raises ImportError if the extension is there but does not load."""
     global _ops
     if _ops is None:
         load()
+        if not EXT_PATH.exists():
+            from . import _ops as mirror
+            _ops = mirror
+            return _ops
         try:
             from . import _ext
         except ImportError as e:
-            raise ImportError(f"paroatten_amd/_ext.so is not built: run `python paroatten_amd/build.py` ({e})") from e
+            raise ImportError(f"paroatten_amd/_ext.so does not load: run `python paroatten_amd/build.py` ({e})") from e
         _ops = _ext._ops
     return _ops
 

@@ -1,7 +1,9 @@
 """Build libparoatten_hip.so (device code for gfx950 only) with hipcc, and the PyTorch-ROCm C++
 extension paroatten_amd/_ext.so (host code only, binds the library's C ABI) with g++, both in-tree.
 
-    python paroatten_amd/build.py
+    python paroatten_amd/build.py [--no-ext]
+
+(--no-ext: the library alone; the package then makes the same calls through ctypes.)
 
 (run as a script, not with -m: importing the package loads the library, which fails while the
 library is missing or older than the header)

@@ -150,6 +150,20 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     L.load()
 
 
+def test_library_alone_is_a_working_package(monkeypatch, tmp_path):
+    """Without _ext.so the package's calls go through ctypes; with one that does not load they fail loudly."""
+    import paroatten_amd._lib as L
+    from paroatten_amd import _ops
+    monkeypatch.setattr(L, "_ops", None)
+    monkeypatch.setattr(L, "EXT_PATH", tmp_path / "none.so")
+    assert L.ops() is _ops
+    x = torch.zeros(1, 1, 64, 64, dtype=torch.float16)
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
+        L.ops().permute_inverse(x, torch.zeros(1, dtype=torch.int32), 1, 8, 8, 0, None)
+    with pytest.raises(RuntimeError, match="must be on CUDA"):
+        L.ops().attn_operator(x, x, x, torch.ones(1, 1, 1, dtype=torch.bool), 1, False, 2, 0.125, False, False, True, 0)
+
+
 def test_chosen_library_is_the_only_one_mapped(tmp_path):
     """PAROATTEN_LIB chooses the library for the compiled extension's calls too: one copy in the process."""
     import paroatten_amd._lib as L
@@ -161,7 +175,7 @@ def test_chosen_library_is_the_only_one_mapped(tmp_path):
     for chosen in (copy, L.LIB_PATH):
         r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PAROATTEN_LIB=str(chosen)), text=True,
                            capture_output=True, timeout=300, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-        if "_ext.so is not built" in r.stderr:
+        if "_ext.so does not load" in r.stderr:
             pytest.skip("compiled extension unavailable")
         assert r.stdout.strip() == str([str(chosen)]), r.stdout + r.stderr
 

@@ -149,3 +149,40 @@ def test_unsupported_combinations_raise_without_the_interpreter_lock(ext, dev):
             ext._ops.attn_sparse_prepacked(q8, k8, qattn.v_f16_tiles(v), None, None, torch.empty_like(q), qs, ks, D ** -0.5, mask,
                                            0, False, flags | _lib.PARO_ATTN_QK_PER_THREAD, None, 0, 0, 0, 0)
     assert torch.isfinite(P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask).float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,mode", [(64, "smooth"), (128, "lse"), (64, "pv_f16"), (64, "per_thread")])
+def test_operators_through_ctypes_bit_for_bit(ext, dev, monkeypatch, D, mode):
+    """A tree with the library alone runs the same calls through ctypes: the operator, the preparation, prepacked attention and
+    the permutations give the same bytes."""
+    import paroatten_amd as P
+    from paroatten_amd import _lib, _ops, _qattn_sm80 as qattn, permute as PM, rope
+    grid, n_text, H = (3, 5, 7), 23, 6
+    N = n_text + grid[0] * grid[1] * grid[2]
+    nb = (N + 63) // 64
+    q, k, v = (t.to(dev) for t in synth.make_qkv(2, H, N, D, torch.float16, seed=9))
+    mask = synth.make_block_mask(H, nb, 0.6, seed=3, device=dev)
+    orders = torch.arange(6, dtype=torch.int32, device=dev)
+    cos, sin = (rope.rope_table_cog if D == 64 else rope.rope_table_wan_real)(D, grid, device=dev)
+    pv_f16 = mode == "pv_f16"
+    got = []
+    for which in (ext._ops, _ops):
+        monkeypatch.setattr(_lib, "_ops", which)
+        outs = [P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, smooth_k=mode != "pv_f16", return_lse=mode == "lse", pv_f16=pv_f16,
+                                                qk_quant_gran="per_thread" if mode == "per_thread" else "per_warp")]
+        prep = PM.rope_permute_quant(q, k, v, orders, grid, n_text, cos, sin, km="mean" if mode == "smooth" else None)
+        o = torch.zeros(2, N, H, D, dtype=q.dtype, device=dev).transpose(1, 2)
+        v8, sc, mn = (qattn.v_f16_tiles(v), None, None) if pv_f16 else (prep.v8, prep.v_scale, prep.v_mean)
+        outs.append(qattn.attn_sparse_prepacked(prep.q8, prep.k8, v8, sc, mn, o, prep.q_scale, prep.k_scale, D ** -0.5, mask,
+                                                return_lse=int(mode == "lse"), unpermute=(orders, grid, n_text), pv_f16=pv_f16))
+        outs += [o, *prep, PM.rope_permute(q, None, v, orders, grid, n_text, cos, sin), PM.permute_inverse(q, orders, grid, n_text)]
+        got.append(outs)
+
+    def same(a, b):
+        if isinstance(a, (tuple, list)):
+            return len(a) == len(b) and all(same(x, y) for x, y in zip(a, b))
+        return (a is None and b is None) or torch.equal(a, b)
+    assert same(got[0], got[1])
+    with pytest.raises(NotImplementedError):
+        _ops.attn_operator(q, k, v, mask, 1, False, 3, 0.125, False, False, True, _lib.PARO_ATTN_PV_F16)

@@ -56,11 +56,14 @@ template <int D> struct AttnLds {
   }
 };
 
-// Waves per SIMD the register budget is set for: the D = 64 variants fit 168 registers (but for the score dump, and the fast
-// path with the causal diagonal).
+// Waves per SIMD the register budget is set for: the D = 64 variants are built for 168 registers (but for the score dump, and
+// the fast path with the causal diagonal).  The plain launch fits; of the paced one the fast path spills five registers (12
+// with per-thread scales), true exponentials two at most.
 #define PARO_ATTN_WAVES_PER_SIMD ((D == 64 && !DUMP && (!CAUSAL || EXACT)) ? 3 : 2)
 
 // One 64-row q-block `vid` (numbered over batch, head, q-block) by one workgroup of two waves.
+//
+// PACED: called from the paced launch, once per generation.
 //
 // PT: the scales have the reference's per-thread granularity (qk_quant_gran 3, csrc/qattn/
 // qk_int_sv_f16_cuda_sm80.cu:112-116 and :129-133): eight q scales per 32-row group, scale g for the rows
@@ -69,7 +72,7 @@ template <int D> struct AttnLds {
 // 2 (lane % 4) + 1 of every 8-wide tile).  Here a lane holds one q-row, so its q scale is its own, and of its
 // 32 keys per block (offsets 4 lh + i % 4 within every group of 8) the even pair i % 4 < 2 has k scale 2 lh and
 // the odd pair 2 lh + 1: two affine maps from score to exponent per block instead of one.
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED>
 __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) {
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
   using Lds = AttnLds<D>;
@@ -548,7 +551,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     // (fetching the K fragments at the head of the iteration instead, so that they arrive under the VALU
     // phase, measured 2 % slower at D = 128, 7 % with the dense mask)
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (!(D == 64 && EXACT && PT)) read_k_frags(sk1);
+    if constexpr (!(D == 64 && EXACT && (PT || PACED))) read_k_frags(sk1);
     if constexpr (D == 64 && !EXACT) read_v_frags(sv);
     __builtin_amdgcn_sched_barrier(0);
     // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
@@ -569,8 +572,11 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     }
     d_acc = d_new;
     if constexpr (LSE) d_exact += rs;
-    if constexpr (D == 64 && EXACT && PT) read_k_frags(sk1);
-    if constexpr (D == 64 && EXACT) read_v_frags(sv);   // (behind the search: its registers)
+    // (behind the search, whose registers they take.  K too where a generation's bookkeeping or the scales of single threads
+    // need some: in front of it the paced launch spilled up to 60 registers, bf16, causal, exact, H = 16, N = 38400, density
+    // 0.3: 2059 instead of 876 us, N = 102400, H = 8, density 0.1: 3588 instead of 1049; not causal 1967 instead of 1883)
+    if constexpr (D == 64 && EXACT && (PT || PACED)) read_k_frags(sk1);
+    if constexpr (D == 64 && EXACT) read_v_frags(sv);
     __builtin_amdgcn_sched_barrier(0);
 
     // -- matrix phase: S^T of the next block first (the next VALU phase waits for it alone), then this
@@ -673,7 +679,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
   // hardware deals workgroup ids round-robin to the 8 XCDs
   const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
-  attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>(p, vid);
+  attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false>(p, vid);
 }
 
 // The same work with a resident set of workgroups per XCD that take the XCD's q-blocks generation by
@@ -705,7 +711,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
   bool waiting = true;   // a workgroup that has once waited in vain goes on without waiting for the rest of the launch
   for (int base = 0; base < per; base += G) {
     const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
-    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>(p, vid);
+    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true>(p, vid);
     if (base + G >= per) break;
     // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
     __syncthreads();   // also: both waves are done with this q-block's lists in LDS

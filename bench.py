@@ -415,8 +415,8 @@ def main():
             dens[str(d)]["attn_kernel_ms_median"] = round(med, 4)
             dens[str(d)]["attn_kernel_ms_min"] = round(mn, 4)
             # what the default's choices buy, same launch otherwise: exact exponentials instead of the direct
-            # construction of the e4m3 byte; at head size 64 the two-waves-per-q-block kernel instead of the
-            # one-wave one (bit-identical results)
+            # construction of the e4m3 byte; at head size 64 the two-waves-per-q-block kernel instead of what the
+            # library takes there (roofline.kernel)
             t_ex = event_time_ms(lambda: attn_only(masks[d], attn_flags | L.PARO_ATTN_EXACT_EXP), reps, 2)
             dens[str(d)]["attn_kernel_ms_exact_exp"] = round(t_ex, 4)
             if D == 64:
@@ -469,7 +469,9 @@ def main():
     hk = dens[str(HEADLINE_DENSITY)]
     achieved = hk["executed_tops_kernel"]
     roofline = {
-        "kernel": "attn_sparse_w64_kernel" if D == 64 and not args.two_waves and args.pacing != "on" else f"attn_sparse_kernel<{D}>",
+        "kernel": {L.PARO_ATTN_FORM_TWO_WAVES: f"attn_sparse_kernel<{D}>", L.PARO_ATTN_FORM_PACED: f"attn_sparse_paced_kernel<{D}>",
+                   L.PARO_ATTN_FORM_ONE_WAVE: "attn_sparse_w64_kernel", L.PARO_ATTN_FORM_SPLIT: f"attn_sparse_split_kernel<{D}>",
+                   }[lib.paro_attn_kernel_form(B, H, N, N, D, 0, 0, attn_flags)],
         "bound": "mfma",
         "achieved": achieved,
         "peak": PEAK_MFMA_TOPS,

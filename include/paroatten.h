@@ -207,6 +207,16 @@ int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8, const uin
                                    const int32_t* orders, int n_text, int F, int Hh, int W,
                                    void* stream);
 
+/* The form of the attention kernel that a call of these sizes and flags gets: one of PARO_ATTN_FORM_* (host only, no GPU is
+ * needed), or a negative error code.  A measurement names the kernel it timed by this, a test the one it means to run.
+ * PARO_ATTN_FORM_PACED: a launch of a single generation of workgroups is the plain one all the same. */
+#define PARO_ATTN_FORM_TWO_WAVES 0 /* two waves per q-block, plain launch */
+#define PARO_ATTN_FORM_PACED 1     /* the same kernel, paced launch */
+#define PARO_ATTN_FORM_ONE_WAVE 2  /* head size 64: one wave per q-block */
+#define PARO_ATTN_FORM_SPLIT 3     /* several key blocks of a q-block at a time */
+#define PARO_ATTN_FORM_PV_F16 4    /* float16 P.V product */
+int paro_attn_kernel_form(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags);
+
 /* ---------------------------------------------------------------------------------------------
  * (2c) The reference's extension entry point in one call: V (fp16/bf16) -> FP8 tiles, then (2b).
  * Stands in for qk_int8_sv_f16_accum_f16_attn as bound at csrc/qattn/pybind_sm80.cpp:23 /

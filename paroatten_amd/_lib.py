@@ -25,6 +25,11 @@ PARO_ATTN_UNPACED = 4
 PARO_ATTN_TWO_WAVES = 8
 PARO_ATTN_PV_F16 = 16
 PARO_ATTN_QK_PER_THREAD = 32
+PARO_ATTN_FORM_TWO_WAVES = 0
+PARO_ATTN_FORM_PACED = 1
+PARO_ATTN_FORM_ONE_WAVE = 2
+PARO_ATTN_FORM_SPLIT = 3
+PARO_ATTN_FORM_PV_F16 = 4
 
 DTYPE_CODE = {torch.float16: 0, torch.bfloat16: 1}
 
@@ -52,6 +57,7 @@ SIGNATURES = {
                                                _I, _I, _I, _I, _I, _I,
                                                _L, _L, _L, _L, _L, _L, _L, _L, _L, _F, _I, _I,
                                                _P, _I, _I, _I, _I, _P]),
+    "paro_attn_kernel_form": (c_int, [_I, _I, _I, _I, _I, _I, _I, _I]),
     "paro_attn_workspace_bytes": (c_int64, [_I, _I, _I, _I]),
     "paro_attn_workspace_bytes_for": (c_int64, [_I, _I, _I, _I, _I]),
     "paro_v_f16_bytes": (c_int64, [_I, _I, _I, _I]),

@@ -789,12 +789,21 @@ static size_t attn_list_bytes(int nbk, int list_pad, bool per_thread) {
   return (((size_t)(nbk + list_pad + 1) * (per_thread ? 18 : 6) + 15) & ~(size_t)15);
 }
 
+template <int D>
+static size_t attn_smem(int nbk, bool per_thread) {
+  return AttnLds<D>::LIST_OFF + attn_list_bytes(nbk, AttnLds<D>::LIST_PAD, per_thread);
+}
+
+// Per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup, Wan 720p, the
+// paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms.
+static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
+  return !per_thread || (D == 64 ? attn_smem<64>(p.nbk, true) : attn_smem<128>(p.nbk, true)) <= 40 * 1024;
+}
+
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
 static int launch_attn(const AttnParams& p, hipStream_t st) {
-  const size_t smem = AttnLds<D>::LIST_OFF + attn_list_bytes(p.nbk, AttnLds<D>::LIST_PAD, PT);
-  // (per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup,
-  // Wan 720p, the paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms)
-  if (!DUMP && want_pacing(p, D, CAUSAL) && (!PT || smem <= 40 * 1024)) {
+  const size_t smem = attn_smem<D>(p.nbk, PT);
+  if (!DUMP && want_pacing(p, D, CAUSAL) && pace_list_fits(p, D, PT)) {
     auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>;
     if (smem > 48 * 1024)
       PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
@@ -877,6 +886,20 @@ static bool two_waves_fill_better(const AttnParams& p, bool causal, bool exact) 
   return p.nbk <= 340 && (p.total <= 1536 || (p.total > 2048 && p.total <= 3072));
 }
 
+// The kernel that a call gets (PARO_ATTN_FORM_*).
+static int attn_form(const AttnParams& p, int D, bool causal, bool exact, bool dump, int flags) {
+  if (flags & PARO_ATTN_PV_F16) return PARO_ATTN_FORM_PV_F16;   // a kernel of its own (true exponentials, plain launch)
+  const bool per_thread = (flags & PARO_ATTN_QK_PER_THREAD) != 0, paced = !dump && want_pacing(p, D, causal);
+  if (!per_thread && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0) {
+    // too few q-blocks to fill the card: several kept blocks of each at a time (attn_sparse_split.hip)
+    if (p.pacing == 0 && split_width(p, D) != 0) return PARO_ATTN_FORM_SPLIT;
+    // D = 64: one wave per q-block (attn_sparse_w64.hip), unless the launch is to be paced (only the two-wave kernel has
+    // the paced form) or two waves fill the card better
+    if (D == 64 && !paced && !two_waves_fill_better(p, causal, exact || p.lse != nullptr)) return PARO_ATTN_FORM_ONE_WAVE;
+  }
+  return paced && pace_list_fits(p, D, per_thread) ? PARO_ATTN_FORM_PACED : PARO_ATTN_FORM_TWO_WAVES;
+}
+
 }  // namespace paro
 
 namespace paro {
@@ -943,7 +966,6 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   hipStream_t st = (hipStream_t)stream;
   const bool dump = s_dump != nullptr;
   const bool exact = (flags & PARO_ATTN_EXACT_EXP) != 0;
-  // float16 P.V product: a kernel of its own (true exponentials, plain launch)
   if (pv16) return launch_attn_pv16(p, D, out_dtype, is_causal != 0, st);
   if (per_thread) {
     if (D == 64)
@@ -952,14 +974,11 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
     return out_dtype == PARO_DTYPE_F16 ? dispatch_attn_per_thread<128, PARO_DTYPE_F16>(p, is_causal, exact, st)
                                        : dispatch_attn_per_thread<128, PARO_DTYPE_BF16>(p, is_causal, exact, st);
   }
-  // too few q-blocks to fill the card: several kept blocks of each at a time (attn_sparse_split.hip)
-  if (!dump && p.pacing == 0 && (flags & PARO_ATTN_TWO_WAVES) == 0 && split_width(p, D) != 0)
-    return launch_attn_split(p, D, out_dtype, is_causal != 0, exact, st);
-  // D = 64 without score dump: one wave per q-block (attn_sparse_w64.hip), unless the caller asks for the two-wave
-  // kernel, the launch is to be paced (only the two-wave kernel has the paced form), or two waves fill the card better
-  if (D == 64 && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0 && !want_pacing(p, D, is_causal != 0) &&
-      !two_waves_fill_better(p, is_causal != 0, exact || lse != nullptr))
-    return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
+  switch (attn_form(p, D, is_causal != 0, exact, dump, flags)) {
+    case PARO_ATTN_FORM_SPLIT: return launch_attn_split(p, D, out_dtype, is_causal != 0, exact, st);
+    case PARO_ATTN_FORM_ONE_WAVE: return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
+    default: break;   // two waves per q-block, below; launch_attn chooses plain or paced
+  }
   if (D == 64) {
     if (out_dtype == PARO_DTYPE_F16) return dispatch_attn<64, PARO_DTYPE_F16>(p, is_causal, dump, exact, st);
     return dispatch_attn<64, PARO_DTYPE_BF16>(p, is_causal, dump, exact, st);
@@ -968,6 +987,22 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   return dispatch_attn<128, PARO_DTYPE_BF16>(p, is_causal, dump, exact, st);
 }
 }  // namespace paro
+
+extern "C" int paro_attn_kernel_form(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags) {
+  using namespace paro;
+  PARO_CHECK(B > 0 && H > 0 && Nq > 0 && Nk > 0, PARO_ERR_RUNTIME, "paro_attn_kernel_form: empty shape");
+  PARO_CHECK(D == 64 || D == 128, PARO_ERR_INVALID_VALUE, "Unsupported head dim: %d", D);
+  PARO_CHECK((flags & (PARO_ATTN_PACED | PARO_ATTN_UNPACED)) != (PARO_ATTN_PACED | PARO_ATTN_UNPACED), PARO_ERR_INVALID_VALUE,
+             "Unsupported attention flags: %d", flags);
+  float lse = 0.f;
+  AttnParams p = {};
+  p.nbq = ceil_div(Nq, 64); p.nbk = ceil_div(Nk, 64);
+  PARO_CHECK((int64_t)B * H * p.nbq < (int64_t)1 << 31, PARO_ERR_RUNTIME, "paro_attn_kernel_form: too many q-blocks");
+  p.total = B * H * p.nbq;
+  p.lse = with_lse ? &lse : nullptr;
+  p.pacing = (flags & PARO_ATTN_PACED) ? 1 : ((flags & PARO_ATTN_UNPACED) ? -1 : 0);
+  return attn_form(p, D, is_causal != 0, (flags & PARO_ATTN_EXACT_EXP) != 0, false, flags);
+}
 
 extern "C" int paro_attn_sparse_fwd(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale,
                                     const float* k_scale, const float* v_scale, const float* v_mean,

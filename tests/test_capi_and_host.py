@@ -68,6 +68,31 @@ def test_size_queries_need_no_gpu():
     assert ws >= lib.paro_v_fp8_bytes(2, 48, 17776, 64) and ws % 256 == 0
 
 
+def test_kernel_form_query_needs_no_gpu(monkeypatch):
+    """which attention kernel a call gets, by head size, number of q-blocks and key blocks, and flags"""
+    import paroatten_amd._lib as L
+    monkeypatch.delenv("PARO_ATTN_PACING", raising=False)
+    form = L.load().paro_attn_kernel_form
+    assert form(1, 2, 4096, 4096, 64, 0, 0, 0) == L.PARO_ATTN_FORM_SPLIT
+    assert form(1, 2, 4096, 4096, 64, 0, 0, L.PARO_ATTN_TWO_WAVES) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(1, 2, 4096, 4096, 64, 0, 0, L.PARO_ATTN_UNPACED) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(1, 8, 4096, 4096, 64, 0, 1, 0) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(2, 48, 17776, 17776, 64, 0, 0, 0) == L.PARO_ATTN_FORM_ONE_WAVE
+    assert form(2, 48, 17776, 17776, 64, 0, 0, L.PARO_ATTN_PACED) == L.PARO_ATTN_FORM_PACED
+    assert form(2, 48, 17776, 17776, 64, 0, 0, L.PARO_ATTN_PV_F16) == L.PARO_ATTN_FORM_PV_F16
+    assert form(1, 40, 17776, 17776, 128, 0, 0, 0) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(1, 40, 75600, 75600, 128, 0, 0, 0) == L.PARO_ATTN_FORM_PACED
+    assert form(1, 40, 75600, 75600, 128, 0, 0, L.PARO_ATTN_UNPACED) == L.PARO_ATTN_FORM_TWO_WAVES
+    for flags in (0, L.PARO_ATTN_PACED):   # per-thread scales: the list of 1182 key blocks is too long to pace
+        assert form(1, 40, 75600, 75600, 128, 0, 0, flags | L.PARO_ATTN_QK_PER_THREAD) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(1, 40, 16384, 16384, 128, 0, 0, L.PARO_ATTN_PACED | L.PARO_ATTN_QK_PER_THREAD) == L.PARO_ATTN_FORM_PACED
+    monkeypatch.setenv("PARO_ATTN_PACING", "0")
+    assert form(1, 40, 75600, 75600, 128, 0, 0, 0) == L.PARO_ATTN_FORM_TWO_WAVES
+    assert form(1, 40, 75600, 75600, 96, 0, 0, 0) == L.PARO_ERR_INVALID_VALUE
+    assert form(1, 0, 64, 64, 64, 0, 0, 0) == L.PARO_ERR_RUNTIME
+    assert form(1, 1, 64, 64, 64, 0, 0, L.PARO_ATTN_PACED | L.PARO_ATTN_UNPACED) == L.PARO_ERR_INVALID_VALUE
+
+
 def test_c_abi_argument_errors_without_gpu():
     """argument validation happens before any launch: codes and messages come back on CPU"""
     import paroatten_amd._lib as L

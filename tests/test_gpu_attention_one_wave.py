@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from oracle import paro_oracle as O
+from paroatten_amd import _lib as L
 from paroatten_amd import _qattn_sm80 as qattn
 from paroatten_amd import permute as PM
 
@@ -17,6 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("B,H", [(1, 448), (1, 451)])
 def test_one_wave_equals_two_waves(dev, mode, causal, B, H):
     N, D, nb = 64 * 11 - 21, 64, 11
+    assert L.load().paro_attn_kernel_form(B, H, N, N, D, int(causal), int(mode == "lse"),
+                                          L.PARO_ATTN_EXACT_EXP if mode == "exact" else 0) == L.PARO_ATTN_FORM_ONE_WAVE
     g = torch.Generator().manual_seed(17)
     q, k, v = (torch.randn(B, H, N, D, generator=g) for _ in range(3))
     k[:, 1::2] *= torch.linspace(0.1, 4.0, N)[:, None]       # the maxima of these heads grow along the row

@@ -377,6 +377,38 @@ def test_paced_launch_is_bit_identical(dev, D, H, N, monkeypatch):
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", ["fast", "exact", "lse"])
+def test_paced_launch_takes_every_causal_q_block_once(dev, D, mode):
+    """Causal q-blocks are renumbered (the longest of a head first, the heads that do not come out even dealt out one q-block
+    at a time, slots past the end).  89 heads of 41 q-blocks: one head left over, 457 slots an XCD, several generations
+    of at most 192 workgroups, and slots past the end.  Outputs start as NaN: a q-block left out stays NaN."""
+    from paroatten_amd import _lib as L
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    B, H, N = 1, 89, 64 * 41 - 9
+    nb = (N + 63) // 64
+    flags = L.PARO_ATTN_EXACT_EXP if mode == "exact" else 0
+    assert L.load().paro_attn_kernel_form(B, H, N, N, D, 1, int(mode == "lse"), flags | L.PARO_ATTN_PACED) == L.PARO_ATTN_FORM_PACED
+    q, k, v = synth.make_qkv_device(B, H, N, D, torch.bfloat16, seed=15, device=dev)
+    g = torch.Generator().manual_seed(16)
+    mask = torch.rand(H, nb, nb, generator=g) < 0.4
+    mask[5, 7] = False
+    mask = mask.to(dev)
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, None, BLKQ=64, WARPQ=32, BLKK=64)
+    v8, vsc, vm = Q.per_channel_fp8(v)
+    outs = []
+    for pacing in (False, True):
+        out = torch.full_like(q, float("nan"))
+        lse = qattn.attn_sparse_prepacked(q8, k8, v8, vsc, vm, out, qs, ks, D ** -0.5, mask, is_causal=1, exact_exp=mode == "exact",
+                                          return_lse=int(mode == "lse"), pacing=pacing)
+        outs.append((out.cpu(), lse.cpu() if mode == "lse" else torch.zeros(0)))
+    assert torch.isfinite(outs[0][0].float()).all()
+    assert torch.count_nonzero(outs[0][0][0, 5, 7 * 64:8 * 64]) == 0
+    assert torch.equal(outs[0][0].view(torch.int16), outs[1][0].view(torch.int16))
+    assert torch.equal(outs[0][1], outs[1][1])
+
+
 def test_paced_launches_that_overlap_on_two_streams(dev):
     """Two paced launches in flight at once on one GPU (two streams, as a caller that runs the two halves of a
     classifier-free-guidance batch side by side would have them): each takes its own set of the library's pacing

@@ -180,3 +180,17 @@ def test_flag_is_checked(dev):
     with pytest.raises(RuntimeError):
         qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, vd, torch.empty_like(qd), qs, ks, 1, 0, 2, D ** -0.5, 0, md,
                                             pv_f16=True, workspace=small)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_weights_are_normalised_by_their_own_sum(dev, D):
+    """The row sums are those of the float16 weights that the product uses: where V is the same for every key, the output is
+    V itself, whatever the rounding of the weights (sums of unrounded weights leave up to 2^-12 of it)."""
+    import paroatten_amd as P
+    B, H, N = 1, 4, 1000
+    q, k, v, mask = _case(B, H, N, D, torch.float16, seed=91)
+    v = torch.randn(B, H, 1, D, generator=torch.Generator().manual_seed(92)).half().expand(B, H, N, D).contiguous()
+    out = P.paroattn_qk_int8_pv_fp16_cuda((3 * q).to(dev), k.to(dev), v.to(dev), mask.to(dev), pv_f16=True).cpu()
+    # what is left is fp32: two sums of up to 1000 terms and a division, below 1000 * 2^-23 = 2^-13 of the value in the worst
+    # case and far below it with rounding to nearest; V is a float16 number, at least 2^-12 from where rounding would change
+    assert torch.equal(out, v)

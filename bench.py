@@ -277,7 +277,7 @@ def main():
                          "under the kernel from what its instruction mix costs.  Not a benchmark result.")
     ap.add_argument("--pacing", choices=["auto", "on", "off"], default="auto",
                     help="attention launch: generation-paced resident workgroups (on), the plain launch (off), or the "
-                         "library's own choice (auto: paced when one head's K8+V8 exceed 7 MB, D = 64: 12 MB)")
+                         "library's own choice (auto: paced when one head's K8+V8 exceed 7 MB, D = 64: 14 MB)")
     ap.add_argument("--mfma-ceiling", action="store_true",
                     help="only time back-to-back MFMAs (int8 and fp8, random and zero operands): what the matrix pipe "
                          "sustains on this box, the ceiling of any kernel built on it.  Prints its own JSON line.")

@@ -43,12 +43,14 @@ extern "C" {
                                  XCD takes the q-blocks generation by generation, so that workgroups running
                                  together walk the key sequence together and share K8 / V8 tiles in the XCD's L2 */
 #define PARO_ATTN_UNPACED 4   /* one workgroup per q-block, started as the hardware pleases.  With neither flag the
-                                 library paces when one head's K8 + V8 exceed 7 MB at head size 128 (causal 16 MB) or
-                                 12 MB at 64 (environment variable PARO_ATTN_PACING=0/1 overrides that default).  Scattered masks on long sequences gain
-                                 (Wan 720p, uniformly random blocks: 26 -> 39 % of the MFMA peak, 4x fewer L2 fills);
-                                 masks made of one contiguous run per row lose a few per cent.  A generation waits for
-                                 all but a share of its workgroups (PARO_ATTN_PACE_SLACK; default half the L2's share
-                                 of a head, at most a quarter of them) and at most PARO_ATTN_PACE_SPINS rounds. */
+                                 library paces when one head's K8 + V8 exceed 7 MB at head size 128 (causal 20 MB) or
+                                 14 MB at 64 (with true exponentials 40 MB, causal 64 MB), and never with per-thread
+                                 scales (environment variable PARO_ATTN_PACING=0/1 overrides that default).
+                                 Scattered masks on long sequences gain (Wan 720p, uniformly random blocks: 26 -> 39 %
+                                 of the MFMA peak, 4x fewer L2 fills); masks made of one contiguous run per row lose, a
+                                 few per cent at head size 128, up to 15 % at 64.  A generation waits for all but a
+                                 share of its workgroups (PARO_ATTN_PACE_SLACK; default half the L2's share of a head, at
+                                 most a quarter of them) and at most PARO_ATTN_PACE_SPINS rounds. */
 #define PARO_ATTN_TWO_WAVES 8 /* kernel form: two waves per 64-row q-block (32 q-rows each) also where the
                                  library would pick one wave per q-block (head size 64, plain launch, more than
                                  1024 q-blocks; bit-identical results) or several key blocks of a q-block at a

@@ -770,18 +770,29 @@ static int pace_device(PaceDevice* out) {
 // head's K8 + V8 exceed what the plain launch still gets out of the 4 MB L2 of an XCD and the memory-side cache.  A layer
 // (preparation included) with rotary embedding at density 0.3, paced / plain, scattered masks: D = 128, 4.5 MB 893 / 820 us,
 // 5 MB 1061 / 979, 6 MB 1403 / 1362, 6.9 MB 1803 / 1782, 8 MB 3744 / 3903 (40 heads), 18 MB 13131 / 18596; rows of one run,
-// 6.9 MB 1798 / 1689.  D = 64, where plain means the one-wave kernel: 4.6 MB 1915 / 1628, 6.9 MB 2638 / 2430, 8.8 MB 3049 /
-// 3099, 12.3 MB 4503 / 4434, runs 4476 / 3635.  Causal q-blocks differ in length, and a generation lasts as long as its
-// longest: D = 128, density 0.2, the kernel alone, 8 MB 797 / 704, 11 MB 734 / 665, 18 MB 1864 / 1849, density 0.5 there
-// 4238 / 4282.
+// 6.9 MB 1798 / 1689.  D = 64, where plain means the one-wave kernel: 4.6 MB 1915 / 1628, 6.9 MB 2638 / 2430.  The lines
+// further out are from attention and V conversion alone, scattered masks of density 0.2, 8 or 16 heads, paced / plain:
+//   D = 64      12 MB 2851 / 2740, 13 MB 3351 / 3369 (density 0.1 3689 / 3449, 0.3 9591 / 9845), 14 MB 3862 / 4015 (0.1 4185 /
+//               4110, 0.3 10948 / 11748), 16 MB 4957 / 5366, 24 MB 12745 / 13285; rows of one run 16 MB 4861 / 4422, 24 MB
+//               12319 / 10786, which no size makes up for.  Causal the same: 12 MB 2866 / 2562, 14 MB 3734 / 3772, 16 MB 4728 /
+//               4914, 24 MB 5646 / 6103.
+//   D = 64, true exponentials (the two-wave kernel has no third wave per SIMD to give there)
+//               12.5 MB 6860 / 5570, 24 MB 20702 / 15958, log-sum-exp 22553 / 17723; density 0.1, 40 MB 16641 / 12178 and 17678 /
+//               13896; 48 MB, where the lists leave a compute unit three one-wave workgroups, 23967 / 23596 and 25432 / 27011;
+//               64 MB 42163 / 41634 and 44865 / 47700.  Causal 12.5 MB 3580 / 2869, 48 MB 12424 / 9597, 64 MB 21767 / 16924.
+//   D = 128, causal: q-blocks differ in length, and a generation lasts as long as its longest.  8 MB 797 / 704, 11 MB 734 / 665,
+//               16 MB 1157 / 1023, 17 MB 2517 / 2289 (density 0.5 5367 / 5179, 1 10476 / 10046), 18.5 MB, 40 heads, 6853 / 6785
+//               (15130 / 15216), 24 MB 4939 / 5041 (11054 / 11344, 21249 / 21122), 32 MB 8444 / 9624 (19556 / 22061).
 // PARO_ATTN_PACE_SPINS: rounds (about 1 us each) a workgroup
 // waits for its generation at most (default: half the number of key blocks, between 64 and 4096).
 // PARO_ATTN_PACE_SLACK: how many of an XCD's resident workgroups a generation does not wait for (default: half
 // the share of the head's K8 + V8 that the L2 holds, at most a quarter of them).
-static bool want_pacing(const AttnParams& p, int D, bool causal) {
+// exact: true exponentials, also those of a log-sum-exp.
+static bool want_pacing(const AttnParams& p, int D, bool causal, bool exact) {
   if (p.pacing != 0) return p.pacing > 0;
   if (const char* e = getenv("PARO_ATTN_PACING")) return e[0] == '1';
-  return (int64_t)p.nbk * 64 * D * 2 > (int64_t)(D == 64 ? 12 : causal ? 16 : 7) << 20;
+  const int line = D == 64 ? (!exact ? 14 : causal ? 64 : 40) : causal ? 20 : 7;   // MB
+  return (int64_t)p.nbk * 64 * D * 2 > (int64_t)line << 20;
 }
 
 // bytes of the kept-block list in LDS: per key block a 16-bit index and its k scale (four with per-thread scales)
@@ -795,7 +806,11 @@ static size_t attn_smem(int nbk, bool per_thread) {
 }
 
 // Per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup, Wan 720p, the
-// paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms.
+// paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms.  The lists that fit, up to 446 key
+// blocks at D = 128 and 872 at 64, end where the lines above begin, so only PARO_ATTN_PACED paces such a call.  Below, the plain
+// launch is the faster one throughout, paced / plain at density 0.3: D = 128, 40 heads, 4 MB 1244 / 1019 us, 5.3 MB 1813 / 1616,
+// 7 MB 2880 / 2689, rows of one run 2852 / 2622, log-sum-exp at 6 MB 2681 / 2588, causal 1350 / 1125; D = 64, 32 heads, 4.1 MB
+// 2134 / 1742, 6.8 MB 5579 / 5132, log-sum-exp 8949 / 7788.
 static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
   return !per_thread || (D == 64 ? attn_smem<64>(p.nbk, true) : attn_smem<128>(p.nbk, true)) <= 40 * 1024;
 }
@@ -803,7 +818,7 @@ static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
 static int launch_attn(const AttnParams& p, hipStream_t st) {
   const size_t smem = attn_smem<D>(p.nbk, PT);
-  if (!DUMP && want_pacing(p, D, CAUSAL) && pace_list_fits(p, D, PT)) {
+  if (!DUMP && want_pacing(p, D, CAUSAL, EXACT) && pace_list_fits(p, D, PT)) {
     auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>;
     if (smem > 48 * 1024)
       PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
@@ -889,13 +904,14 @@ static bool two_waves_fill_better(const AttnParams& p, bool causal, bool exact) 
 // The kernel that a call gets (PARO_ATTN_FORM_*).
 static int attn_form(const AttnParams& p, int D, bool causal, bool exact, bool dump, int flags) {
   if (flags & PARO_ATTN_PV_F16) return PARO_ATTN_FORM_PV_F16;   // a kernel of its own (true exponentials, plain launch)
-  const bool per_thread = (flags & PARO_ATTN_QK_PER_THREAD) != 0, paced = !dump && want_pacing(p, D, causal);
+  exact = exact || p.lse != nullptr;
+  const bool per_thread = (flags & PARO_ATTN_QK_PER_THREAD) != 0, paced = !dump && want_pacing(p, D, causal, exact);
   if (!per_thread && !dump && (flags & PARO_ATTN_TWO_WAVES) == 0) {
     // too few q-blocks to fill the card: several kept blocks of each at a time (attn_sparse_split.hip)
     if (p.pacing == 0 && split_width(p, D) != 0) return PARO_ATTN_FORM_SPLIT;
     // D = 64: one wave per q-block (attn_sparse_w64.hip), unless the launch is to be paced (only the two-wave kernel has
     // the paced form) or two waves fill the card better
-    if (D == 64 && !paced && !two_waves_fill_better(p, causal, exact || p.lse != nullptr)) return PARO_ATTN_FORM_ONE_WAVE;
+    if (D == 64 && !paced && !two_waves_fill_better(p, causal, exact)) return PARO_ATTN_FORM_ONE_WAVE;
   }
   return paced && pace_list_fits(p, D, per_thread) ? PARO_ATTN_FORM_PACED : PARO_ATTN_FORM_TWO_WAVES;
 }

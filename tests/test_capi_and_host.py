@@ -86,6 +86,12 @@ def test_kernel_form_query_needs_no_gpu(monkeypatch):
     for flags in (0, L.PARO_ATTN_PACED):   # per-thread scales: the list of 1182 key blocks is too long to pace
         assert form(1, 40, 75600, 75600, 128, 0, 0, flags | L.PARO_ATTN_QK_PER_THREAD) == L.PARO_ATTN_FORM_TWO_WAVES
     assert form(1, 40, 16384, 16384, 128, 0, 0, L.PARO_ATTN_PACED | L.PARO_ATTN_QK_PER_THREAD) == L.PARO_ATTN_FORM_PACED
+    # what a head's K8 + V8 have to exceed for the paced launch, in MB: the key blocks at the line and one more
+    for D, causal, lse, flags, mb in ((128, 0, 0, 0, 7), (128, 0, 1, 0, 7), (128, 1, 0, 0, 20), (64, 0, 0, 0, 14), (64, 1, 0, 0, 14),
+                                      (64, 0, 1, 0, 40), (64, 0, 0, L.PARO_ATTN_EXACT_EXP, 40), (64, 1, 1, 0, 64)):
+        n = mb * 2 ** 20 // (2 * D)
+        assert form(1, 40, n, n, D, causal, lse, flags) != L.PARO_ATTN_FORM_PACED, (D, causal, lse, flags)
+        assert form(1, 40, n + 1, n + 1, D, causal, lse, flags) == L.PARO_ATTN_FORM_PACED, (D, causal, lse, flags)
     monkeypatch.setenv("PARO_ATTN_PACING", "0")
     assert form(1, 40, 75600, 75600, 128, 0, 0, 0) == L.PARO_ATTN_FORM_TWO_WAVES
     assert form(1, 40, 75600, 75600, 96, 0, 0, 0) == L.PARO_ERR_INVALID_VALUE

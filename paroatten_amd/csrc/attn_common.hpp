@@ -1,5 +1,6 @@
-// Shared by the two attention kernels of this library (attn_sparse.hip: two waves per 64-row q-block, any head
-// size and variant; attn_sparse_w64.hip: one wave per q-block, D = 64): launch parameters, the constants of the
+// Shared by the attention kernels of this library (attn_sparse.hip: two waves per 64-row q-block, any head
+// size and variant; attn_sparse_w64.hip: one wave per q-block, D = 64; attn_sparse_split.hip: several kept blocks of a
+// q-block at a time; attn_sparse_pv16.hip: float16 P.V product): launch parameters, the constants of the
 // softmax-weight arithmetic and small device helpers.  gfx950 only.
 #pragma once
 #include "paro_device.hpp"

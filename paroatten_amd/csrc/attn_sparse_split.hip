@@ -455,8 +455,15 @@ static int launch_split(const AttnParams& p, bool causal, bool exact, hipStream_
 //   D = 128   W = 4                         17.9   18.3   32.2   33.7   46.2
 //             W = 2                                22.7   24.5   25.6   40.4
 //             two waves                            29.0          31.7   32
-// i.e. W such that every workgroup of four waves, or two of two waves, has a compute unit.  Lists of sixteen blocks gain
-// 1 us of 9 (shorter ones nothing): the walk is a few rounds then, and below twenty it stays with the other kernels.
+// i.e. W such that every workgroup of four waves, or two of two waves, has a compute unit.  What gains is the length of the
+// lists, of which the host knows only the bound, the number of key blocks.  This / two waves per q-block, us, by the
+// share of the blocks that is kept (two heads of 64, one to twelve of 20 key blocks):   0.05        0.1         0.2         0.5
+//   D = 64    64 key blocks                        8.7/8.9   9.6/11.0    11.0/13.6   14.3/21.1
+//             20 key blocks, lists of 2 to 10      7.9/7.4   8.6/8.0      8.7/8.6     9.7/11.3
+//   D = 128   64 key blocks                       12.0/14.0 13.3/16.7    15.5/20.4   21.0/30.8
+//             20 key blocks                       10.8/11.5 11.0/12.1    12.0/13.7   13.7/17.6
+// so at D = 64 lists of two or three blocks lose 0.5 to 0.8 us and those from four on gain, and below twenty key blocks it
+// stays with the other kernels.
 int split_width(const AttnParams& p, int D) {
   if (p.nbk < 20 || p.total > 256) return 0;
   const int W = p.total <= 128 ? 4 : 2;

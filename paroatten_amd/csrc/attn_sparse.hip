@@ -780,6 +780,9 @@ static int pace_device(PaceDevice* out) {
 //               12.5 MB 6860 / 5570, 24 MB 20702 / 15958, log-sum-exp 22553 / 17723; density 0.1, 40 MB 16641 / 12178 and 17678 /
 //               13896; 48 MB, where the lists leave a compute unit three one-wave workgroups, 23967 / 23596 and 25432 / 27011;
 //               64 MB 42163 / 41634 and 44865 / 47700.  Causal 12.5 MB 3580 / 2869, 48 MB 12424 / 9597, 64 MB 21767 / 16924.
+//   D = 128, 40 heads, density 0.3: 7.2 MB 2976 / 2943, 8 MB 3573 / 3647, 9 MB 4412 / 4732, 10 MB 5365 / 6146; the log-sum-exp 7.2 MB
+//               3742 / 3748, 9 MB 5657 / 5895; true exponentials without it gain least, 7.2 MB 3568 / 3429, 9 MB 5445 / 5434, 10 MB
+//               6660 / 6730, 18.5 MB, 16 heads, 9196 / 10724: 3 to 4 % between 7 and 9 MB, not worth a line of their own.
 //   D = 128, causal: q-blocks differ in length, and a generation lasts as long as its longest.  8 MB 797 / 704, 11 MB 734 / 665,
 //               16 MB 1157 / 1023, 17 MB 2517 / 2289 (density 0.5 5367 / 5179, 1 10476 / 10046), 18.5 MB, 40 heads, 6853 / 6785
 //               (15130 / 15216), 24 MB 4939 / 5041 (11054 / 11344, 21249 / 21122), 32 MB 8444 / 9624 (19556 / 22061).

@@ -18,9 +18,9 @@ struct AttnParams {
   const float* v_mean;
   const uint8_t* sparse;
   void* out;
-  float* lse;            // what is stored: base-2 log-sum-exp * lse_scale (+ lse_add[row], if given)
+  float* lse;            // what is stored: base-2 log-sum-exp * lse_scale (+ what the row holds before, with lse_add)
   float lse_scale;
-  const float* lse_add;
+  int lse_add;
   int32_t* s_dump;
   int64_t sparse_bs;
   int64_t qs_b, qs_h, qs_n;
@@ -34,6 +34,12 @@ struct AttnParams {
   const int* orders;
   int n_text, F, Hh, W;
   int pacing;  // +1: paced launch asked for, -1: plain launch asked for, 0: the library chooses
+  // Q as the 16-bit tensor (of the output's type; qs_* are its strides, q8 and q_scale are not read): the kernels quantise
+  // the rows of their q-block themselves (QRows).  k_mean [B,Hkv,D] (may be null; with lse): the mean that has been taken
+  // off K, the row's log-sum-exp gets lse_dot_scale * q . k_mean
+  const unsigned short* q16;
+  const unsigned short* k_mean;
+  float lse_dot_scale;
 };
 
 // P~ = 2^(S*c - m + P_EXP_OFFSET).  m is the running row maximum, refreshed lazily: only when a
@@ -67,7 +73,7 @@ __device__ __forceinline__ int qblock_of(const AttnParams& p, int xcd, int slot,
 }
 
 __device__ __forceinline__ void store_lse(const AttnParams& p, int64_t row, float lse2) {
-  p.lse[row] = p.lse_add != nullptr ? fmaf(lse2, p.lse_scale, p.lse_add[row]) : lse2 * p.lse_scale;
+  p.lse[row] = p.lse_add ? fmaf(lse2, p.lse_scale, p.lse[row]) : lse2 * p.lse_scale;
 }
 
 __device__ __forceinline__ float max3(float a, float b, float c) {
@@ -75,6 +81,70 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+
+__device__ __forceinline__ float max3_abs(float a, float b, float c) {   // max(|a|, |b|, c)
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// The 32 q-rows of one wave (or half of one), from 16 bits: INT8 codes in the B operand's order, and their scale.  Lane: row
+// lane % 32, channels 32 ks + 16 (lane / 32) .. + 15 of k-step ks.  Codes and scale are those of quant_group_body, to the
+// bit (rows past the end repeat the last one, which leaves the maximum as it is; their results are never stored).
+// A pass of its own for Q (3 bytes per element, and a fourth to read the codes back) is bound by HBM, the attention
+// kernel is not.
+template <int DT, int D>
+struct QRows {
+  v4i raw[D / 16];
+  // p: the row's first channel, plus 16 (lane / 32).  (Ordinary loads: a line of memory is fetched in pieces by two to four
+  // of them; with non-temporal ones the operator lost 1 to 2 %)
+  __device__ __forceinline__ void load(const unsigned short* p) {
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ks++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+        raw[2 * ks + i] = *reinterpret_cast<const v4i*>(p + 32 * ks + 8 * i);
+  }
+  // the codes; returns the scale (the same in every lane)
+  __device__ __forceinline__ float quantise(v4i (&qf)[D / 32]) const {
+    float amax = 0.0000001f;
+#pragma unroll
+    for (int c = 0; c < D / 16; c++)
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) amax = max3_abs(elem16_to_f32<DT>(raw[c], j), elem16_to_f32<DT>(raw[c], j + 1), amax);
+    amax = wave_max(amax);
+    const float inv = 127.0f / amax;
+#pragma unroll
+    for (int c = 0; c < D / 16; c++) {
+      float y[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) y[j] = elem16_to_f32<DT>(raw[c], j) * inv;
+      qf[c >> 1][2 * (c & 1)] = (int)pack4_rint_i8(y[0], y[1], y[2], y[3]);
+      qf[c >> 1][2 * (c & 1) + 1] = (int)pack4_rint_i8(y[4], y[5], y[6], y[7]);
+    }
+    return amax / 127.0f;
+  }
+  // the row's product with w[0..D) (w: plus 16 (lane / 32)), in the order of quant_group_body
+  __device__ __forceinline__ float dot(const unsigned short* w) const {
+    float t[D / 32];
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ks++) {
+      float d[2];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const v4i wr = *reinterpret_cast<const v4i*>(w + 32 * ks + 8 * i);
+        d[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) d[i] = fmaf(elem16_to_f32<DT>(raw[2 * ks + i], j), elem16_to_f32<DT>(wr, j), d[i]);
+      }
+      float a, b;
+      with_lane_xor32(d[0] + d[1], a, b);
+      t[ks] = a + b;
+    }
+    if constexpr (D == 64) return t[0] + t[1];
+    else return (t[0] + t[1]) + (t[2] + t[3]);
+  }
+};
 
 // two floats -> two e4m3 bytes in the low (HI = false) or high half of a word; the other half of the
 // destination is left as it is, so a full word takes one call of each kind
@@ -147,10 +217,20 @@ int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hip
 int split_width(const AttnParams& p, int D);
 int launch_attn_split(const AttnParams& p, int D, int out_dtype, bool causal, bool exact, hipStream_t st);
 
-// paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip) with the two values that go into a stored log-sum-exp.
+// Q from 16 bits, and what goes into a stored log-sum-exp (AttnParams says what they are)
+struct AttnExtra {
+  float lse_scale = 1.0f;
+  bool lse_add = false;
+  const unsigned short* q16 = nullptr;
+  const unsigned short* k_mean = nullptr;
+  float lse_dot_scale = 0.f;
+};
+
+// paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip).  extra.q16: q8 and q_scale are not read, the q strides are those of
+// the 16-bit tensor, which is of the type out_dtype.
 int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
                      const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
-                     void* out, int out_dtype, float* lse, float lse_scale, const float* lse_add, int32_t* s_dump, int B,
+                     void* out, int out_dtype, float* lse, const AttnExtra& extra, int32_t* s_dump, int B,
                      int H, int Hkv, int Nq, int Nk, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
                      int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
                      int64_t o_stride_n, float sm_scale, int is_causal, int flags, const int32_t* orders, int n_text, int F,

@@ -143,14 +143,20 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   // ---- Q fragments (B operand: column = q-row, 16 channels per lane and k-step) -----------
   const int qrow = qb * 64 + wave * 32 + l32;
   v4i qf[KS];
+  float qsc = 0.f;
+  QRows<OUT_DT, D> q16;
   {
     // rows past the end re-read the last row; their results are never stored
-    const int8_t* qp = p.q8 + b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave;
+    if (!PT && p.q16 != nullptr) {
+      q16.load(p.q16 + qoff);
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(qp + 32 * ks);
+      for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
+      qsc = PT ? p.q_scale[qs_group * 8 + (l32 & 7)] : p.q_scale[qs_group];
+    }
   }
-  const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave;
-  const float qsc = (PT ? p.q_scale[qs_group * 8 + (l32 & 7)] : p.q_scale[qs_group]) * p.sm_scale_log2e;
 
   float* epi = reinterpret_cast<float*>(smem + Lds::EPI_OFF);   // [2][D]: v_scale, v_mean (D = 64)
   float epi_sc = 0.f, epi_mn = 0.f;
@@ -179,7 +185,6 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 
   __syncthreads();
 
-
   using OutT = F16x<OUT_DT>;
   // where this lane's q-row goes (evaluated where it is needed: nothing of it lives across the loop)
   auto out_row_ptr = [&]() {
@@ -194,7 +199,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
-      if (p.lse && lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, -INFINITY);
+      if (p.lse && lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = -INFINITY;
     }
     return;
   }
@@ -333,6 +338,19 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     load_k(kb_2, 2);
     load_v(kb_1, 1);
   }
+  // (Q from 16 bits: quantised while the tiles are on their way)
+  if constexpr (!PT) {
+    if (p.q16 != nullptr) {
+      qsc = q16.quantise(qf);
+      if constexpr (LSE) {
+        if (p.k_mean != nullptr) {
+          const float d = q16.dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
+          if (lh == 0 && qrow < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = d;
+        }
+      }
+    }
+  }
+  qsc *= p.sm_scale_log2e;
   // (PT: the lane's two k scales of the block, for its even and its odd pairs of keys)
   // (everything the odd pairs need is declared for PT only in effect: without PT the names below are never read,
   // so the per-warp kernels are the instruction streams they were)
@@ -924,7 +942,7 @@ static int attn_form(const AttnParams& p, int D, bool causal, bool exact, bool d
 namespace paro {
 int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
                      const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
-                     void* out, int out_dtype, float* lse, float lse_scale, const float* lse_add, int32_t* s_dump, int B,
+                     void* out, int out_dtype, float* lse, const AttnExtra& extra, int32_t* s_dump, int B,
                      int H, int Hkv, int Nq, int Nk, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
                      int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
                      int64_t o_stride_n, float sm_scale, int is_causal, int flags, const int32_t* orders, int n_text, int F,
@@ -939,8 +957,10 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
              "per-thread scales (PARO_ATTN_QK_PER_THREAD) go with neither PARO_ATTN_PV_F16 nor the score dump");
   PARO_CHECK(!per_thread || ((uintptr_t)k_scale % 16) == 0, PARO_ERR_RUNTIME,
              "paro_attn_sparse_fwd: per-thread key scales must be 16-byte aligned");
-  PARO_CHECK(q8 && k8 && v8 && q_scale && k_scale && (v_scale || pv16) && sparse && out, PARO_ERR_RUNTIME,
+  PARO_CHECK(((q8 && q_scale) || extra.q16) && k8 && v8 && k_scale && (v_scale || pv16) && sparse && out, PARO_ERR_RUNTIME,
              "paro_attn_sparse_fwd: null tensor pointer");
+  PARO_CHECK(!extra.q16 || (!per_thread && s_dump == nullptr), PARO_ERR_UNSUPPORTED,
+             "16-bit queries go with neither per-thread scales nor the score dump");
   PARO_CHECK(!pv16 || s_dump == nullptr, PARO_ERR_UNSUPPORTED, "the score dump is not available with PARO_ATTN_PV_F16");
   PARO_CHECK(B > 0 && H > 0 && Hkv > 0 && Nq > 0 && Nk > 0, PARO_ERR_RUNTIME, "paro_attn_sparse_fwd: empty shape");
   PARO_CHECK(D == 64 || D == 128, PARO_ERR_INVALID_VALUE, "Unsupported head dim: %d", D);
@@ -950,8 +970,8 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   PARO_CHECK(out_dtype == PARO_DTYPE_F16 || out_dtype == PARO_DTYPE_BF16, PARO_ERR_RUNTIME,
              "Unsupported output dtype (expect float16 or bfloat16)");
   PARO_CHECK(((uintptr_t)q8 % 16) == 0 && ((uintptr_t)k8 % 16) == 0 && ((uintptr_t)v8 % 16) == 0 &&
-                 q_stride_b % 16 == 0 && q_stride_h % 16 == 0 && q_stride_n % 16 == 0 && k_stride_b % 16 == 0 &&
-                 k_stride_h % 16 == 0 && k_stride_n % 16 == 0,
+                 ((uintptr_t)extra.q16 % 16) == 0 && (q_stride_b | q_stride_h | q_stride_n) % (extra.q16 ? 8 : 16) == 0 &&
+                 k_stride_b % 16 == 0 && k_stride_h % 16 == 0 && k_stride_n % 16 == 0,
              PARO_ERR_RUNTIME, "Tensor query/key must be 16-byte aligned with strides that are multiples of 16");
   PARO_CHECK(((uintptr_t)out % 16) == 0 && o_stride_b % 8 == 0 && o_stride_h % 8 == 0 && o_stride_n % 8 == 0,
              PARO_ERR_RUNTIME, "Tensor output must be 16-byte aligned with strides that are multiples of 8");
@@ -973,7 +993,9 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   }
   AttnParams p;
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.v_mean = v_mean;
-  p.sparse = sparse; p.out = out; p.lse = lse; p.lse_scale = lse_scale; p.lse_add = lse_add; p.s_dump = s_dump; p.sparse_bs = sparse_batch_stride;
+  p.sparse = sparse; p.out = out; p.lse = lse; p.s_dump = s_dump; p.sparse_bs = sparse_batch_stride;
+  p.lse_scale = extra.lse_scale; p.k_mean = lse ? extra.k_mean : nullptr; p.lse_add = extra.lse_add || p.k_mean != nullptr;
+  p.q16 = extra.q16; p.lse_dot_scale = extra.lse_dot_scale;
   p.qs_b = q_stride_b; p.qs_h = q_stride_h; p.qs_n = q_stride_n;
   p.ks_b = k_stride_b; p.ks_h = k_stride_h; p.ks_n = k_stride_n;
   p.os_b = o_stride_b; p.os_h = o_stride_h; p.os_n = o_stride_n;
@@ -1031,7 +1053,7 @@ extern "C" int paro_attn_sparse_fwd(const int8_t* q8, const int8_t* k8, const ui
                                     int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
                                     int64_t o_stride_n, float sm_scale, int is_causal, int flags, void* stream) {
   return paro::attn_sparse_impl(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out,
-                                out_dtype, lse, 1.0f, nullptr, s_dump, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n,
+                                out_dtype, lse, paro::AttnExtra(), s_dump, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n,
                                 k_stride_b, k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale,
                                 is_causal, flags, nullptr, 0, 0, 0, 0, stream);
 }
@@ -1052,7 +1074,7 @@ extern "C" int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8
              "paro_attn_sparse_unpermute_fwd: n_text + F*H*W = %d + %d*%d*%d does not equal the token count %d",
              n_text, F, Hh, W, Nq);
   return attn_sparse_impl(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out, out_dtype,
-                          lse, 1.0f, nullptr, nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
+                          lse, AttnExtra(), nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
                           k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale, is_causal, flags,
                           orders, n_text, F, Hh, W, stream);
 }

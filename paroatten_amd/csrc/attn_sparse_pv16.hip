@@ -135,12 +135,18 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   // ---- Q fragments and scale of this wave's 32 rows ----
   const int qrow = qb * 64 + wave * 32 + l32;
   v4i qf[KS];
+  float qsc = 0.f;
+  QRows<OUT_DT, D> q16;
   {
-    const int8_t* qp = p.q8 + b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    if (p.q16 != nullptr) {
+      q16.load(p.q16 + qoff);
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(qp + 32 * ks);
+      for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
+      qsc = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave];
+    }
   }
-  const float qsc = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave] * (p.sm_scale_log2e * S_INV2PI_SCALE);
 
   list_take(0);
   for (int base = 64 * MU; base < kmax; base += 64 * MU) {
@@ -165,7 +171,7 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
-      if (LSE && lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow, -INFINITY);
+      if (LSE && lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = -INFINITY;
     }
     return;
   }
@@ -262,6 +268,17 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   load_k(kb_c, 0);
   load_k(kb_1, 1);
   load_v(kb_c, 0);
+  // (Q from 16 bits: quantised while the tiles are on their way)
+  if (p.q16 != nullptr) {
+    qsc = q16.quantise(qf);
+    if constexpr (LSE) {
+      if (p.k_mean != nullptr) {
+        const float d = q16.dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
+        if (lh == 0 && qrow < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = d;
+      }
+    }
+  }
+  qsc *= p.sm_scale_log2e * S_INV2PI_SCALE;
   float c_cur = qsc * clist[0];
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();

@@ -82,12 +82,18 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   list_load(0);
   const int qrow = qb * 64 + half * 32 + l32;
   v4i qf[KS];
+  float qsc = 0.f;
+  QRows<OUT_DT, D> q16;
   {
-    const int8_t* qp = p.q8 + b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
+    if (p.q16 != nullptr) {
+      q16.load(p.q16 + qoff);
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(qp + 32 * ks);
+      for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
+      qsc = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + half];
+    }
   }
-  const float qsc = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + half] * p.sm_scale_log2e;
   float* epi = reinterpret_cast<float*>(smem + Lds::EPI_OFF);
   float epi_sc = 0.f, epi_mn = 0.f;
   const int epi_ch = t % D;   // (W * 64 >= D; every wave writes the same values)
@@ -119,7 +125,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
-      if (LSE && lh == 0) store_lse(p, lse_row, -INFINITY);
+      if (LSE && lh == 0) p.lse[lse_row] = -INFINITY;
     }
     return;
   }
@@ -288,6 +294,18 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   };
 
   // ---- prologue: round 0's scores ----
+  auto quantise_q = [&]() __attribute__((always_inline)) {   // (Q from 16 bits: while the tiles are on their way)
+    if (p.q16 != nullptr) {
+      qsc = q16.quantise(qf);
+      if constexpr (LSE) {
+        if (wave == 0 && p.k_mean != nullptr) {
+          const float d = q16.dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
+          if (lh == 0 && qrow < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = d;
+        }
+      }
+    }
+    qsc *= p.sm_scale_log2e;
+  };
   const int rounds = (cnt + W - 1) / W;
   auto block_of = [&](int r) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)klist[r * W + wave]); };
   int kb_c = block_of(0), kb_1 = block_of(1), kb_2 = block_of(2);
@@ -298,6 +316,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     dma_k(kb_1, 1);
     load_v(kb_c, vfrag[0]);
     __builtin_amdgcn_sched_barrier(0);
+    quantise_q();
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D / 16 + 2 * DT) : "memory");
     read_k(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -305,6 +324,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     load_k(kb_c, kfrag[0]);
     load_k(kb_1, kfrag[1]);
     load_v(kb_c, vfrag[0]);
+    quantise_q();
   }
   v16i acc[2][2];   // [round parity][row tile of the 64 keys]: the next round's products are issued before the barrier
   qk(acc[0], kfrag[0]);

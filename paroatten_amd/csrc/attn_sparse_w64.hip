@@ -103,14 +103,19 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   int qrow[2];
   v4i qf[2][2];
   float qsc[2];
+  QRows<OUT_DT, D> q16[2];
 #pragma unroll
   for (int hf = 0; hf < 2; hf++) {
     qrow[hf] = qb * 64 + hf * 32 + l32;
     // rows past the end re-read the last row; their results are never stored
-    const int8_t* qp = p.q8 + b * p.qs_b + h * p.qs_h + (int64_t)min(qrow[hf], p.Nq - 1) * p.qs_n + 16 * lh;
+    const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow[hf], p.Nq - 1) * p.qs_n + 16 * lh;
+    if (p.q16 != nullptr) {
+      q16[hf].load(p.q16 + qoff);
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) qf[hf][ks] = *reinterpret_cast<const v4i*>(qp + 32 * ks);
-    qsc[hf] = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + hf] * p.sm_scale_log2e;
+      for (int ks = 0; ks < 2; ks++) qf[hf][ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
+      qsc[hf] = p.q_scale[((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + hf];
+    }
   }
   float* epi = reinterpret_cast<float*>(smem + Lds::EPI_OFF);   // [2][D]: v_scale, v_mean
   const float epi_sc = p.v_scale[bhk * D + lane];
@@ -146,7 +151,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
 #pragma unroll
         for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
         if constexpr (LSE)
-          if (lh == 0) store_lse(p, ((int64_t)b * p.H + h) * p.Nq + qrow[hf], -INFINITY);
+          if (lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow[hf]] = -INFINITY;
       }
     return;
   }
@@ -372,9 +377,6 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   int kb_1 = __builtin_amdgcn_readfirstlane((int)klist[1]);
   int kb_2 = __builtin_amdgcn_readfirstlane((int)klist[2]);
   int kb_3 = __builtin_amdgcn_readfirstlane((int)klist[3]);
-  // (the q scales are the same in every lane: scalar registers from here on)
-  qsc[0] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(qsc[0])));
-  qsc[1] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(qsc[1])));
 
   // One phase.  X: the half whose products are issued (S_X of the next block, O_X of this one); Y = 1 - X: the
   // half whose weights are computed, from the scores of block list entry `yi` (block number kb_y).  xi: list
@@ -485,6 +487,23 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   load_k(kb_1, 1);
   load_v(kb_c, 0);
   load_v(kb_1, 1);
+  // (Q from 16 bits: quantised while the tiles are on their way)
+  if (p.q16 != nullptr) {
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+      qsc[hf] = q16[hf].quantise(qf[hf]);
+      if constexpr (LSE) {
+        if (p.k_mean != nullptr) {
+          const float d = q16[hf].dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
+          if (lh == 0 && qrow[hf] < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow[hf]] = d;
+        }
+      }
+    }
+  }
+  // (the q scales are the same in every lane: scalar registers from here on)
+#pragma unroll
+  for (int hf = 0; hf < 2; hf++)
+    qsc[hf] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(qsc[hf] * p.sm_scale_log2e)));
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   read_k_frags(0);
 #pragma unroll

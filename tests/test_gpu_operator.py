@@ -88,3 +88,33 @@ def test_operator_batch_and_head_counts_of_16_bits(dev, B, H, smooth_k):
     part = P.paroattn_qk_int8_pv_fp16_cuda(q[tail].contiguous(), k[tail].contiguous(), v[tail].contiguous(),
                                            mask if B > 1 else mask[-1100:], **kw)
     assert torch.equal(o[tail], part)
+
+
+@pytest.mark.parametrize("H,N,D,form,causal", [
+    (2, 1345, 64, "SPLIT", False), (2, 1345, 128, "SPLIT", True), (6, 1345, 128, "SPLIT", False),
+    (75, 1345, 64, "ONE_WAVE", False), (200, 1345, 64, "ONE_WAVE", True), (30, 700, 64, "TWO_WAVES", True),
+    (90, 1345, 64, "PACED", False), (60, 1345, 128, "PACED", True),
+])
+@pytest.mark.parametrize("lse", [False, True])
+def test_queries_quantised_by_every_kernel_form(dev, monkeypatch, H, N, D, form, causal, lse):
+    """The operator's attention kernels read 16-bit queries and quantise them themselves: the same bits as on queries that
+    the quantiser has made, in every form, with a last q-block of one row, an empty row of the mask and queries of zero."""
+    import paroatten_amd as P
+    from paroatten_amd import _lib
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    if form == "PACED":
+        monkeypatch.setenv("PARO_ATTN_PACING", "1")
+    assert _lib.load().paro_attn_kernel_form(1, H, N, N, D, int(causal), int(lse), 0) == getattr(_lib, "PARO_ATTN_FORM_" + form)
+    g = torch.Generator(device=dev).manual_seed(N + D + H)
+    q, k, v = (torch.randn(1, H, N, D, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
+    q[:, 0, 64:96] = 0
+    mask = synth.make_block_mask(H, (N + 63) // 64, 0.4, seed=N, device=dev)
+    mask[1, 2] = False
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, None, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="HND")
+    o_ref = torch.empty_like(q)
+    lse2 = qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, 1, int(causal), 2, D ** -0.5, int(lse), mask)
+    got = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, is_causal=causal, smooth_k=False, return_lse=lse)
+    assert torch.equal(got[0] if lse else got, o_ref)
+    if lse:
+        assert torch.equal(got[1], lse2 * 0.6931471805599453)

@@ -4,6 +4,7 @@
 //   op_finalize  their second steps
 //   op_prep      quantised K and the V tiles, side by side (per-thread scales: quantised Q too)
 //   v_residual   (FP8 product with smooth_v)
+// (op_head, one launch, in the place of these for up to 1024 tokens)
 //   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; per-thread scales: on INT8 Q); the
 //                log-sum-exp leaves as the natural one of the scores of q and k as given
 // The first four are bound by HBM: at B = 2, H = 48, N = 17776, D = 64 they move 16-bit K and V twice and write their 8-bit
@@ -37,6 +38,8 @@ struct OpParams {
   int stats_k, stats_v;         // which statistics are taken
   int kv_blocks;                // workgroups of op_prep that take K or V; the rest (per-thread scales) take Q
   float sm_scale;
+  bool one_launch;              // op_head does it all
+  int k_parts, k_rounds;        // of it: workgroups that share the K of a head, 256 tokens they take one after the other
 };
 
 template <int DT, int D>
@@ -104,6 +107,260 @@ __global__ void __launch_bounds__(256) op_prep_kernel(const OpParams p) {
   }
 }
 
+// Everything in front of the attention launch, up to OP_HEAD_TOKENS tokens, in one launch: such a call consists of launches of
+// a few microseconds that wait for each other, not of bytes.  Workgroups of 16 waves that need nothing of each other:
+//   V: 32 channels of a (batch, kv-head) over all tokens, read once and held in registers between the statistics and the
+//      codes.  A lane has two channels of four neighbouring tokens, which are a word of the tiles each.
+//   K: four 64-token groups, four waves to each; with smooth_k every workgroup takes the mean over all tokens for itself.
+// What bounds it is the vector work and the latencies of one compute unit: with one workgroup to K and one to V of a head the
+// launch took 10.5 us at N = 416, D = 64, two heads, 3 of them for adding up across lanes and 4 for the codes of V; this way
+// 5.8.  The operator, start to end, separate launches / this one, smooth_k, us:
+//   D = 64   N = 416   2 heads 19.4 / 13.2   16 heads 20.7 / 13.4     D = 128  N = 512   8 heads 24.9 / 18.4   48 heads 31.5 / 26.0
+//            N = 1024  8 heads 22.6 / 19.9   48 heads 29.6 / 24.6              N = 1024  8 heads 29.4 / 25.2   48 heads 45.8 / 40.6
+//            N = 1024 160 heads 63.0 / 54.1                                    N = 1024 96 heads 75.0 / 73.4
+constexpr int OP_HEAD_TOKENS = 1024;
+
+template <int DT, int D, bool F16V>
+__global__ void __launch_bounds__(1024) op_head_kernel(const OpParams p) {
+  constexpr int LPR = D / 8;                // lanes per token row (K)
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int k_parts = p.k_parts, parts = k_parts + (F16V ? (p.nbk + 3) / 4 : D / 32);
+  const int bh = blockIdx.x / parts, b = bh / p.Hkv, h = bh % p.Hkv;
+  int part = blockIdx.x % parts;
+  const int N = p.Nk;
+  constexpr int V_BYTES = F16V ? 4 * 64 * (D + 8) * 2 : OP_HEAD_TOKENS * 64 + 32 * 3 * 32 * 4 + 2 * 32 * 4;
+  constexpr int K_BYTES = 16 * D * 4 + D * 2 + 2 * 16 * 4;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[V_BYTES > K_BYTES ? V_BYTES : K_BYTES];
+
+  if (part < k_parts) {
+    constexpr int RPI = 64 / LPR, CH = 16 / RPI;   // rows per load, loads per lane of a wave's 16 rows
+    constexpr int ROWS = 1024 / LPR, BATCH = 8;
+    const int col = (lane % LPR) * 8;
+    const unsigned short* k = p.k + b * p.ks_b + h * p.ks_h + col;
+    int grp = part * 4 * p.k_rounds + (wave >> 2);
+    v4i raw[CH];
+    auto load = [&]() {
+#pragma unroll
+      for (int i = 0; i < CH; i++) {
+        const int tok = grp * 64 + (wave & 3) * 16 + lane / LPR + i * RPI;
+        raw[i] = tok < N ? *reinterpret_cast<const v4i*>(k + (int64_t)tok * p.ks_n) : v4i{0, 0, 0, 0};
+      }
+    };
+    load();
+    float mv[8] = {};
+    if (p.stats_k) {
+      auto* red = reinterpret_cast<float(*)[D]>(smem);
+      unsigned short* mean = reinterpret_cast<unsigned short*>(smem + 16 * D * 4);
+      float s[8] = {};
+      for (int r = t / LPR; r < N; r += ROWS * BATCH) {
+        v4i x[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++)
+          x[u] = *reinterpret_cast<const v4i*>(k + (int64_t)min(r + u * ROWS, N - 1) * p.ks_n);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          float f[BATCH];
+#pragma unroll
+          for (int u = 0; u < BATCH; u++) f[u] = r + u * ROWS < N ? elem16_to_f32<DT>(x[u], j) : 0.f;
+          s[j] += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        float a, c;
+        if constexpr (LPR == 8) s[j] += row_dpp<0x128>(s[j]);
+        with_lane_xor16(s[j], a, c);
+        s[j] = a + c;
+        with_lane_xor32(s[j], a, c);
+        s[j] = a + c;
+      }
+      if (lane < LPR) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) red[wave][col + j] = s[j];
+      }
+      __syncthreads();
+      if (t < D) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) sum += red[w][t];
+        mean[t] = (unsigned short)(pack2_from_f32<DT>((float)(sum / (double)N), 0.f) & 0xffffu);
+        if (part == 0) p.k_mean[(int64_t)bh * D + t] = mean[t];
+      }
+      __syncthreads();
+      load8_f32<DT>(mean + col, mv);
+    }
+    // (the rest is quant_group_body, with the maximum of four waves)
+    auto* gmax = reinterpret_cast<float(*)[16]>(smem + 16 * D * 4 + D * 2);
+    int8_t* out = p.k8 + (int64_t)bh * N * D + col;
+    for (int r = 0; r < p.k_rounds; r++) {
+      const int tok0 = grp * 64 + (wave & 3) * 16 + lane / LPR;
+      float amax = 0.0000001f;
+#pragma unroll
+      for (int i = 0; i < CH; i++)
+        if (tok0 + i * RPI < N) {
+#pragma unroll
+          for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(elem16_to_f32<DT>(raw[i], j) - mv[j]));
+        }
+      float* gm = gmax[r & 1];   // (a wave may be one round ahead of the others, not two)
+      gm[wave] = wave_max(amax);
+      __syncthreads();
+      const int w0 = wave & ~3;
+      amax = fmaxf(fmaxf(gm[w0], gm[w0 + 1]), fmaxf(gm[w0 + 2], gm[w0 + 3]));
+      if (t % 256 == 0 && grp < p.nbk) p.k_scale[(int64_t)bh * p.nbk + grp] = amax / 127.0f;
+      const float inv = 127.0f / amax;
+#pragma unroll
+      for (int i = 0; i < CH; i++) {
+        const int tok = tok0 + i * RPI;
+        float y[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) y[j] = (elem16_to_f32<DT>(raw[i], j) - mv[j]) * inv;
+        if (tok < N)
+          *reinterpret_cast<v2i*>(out + (int64_t)tok * D) =
+              v2i{(int)pack4_rint_i8(y[0], y[1], y[2], y[3]), (int)pack4_rint_i8(y[4], y[5], y[6], y[7])};
+      }
+      grp += 4;
+      if (r + 1 < p.k_rounds) load();
+    }
+    return;
+  }
+  part -= k_parts;
+
+  if constexpr (F16V) {
+    auto* tiles = reinterpret_cast<unsigned short(*)[64 * (D + 8)]>(smem);
+    const int g = t >> 8, tg = t & 255, kb = part * 4 + g;
+    const unsigned short* v = p.v + b * p.vs_b + h * p.vs_h;
+    v_f16_load_tile<D>(v, tiles[g], N, p.vs_n, kb, tg);
+    __syncthreads();
+    if (kb < p.nbk) v_f16_store_tile<DT, D>(tiles[g], (unsigned short*)p.v_tiles + ((int64_t)bh * p.nbk + kb) * (64 * D), tg);
+  } else {
+    // The 32 channels go to LDS once, four tokens of 64 bytes to a group; token q of group a lies at place q ^ (a / 2 % 4), so
+    // that both the statistics (four tokens of a group at a time) and the codes (the same token of every other group) read
+    // each bank once.  Sums are taken in the order of v_stats_body, v_finalize_body, pack_v_tile and v_residual, to the bit.
+    auto* red = reinterpret_cast<float(*)[3][32]>(smem + OP_HEAD_TOKENS * 64);          // [chunk][group][3][32]
+    auto* resid = reinterpret_cast<float(*)[2][32]>(smem + OP_HEAD_TOKENS * 64);        // (later) [row tile][lane half][32]
+    auto* chan = reinterpret_cast<float(*)[32]>(smem + OP_HEAD_TOKENS * 64 + 32 * 3 * 32 * 4);   // reciprocal scale, mean
+    constexpr int U = D / 8, GROUPS = 64 / U;   // tokens that v_stats_body adds up one after the other; groups of four such rows
+    const unsigned short* v = p.v + b * p.vs_b + h * p.vs_h + 32 * part;
+    v4i raw[OP_HEAD_TOKENS / 256];
+#pragma unroll
+    for (int i = 0; i < OP_HEAD_TOKENS / 256; i++) {
+      const int tok = t / 4 + 256 * i;
+      raw[i] = tok < N ? *reinterpret_cast<const v4i*>(v + (int64_t)tok * p.vs_n + t % 4 * 8) : v4i{0, 0, 0, 0};
+    }
+    auto at = [&](int group, int q) { return smem + group * 256 + ((q ^ (group >> 1)) & 3) * 64; };
+#pragma unroll
+    for (int i = 0; i < OP_HEAD_TOKENS / 256; i++) {
+      const int tok = t / 4 + 256 * i;
+      *reinterpret_cast<v4i*>(at(tok >> 2, tok & 3) + t % 4 * 16) = raw[i];
+    }
+    __syncthreads();
+    const int cp = 2 * (lane & 15);
+    for (int sc = wave; sc < OP_HEAD_TOKENS / 256 * GROUPS; sc += 16) {
+      const int chunk = sc / GROUPS, q = lane >> 4;
+      if (256 * chunk >= N) break;
+      float s[2] = {0.f, 0.f}, mn[2] = {INFINITY, INFINITY}, mx[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int group = 64 * chunk + GROUPS * u + sc % GROUPS;
+        const unsigned w = *reinterpret_cast<const unsigned*>(at(group, q) + 2 * cp);
+        const float f[2] = {lo16_to_f32<DT>(w), hi16_to_f32<DT>(w)};
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          s[c] += f[c];
+          if (4 * group + q < N) {
+            mn[c] = fminf(mn[c], f[c]);
+            mx[c] = fmaxf(mx[c], f[c]);
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        float x, y;
+        with_lane_xor16(s[c], x, y);  s[c] = x + y;
+        with_lane_xor16(mn[c], x, y); mn[c] = fminf(x, y);
+        with_lane_xor16(mx[c], x, y); mx[c] = fmaxf(x, y);
+        with_lane_xor32(s[c], x, y);  s[c] = x + y;
+        with_lane_xor32(mn[c], x, y); mn[c] = fminf(x, y);
+        with_lane_xor32(mx[c], x, y); mx[c] = fmaxf(x, y);
+        if (lane < 16) {
+          red[sc][0][cp + c] = s[c];
+          red[sc][1][cp + c] = mn[c];
+          red[sc][2][cp + c] = mx[c];
+        }
+      }
+    }
+    __syncthreads();
+    float mean_t = 0.f, scale_t = 0.f;   // threads below 32: their channel's
+    if (wave == 0) {
+      const int ch = lane & 31;          // lower half: sum and minimum, upper half: maximum
+      double sum = 0.0;
+      float ext = lane < 32 ? INFINITY : -INFINITY;
+#pragma unroll
+      for (int c = 0; c < OP_HEAD_TOKENS / 256; c++) {
+        if (256 * c >= N) break;
+        float x[GROUPS];
+#pragma unroll
+        for (int g = 0; g < GROUPS; g++) {
+          x[g] = red[GROUPS * c + g][0][ch];
+          const float e = red[GROUPS * c + g][lane < 32 ? 1 : 2][ch];
+          ext = lane < 32 ? fminf(ext, e) : fmaxf(ext, e);
+        }
+#pragma unroll
+        for (int n = 1; n < GROUPS; n *= 2)
+#pragma unroll
+          for (int g = 0; g < GROUPS; g += 2 * n) x[g] += x[g + n];
+        sum += x[0];
+      }
+      float lo, hi;
+      with_lane_xor32(ext, lo, hi);
+      mean_t = p.smooth_v ? (float)(sum / (double)N) : 0.f;
+      const float amax = fmaxf(hi - mean_t, mean_t - lo);
+      scale_t = amax / 448.0f;
+      if (lane < 32) {
+        chan[0][ch] = amax > 0.f ? 448.0f / amax : 0.f;
+        chan[1][ch] = mean_t;
+      }
+    }
+    __syncthreads();
+    const float recp[2] = {chan[0][cp], chan[0][cp + 1]}, mean[2] = {chan[1][cp], chan[1][cp + 1]};
+    for (int pc = wave; pc < 4 * p.nbk; pc += 16) {
+      const int kb = pc >> 2, mt = (pc >> 1) & 1, lh = pc & 1, g = lane >> 4;
+      const int group = kb * 16 + mt * 8 + 2 * g + lh;
+      float f[2][4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const unsigned w = *reinterpret_cast<const unsigned*>(at(group, q) + 2 * cp);
+        const bool in = 4 * group + q < N;
+        f[0][q] = in ? (lo16_to_f32<DT>(w) - mean[0]) * recp[0] : 0.f;
+        f[1][q] = in ? (hi16_to_f32<DT>(w) - mean[1]) * recp[1] : 0.f;
+      }
+      uint8_t* out = p.v_tiles + ((int64_t)bh * p.nbk + kb) * (64 * D) + part * 2048 + mt * 1024 + (lh * 32 + cp) * 16 + 4 * g;
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        int w = __builtin_amdgcn_cvt_pk_fp8_f32(f[c][0], f[c][1], 0, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(f[c][2], f[c][3], w, true);
+        *reinterpret_cast<int*>(out + 16 * c) = w;
+        const float e = ((f[c][0] - __builtin_amdgcn_cvt_f32_fp8(w, 0)) + (f[c][1] - __builtin_amdgcn_cvt_f32_fp8(w, 1))) +
+                        ((f[c][2] - __builtin_amdgcn_cvt_f32_fp8(w, 2)) + (f[c][3] - __builtin_amdgcn_cvt_f32_fp8(w, 3)));
+        // the four words of a piece one after the other (lanes 0..15)
+        float own, e1, e2, e3;
+        with_lane_xor16(e, own, e1);
+        with_lane_xor32(e, own, e2);
+        with_lane_xor32(e1, own, e3);
+        if (lane < 16) resid[2 * kb + mt][lh][cp + c] = ((e + e1) + e2) + e3;
+      }
+    }
+    __syncthreads();
+    if (t < 32) {
+      float r = 0.f;
+      for (int i = 0; i < 2 * p.nbk; i++) r += resid[i][0][t] + resid[i][1][t];
+      const int64_t ch = (int64_t)bh * D + 32 * part + t;
+      p.v_scale[ch] = scale_t;
+      p.v_mean[ch] = p.smooth_v ? mean_t + scale_t * (r / (float)N) : mean_t;
+    }
+  }
+}
+
 // Where the intermediate tensors lie in the workspace (256-byte aligned pieces).
 struct OpLayout {
   int64_t q8, k8, v_tiles, q_scale, k_scale, v_scale, v_mean, v_work, k_partial, k_mean, bytes;
@@ -128,8 +385,17 @@ struct OpLayout {
   }
 };
 
+template <int DT, int D, bool F16V>
+static int launch_op_head(const OpParams& p, hipStream_t st) {
+  const int parts = p.k_parts + (F16V ? ceil_div(p.nbk, 4) : D / 32);
+  hipLaunchKernelGGL((op_head_kernel<DT, D, F16V>), dim3(p.B * p.Hkv * parts), dim3(1024), 0, st, p);
+  PARO_HIP(hipGetLastError());
+  return PARO_OK;
+}
+
 template <int DT, int D>
 static int launch_op_prep(const OpParams& p, bool per_thread, bool f16v, hipStream_t st) {
+  if (p.one_launch) return f16v ? launch_op_head<DT, D, true>(p, st) : launch_op_head<DT, D, false>(p, st);
   if (p.stats_k + p.stats_v > 0) {
     hipLaunchKernelGGL((op_stats_kernel<DT, D>), dim3(p.chunks * (p.stats_k + p.stats_v), p.Hkv, p.B), dim3(256), 0, st, p);
     hipLaunchKernelGGL((op_finalize_kernel<DT, D>), dim3(p.B * p.Hkv * (p.stats_k + p.stats_v)), dim3(1024), 0, st, p);
@@ -203,6 +469,14 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   p.stats_k = smooth_k != 0; p.stats_v = !f16v;
   p.kv_blocks = B * Hkv * (p.nbk + ceil_div(p.nbk, 4));
   p.sm_scale = sm_scale;
+  const int64_t BK = (int64_t)B * Hkv, v_parts = f16v ? ceil_div(p.nbk, 4) : D / 32;
+  // op_head: its workgroups have to run at the same time, two to a compute unit.  K's take 256 tokens each as long as all of
+  // them find a compute unit to themselves, and otherwise a whole head, since with smooth_k each reads all of it for the mean:
+  // 48 heads, N = 1024, D = 64 24.6 us by heads and 29.5 by 256 tokens, 32 heads 23.3 and 22.4; D = 128 48 heads 40.9 and 43.7,
+  // 24 heads 35.7 and 31.2
+  p.one_launch = !per_thread && Nk <= OP_HEAD_TOKENS && p.stats_k + p.stats_v > 0 && BK * (1 + v_parts) <= 512;
+  p.k_rounds = p.stats_k && BK * (ceil_div(p.nbk, 4) + v_parts) > 256 ? ceil_div(p.nbk, 4) : 1;
+  p.k_parts = ceil_div(p.nbk, 4 * p.k_rounds);
   hipStream_t st = (hipStream_t)stream;
   int rc;
   if (dtype == PARO_DTYPE_F16)
@@ -210,7 +484,7 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   else
     rc = D == 64 ? launch_op_prep<PARO_DTYPE_BF16, 64>(p, per_thread, f16v, st) : launch_op_prep<PARO_DTYPE_BF16, 128>(p, per_thread, f16v, st);
   if (rc) return rc;
-  if (p.v_resid)
+  if (p.v_resid && !p.one_launch)
     if ((rc = v_fp8_add_residual(p.v_resid, p.v_scale, p.v_mean, B, Hkv, Nk, D, st))) return rc;
   AttnExtra extra;
   extra.lse_scale = 0.6931471805599453f;

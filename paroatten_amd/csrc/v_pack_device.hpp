@@ -37,25 +37,11 @@ __device__ __forceinline__ void v_pack_body(const unsigned short* __restrict__ v
   }
 }
 
-// float16 tiles: the block goes through LDS row by row (16-byte loads) and leaves as D/32 x 4 pieces of 1 KB (16 bytes
-// per lane).
+// One block, in LDS as rows of D + 8 elements, as a float16 tile: 256 threads.
 template <int DT, int D>
-__device__ __forceinline__ void v_f16_pack_body(const unsigned short* __restrict__ v, unsigned short* __restrict__ out,
-                                                int N, int nb, int64_t vs_n, int kb, int64_t bh) {
-  __shared__ __attribute__((aligned(16))) unsigned short tile[64 * (D + 8)];   // rows padded by 16 bytes
-  constexpr int CPR = D / 8;   // 16-byte chunks per row
+__device__ __forceinline__ void v_f16_store_tile(const unsigned short* tile, unsigned short* __restrict__ dst, int t) {
 #pragma unroll
-  for (int c = threadIdx.x; c < 64 * CPR; c += 256) {
-    const int row = c / CPR, ch = c % CPR;
-    const int tok = kb * 64 + row;
-    v4i x = {0, 0, 0, 0};
-    if (tok < N) x = *reinterpret_cast<const v4i*>(v + (int64_t)tok * vs_n + ch * 8);
-    *reinterpret_cast<v4i*>(tile + row * (D + 8) + ch * 8) = x;
-  }
-  __syncthreads();
-  unsigned short* dst = out + (bh * nb + kb) * (64 * D);
-#pragma unroll
-  for (int pl = threadIdx.x; pl < (D / 32) * 4 * 64; pl += 256) {
+  for (int pl = t; pl < (D / 32) * 4 * 64; pl += 256) {
     const int lane = pl & 63, piece = pl >> 6;
     const int dt = piece >> 2, s = piece & 3;
     const int chn = 32 * dt + (lane & 31);
@@ -70,6 +56,32 @@ __device__ __forceinline__ void v_f16_pack_body(const unsigned short* __restrict
         v4i{(int)(r[0] | ((unsigned)r[1] << 16)), (int)(r[2] | ((unsigned)r[3] << 16)),
             (int)(r[4] | ((unsigned)r[5] << 16)), (int)(r[6] | ((unsigned)r[7] << 16))};
   }
+}
+
+// Its way there: 256 threads, rows past the end are zero.
+template <int D>
+__device__ __forceinline__ void v_f16_load_tile(const unsigned short* __restrict__ v, unsigned short* tile, int N, int64_t vs_n,
+                                                int kb, int t) {
+  constexpr int CPR = D / 8;   // 16-byte chunks per row
+#pragma unroll
+  for (int c = t; c < 64 * CPR; c += 256) {
+    const int row = c / CPR, ch = c % CPR;
+    const int tok = kb * 64 + row;
+    v4i x = {0, 0, 0, 0};
+    if (tok < N) x = *reinterpret_cast<const v4i*>(v + (int64_t)tok * vs_n + ch * 8);
+    *reinterpret_cast<v4i*>(tile + row * (D + 8) + ch * 8) = x;
+  }
+}
+
+// float16 tiles: the block goes through LDS row by row (16-byte loads) and leaves as D/32 x 4 pieces of 1 KB (16 bytes
+// per lane).
+template <int DT, int D>
+__device__ __forceinline__ void v_f16_pack_body(const unsigned short* __restrict__ v, unsigned short* __restrict__ out,
+                                                int N, int nb, int64_t vs_n, int kb, int64_t bh) {
+  __shared__ __attribute__((aligned(16))) unsigned short tile[64 * (D + 8)];   // rows padded by 16 bytes
+  v_f16_load_tile<D>(v, tile, N, vs_n, kb, threadIdx.x);
+  __syncthreads();
+  v_f16_store_tile<DT, D>(tile, out + (bh * nb + kb) * (64 * D), threadIdx.x);
 }
 
 }  // namespace paro

@@ -55,6 +55,33 @@ def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode,
     assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()
 
 
+@pytest.mark.parametrize("N,D,H,mode", [
+    (1, 64, 3, "fp8"), (64, 128, 3, "f16"), (255, 64, 3, "fp8"), (256, 128, 3, "fp8"), (257, 64, 3, "f16"), (513, 128, 3, "fp8"),
+    (1023, 64, 3, "fp8"), (1024, 64, 3, "fp8"), (1024, 128, 3, "fp8"), (1025, 64, 3, "fp8"),
+    (1000, 64, 60, "fp8"), (1024, 128, 60, "f16"), (700, 128, 60, "fp8"), (300, 128, 110, "fp8"), (300, 64, 180, "fp8"),
+])
+@pytest.mark.parametrize("smooth_k,smooth_v", [(False, True), (True, True), (True, False)])
+def test_one_launch_preparation_equals_the_separate_ones(dev, N, D, H, mode, smooth_k, smooth_v):
+    """Edges of the 64-token tiles, the 256-token chunks and the 1024 tokens of the one-launch preparation; K by 256 tokens
+    (3 heads), by heads (60) and separate launches (110, 180).  K's sums are exact, V is arbitrary: the same bits."""
+    import paroatten_amd as P
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    dtype = torch.bfloat16 if N % 2 else torch.float16
+    g = torch.Generator(device=dev).manual_seed(N + D + H)
+    q, v = (torch.randn(1, H, N, D, generator=g, device=dev).to(dtype) for _ in range(2))
+    v = v + torch.randn(1, H, 1, D, generator=g, device=dev).to(dtype)
+    k = (torch.randint(-63, 64, (1, H, N, D), generator=g, device=dev) / 8).to(dtype)
+    mask = synth.make_block_mask(H, (N + 63) // 64, 0.6, seed=N, device=dev)
+    km = k.double().mean(dim=2, keepdim=True).float().to(dtype) if smooth_k else None
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, km, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="HND")
+    o_ref = torch.empty_like(q)
+    qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, 1, 0, 2, D ** -0.5, 0, mask, pv_f16=mode == "f16",
+                                        smooth_v=smooth_v)
+    got = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, smooth_k=smooth_k, smooth_v=smooth_v, pv_f16=mode == "f16")
+    assert torch.equal(got, o_ref)
+
+
 @pytest.mark.parametrize("N,D,dtype", [(416, 64, torch.float16), (2000, 128, torch.bfloat16), (32760, 128, torch.float16)])
 def test_k_mean_is_the_rounded_mean(dev, N, D, dtype):
     """The K mean that the operator takes is the one that 64-bit sums round to, on inputs of which sums in one fp32

@@ -4,7 +4,7 @@
 //   op_finalize  their second steps
 //   op_prep      quantised K and the V tiles, side by side (per-thread scales: quantised Q too)
 //   v_residual   (FP8 product with smooth_v)
-// (op_head, one launch, in the place of these for up to 1024 tokens)
+// (op_head, one launch, in the place of these for up to 1024 tokens; op_prep_short in that of the second and third beyond)
 //   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; per-thread scales: on INT8 Q); the
 //                log-sum-exp leaves as the natural one of the scores of q and k as given
 // The first four are bound by HBM: at B = 2, H = 48, N = 17776, D = 64 they move 16-bit K and V twice and write their 8-bit
@@ -39,6 +39,7 @@ struct OpParams {
   int kv_blocks;                // workgroups of op_prep that take K or V; the rest (per-thread scales) take Q
   float sm_scale;
   bool one_launch;              // op_head does it all
+  bool short_prep;              // op_prep_short does what comes after the statistics
   int k_parts, k_rounds;        // of it: workgroups that share the K of a head, 256 tokens they take one after the other
 };
 
@@ -361,9 +362,114 @@ __global__ void __launch_bounds__(1024) op_head_kernel(const OpParams p) {
   }
 }
 
+// op_finalize and op_prep in one, for sequences of few statistics chunks: every workgroup adds the chunks up for itself.  256
+// threads take one V tile or 256 tokens of K.  To the bit the results of the two launches (sums of short chunks are added up
+// in fp64).  (Tried as well: the last V tile of a head to get there adds up the residuals, instead of a launch of its own.
+// Rows that other compute units have just written have to be read past the caches: N = 4096, two heads, 31.6 us instead of 25.0.)
+template <int DT, int D, bool F16V>
+__global__ void __launch_bounds__(256) op_prep_short_kernel(const OpParams p) {
+  constexpr int LPR = D / 8, ROWS = 256 / LPR, SL = 256 / D, PITCH = D + 8;
+  const int t = threadIdx.x, wave = t >> 6;
+  const int per_k = (p.nbk + 3) / 4, per = p.nbk + per_k;
+  const int bh = blockIdx.x / per, j = blockIdx.x % per;
+  const int b = bh / p.Hkv, h = bh % p.Hkv, N = p.Nk;
+  const int ch = t % D, sl = t / D;
+  __shared__ double red_s[SL][D];
+  __shared__ __attribute__((aligned(16))) unsigned short tile[64 * PITCH];
+  if (j >= p.nbk) {
+    unsigned short* mean = tile;
+    if (p.stats_k) {
+      const float* x = p.k_partial + (int64_t)bh * p.chunks * D + ch;
+      double s = 0.0;
+      for (int c = sl; c < p.chunks; c += SL) s += x[c * D];
+      red_s[sl][ch] = s;
+      __syncthreads();
+      if (t < D) {
+        for (int i = 1; i < SL; i++) s += red_s[i][ch];
+        mean[ch] = (unsigned short)(pack2_from_f32<DT>((float)(s / (double)N), 0.f) & 0xffffu);
+        if (j == p.nbk) p.k_mean[(int64_t)bh * D + ch] = mean[ch];
+      }
+      __syncthreads();
+    }
+    const int g = (j - p.nbk) * 4 + wave;
+    if (g >= p.nbk) return;
+    const unsigned short* k = p.k + b * p.ks_b + h * p.ks_h;
+    int8_t* out = p.k8 + (int64_t)bh * N * D;
+    float* scale = p.k_scale + (int64_t)bh * p.nbk;
+    if (p.stats_k) quant_group_body<DT, D, 64, true, false>(k, mean, out, scale, N, g, p.ks_n, D, 0.f);
+    else quant_group_body<DT, D, 64, false, false>(k, nullptr, out, scale, N, g, p.ks_n, D, 0.f);
+    return;
+  }
+  const unsigned short* v = p.v + b * p.vs_b + h * p.vs_h;
+  if constexpr (F16V) {
+    v_f16_load_tile<D>(v, tile, N, p.vs_n, j, t);
+    __syncthreads();
+    v_f16_store_tile<DT, D>(tile, (unsigned short*)p.v_tiles + ((int64_t)bh * p.nbk + j) * (64 * D), t);
+  } else {
+    __shared__ float red[2][SL][D];
+    __shared__ float chan[2][D];        // reciprocal scale, mean
+    const int col = (t % LPR) * 8, row = t / LPR;
+    v4i raw[64 / ROWS];
+#pragma unroll
+    for (int u = 0; u < 64 / ROWS; u++) {
+      const int tok = j * 64 + row + u * ROWS;
+      raw[u] = tok < N ? *reinterpret_cast<const v4i*>(v + (int64_t)tok * p.vs_n + col) : v4i{0, 0, 0, 0};
+    }
+    const float* x = p.v_work + v_stats_offset((int64_t)p.B * p.Hkv, N, D) + (int64_t)bh * p.chunks * 3 * D + ch;
+    double s = 0.0;
+    float mn = INFINITY, mx = -INFINITY;
+#pragma unroll 4
+    for (int c = sl; c < p.chunks; c += SL) {
+      s += x[(c * 3 + 0) * D];
+      mn = fminf(mn, x[(c * 3 + 1) * D]);
+      mx = fmaxf(mx, x[(c * 3 + 2) * D]);
+    }
+    red_s[sl][ch] = s;
+    red[0][sl][ch] = mn;
+    red[1][sl][ch] = mx;
+#pragma unroll
+    for (int u = 0; u < 64 / ROWS; u++) *reinterpret_cast<v4i*>(&tile[(row + u * ROWS) * PITCH + col]) = raw[u];
+    __syncthreads();
+    if (t < D) {
+      for (int i = 1; i < SL; i++) {
+        s += red_s[i][ch];
+        mn = fminf(mn, red[0][i][ch]);
+        mx = fmaxf(mx, red[1][i][ch]);
+      }
+      const float mean = p.smooth_v ? (float)(s / (double)N) : 0.f;
+      const float amax = fmaxf(mx - mean, mean - mn);
+      chan[0][ch] = amax > 0.f ? 448.0f / amax : 0.f;
+      chan[1][ch] = mean;
+      if (j == 0) {
+        p.v_scale[(int64_t)bh * D + ch] = amax / 448.0f;
+        p.v_mean[(int64_t)bh * D + ch] = mean;
+      }
+    }
+    __syncthreads();
+    float rs[D / 64];
+    pack_v_tile<DT, D, PITCH>(tile, p.v_tiles + ((int64_t)bh * p.nbk + j) * (64 * D), chan[0], p.smooth_v ? chan[1] : nullptr,
+                              j * 64, N, t, rs);
+    if (!p.smooth_v) return;
+    float* resid = p.v_resid + (int64_t)bh * p.nbk * 2 * D;
+    if ((t & 63) < 32) {
+#pragma unroll
+      for (int n = 0; n < D / 64; n++)
+        resid[(j * 2 + (wave & 1)) * D + 32 * ((wave >> 1) + 2 * n) + (t & 31)] = rs[n];
+    }
+  }
+}
+
+// What a launch less is worth, 2 to 3 us, against the chunks (768 bytes per 256 tokens, of V at D = 64) that every workgroup
+// reads.  Operator, smooth_k, with op_finalize / without it, us: D = 64 N = 1100 2 heads 22.2 / 20.0, 96 heads 44.2 / 41.1;
+// N = 4096 2 heads 26.6 / 24.6, 24 heads 63.1 / 59.6, 96 heads 182.2 / 180.5; N = 8192 8 heads 68.9 / 67.2, 48 heads 288.8 / 289.9;
+// D = 128 N = 4096 2 heads 35.0 / 33.7, 48 heads 183.6 / 183.8; N = 8192 2 heads 60.2 / 59.2, 24 heads 288.3 / 292.9.
+static bool op_short(int64_t BK, int Nk, int D, bool per_thread) {
+  return !per_thread && Nk > OP_HEAD_TOKENS && (Nk <= 4096 || (Nk <= 8192 && BK * D <= 512));
+}
+
 // Where the intermediate tensors lie in the workspace (256-byte aligned pieces).
 struct OpLayout {
-  int64_t q8, k8, v_tiles, q_scale, k_scale, v_scale, v_mean, v_work, k_partial, k_mean, bytes;
+  int64_t q8, k8, v_tiles, q_scale, k_scale, v_scale, v_mean, v_work, k_partial, k_mean, resid, bytes;
   OpLayout(int B, int H, int Hkv, int Nq, int Nk, int D, bool smooth_k, bool per_thread, bool f16v) {
     bytes = 0;
     auto take = [&](int64_t n) {
@@ -382,6 +488,8 @@ struct OpLayout {
     v_work = take(f16v ? 0 : paro_v_fp8_partial_floats(B, Hkv, Nk, D) * 4);
     k_partial = take(smooth_k ? BK * ceil_div(Nk, v_chunk(Nk)) * D * 4 : 0);
     k_mean = take(smooth_k ? BK * D * 2 : 0);
+    const bool s = op_short(BK, Nk, D, per_thread) && !f16v;
+    resid = take(s ? BK * nbk * 2 * D * 4 : 0);   // (the chunks in v_work are read until the last tile)
   }
 };
 
@@ -398,6 +506,13 @@ static int launch_op_prep(const OpParams& p, bool per_thread, bool f16v, hipStre
   if (p.one_launch) return f16v ? launch_op_head<DT, D, true>(p, st) : launch_op_head<DT, D, false>(p, st);
   if (p.stats_k + p.stats_v > 0) {
     hipLaunchKernelGGL((op_stats_kernel<DT, D>), dim3(p.chunks * (p.stats_k + p.stats_v), p.Hkv, p.B), dim3(256), 0, st, p);
+    if (p.short_prep) {
+      const dim3 all(p.kv_blocks);
+      if (f16v) hipLaunchKernelGGL((op_prep_short_kernel<DT, D, true>), all, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((op_prep_short_kernel<DT, D, false>), all, dim3(256), 0, st, p);
+      PARO_HIP(hipGetLastError());
+      return PARO_OK;
+    }
     hipLaunchKernelGGL((op_finalize_kernel<DT, D>), dim3(p.B * p.Hkv * (p.stats_k + p.stats_v)), dim3(1024), 0, st, p);
   }
   const int q_blocks = per_thread ? p.B * p.H * ceil_div(p.nbq, 4) : 0;
@@ -477,6 +592,8 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   p.one_launch = !per_thread && Nk <= OP_HEAD_TOKENS && p.stats_k + p.stats_v > 0 && BK * (1 + v_parts) <= 512;
   p.k_rounds = p.stats_k && BK * (ceil_div(p.nbk, 4) + v_parts) > 256 ? ceil_div(p.nbk, 4) : 1;
   p.k_parts = ceil_div(p.nbk, 4 * p.k_rounds);
+  p.short_prep = op_short(BK, Nk, D, per_thread);
+  if (p.short_prep && p.v_resid) p.v_resid = (float*)(ws + at.resid);
   hipStream_t st = (hipStream_t)stream;
   int rc;
   if (dtype == PARO_DTYPE_F16)

@@ -57,13 +57,15 @@ def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode,
 
 @pytest.mark.parametrize("N,D,H,mode", [
     (1, 64, 3, "fp8"), (64, 128, 3, "f16"), (255, 64, 3, "fp8"), (256, 128, 3, "fp8"), (257, 64, 3, "f16"), (513, 128, 3, "fp8"),
-    (1023, 64, 3, "fp8"), (1024, 64, 3, "fp8"), (1024, 128, 3, "fp8"), (1025, 64, 3, "fp8"),
+    (1023, 64, 3, "fp8"), (1024, 64, 3, "fp8"), (1024, 128, 3, "fp8"),
+    (1025, 64, 3, "fp8"), (2000, 64, 3, "f16"), (4096, 128, 3, "fp8"), (4097, 64, 3, "fp8"), (8192, 64, 9, "fp8"),
     (1000, 64, 60, "fp8"), (1024, 128, 60, "f16"), (700, 128, 60, "fp8"), (300, 128, 110, "fp8"), (300, 64, 180, "fp8"),
 ])
 @pytest.mark.parametrize("smooth_k,smooth_v", [(False, True), (True, True), (True, False)])
 def test_one_launch_preparation_equals_the_separate_ones(dev, N, D, H, mode, smooth_k, smooth_v):
     """Edges of the 64-token tiles, the 256-token chunks and the 1024 tokens of the one-launch preparation; K by 256 tokens
-    (3 heads), by heads (60) and separate launches (110, 180).  K's sums are exact, V is arbitrary: the same bits."""
+    (3 heads), by heads (60) and separate launches (110, 180); beyond, the preparation that adds up the chunks itself, at its
+    edges of 4096 and (512 channels) 8192 tokens.  K's sums are exact, V is arbitrary: the same bits."""
     import paroatten_amd as P
     from paroatten_amd import _qattn_sm80 as qattn
     from paroatten_amd import quant as Q

@@ -138,3 +138,25 @@ def test_processor_grid_and_table_cache_rules():
     import gc
     gc.collect()
     assert any(r() is None for _, refs, _, _ in SHARED_TABLES._entries for r, _ in refs)
+
+
+@pytest.mark.parametrize("kind", ["layer", "layer_with_hook", "two_dims", "other"])
+def test_head_norm_is_the_norm_of_the_view(kind):
+    """A LayerNorm over the channels may be called in the projection's order of rows; hooks and other modules see the
+    [B,H,N,D] view that they are written for."""
+    from paroatten_amd.cogvideox import _head_norm
+    B, H, N, D = 2, 3, 5, 64
+    x = torch.randn(B, N, H, D, generator=torch.Generator().manual_seed(1)).transpose(1, 2)
+    seen = []
+
+    class Other(torch.nn.Module):
+        def forward(self, t):
+            seen.append(tuple(t.shape))
+            return t * torch.arange(1, H + 1).view(1, H, 1, 1)
+    norm = Other() if kind == "other" else torch.nn.LayerNorm((N, D) if kind == "two_dims" else D)
+    if kind == "layer_with_hook":
+        norm.register_forward_hook(lambda mod, args, out: seen.append(tuple(args[0].shape)))
+    got = _head_norm(norm, x)
+    assert all(s == (B, H, N, D) for s in seen) and len(seen) == (kind in ("other", "layer_with_hook"))
+    assert torch.equal(got, norm(x))
+    assert (got.stride() == x.stride()) == (kind in ("layer", "other"))

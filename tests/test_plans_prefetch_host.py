@@ -160,3 +160,48 @@ def test_head_norm_is_the_norm_of_the_view(kind):
     assert all(s == (B, H, N, D) for s in seen) and len(seen) == (kind in ("other", "layer_with_hook"))
     assert torch.equal(got, norm(x))
     assert (got.stride() == x.stride()) == (kind in ("layer", "other"))
+
+
+@pytest.mark.parametrize("kind", ["forward", "class_forward", "forward_of_another", "global_pre_hook", "global_hook",
+                                  "global_backward_hook", "pre_hook", "compiled"])
+def test_head_norm_in_other_hands_gets_the_view(kind, monkeypatch):
+    """Whatever else runs when the norm is called, a forward that has been put in its place or a hook on all modules among
+    it, is given the [B,H,N,D] view, and its result is the processor's."""
+    from torch.nn.modules import module as M
+
+    from paroatten_amd.cogvideox import _head_norm
+    B, H, N, D = 2, 3, 5, 64
+    x = torch.randn(B, N, H, D, generator=torch.Generator().manual_seed(1)).transpose(1, 2)
+    norm, seen, plain = torch.nn.LayerNorm(D), [], torch.nn.LayerNorm.forward
+
+    def by_head(t):
+        seen.append(tuple(t.shape))
+        return plain(norm, t) * torch.arange(1, H + 1).view(1, H, 1, 1)
+    handle = None
+    if kind == "forward":
+        norm.forward = by_head
+    elif kind == "class_forward":
+        monkeypatch.setattr(torch.nn.LayerNorm, "forward", lambda self, t: by_head(t))
+    elif kind == "forward_of_another":
+        other = torch.nn.LayerNorm(D)
+        torch.nn.init.constant_(other.weight, 2.0)
+        norm.forward = other.forward
+    elif kind == "global_pre_hook":
+        handle = M.register_module_forward_pre_hook(lambda mod, args: seen.append(tuple(args[0].shape)))
+    elif kind == "global_hook":
+        handle = M.register_module_forward_hook(lambda mod, args, out: seen.append(tuple(out.shape)))
+    elif kind == "global_backward_hook":
+        handle = M.register_module_full_backward_hook(lambda mod, gi, go: seen.append(tuple(go[0].shape)))
+    elif kind == "pre_hook":
+        norm.register_forward_pre_hook(lambda mod, args: (by_head(args[0]),))
+    else:
+        norm._compiled_call_impl = by_head   # what Module.compile() sets
+    try:
+        got = _head_norm(norm, x)
+        got.sum().backward()
+        calls, want = list(seen), norm(x)
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert all(s == (B, H, N, D) for s in calls) and len(calls) == (kind != "forward_of_another")
+    assert torch.equal(got, want) and got.is_contiguous()

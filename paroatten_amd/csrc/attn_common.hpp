@@ -36,7 +36,10 @@ struct AttnParams {
   int pacing;  // +1: paced launch asked for, -1: plain launch asked for, 0: the library chooses
   // Q as the 16-bit tensor (of the output's type; qs_* are its strides, q8 and q_scale are not read): the kernels quantise
   // the rows of their q-block themselves (QRows).  k_mean [B,Hkv,D] (may be null; with lse): the mean that has been taken
-  // off K, the row's log-sum-exp gets lse_dot_scale * q . k_mean
+  // off K, the row's log-sum-exp gets lse_dot_scale * q . k_mean.
+  // (Which of the two a kernel reads is a template parameter, Q16.  As a branch at run time it cost calls on INT8 Q 0.1 to 0.5 us
+  // in front of the loop, 1 to 2 % of those below 50 us: 48 heads, N = 1024, D = 64 9.07 / 8.92 us, 40 heads, N = 2048,
+  // D = 128 38.2 / 37.45, two heads, N = 4096 12.40 / 12.28 and 18.58 / 18.21; calls on 16-bit Q are the same.)
   const unsigned short* q16;
   const unsigned short* k_mean;
   float lse_dot_scale;

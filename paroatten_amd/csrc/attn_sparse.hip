@@ -72,9 +72,12 @@ template <int D> struct AttnLds {
 // 2 (lane % 4) + 1 of every 8-wide tile).  Here a lane holds one q-row, so its q scale is its own, and of its
 // 32 keys per block (offsets 4 lh + i % 4 within every group of 8) the even pair i % 4 < 2 has k scale 2 lh and
 // the odd pair 2 lh + 1: two affine maps from score to exponent per block instead of one.
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED>
+//
+// Q16: Q as 16-bit rows (AttnParams::q16).
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED, bool Q16>
 __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) {
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
+  static_assert(!Q16 || (!PT && !DUMP), "16-bit queries: neither per-thread scales nor the score dump");
   using Lds = AttnLds<D>;
   constexpr int CW = PT ? 4 : 1;    // k scales per key block
   constexpr int KS = D / 32;        // k-steps of the QK MFMA (32 channels each)
@@ -144,14 +147,14 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   const int qrow = qb * 64 + wave * 32 + l32;
   v4i qf[KS];
   float qsc = 0.f;
-  QRows<OUT_DT, D> q16;
+  [[maybe_unused]] QRows<OUT_DT, D> q16;
   {
     // rows past the end re-read the last row; their results are never stored
     const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
-    const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave;
-    if (!PT && p.q16 != nullptr) {
+    if constexpr (Q16) {
       q16.load(p.q16 + qoff);
     } else {
+      const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
       qsc = PT ? p.q_scale[qs_group * 8 + (l32 & 7)] : p.q_scale[qs_group];
@@ -339,14 +342,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     load_v(kb_1, 1);
   }
   // (Q from 16 bits: quantised while the tiles are on their way)
-  if constexpr (!PT) {
-    if (p.q16 != nullptr) {
-      qsc = q16.quantise(qf);
-      if constexpr (LSE) {
-        if (p.k_mean != nullptr) {
-          const float d = q16.dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
-          if (lh == 0 && qrow < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = d;
-        }
+  if constexpr (Q16) {
+    qsc = q16.quantise(qf);
+    if constexpr (LSE) {
+      if (p.k_mean != nullptr) {
+        const float d = q16.dot(p.k_mean + bhk * D + 16 * lh) * p.lse_dot_scale;
+        if (lh == 0 && qrow < p.Nq) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = d;
       }
     }
   }
@@ -692,12 +693,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   }
 }
 
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
 __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_kernel(const AttnParams p) {
   // hardware deals workgroup ids round-robin to the 8 XCDs
   const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
-  attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false>(p, vid);
+  attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false, Q16>(p, vid);
 }
 
 // The same work with a resident set of workgroups per XCD that take the XCD's q-blocks generation by
@@ -720,7 +721,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
 // q-blocks of equal length, sorted by a pre-pass over the mask, changed nothing: a workgroup that waits leaves
 // the matrix pipe to its neighbours on the compute unit, so the waiting itself costs little.)
 constexpr int PACE_PAD = 32;   // counters 128 bytes apart: one per XCD
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
 __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
     attn_sparse_paced_kernel(const AttnParams p, unsigned* __restrict__ counters, const int per, const int spin_limit,
                              const int slack) {
@@ -729,7 +730,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
   bool waiting = true;   // a workgroup that has once waited in vain goes on without waiting for the rest of the launch
   for (int base = 0; base < per; base += G) {
     const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
-    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true>(p, vid);
+    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true, Q16>(p, vid);
     if (base + G >= per) break;
     // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
     __syncthreads();   // also: both waves are done with this q-block's lists in LDS
@@ -836,11 +837,11 @@ static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
   return !per_thread || (D == 64 ? attn_smem<64>(p.nbk, true) : attn_smem<128>(p.nbk, true)) <= 40 * 1024;
 }
 
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT = false>
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
 static int launch_attn(const AttnParams& p, hipStream_t st) {
   const size_t smem = attn_smem<D>(p.nbk, PT);
   if (!DUMP && want_pacing(p, D, CAUSAL, EXACT) && pace_list_fits(p, D, PT)) {
-    auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>;
+    auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, Q16>;
     if (smem > 48 * 1024)
       PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     PaceDevice pd;
@@ -868,7 +869,7 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
     }
   }
   const int grid = ((p.total + 7) / 8) * 8;
-  auto kern = attn_sparse_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT>;
+  auto kern = attn_sparse_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, Q16>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(128), smem, st, p);
@@ -880,29 +881,39 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
 template <int D, int OUT_DT>
 static int dispatch_attn_per_thread(const AttnParams& p, int is_causal, bool exact, hipStream_t st) {
   if (p.lse != nullptr)
-    return is_causal ? launch_attn<D, OUT_DT, true, false, true, true, true>(p, st)
-                     : launch_attn<D, OUT_DT, false, false, true, true, true>(p, st);
+    return is_causal ? launch_attn<D, OUT_DT, true, false, true, true, true, false>(p, st)
+                     : launch_attn<D, OUT_DT, false, false, true, true, true, false>(p, st);
   if (exact)
-    return is_causal ? launch_attn<D, OUT_DT, true, false, false, true, true>(p, st)
-                     : launch_attn<D, OUT_DT, false, false, false, true, true>(p, st);
-  return is_causal ? launch_attn<D, OUT_DT, true, false, false, false, true>(p, st)
-                   : launch_attn<D, OUT_DT, false, false, false, false, true>(p, st);
+    return is_causal ? launch_attn<D, OUT_DT, true, false, false, true, true, false>(p, st)
+                     : launch_attn<D, OUT_DT, false, false, false, true, true, false>(p, st);
+  return is_causal ? launch_attn<D, OUT_DT, true, false, false, false, true, false>(p, st)
+                   : launch_attn<D, OUT_DT, false, false, false, false, true, false>(p, st);
 }
 
-template <int D, int OUT_DT>
+template <int D, int OUT_DT, bool Q16>
 static int dispatch_attn(const AttnParams& p, int is_causal, bool dump, bool exact, hipStream_t st) {
   // the log-sum-exp needs true exponentials; the debug dump rides on the same instantiation
   if (p.lse != nullptr || dump) {
-    if (dump) return is_causal ? launch_attn<D, OUT_DT, true, true, true, true>(p, st)
-                               : launch_attn<D, OUT_DT, false, true, true, true>(p, st);
-    return is_causal ? launch_attn<D, OUT_DT, true, false, true, true>(p, st)
-                     : launch_attn<D, OUT_DT, false, false, true, true>(p, st);
+    if constexpr (!Q16)
+      if (dump) return is_causal ? launch_attn<D, OUT_DT, true, true, true, true, false, false>(p, st)
+                                 : launch_attn<D, OUT_DT, false, true, true, true, false, false>(p, st);
+    return is_causal ? launch_attn<D, OUT_DT, true, false, true, true, false, Q16>(p, st)
+                     : launch_attn<D, OUT_DT, false, false, true, true, false, Q16>(p, st);
   }
   if (exact)
-    return is_causal ? launch_attn<D, OUT_DT, true, false, false, true>(p, st)
-                     : launch_attn<D, OUT_DT, false, false, false, true>(p, st);
-  return is_causal ? launch_attn<D, OUT_DT, true, false, false, false>(p, st)
-                   : launch_attn<D, OUT_DT, false, false, false, false>(p, st);
+    return is_causal ? launch_attn<D, OUT_DT, true, false, false, true, false, Q16>(p, st)
+                     : launch_attn<D, OUT_DT, false, false, false, true, false, Q16>(p, st);
+  return is_causal ? launch_attn<D, OUT_DT, true, false, false, false, false, Q16>(p, st)
+                   : launch_attn<D, OUT_DT, false, false, false, false, false, Q16>(p, st);
+}
+
+template <int D>
+static int dispatch_attn(const AttnParams& p, int out_dtype, int is_causal, bool dump, bool exact, hipStream_t st) {
+  if (p.q16 != nullptr)   // (no dump with them)
+    return out_dtype == PARO_DTYPE_F16 ? dispatch_attn<D, PARO_DTYPE_F16, true>(p, is_causal, false, exact, st)
+                                       : dispatch_attn<D, PARO_DTYPE_BF16, true>(p, is_causal, false, exact, st);
+  return out_dtype == PARO_DTYPE_F16 ? dispatch_attn<D, PARO_DTYPE_F16, false>(p, is_causal, dump, exact, st)
+                                     : dispatch_attn<D, PARO_DTYPE_BF16, false>(p, is_causal, dump, exact, st);
 }
 
 // Whether the two-wave kernel is the faster one for so few q-blocks at D = 64.  Up to one q-block per SIMD the latency of a
@@ -1020,12 +1031,8 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
     case PARO_ATTN_FORM_ONE_WAVE: return launch_attn_w64(p, out_dtype, is_causal != 0, exact, st);
     default: break;   // two waves per q-block, below; launch_attn chooses plain or paced
   }
-  if (D == 64) {
-    if (out_dtype == PARO_DTYPE_F16) return dispatch_attn<64, PARO_DTYPE_F16>(p, is_causal, dump, exact, st);
-    return dispatch_attn<64, PARO_DTYPE_BF16>(p, is_causal, dump, exact, st);
-  }
-  if (out_dtype == PARO_DTYPE_F16) return dispatch_attn<128, PARO_DTYPE_F16>(p, is_causal, dump, exact, st);
-  return dispatch_attn<128, PARO_DTYPE_BF16>(p, is_causal, dump, exact, st);
+  return D == 64 ? dispatch_attn<64>(p, out_dtype, is_causal, dump, exact, st)
+                 : dispatch_attn<128>(p, out_dtype, is_causal, dump, exact, st);
 }
 }  // namespace paro
 

@@ -76,7 +76,7 @@ __device__ __forceinline__ void qk_first(v16i (&acc)[2], const v4i& k0, const v4
       : "=&v"(acc[0]), "=&v"(acc[1]) : "v"(k0), "v"(k1), "v"(q));
 }
 
-template <int D, int OUT_DT, bool LSE>
+template <int D, int OUT_DT, bool LSE, bool Q16>
 __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kernel(const AttnParams p, const int causal) {
   using Lds = Pv16Lds<D>;
   constexpr int KS = D / 32;         // k-steps of the QK MFMA
@@ -136,10 +136,10 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   const int qrow = qb * 64 + wave * 32 + l32;
   v4i qf[KS];
   float qsc = 0.f;
-  QRows<OUT_DT, D> q16;
+  [[maybe_unused]] QRows<OUT_DT, D> q16;
   {
     const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
-    if (p.q16 != nullptr) {
+    if constexpr (Q16) {
       q16.load(p.q16 + qoff);
     } else {
 #pragma unroll
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   load_k(kb_1, 1);
   load_v(kb_c, 0);
   // (Q from 16 bits: quantised while the tiles are on their way)
-  if (p.q16 != nullptr) {
+  if constexpr (Q16) {
     qsc = q16.quantise(qf);
     if constexpr (LSE) {
       if (p.k_mean != nullptr) {
@@ -440,13 +440,13 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   }
 }
 
-template <int D, int OUT_DT, bool LSE>
+template <int D, int OUT_DT, bool LSE, bool Q16>
 static int launch_pv16(const AttnParams& p, bool causal, hipStream_t st) {
   const size_t smem = Pv16Lds<D>::LIST_OFF + (((size_t)(p.nbk + Pv16Lds<D>::LIST_PAD + 1) * 6 + 15) & ~(size_t)15);
   PARO_CHECK(smem <= 160 * 1024, PARO_ERR_RUNTIME, "kv_len %d: the list of %d key blocks does not fit the local data share",
              p.Nk, p.nbk);
   const int grid = ((p.total + 7) / 8) * 8;
-  auto kern = attn_sparse_pv16_kernel<D, OUT_DT, LSE>;
+  auto kern = attn_sparse_pv16_kernel<D, OUT_DT, LSE, Q16>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(128), smem, st, p, causal ? 1 : 0);
@@ -456,7 +456,9 @@ static int launch_pv16(const AttnParams& p, bool causal, hipStream_t st) {
 
 template <int D, int OUT_DT>
 static int dispatch_pv16(const AttnParams& p, bool causal, hipStream_t st) {
-  return p.lse != nullptr ? launch_pv16<D, OUT_DT, true>(p, causal, st) : launch_pv16<D, OUT_DT, false>(p, causal, st);
+  if (p.q16 != nullptr)
+    return p.lse != nullptr ? launch_pv16<D, OUT_DT, true, true>(p, causal, st) : launch_pv16<D, OUT_DT, false, true>(p, causal, st);
+  return p.lse != nullptr ? launch_pv16<D, OUT_DT, true, false>(p, causal, st) : launch_pv16<D, OUT_DT, false, false>(p, causal, st);
 }
 
 int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hipStream_t st) {

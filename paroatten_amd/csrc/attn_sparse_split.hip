@@ -29,7 +29,7 @@ template <int D, int W> struct SplitLds {
   static constexpr int LIST_PAD = 4 * W;                         // a wave looks up to 4 rounds ahead
 };
 
-template <int D, int OUT_DT, bool LSE, bool EXACT, int W>
+template <int D, int OUT_DT, bool LSE, bool EXACT, int W, bool Q16>
 __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const AttnParams p, const int causal) {
   using Lds = SplitLds<D, W>;
   constexpr int KS = D / 32;      // k-steps of the QK product
@@ -83,10 +83,10 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   const int qrow = qb * 64 + half * 32 + l32;
   v4i qf[KS];
   float qsc = 0.f;
-  QRows<OUT_DT, D> q16;
+  [[maybe_unused]] QRows<OUT_DT, D> q16;
   {
     const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow, p.Nq - 1) * p.qs_n + 16 * lh;
-    if (p.q16 != nullptr) {
+    if constexpr (Q16) {
       q16.load(p.q16 + qoff);
     } else {
 #pragma unroll
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
 
   // ---- prologue: round 0's scores ----
   auto quantise_q = [&]() __attribute__((always_inline)) {   // (Q from 16 bits: while the tiles are on their way)
-    if (p.q16 != nullptr) {
+    if constexpr (Q16) {
       qsc = q16.quantise(qf);
       if constexpr (LSE) {
         if (wave == 0 && p.k_mean != nullptr) {
@@ -454,12 +454,12 @@ static size_t split_lds(int nbk, int W) {
   return list + (((size_t)(nbk + 4 * W + 1) * 6 + 15) & ~(size_t)15);
 }
 
-template <int D, int OUT_DT, int W>
+template <int D, int OUT_DT, int W, bool Q16>
 static int launch_split(const AttnParams& p, bool causal, bool exact, hipStream_t st) {
   const size_t smem = split_lds<D>(p.nbk, W);
-  auto kern = p.lse != nullptr ? attn_sparse_split_kernel<D, OUT_DT, true, true, W>
-              : exact          ? attn_sparse_split_kernel<D, OUT_DT, false, true, W>
-                               : attn_sparse_split_kernel<D, OUT_DT, false, false, W>;
+  auto kern = p.lse != nullptr ? attn_sparse_split_kernel<D, OUT_DT, true, true, W, Q16>
+              : exact          ? attn_sparse_split_kernel<D, OUT_DT, false, true, W, Q16>
+                               : attn_sparse_split_kernel<D, OUT_DT, false, false, W, Q16>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3(((2 * p.total + 7) / 8) * 8), dim3(64 * W), smem, st, p, causal ? 1 : 0);
@@ -493,10 +493,13 @@ int split_width(const AttnParams& p, int D) {
 
 int launch_attn_split(const AttnParams& p, int D, int out_dtype, bool causal, bool exact, hipStream_t st) {
   const int W = split_width(p, D);
-#define PARO_SPLIT(DV, OV) (W == 4 ? launch_split<DV, OV, 4>(p, causal, exact, st) : launch_split<DV, OV, 2>(p, causal, exact, st))
+#define PARO_SPLIT_Q(DV, OV, QV) \
+  (W == 4 ? launch_split<DV, OV, 4, QV>(p, causal, exact, st) : launch_split<DV, OV, 2, QV>(p, causal, exact, st))
+#define PARO_SPLIT(DV, OV) (p.q16 != nullptr ? PARO_SPLIT_Q(DV, OV, true) : PARO_SPLIT_Q(DV, OV, false))
   if (D == 64) return out_dtype == PARO_DTYPE_F16 ? PARO_SPLIT(64, PARO_DTYPE_F16) : PARO_SPLIT(64, PARO_DTYPE_BF16);
   return out_dtype == PARO_DTYPE_F16 ? PARO_SPLIT(128, PARO_DTYPE_F16) : PARO_SPLIT(128, PARO_DTYPE_BF16);
 #undef PARO_SPLIT
+#undef PARO_SPLIT_Q
 }
 
 }  // namespace paro

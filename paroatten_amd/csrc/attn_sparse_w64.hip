@@ -50,7 +50,7 @@ __device__ __forceinline__ int lane_here() {
   return x;
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE, bool Q16>
 __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int vid) {
   using Lds = W64Lds;
   constexpr int D = 64;
@@ -103,13 +103,13 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   int qrow[2];
   v4i qf[2][2];
   float qsc[2];
-  QRows<OUT_DT, D> q16[2];
+  [[maybe_unused]] QRows<OUT_DT, D> q16[2];
 #pragma unroll
   for (int hf = 0; hf < 2; hf++) {
     qrow[hf] = qb * 64 + hf * 32 + l32;
     // rows past the end re-read the last row; their results are never stored
     const int64_t qoff = b * p.qs_b + h * p.qs_h + (int64_t)min(qrow[hf], p.Nq - 1) * p.qs_n + 16 * lh;
-    if (p.q16 != nullptr) {
+    if constexpr (Q16) {
       q16[hf].load(p.q16 + qoff);
     } else {
 #pragma unroll
@@ -488,7 +488,7 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   load_v(kb_c, 0);
   load_v(kb_1, 1);
   // (Q from 16 bits: quantised while the tiles are on their way)
-  if (p.q16 != nullptr) {
+  if constexpr (Q16) {
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
       qsc[hf] = q16[hf].quantise(qf[hf]);
@@ -589,19 +589,19 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
   }
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE, bool Q16>
 __global__ void __launch_bounds__(64, 2) attn_sparse_w64_kernel(const AttnParams p) {
   // hardware deals workgroup ids round-robin to the 8 XCDs
   const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
-  attn_qblock_w64<OUT_DT, CAUSAL, EXACT, LSE>(p, vid);
+  attn_qblock_w64<OUT_DT, CAUSAL, EXACT, LSE, Q16>(p, vid);
 }
 
-template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE>
+template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE, bool Q16>
 static int launch_w64(const AttnParams& p, hipStream_t st) {
   const size_t smem = W64Lds::LIST_OFF + (((size_t)(p.nbk + W64Lds::LIST_PAD + 1) * 6 + 15) & ~(size_t)15);
   const int grid = ((p.total + 7) / 8) * 8;
-  auto kern = attn_sparse_w64_kernel<OUT_DT, CAUSAL, EXACT, LSE>;
+  auto kern = attn_sparse_w64_kernel<OUT_DT, CAUSAL, EXACT, LSE, Q16>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64), smem, st, p);
@@ -609,16 +609,21 @@ static int launch_w64(const AttnParams& p, hipStream_t st) {
   return PARO_OK;
 }
 
-template <int OUT_DT>
+template <int OUT_DT, bool Q16>
 static int dispatch_w64(const AttnParams& p, bool causal, bool exact, hipStream_t st) {
-  if (p.lse != nullptr) return causal ? launch_w64<OUT_DT, true, true, true>(p, st) : launch_w64<OUT_DT, false, true, true>(p, st);
-  if (exact) return causal ? launch_w64<OUT_DT, true, true, false>(p, st) : launch_w64<OUT_DT, false, true, false>(p, st);
-  return causal ? launch_w64<OUT_DT, true, false, false>(p, st) : launch_w64<OUT_DT, false, false, false>(p, st);
+  if (p.lse != nullptr)
+    return causal ? launch_w64<OUT_DT, true, true, true, Q16>(p, st) : launch_w64<OUT_DT, false, true, true, Q16>(p, st);
+  if (exact)
+    return causal ? launch_w64<OUT_DT, true, true, false, Q16>(p, st) : launch_w64<OUT_DT, false, true, false, Q16>(p, st);
+  return causal ? launch_w64<OUT_DT, true, false, false, Q16>(p, st) : launch_w64<OUT_DT, false, false, false, Q16>(p, st);
 }
 
 int launch_attn_w64(const AttnParams& p, int out_dtype, bool causal, bool exact, hipStream_t st) {
-  return out_dtype == PARO_DTYPE_F16 ? dispatch_w64<PARO_DTYPE_F16>(p, causal, exact, st)
-                                     : dispatch_w64<PARO_DTYPE_BF16>(p, causal, exact, st);
+  if (p.q16 != nullptr)
+    return out_dtype == PARO_DTYPE_F16 ? dispatch_w64<PARO_DTYPE_F16, true>(p, causal, exact, st)
+                                       : dispatch_w64<PARO_DTYPE_BF16, true>(p, causal, exact, st);
+  return out_dtype == PARO_DTYPE_F16 ? dispatch_w64<PARO_DTYPE_F16, false>(p, causal, exact, st)
+                                     : dispatch_w64<PARO_DTYPE_BF16, false>(p, causal, exact, st);
 }
 
 }  // namespace paro

@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(256) op_prep_short_kernel(const OpParams p) {
 // N = 4096 2 heads 26.6 / 24.6, 24 heads 63.1 / 59.6, 96 heads 182.2 / 180.5; N = 8192 8 heads 68.9 / 67.2, 48 heads 288.8 / 289.9;
 // D = 128 N = 4096 2 heads 35.0 / 33.7, 48 heads 183.6 / 183.8; N = 8192 2 heads 60.2 / 59.2, 24 heads 288.3 / 292.9.
 static bool op_short(int64_t BK, int Nk, int D, bool per_thread) {
-  return !per_thread && Nk > OP_HEAD_TOKENS && (Nk <= 4096 || (Nk <= 8192 && BK * D <= 512));
+  return !per_thread && (Nk <= 4096 || (Nk <= 8192 && BK * D <= 512));
 }
 
 // Where the intermediate tensors lie in the workspace (256-byte aligned pieces).
@@ -492,6 +492,33 @@ struct OpLayout {
     resid = take(s ? BK * nbk * 2 * D * 4 : 0);   // (the chunks in v_work are read until the last tile)
   }
 };
+
+// Whether op_head does it all, and how it divides K (op_prep_short is what it stands against).  A compute unit holds one of its
+// workgroups (16 waves of 92 to 101 registers), so what counts is how many rounds of 256 they come to.  K by 256 tokens is
+// taken where all fit into one round.  Otherwise a workgroup takes the K of a whole head (with smooth_k all of those that share
+// a head would read it all for the mean): in one round up to 768 tokens, beyond that not where such a workgroup has the
+// longest time of its own (D = 128 with the mean) nor with float16 tiles; in two rounds up to 512 tokens, beyond that at D = 64
+// where the second is more than half full.  Without the mean two rounds of 256 tokens are the better ones up to 768 tokens.
+// Operator, us, op_prep_short / op_head:
+//   smooth_k       D = 64   N = 512   60 heads 21.1 / 16.2   85 heads 23.1 / 18.5   100 heads 24.4 / 24.5   170 heads 30.9 / 29.6
+//                           N = 1024  32 heads 23.5 / 22.9   85 heads 33.3 / 30.9   100 heads 38.3 / 40.0   170 heads 54.6 / 53.0
+//                  D = 128  N = 320   43 heads 25.7 / 21.2   85 heads 30.3 / 29.4   100 heads 31.3 / 31.8
+//                           N = 1024  16 heads 29.4 / 25.8   43 heads 37.1 / 39.2    60 heads 44.4 / 50.2   100 heads 67.1 / 72.7
+//   without (and with K by 256 tokens in two or three rounds)
+//                  D = 64   N = 1024  60 heads 27.6 / 26.0 (27.5)   100 heads 36.4 / 37.0 (37.7)
+//                  D = 128  N = 512   70 heads 31.7 / 31.5 (30.5)   N = 1024 51 heads 37.5 / 36.8 (44.0)
+//   float16 tiles  D = 64   N = 700   64 heads 26.0 / 24.6   90 heads 28.8 / 34.3
+//                  D = 128  N = 384   90 heads 34.7 / 29.8   N = 1024 43 heads 39.1 / 43.3
+static void op_head_plan(OpParams& p, int64_t BK, int D, bool per_thread, bool f16v) {
+  const int64_t k_parts = ceil_div(p.nbk, 4), v_parts = f16v ? k_parts : D / 32, by_tokens = BK * (k_parts + v_parts),
+                by_heads = BK * (1 + v_parts);
+  bool fits = by_tokens <= 256 || (by_tokens <= 512 && by_heads > 256 && !p.stats_k && p.Nk <= 768);
+  p.k_rounds = fits ? 1 : (int)k_parts;
+  if (!fits && by_heads <= 256) fits = p.Nk <= 768 || (!f16v && (D == 64 || !p.stats_k));
+  else if (!fits && by_heads <= 512) fits = p.Nk <= 512 || (!f16v && D == 64 && by_heads > 400);
+  p.k_parts = ceil_div(p.nbk, 4 * p.k_rounds);
+  p.one_launch = fits && !per_thread && p.Nk <= OP_HEAD_TOKENS && p.stats_k + p.stats_v > 0;
+}
 
 template <int DT, int D, bool F16V>
 static int launch_op_head(const OpParams& p, hipStream_t st) {
@@ -584,15 +611,8 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   p.stats_k = smooth_k != 0; p.stats_v = !f16v;
   p.kv_blocks = B * Hkv * (p.nbk + ceil_div(p.nbk, 4));
   p.sm_scale = sm_scale;
-  const int64_t BK = (int64_t)B * Hkv, v_parts = f16v ? ceil_div(p.nbk, 4) : D / 32;
-  // op_head: its workgroups have to run at the same time, two to a compute unit.  K's take 256 tokens each as long as all of
-  // them find a compute unit to themselves, and otherwise a whole head, since with smooth_k each reads all of it for the mean:
-  // 48 heads, N = 1024, D = 64 24.6 us by heads and 29.5 by 256 tokens, 32 heads 23.3 and 22.4; D = 128 48 heads 40.9 and 43.7,
-  // 24 heads 35.7 and 31.2
-  p.one_launch = !per_thread && Nk <= OP_HEAD_TOKENS && p.stats_k + p.stats_v > 0 && BK * (1 + v_parts) <= 512;
-  p.k_rounds = p.stats_k && BK * (ceil_div(p.nbk, 4) + v_parts) > 256 ? ceil_div(p.nbk, 4) : 1;
-  p.k_parts = ceil_div(p.nbk, 4 * p.k_rounds);
-  p.short_prep = op_short(BK, Nk, D, per_thread);
+  op_head_plan(p, (int64_t)B * Hkv, D, per_thread, f16v);
+  p.short_prep = op_short((int64_t)B * Hkv, Nk, D, per_thread);
   if (p.short_prep && p.v_resid) p.v_resid = (float*)(ws + at.resid);
   hipStream_t st = (hipStream_t)stream;
   int rc;

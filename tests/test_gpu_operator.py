@@ -60,12 +60,15 @@ def test_operator_equals_the_chain_of_its_parts(dev, N, D, layout, groups, mode,
     (1023, 64, 3, "fp8"), (1024, 64, 3, "fp8"), (1024, 128, 3, "fp8"),
     (1025, 64, 3, "fp8"), (2000, 64, 3, "f16"), (4096, 128, 3, "fp8"), (4097, 64, 3, "fp8"), (8192, 64, 9, "fp8"),
     (1000, 64, 60, "fp8"), (1024, 128, 60, "f16"), (700, 128, 60, "fp8"), (300, 128, 110, "fp8"), (300, 64, 180, "fp8"),
+    (1024, 64, 42, "fp8"), (1024, 64, 43, "fp8"), (1024, 64, 86, "fp8"), (1024, 64, 150, "fp8"), (769, 128, 51, "fp8"),
+    (512, 128, 102, "fp8"), (513, 128, 52, "fp8"), (768, 64, 64, "f16"), (769, 64, 51, "f16"), (512, 128, 170, "f16"), (1, 64, 180, "fp8"),
 ])
 @pytest.mark.parametrize("smooth_k,smooth_v", [(False, True), (True, True), (True, False)])
 def test_one_launch_preparation_equals_the_separate_ones(dev, N, D, H, mode, smooth_k, smooth_v):
     """Edges of the 64-token tiles, the 256-token chunks and the 1024 tokens of the one-launch preparation; K by 256 tokens
-    (3 heads), by heads (60) and separate launches (110, 180); beyond, the preparation that adds up the chunks itself, at its
-    edges of 4096 and (512 channels) 8192 tokens.  K's sums are exact, V is arbitrary: the same bits."""
+    (3 heads, 42 at N = 1024), by heads (43, 60; in two rounds 102, 150), and more heads than it takes; there and beyond, the
+    preparation that adds up the chunks itself, at its edges of 4096 and (512 channels) 8192 tokens.  K's sums are exact, V is
+    arbitrary: the same bits."""
     import paroatten_amd as P
     from paroatten_amd import _qattn_sm80 as qattn
     from paroatten_amd import quant as Q

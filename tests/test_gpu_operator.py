@@ -150,3 +150,45 @@ def test_queries_quantised_by_every_kernel_form(dev, monkeypatch, H, N, D, form,
     assert torch.equal(got[0] if lse else got, o_ref)
     if lse:
         assert torch.equal(got[1], lse2 * 0.6931471805599453)
+
+
+@pytest.mark.parametrize("B,H,Hkv,N,D,form,causal", [
+    (1, 4, 2, 1345, 64, "SPLIT", False), (2, 3, 1, 1345, 128, "SPLIT", True), (2, 15, 5, 700, 64, "TWO_WAVES", False),
+    (3, 20, 10, 700, 128, "TWO_WAVES", True), (3, 25, 5, 1345, 64, "ONE_WAVE", False), (2, 100, 25, 1345, 64, "ONE_WAVE", True),
+    (3, 30, 6, 1345, 64, "PACED", False), (3, 32, 8, 1345, 64, "PACED", True), (2, 30, 10, 1345, 128, "PACED", False),
+    (2, 6, 2, 700, 64, "PV_F16", False), (2, 6, 3, 700, 128, "PV_F16", True),
+])
+def test_log_sum_exp_with_the_k_mean_in_every_kernel_form(dev, monkeypatch, B, H, Hkv, N, D, form, causal):
+    """sm_scale * q . k_mean, which the attention kernels put into the row of the log-sum-exp before their loop and add to at
+    its end: every form, grouped heads in a batch (the mean is that of the row's key head), token-major, a last q-block of
+    one row (N = 1345) and an empty row of the mask.  K's sums are exact, so that its mean, and the outputs, are the same bits."""
+    import paroatten_amd as P
+    from paroatten_amd import _lib
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    pv_f16 = form == "PV_F16"
+    if form == "PACED":
+        monkeypatch.setenv("PARO_ATTN_PACING", "1")
+    flags = qattn._flags(False, None, False, pv_f16)
+    assert _lib.load().paro_attn_kernel_form(B, H, N, N, D, int(causal), 1, flags) == getattr(_lib, "PARO_ATTN_FORM_" + form)
+    dtype = torch.float16 if D == 64 else torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(N + D + H)
+    q, v = (torch.randn(B, N, h, D, generator=g, device=dev).to(dtype) for h in (H, Hkv))
+    k = ((torch.randint(-40, 41, (B, N, Hkv, D), generator=g, device=dev)
+          + torch.randint(-20, 21, (B, 1, Hkv, D), generator=g, device=dev)) / 8).to(dtype)
+    mask = synth.make_block_mask(H, (N + 63) // 64, 0.4, seed=N, device=dev)
+    mask[1, 2] = False
+    km = k.double().mean(dim=1, keepdim=True).float().to(dtype)
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, km, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="NHD")
+    o_ref = torch.empty_like(q)
+    lse2 = qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, 0, int(causal), 2, D ** -0.5, 1, mask, pv_f16=pv_f16)
+    o, lse = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, tensor_layout="NHD", is_causal=causal, smooth_k=True,
+                                             return_lse=True, pv_f16=pv_f16)
+    assert torch.equal(o, o_ref)
+    terms = q.transpose(1, 2).double() * km.transpose(1, 2).repeat_interleave(H // Hkv, dim=1).double()
+    want = lse2.double() * 0.6931471805599453 + terms.sum(-1) * D ** -0.5
+    empty = lse2 == -float("inf")
+    assert empty[:, 1, 128:192].all() and torch.equal(lse == -float("inf"), empty)
+    # one product and one sum in fp32, and an fp32 dot product of D terms
+    bound = (D + 4) * 2.0 ** -24 * (lse2.double().abs() + terms.abs().sum(-1) * D ** -0.5)
+    assert ((lse.double() - want).abs() <= bound)[~empty].all()

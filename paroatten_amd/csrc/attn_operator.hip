@@ -1,13 +1,15 @@
 // The whole attention operator on 16-bit q, k, v in one call: INT8 quantisation of Q and K (K's token mean taken off
-// first if asked for), the V conversion, block-sparse attention.  Five launches:
+// first if asked for), the V conversion, block-sparse attention.  Two to five launches:
 //   op_stats     K sums (smooth_k) and V statistics (FP8 product), side by side
 //   op_finalize  their second steps
 //   op_prep      quantised K and the V tiles, side by side (per-thread scales: quantised Q too)
 //   v_residual   (FP8 product with smooth_v)
-// (op_head, one launch, in the place of these for up to 1024 tokens; op_prep_short in that of the second and third beyond)
 //   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; per-thread scales: on INT8 Q); the
 //                log-sum-exp leaves as the natural one of the scores of q and k as given
-// The first four are bound by HBM: at B = 2, H = 48, N = 17776, D = 64 they move 16-bit K and V twice and write their 8-bit
+// Short sequences take one launch for the first four (op_head: up to 1024 tokens, as many heads as op_head_plan says) or one for
+// the second and third (op_prep_short: the rest up to 4096 tokens, op_short).  Calls with nothing to sum up (float16 product
+// without smooth_k) have op_prep and the attention alone, and those with per-thread scales all five.
+// The first four are bound by HBM where they are long: at B = 2, H = 48, N = 17776, D = 64 they move 16-bit K and V twice and write their 8-bit
 // forms, 1.09 GB.  Q as a pass in op_prep moved 3 bytes per element and the attention launch read a fourth; quantised there,
 // behind the requests for the first tiles, start to end of the operator: 1521 -> 1488 us at that shape, 212 -> 205 us at
 // N = 8192, B = 1, 502 -> 494 us at N = 9001 with the log-sum-exp, 655 -> 636 us at B = 2, H = 32, Hkv = 8, N = 8192, D = 128, causal,
@@ -38,9 +40,9 @@ struct OpParams {
   int stats_k, stats_v;         // which statistics are taken
   int kv_blocks;                // workgroups of op_prep that take K or V; the rest (per-thread scales) take Q
   float sm_scale;
-  bool one_launch;              // op_head does it all
-  bool short_prep;              // op_prep_short does what comes after the statistics
-  int k_parts, k_rounds;        // of it: workgroups that share the K of a head, 256 tokens they take one after the other
+  bool one_launch;              // op_head does it all (op_head_plan)
+  int k_parts, k_rounds;        // of op_head: workgroups that share the K of a head, 256 tokens they take one after the other
+  bool short_prep;              // op_prep_short does what comes after the statistics (op_short)
 };
 
 template <int DT, int D>
@@ -110,15 +112,15 @@ __global__ void __launch_bounds__(256) op_prep_kernel(const OpParams p) {
 
 // Everything in front of the attention launch, up to OP_HEAD_TOKENS tokens, in one launch: such a call consists of launches of
 // a few microseconds that wait for each other, not of bytes.  Workgroups of 16 waves that need nothing of each other:
-//   V: 32 channels of a (batch, kv-head) over all tokens, read once and held in registers between the statistics and the
-//      codes.  A lane has two channels of four neighbouring tokens, which are a word of the tiles each.
+//   V: 32 channels of a (batch, kv-head) over all tokens, read once and kept in LDS for the statistics and the codes.  A lane
+//      has two channels of four neighbouring tokens, which are a word of the tiles each.
 //   K: four 64-token groups, four waves to each; with smooth_k every workgroup takes the mean over all tokens for itself.
 // What bounds it is the vector work and the latencies of one compute unit: with one workgroup to K and one to V of a head the
-// launch took 10.5 us at N = 416, D = 64, two heads, 3 of them for adding up across lanes and 4 for the codes of V; this way
-// 5.8.  The operator, start to end, separate launches / this one, smooth_k, us:
+// launch took 4.7 us longer at N = 416, D = 64, two heads, for adding up across lanes and for the codes of V; this way it
+// is 7.1 us (6.6 at the least) in a kernel trace.  The operator, start to end, separate launches / this one, smooth_k, us:
 //   D = 64   N = 416   2 heads 19.4 / 13.2   16 heads 20.7 / 13.4     D = 128  N = 512   8 heads 24.9 / 18.4   48 heads 31.5 / 26.0
-//            N = 1024  8 heads 22.6 / 19.9   48 heads 29.6 / 24.6              N = 1024  8 heads 29.4 / 25.2   48 heads 45.8 / 40.6
-//            N = 1024 160 heads 63.0 / 54.1                                    N = 1024 96 heads 75.0 / 73.4
+//            N = 1024  8 heads 22.6 / 19.9   48 heads 29.6 / 24.6              N = 1024  8 heads 29.4 / 25.2   24 heads 34.0 / 31.5
+// (which calls: op_head_plan)
 constexpr int OP_HEAD_TOKENS = 1024;
 
 template <int DT, int D, bool F16V>
@@ -460,7 +462,8 @@ __global__ void __launch_bounds__(256) op_prep_short_kernel(const OpParams p) {
 }
 
 // What a launch less is worth, 2 to 3 us, against the chunks (768 bytes per 256 tokens, of V at D = 64) that every workgroup
-// reads.  Operator, smooth_k, with op_finalize / without it, us: D = 64 N = 1100 2 heads 22.2 / 20.0, 96 heads 44.2 / 41.1;
+// reads.  Operator, smooth_k, with op_finalize / without it, us: D = 64 N = 320 256 heads 32.9 / 29.7, N = 1024 100 heads 42.0 /
+// 38.5 (D = 128 70.6 / 67.0); N = 1100 2 heads 22.2 / 20.0, 96 heads 44.2 / 41.1;
 // N = 4096 2 heads 26.6 / 24.6, 24 heads 63.1 / 59.6, 96 heads 182.2 / 180.5; N = 8192 8 heads 68.9 / 67.2, 48 heads 288.8 / 289.9;
 // D = 128 N = 4096 2 heads 35.0 / 33.7, 48 heads 183.6 / 183.8; N = 8192 2 heads 60.2 / 59.2, 24 heads 288.3 / 292.9.
 static bool op_short(int64_t BK, int Nk, int D, bool per_thread) {

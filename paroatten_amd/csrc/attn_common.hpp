@@ -127,8 +127,7 @@ struct QRows {
     }
     return amax / 127.0f;
   }
-  // the row's product with w[0..D) (w: plus 16 (lane / 32)): eight neighbouring channels one after the other, fused, and the
-  // sums of eights added up in pairs, as quant_per_thread_body does
+  // the row's product with w[0..D) (w: plus 16 (lane / 32)), in the order of quant_group_body
   __device__ __forceinline__ float dot(const unsigned short* w) const {
     float t[D / 32];
 #pragma unroll

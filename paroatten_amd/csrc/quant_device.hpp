@@ -1,6 +1,5 @@
 // Bodies of the INT8 quantisation of Q and K as device functions, so that one launch can run several of them side by
-// side.  The launches that use them: quant_int8.hip (one tensor), attn_operator.hip (K and the V conversion; with per-thread
-// scales Q too, which otherwise the attention kernels quantise).
+// side.  The launches that use them: quant_int8.hip (one tensor), attn_operator.hip (Q, K and the V conversion).
 //
 // One 64-lane wave owns one group of G tokens x D channels: every lane holds G*D/64 values in
 // registers (16-byte loads, consecutive lanes on consecutive addresses), the group maximum is a
@@ -21,12 +20,14 @@ __device__ __forceinline__ void load8_f32(const unsigned short* p, float (&f)[8]
 }
 
 // Group g of one (batch, head): x, out and scale point at its first token, mean (MEAN) at its D channel means.
-// SMS: the values are multiplied by sm_scale first.
+// SMS: the values are multiplied by sm_scale first.  dot (may be null): dot[token] = sm_scale * x[token] . dot_with, in
+// fp32, for tokens below N (SMS and dot do not go together).
 template <int DT, int D, int G, bool MEAN, bool SMS>
 __device__ __forceinline__ void quant_group_body(const unsigned short* __restrict__ x,
                                                  const unsigned short* __restrict__ mean, int8_t* __restrict__ out,
                                                  float* __restrict__ scale, int N, int g, int64_t xs_n, int64_t os_n,
-                                                 float sm_scale) {
+                                                 float sm_scale, float* __restrict__ dot = nullptr,
+                                                 const unsigned short* __restrict__ dot_with = nullptr) {
   constexpr int LPR = D / 8;          // lanes per token row (16-byte chunks)
   constexpr int CH = G * D / 512;     // 16-byte chunks per lane
   constexpr int ROWS_PER_IT = 64 / LPR;
@@ -72,6 +73,24 @@ __device__ __forceinline__ void quant_group_body(const unsigned short* __restric
   if (lane == 0) scale[g] = amax / 127.0f;
   const float inv = 127.0f / amax;
 
+  if (dot != nullptr) {   // (uniform)
+    float w[8];
+    load8_f32<DT>(dot_with + col, w);
+#pragma unroll
+    for (int i = 0; i < CH; i++) {
+      float d = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; j++) d = fmaf(elem16_to_f32<DT>(raw[i], j), w[j], d);
+      // the LPR lanes of a row: lane ^ 1, ^ 2, then the other quad of eight, then the other eight of sixteen (mirrors)
+      d += row_dpp<0xB1>(d);
+      d += row_dpp<0x4E>(d);
+      d += row_dpp<0x141>(d);
+      if constexpr (LPR == 16) d += row_dpp<0x140>(d);
+      const int tok = g * G + i * ROWS_PER_IT + row0;
+      if (lane % LPR == 0 && tok < N) dot[tok] = d * sm_scale;
+    }
+  }
+
   int8_t* ob = out + col;
 #pragma unroll
   for (int i = 0; i < CH; i++) {
@@ -91,8 +110,7 @@ __device__ __forceinline__ void quant_group_body(const unsigned short* __restric
 // 32-token groups of 8) or 4 (K) scales.  Token row r of the 64 belongs to group
 //   Q: (r / 32) * 8 + r % 8        K: (r % 8) / 2
 // A lane's chunks sit in rows row0 + i * ROWS_PER_IT; every group maximum is a full wave reduction of the
-// lanes' contributions to that group (the kernel is bound by HBM, not by these).  dot (may be null): dot[token] =
-// sm_scale * x[token] . dot_with, in fp32, for tokens below N.
+// lanes' contributions to that group (the kernel is bound by HBM, not by these).
 template <int DT, int D, bool KEY, bool MEAN>
 __device__ __forceinline__ void quant_per_thread_body(const unsigned short* __restrict__ x,
                                                       const unsigned short* __restrict__ mean,
@@ -150,7 +168,7 @@ __device__ __forceinline__ void quant_per_thread_body(const unsigned short* __re
     for (int i = 0; i < CH; i++)
       if (group_of(i * ROWS_PER_IT + row0) == g) inv[i] = 127.0f / a;
   }
-  if (dot != nullptr) {   // (uniform)
+  if (dot != nullptr) {   // (uniform; as in quant_group_body)
     float wv[8];
     load8_f32<DT>(dot_with + col, wv);
 #pragma unroll
@@ -158,7 +176,6 @@ __device__ __forceinline__ void quant_per_thread_body(const unsigned short* __re
       float d = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; j++) d = fmaf(elem16_to_f32<DT>(raw[i], j), wv[j], d);
-      // the LPR lanes of a row: lane ^ 1, ^ 2, then the other quad of eight, then the other eight of sixteen (mirrors)
       d += row_dpp<0xB1>(d);
       d += row_dpp<0x4E>(d);
       d += row_dpp<0x141>(d);

@@ -2,9 +2,9 @@
 // first if asked for), the V conversion, block-sparse attention.  Two to five launches:
 //   op_stats     K sums (smooth_k) and V statistics (FP8 product), side by side
 //   op_finalize  their second steps
-//   op_prep      quantised K and the V tiles, side by side (per-thread scales: quantised Q too)
+//   op_prep      quantised K and the V tiles, side by side (op_q_pass: quantised Q too)
 //   v_residual   (FP8 product with smooth_v)
-//   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; per-thread scales: on INT8 Q); the
+//   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; op_q_pass: on INT8 Q); the
 //                log-sum-exp leaves as the natural one of the scores of q and k as given
 // Short sequences take one launch for the first four (op_head: up to 1024 tokens, as many heads as op_head_plan says) or one for
 // the second and third (op_prep_short: the rest up to 4096 tokens, op_short).  Calls with nothing to sum up (float16 product
@@ -35,11 +35,12 @@ struct OpParams {
   float *v_scale, *v_mean, *v_work, *v_resid;
   float* k_partial;
   unsigned short* k_mean;       // nullptr: not smoothed
-  float* lse_add;               // per-thread scales: sm_scale * q . k_mean per row; nullptr: not wanted
+  float* lse_add;               // with a pass over Q: sm_scale * q . k_mean per row; nullptr: not wanted
   int B, H, Hkv, Nq, Nk, nbq, nbk, chunks, smooth_v;
   int stats_k, stats_v;         // which statistics are taken
-  int kv_blocks;                // workgroups of op_prep that take K or V; the rest (per-thread scales) take Q
+  int kv_blocks;                // workgroups of op_prep that take K or V; the rest (q_pass) take Q
   float sm_scale;
+  bool q_pass;                  // op_prep quantises Q too (op_q_pass)
   bool one_launch;              // op_head does it all (op_head_plan)
   int k_parts, k_rounds;        // of op_head: workgroups that share the K of a head, 256 tokens they take one after the other
   bool short_prep;              // op_prep_short does what comes after the statistics (op_short)
@@ -66,7 +67,7 @@ __global__ void __launch_bounds__(1024) op_finalize_kernel(const OpParams p) {
     v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.Nk, p.chunks, p.smooth_v, (int64_t)blockIdx.x - BH * p.stats_k, BH);
 }
 
-// PT: per-thread scale granularity.  A workgroup takes one V tile, 256 tokens of K or (PT) 256 tokens of Q.
+// PT: per-thread scale granularity.  A workgroup takes one V tile, 256 tokens of K or 128 (PT: 256) tokens of Q.
 template <int DT, int D, bool PT, bool F16V>
 __global__ void __launch_bounds__(256) op_prep_kernel(const OpParams p) {
   const int wave = threadIdx.x >> 6;
@@ -98,16 +99,21 @@ __global__ void __launch_bounds__(256) op_prep_kernel(const OpParams p) {
     }
     return;
   }
-  if constexpr (PT) {
-    i -= p.kv_blocks;
-    const int per = (p.nbq + 3) / 4, bh = i / per, g = i % per * 4 + wave;
-    if (g >= p.nbq) return;
-    const int b = bh / p.H, h = bh % p.H;
-    float* dot = p.lse_add ? p.lse_add + (int64_t)bh * p.Nq : nullptr;
-    const unsigned short* with = p.lse_add ? p.k_mean + ((int64_t)b * p.Hkv + h / (p.H / p.Hkv)) * D : nullptr;
-    quant_per_thread_body<DT, D, false, false>(p.q + b * p.qs_b + h * p.qs_h, nullptr, p.q8 + (int64_t)bh * p.Nq * D,
-                                               p.q_scale + (int64_t)bh * p.nbq * 16, p.Nq, g, p.qs_n, D, p.sm_scale, dot, with);
-  }
+  i -= p.kv_blocks;
+  const int groups = PT ? p.nbq : 2 * p.nbq;   // of 64 or 32 tokens
+  const int per = (groups + 3) / 4, bh = i / per, g = i % per * 4 + wave;
+  if (g >= groups) return;
+  const int b = bh / p.H, h = bh % p.H;
+  const unsigned short* q = p.q + b * p.qs_b + h * p.qs_h;
+  int8_t* out = p.q8 + (int64_t)bh * p.Nq * D;
+  float* dot = p.lse_add ? p.lse_add + (int64_t)bh * p.Nq : nullptr;
+  const unsigned short* with = p.lse_add ? p.k_mean + ((int64_t)b * p.Hkv + h / (p.H / p.Hkv)) * D : nullptr;
+  if constexpr (PT)
+    quant_per_thread_body<DT, D, false, false>(q, nullptr, out, p.q_scale + (int64_t)bh * p.nbq * 16, p.Nq, g, p.qs_n, D, p.sm_scale,
+                                               dot, with);
+  else
+    quant_group_body<DT, D, 32, false, false>(q, nullptr, out, p.q_scale + (int64_t)bh * p.nbq * 2, p.Nq, g, p.qs_n, D, p.sm_scale,
+                                              dot, with);
 }
 
 // Everything in front of the attention launch, up to OP_HEAD_TOKENS tokens, in one launch: such a call consists of launches of
@@ -470,6 +476,22 @@ static bool op_short(int64_t BK, int Nk, int D, bool per_thread) {
   return !per_thread && (Nk <= 4096 || (Nk <= 8192 && BK * D <= 512));
 }
 
+// Whether Q has a pass of its own, in op_prep.  The attention kernels quantise 16-bit Q at next to no cost where a compute unit
+// has other waves to work on meanwhile (QRows); with few q-blocks it is 0.3 us (D = 64) to 2 us on the way of each, while op_prep
+// has compute units to spare for it.  Operator, in the attention kernel / in op_prep, shares of the time, by q-blocks:
+//                                             up to 64        65 to 128      129 to 256     601 to 1024    above 1536
+//   float16 tiles without smooth_k  D = 64   1.01 to 1.04    1.01 to 1.04   0.99 to 0.99   0.96 to 0.99   0.94 to 0.97
+//     (N = 8 .. 4000; 9.4 / 9.1 us)  D = 128  1.02 to 1.06    1.01 to 1.02   0.99 to 1.01   0.97 to 1.00   0.95 to 0.97
+//   4500 and 9000 keys, FP8         D = 64   0.99 to 1.00    0.99 to 1.00   0.99 to 1.00   0.97 to 0.99   0.97
+//                                    D = 128  0.99 to 1.03    1.00 to 1.02   1.00 to 1.01   0.98 to 0.99   0.98
+//     with the log-sum-exp          D = 64   0.98 to 1.03    1.00 to 1.02   1.00 to 1.01   0.99 to 1.00   0.98
+//                                    D = 128  1.00 to 1.03    1.00 to 1.01   1.01 to 1.02   0.98 to 1.00   0.97 to 0.99
+// Calls that have no op_prep keep it in the attention kernel: the launch they lack is worth more.
+static bool op_q_pass(int64_t q_blocks, int64_t BK, int Nk, int D, bool smooth_k, bool per_thread, bool f16v) {
+  if (per_thread) return true;
+  return q_blocks <= 2 * D && !((smooth_k || !f16v) && op_short(BK, Nk, D, false));
+}
+
 // Where the intermediate tensors lie in the workspace (256-byte aligned pieces).
 struct OpLayout {
   int64_t q8, k8, v_tiles, q_scale, k_scale, v_scale, v_mean, v_work, k_partial, k_mean, resid, bytes;
@@ -481,10 +503,11 @@ struct OpLayout {
       return at;
     };
     const int64_t nbq = ceil_div(Nq, 64), nbk = ceil_div(Nk, 64), BK = (int64_t)B * Hkv, BQ = (int64_t)B * H;
-    q8 = take(per_thread ? BQ * Nq * D : 0);   // (per warp: the attention kernels quantise Q themselves)
+    const bool q_pass = op_q_pass(BQ * nbq, BK, Nk, D, smooth_k, per_thread, f16v);
+    q8 = take(q_pass ? BQ * Nq * D : 0);   // (otherwise the attention kernels quantise Q themselves)
     k8 = take(BK * Nk * D);
     v_tiles = take(BK * nbk * 64 * D * (f16v ? 2 : 1));
-    q_scale = take(per_thread ? BQ * nbq * 16 * 4 : 0);
+    q_scale = take(q_pass ? BQ * nbq * (per_thread ? 16 : 2) * 4 : 0);
     k_scale = take(BK * nbk * (per_thread ? 4 : 1) * 4);
     v_scale = take(f16v ? 0 : BK * D * 4);
     v_mean = take(f16v ? 0 : BK * D * 4);
@@ -545,7 +568,7 @@ static int launch_op_prep(const OpParams& p, bool per_thread, bool f16v, hipStre
     }
     hipLaunchKernelGGL((op_finalize_kernel<DT, D>), dim3(p.B * p.Hkv * (p.stats_k + p.stats_v)), dim3(1024), 0, st, p);
   }
-  const int q_blocks = per_thread ? p.B * p.H * ceil_div(p.nbq, 4) : 0;
+  const int q_blocks = p.q_pass ? p.B * p.H * ceil_div(per_thread ? p.nbq : 2 * p.nbq, 4) : 0;
   const dim3 grid(p.kv_blocks + q_blocks);
   if (per_thread) hipLaunchKernelGGL((op_prep_kernel<DT, D, true, false>), grid, dim3(256), 0, st, p);
   else if (f16v) hipLaunchKernelGGL((op_prep_kernel<DT, D, false, true>), grid, dim3(256), 0, st, p);
@@ -609,7 +632,8 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   p.v_resid = !f16v && smooth_v ? p.v_work + v_resid_offset((int64_t)B * Hkv, Nk, D) : nullptr;
   p.k_partial = (float*)(ws + at.k_partial);
   p.k_mean = smooth_k ? (unsigned short*)(ws + at.k_mean) : nullptr;
-  p.lse_add = per_thread && smooth_k ? lse : nullptr;   // (the attention kernel adds to what the row holds)
+  p.q_pass = op_q_pass((int64_t)B * H * p.nbq, (int64_t)B * Hkv, Nk, D, smooth_k != 0, per_thread, f16v);
+  p.lse_add = p.q_pass && smooth_k ? lse : nullptr;   // (the attention kernel adds to what the row holds)
   p.chunks = ceil_div(Nk, v_chunk(Nk));
   p.stats_k = smooth_k != 0; p.stats_v = !f16v;
   p.kv_blocks = B * Hkv * (p.nbk + ceil_div(p.nbk, 4));
@@ -629,15 +653,15 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   AttnExtra extra;
   extra.lse_scale = 0.6931471805599453f;
   extra.lse_add = p.lse_add != nullptr;
-  if (!per_thread) {
+  if (!p.q_pass) {
     extra.q16 = p.q;
     extra.k_mean = p.k_mean;
     extra.lse_dot_scale = sm_scale;
   }
-  const int64_t qs_b = per_thread ? (int64_t)H * Nq * D : q_stride_b, qs_h = per_thread ? (int64_t)Nq * D : q_stride_h;
+  const int64_t qs_b = p.q_pass ? (int64_t)H * Nq * D : q_stride_b, qs_h = p.q_pass ? (int64_t)Nq * D : q_stride_h;
   return attn_sparse_impl(p.q8, p.k8, p.v_tiles, p.q_scale, p.k_scale, p.v_scale, smooth_v ? p.v_mean : nullptr, sparse,
                           sparse_batch_stride, out, dtype, lse, extra, nullptr, B, H, Hkv, Nq, Nk, D, qs_b, qs_h,
-                          per_thread ? D : q_stride_n, (int64_t)Hkv * Nk * D, (int64_t)Nk * D, D, o_stride_b, o_stride_h,
+                          p.q_pass ? D : q_stride_n, (int64_t)Hkv * Nk * D, (int64_t)Nk * D, D, o_stride_b, o_stride_h,
                           o_stride_n, sm_scale, is_causal, flags | (per_thread ? PARO_ATTN_QK_PER_THREAD : 0), nullptr, 0, 0, 0,
                           0, stream);
 }

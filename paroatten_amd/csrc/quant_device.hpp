@@ -1,5 +1,6 @@
 // Bodies of the INT8 quantisation of Q and K as device functions, so that one launch can run several of them side by
-// side.  The launches that use them: quant_int8.hip (one tensor), attn_operator.hip (Q, K and the V conversion).
+// side.  The launches that use them: quant_int8.hip (one tensor), attn_operator.hip (K and the V conversion; with few
+// q-blocks or per-thread scales Q too, which otherwise the attention kernels quantise).
 //
 // One 64-lane wave owns one group of G tokens x D channels: every lane holds G*D/64 values in
 // registers (16-byte loads, consecutive lanes on consecutive addresses), the group maximum is a

@@ -1,6 +1,6 @@
 // Bodies of the two V conversions as device functions (v_fp8.hip, attn_sparse_pv16.hip: V alone; attn_operator.hip:
-// next to the quantisation of K, and with per-thread scales of Q, in one launch).  256 threads take one 64-token block kb of
-// (batch, kv-head) bh; v points at the first token of that (batch, kv-head).
+// next to the quantisation of K, or of Q and K, in one launch).  256 threads take one 64-token block kb of (batch, kv-head)
+// bh; v points at the first token of that (batch, kv-head).
 #pragma once
 #include "paro_device.hpp"
 

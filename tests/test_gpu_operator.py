@@ -192,3 +192,44 @@ def test_log_sum_exp_with_the_k_mean_in_every_kernel_form(dev, monkeypatch, B, H
     # one product and one sum in fp32, and an fp32 dot product of D terms
     bound = (D + 4) * 2.0 ** -24 * (lse2.double().abs() + terms.abs().sum(-1) * D ** -0.5)
     assert ((lse.double() - want).abs() <= bound)[~empty].all()
+
+
+@pytest.mark.parametrize("H,Hkv,Nq,Nk,D,mode", [
+    (4, 2, 1, 1, 64, "f16"), (3, 1, 33, 33, 128, "f16"), (2, 2, 4096, 4096, 64, "f16"), (3, 3, 2752, 2752, 64, "f16"),
+    (4, 4, 4096, 4096, 128, "f16"), (4, 2, 65, 4200, 64, "fp8"), (6, 3, 1, 4097, 128, "fp8"), (9, 3, 129, 8200, 128, "exact"),
+    (2, 1, 4097, 4097, 64, "fp8"), (1, 1, 8200, 8200, 64, "fp8"), (3, 1, 95, 5000, 64, "f16"),
+])
+@pytest.mark.parametrize("smooth_k", [False, True])
+def test_queries_in_a_pass_of_their_own(dev, H, Hkv, Nq, Nk, D, mode, smooth_k):
+    """With few q-blocks and a preparation launch that takes K and V tile by tile, Q is quantised in that launch: token-major,
+    grouped heads, last groups of one row, both sides of the lines (128 q-blocks at D = 64, 256 at 128; 4096 keys where there is
+    something to sum up).  K's sums are exact: the same bits as the chain of its parts, and the log-sum-exp within its bound."""
+    import paroatten_amd as P
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    dtype = torch.bfloat16 if Nk % 2 else torch.float16
+    g = torch.Generator(device=dev).manual_seed(Nq + Nk + D + H)
+    q = torch.randn(2 if Nq < 4000 else 1, Nq, H, D, generator=g, device=dev).to(dtype)
+    B = q.size(0)
+    v = torch.randn(B, Nk, Hkv, D, generator=g, device=dev).to(dtype)
+    k = (torch.randint(-63, 64, (B, Nk, Hkv, D), generator=g, device=dev) / 8).to(dtype)
+    mask = torch.rand(H, (Nq + 63) // 64, (Nk + 63) // 64, generator=g, device=dev) < 0.4
+    mask[:, :, 0] = True
+    km = k.double().mean(dim=1, keepdim=True).float().to(dtype) if smooth_k else None
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, km, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="NHD")
+    kw = dict(pv_f16=mode == "f16", exact_exp=mode == "exact")
+    o_ref, o_lse_ref = torch.empty_like(q), torch.empty_like(q)
+    args = (0, 0, 2, D ** -0.5)
+    qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_ref, qs, ks, *args, 0, mask, **kw)
+    lse2 = qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o_lse_ref, qs, ks, *args, 1, mask, **kw)
+    call = dict(tensor_layout="NHD", smooth_k=smooth_k, **kw)
+    assert torch.equal(P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, **call), o_ref)
+    o, lse = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, return_lse=True, **call)
+    assert torch.equal(o, o_lse_ref)
+    want, scale = lse2.double() * 0.6931471805599453, lse2.double().abs()
+    if smooth_k:
+        terms = q.transpose(1, 2).double() * km.transpose(1, 2).repeat_interleave(H // Hkv, dim=1).double()
+        want = want + terms.sum(-1) * D ** -0.5
+        scale = scale + terms.abs().sum(-1) * D ** -0.5
+    # one product and one sum in fp32, and an fp32 dot product of D terms
+    assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()

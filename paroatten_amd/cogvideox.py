@@ -21,6 +21,7 @@ from typing import Optional, Sequence, Tuple
 
 import torch
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _qattn_sm80 as qattn
 from . import permute as PM
@@ -199,11 +200,12 @@ _LAYER_NORM_FORWARD = torch.nn.LayerNorm.forward
 def _is_plain_layer_norm(norm) -> bool:
     """Whether calling norm runs torch's LayerNorm and nothing else: no hook of its own or on all modules, no other forward
     (set on the instance, as offloading and instrumentation wrappers do, or on the class), not compiled by itself."""
-    return (type(norm) is torch.nn.LayerNorm
-            and getattr(norm.forward, "__func__", None) is _LAYER_NORM_FORWARD and norm.forward.__self__ is norm
-            and norm._compiled_call_impl is None
-            and not (norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks)
-            and not torch.nn.modules.module._has_any_global_hook())
+    if type(norm) is not torch.nn.LayerNorm or torch.nn.LayerNorm.forward is not _LAYER_NORM_FORWARD:
+        return False
+    own = norm.__dict__   # (looked up once: twice a layer, 0.8 us each time, through the attributes 1.4)
+    return not ("forward" in own or own.get("_compiled_call_impl") is not None
+                or own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or _has_any_global_hook())
 
 
 def _head_norm(norm, x: torch.Tensor) -> torch.Tensor:

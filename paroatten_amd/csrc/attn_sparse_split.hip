@@ -12,6 +12,14 @@
 // order would have: it changes only when a weight leaves its range (rarely, and in the first block), each wave says so in LDS
 // before the round's barrier, and the waves of such a round settle it in list order.  A wave before the block that
 // moved the maximum keeps its weights and is rescaled after its product, one behind it computes its own again.
+//
+// What bounds it, by the clock inside the kernel at N = 4096, two heads, D = 64, W = 4, 11 us: 3.4 us until the first scores (a
+// microsecond of it before the first load), 0.7 us a round, in which four waves fetch 32 KB through one compute unit's 64 bytes
+// a clock, 1 us from the last round to the last store.  Each wave taking the first maximum for itself (instead of the first
+// wave for all of them, 0.6 us), the next round's products in front of the look at the row sums and all waves adding up
+// (instead of the first): 12.6 -> 11.8 us.  With the registers of two waves per SIMD at D = 64: 256 q-blocks 17.4 -> 14.3 us,
+// 384 21.9 -> 18.4.  (Tried: eight blocks a round, no faster at 64 q-blocks; K through LDS at D = 64, 12.3; D = 128 in the
+// registers of two waves per SIMD spills 70 of them, three times the time.)
 #include "attn_common.hpp"
 
 namespace paro {
@@ -21,7 +29,7 @@ template <int D, int W> struct SplitLds {
   // of fragments takes 32 bytes: straight into registers it measured 22.8 instead of 18.0 us at N = 4096, two heads.)
   static constexpr int RING = D == 128 ? 2 * 64 * D : 0;
   static constexpr int PIECES = D / 32 * 4 + 1;                  // a wave's share of the result: O, and (d[0], d[1], d_exact, -)
-  static constexpr int SHARES = (W - 1) * PIECES * 1024;
+  static constexpr int SHARES = W * PIECES * 1024;
   static constexpr int EPI_OFF = W * RING > SHARES ? W * RING : SHARES;   // v_scale and v_mean of the head
   static constexpr int M_OFF = EPI_OFF + 2 * D * 4;              // the settled maximum of the 32 rows
   static constexpr int FLAG_OFF = M_OFF + 32 * 4;                // [round parity][8] bytes, one per wave
@@ -30,7 +38,7 @@ template <int D, int W> struct SplitLds {
 };
 
 template <int D, int OUT_DT, bool LSE, bool EXACT, int W, bool Q16>
-__global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const AttnParams p, const int causal) {
+__global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_kernel(const AttnParams p, const int causal) {
   using Lds = SplitLds<D, W>;
   constexpr int KS = D / 32;      // k-steps of the QK product
   constexpr int DT = D / 32;      // 32-channel tiles of O^T
@@ -309,8 +317,11 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
   const int rounds = (cnt + W - 1) / W;
   auto block_of = [&](int r) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane((int)klist[r * W + wave]); };
   int kb_c = block_of(0), kb_1 = block_of(1), kb_2 = block_of(2);
+  const int kb_first = __builtin_amdgcn_readfirstlane((int)klist[0]);
+  v4i k_first[2 * KS];
   if constexpr (K_LDS) {
     // (issued in this order: the count below leaves in flight what comes after the first tile)
+    load_k(kb_first, k_first);
     dma_k(kb_c, 0);
     __builtin_amdgcn_sched_barrier(0);
     dma_k(kb_1, 1);
@@ -322,48 +333,62 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   } else {
     load_k(kb_c, kfrag[0]);
+    load_k(kb_first, k_first);
     load_k(kb_1, kfrag[1]);
     load_v(kb_c, vfrag[0]);
     quantise_q();
   }
   v16i acc[2][2];   // [round parity][row tile of the 64 keys]: the next round's products are issued before the barrier
   qk(acc[0], kfrag[0]);
+  // columns past the end of K or above the diagonal leave the softmax
+  auto mask_edge = [&](v16i (&s)[2], int kb) __attribute__((always_inline)) {
+    if ((kb == p.nbk - 1 && (p.Nk & 63) != 0) || (causal && kb == qb)) {
+      int thr = p.Nk - kb * 64 - 4 * lh;
+      if (causal) thr = min(thr, qrow + 1 - kb * 64 - 4 * lh);
+#pragma unroll
+      for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+          if (32 * mt + 8 * (i >> 2) + (i & 3) >= thr) s[mt][i] = (int)0xFF800000u;
+    }
+  };
+  {   // the maximum of the first block of the list: every wave takes it for itself
+    v16i s0[2];
+    qk(s0, k_first);
+    mask_edge(s0, kb_first);
+    set_max(fmaxf(m_i, block_max(s0, qsc * clist[0])));
+  }
 
+  float c_cur = qsc * clist[wave];
   // One round.  cur holds the scores of this round's block, nxt receives those of the next.
   auto round = [&](int r, auto parc) __attribute__((always_inline)) {
     constexpr int par = decltype(parc)::value;
     v16i(&cur)[2] = acc[par];
     v16i(&nxt)[2] = acc[par ^ 1];
+    const int j = r * W + wave;
+    const bool active = j < cnt;
+    const float c = c_cur, c_next = qsc * clist[j + W];
+    const int kidx = (int)klist[j + 3 * W];
+    if constexpr (K_LDS) {   // K(r + 1) has landed: everything older than V(r)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DT) : "memory");
+      read_k(par ^ 1);
+    }
+    if (active) {
+      mask_edge(cur, kb_c);
+      words(cur, c);
+    }
+    // (the next round's products run on while the row sums are looked at and the waves meet)
+    __builtin_amdgcn_sched_barrier(0);
+    qk(nxt, kfrag[K_LDS ? 0 : par ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    uint8_t* flag = flags + par * 8;
+    const bool left = active && left_range(cur, c);
+    if (lane == 0) flag[wave] = left;
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (K_LDS) dma_k(kb_2, par);       // K(r + 2): K(r) has been used
     else load_k(kb_2, kfrag[par]);
     load_v(kb_1, vfrag[par ^ 1]);                // V(r + 1)
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (K_LDS) {   // K(r + 1) has landed: everything older than this round's requests
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D / 16 + 2 * DT) : "memory");
-      read_k(par ^ 1);
-    }
-    const int j = r * W + wave;
-    const bool active = j < cnt;
-    const float c = qsc * clist[j];
-    const int kidx = (int)klist[j + 3 * W];
-    if (active && ((kb_c == p.nbk - 1 && (p.Nk & 63) != 0) || (causal && kb_c == qb))) {
-      // columns past the end of K or above the diagonal leave the softmax
-      int thr = p.Nk - kb_c * 64 - 4 * lh;
-      if (causal) thr = min(thr, qrow + 1 - kb_c * 64 - 4 * lh);
-#pragma unroll
-      for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-          if (32 * mt + 8 * (i >> 2) + (i & 3) >= thr) cur[mt][i] = (int)0xFF800000u;
-    }
-    uint8_t* flag = flags + par * 8;
-    bool left = r == 0 && wave == 0;
-    if (active && r > 0) {
-      words(cur, c);
-      left = left_range(cur, c);
-    }
-    if (lane == 0) flag[wave] = left;
-    qk(nxt, kfrag[K_LDS ? 0 : par ^ 1]);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();   // (a bare one: the loads stay in flight)
     const unsigned f = __builtin_amdgcn_readfirstlane((unsigned)*reinterpret_cast<const Flags*>(flag));
@@ -381,6 +406,7 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
       if constexpr (LSE) d_exact += rs;
     }
     if (f != 0) rescale(post);
+    c_cur = c_next;
     kb_c = kb_1; kb_1 = kb_2; kb_2 = __builtin_amdgcn_readfirstlane(kidx);
   };
   for (int r = 0; r < rounds; r += 2) {
@@ -393,11 +419,12 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
-  // ---- the first wave adds the others up: 16-byte pieces [wave][piece][lane] ----
-  constexpr int PIECES = Lds::PIECES;
+  // ---- every wave adds up its part of the channels, in the order of the waves, and stores it: 16-byte pieces
+  //      [wave][piece][lane], piece (dt, g) channels 32 dt + 8 g + 4 lh .. + 3 of row l32 ----
+  constexpr int PIECES = Lds::PIECES, OWN = DT * 4 / W;
   v4f* parts = reinterpret_cast<v4f*>(smem);
-  if (wave > 0) {
-    v4f* dst = parts + (wave - 1) * PIECES * 64 + lane;
+  {
+    v4f* dst = parts + wave * PIECES * 64 + lane;
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -406,45 +433,42 @@ __global__ void __launch_bounds__(64 * W, 1) attn_sparse_split_kernel(const Attn
     dst[DT * 4 * 64] = v4f{d_acc[0], d_acc[1], d_exact, 0.f};
   }
   __syncthreads();
-  if (wave > 0) return;
+  v4f o_sum[OWN], d_sum = parts[DT * 4 * 64 + lane];
+  const v4f* own = parts + wave * OWN * 64 + lane;
 #pragma unroll
-  for (int o = 0; o < W - 1; o++) {
-    const v4f* src = parts + o * PIECES * 64 + lane;
+  for (int i = 0; i < OWN; i++) o_sum[i] = own[i * 64];
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++)
+  for (int o = 1; o < W; o++) {
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const v4f x = src[(dt * 4 + g) * 64];
+    for (int i = 0; i < OWN; i++) {
+      const v4f x = own[(o * PIECES + i) * 64];
 #pragma unroll
-        for (int q = 0; q < 4; q++) o_acc[dt][4 * g + q] += x[q];
-      }
-    const v4f x = src[DT * 4 * 64];
-    d_acc[0] += x[0];
-    d_acc[1] += x[1];
-    d_exact += x[2];
+      for (int q = 0; q < 4; q++) o_sum[i][q] += x[q];
+    }
+    const v4f x = parts[(o * PIECES + DT * 4) * 64 + lane];
+#pragma unroll
+    for (int q = 0; q < 3; q++) d_sum[q] += x[q];
   }
 
   // ---- epilogue: O = O~/d * v_scale + v_mean ----
-  const float d_lo = __shfl(d_acc[0], l32 & 15, 64), d_hi = __shfl(d_acc[1], l32 & 15, 64);
+  const float d_lo = __shfl(d_sum[0], l32 & 15, 64), d_hi = __shfl(d_sum[1], l32 & 15, 64);
   const float inv = 1.0f / (l32 < 16 ? d_lo : d_hi);
   if (qrow < p.Nq) {
     unsigned short* outp = out_row_ptr();
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++)
+    for (int i = 0; i < OWN; i++) {
+      const int ch = 8 * (wave * OWN + i) + 4 * lh;
+      const v4f sc = *reinterpret_cast<const v4f*>(epi + ch), mn = *reinterpret_cast<const v4f*>(epi + D + ch);
+      unsigned short r[4];
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const int ch = 32 * dt + 8 * g + 4 * lh;
-        const v4f sc = *reinterpret_cast<const v4f*>(epi + ch), mn = *reinterpret_cast<const v4f*>(epi + D + ch);
-        unsigned short r[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) r[q] = OutT::from_f32(fmaf(o_acc[dt][4 * g + q] * inv, sc[q], mn[q]));
-        *reinterpret_cast<v2i*>(outp + ch) =
-            v2i{(int)((unsigned)r[0] | ((unsigned)r[1] << 16)), (int)((unsigned)r[2] | ((unsigned)r[3] << 16))};
-      }
+      for (int q = 0; q < 4; q++) r[q] = OutT::from_f32(fmaf(o_sum[i][q] * inv, sc[q], mn[q]));
+      *reinterpret_cast<v2i*>(outp + ch) =
+          v2i{(int)((unsigned)r[0] | ((unsigned)r[1] << 16)), (int)((unsigned)r[2] | ((unsigned)r[3] << 16))};
+    }
   }
   if constexpr (LSE) {
-    const float d_full = d_exact + __shfl_xor(d_exact, 32, 64);
-    if (qrow < p.Nq && lh == 0) store_lse(p, lse_row, m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET);
+    const float d_full = d_sum[2] + __shfl_xor(d_sum[2], 32, 64);
+    if (wave == 0 && qrow < p.Nq && lh == 0) store_lse(p, lse_row, m_i + __builtin_amdgcn_logf(d_full) - P_EXP_OFFSET);
   }
 }
 
@@ -467,26 +491,35 @@ static int launch_split(const AttnParams& p, bool causal, bool exact, hipStream_
   return PARO_OK;
 }
 
-// Measured at N = 4096 (64 key blocks, half of them kept), one to ten heads of 64 q-blocks, against two waves per q-block
-// (attn_sparse.hip), us:        q-blocks    64     128    192    256    320
-//   D = 64    W = 4                         12.2   12.9   22.1   23.5   30.5
-//             W = 2                                16.4   17.0   17.0   27.4
-//             two waves                            20.3          20.7   21.9
-//   D = 128   W = 4                         17.9   18.3   32.2   33.7   46.2
-//             W = 2                                22.7   24.5   25.6   40.4
-//             two waves                            29.0          31.7   32
-// i.e. W such that every workgroup of four waves, or two of two waves, has a compute unit.  What gains is the length of the
-// lists, of which the host knows only the bound, the number of key blocks.  This / two waves per q-block, us, by the
-// share of the blocks that is kept (two heads of 64, one to twelve of 20 key blocks):   0.05        0.1         0.2         0.5
-//   D = 64    64 key blocks                        8.7/8.9   9.6/11.0    11.0/13.6   14.3/21.1
-//             20 key blocks, lists of 2 to 10      7.9/7.4   8.6/8.0      8.7/8.6     9.7/11.3
-//   D = 128   64 key blocks                       12.0/14.0 13.3/16.7    15.5/20.4   21.0/30.8
-//             20 key blocks                       10.8/11.5 11.0/12.1    12.0/13.7   13.7/17.6
-// so at D = 64 lists of two or three blocks lose 0.5 to 0.8 us and those from four on gain, and below twenty key blocks it
-// stays with the other kernels.
+// Measured against two waves per q-block (attn_sparse.hip), us, lists of 0.3 of the key blocks; q-blocks:
+//                              64            128            192            256            384            512
+//   D = 64   64 key blocks   W = 4 is 1.52, 1.49, 1.55, 1.50, 1.00 and 0.87 times as fast, W = 2 1.25, 1.22, 1.27, 1.27, 1.16, 1.15:
+//            two waves     14.40          14.93          17.93          18.04          18.10          19.03
+//            32 (W = 4)       1.24           1.24           1.22           1.17           0.81           0.76
+//               (W = 2)       1.14           1.16           1.11           1.14           1.09           1.04
+//            20 (W = 4)       1.17           1.15           0.98           0.81           0.71           0.61
+//               (W = 2)       1.13           1.11           1.02           1.07           1.02           0.82 (520)
+//            12 (W = 4)       1.03           1.02           0.92           0.94           0.68           0.56
+//             8 (W = 2, with the operator's other launches)  1.02  1.03
+//   D = 128  64 (W = 4)       1.53           1.52           1.10           0.93
+//               (W = 2)       1.24           1.24           1.12           1.12
+//            12 (W = 4)       1.25           0.78           0.73           0.73
+//               (W = 2)       1.22           1.21           1.11           1.13
+//             4 (W = 2, with the operator's other launches)  1.12  1.12  1.04  1.03
+// A SIMD holds two of these waves at D = 64 and one at D = 128, so W is what fills the card with one round of workgroups.
+// (Beyond: D = 64, 520 q-blocks, W = 2 0.82; D = 128, 260 q-blocks, W = 2 0.87.)  Longer lists gain more, up to 1.9 times at 77
+// blocks of 128; of the lists the host knows only the bound, the number of key blocks.  With less than one block in eight
+// kept (lists of one to four) the lines below lose up to 6 %, at 12 to 20 key blocks.  Calls with the log-sum-exp below 20 key
+// blocks or above 448 q-blocks stay with two waves: their bits are those of the per-thread kernels, which callers may compare.
 int split_width(const AttnParams& p, int D) {
-  if (p.nbk < 20 || p.total > 256) return 0;
-  const int W = p.total <= 128 ? 4 : 2;
+  int W = 0;
+  if (p.lse != nullptr && (p.nbk < 20 || p.total > 448)) return 0;
+  if (D == 64) {
+    if (p.total <= 128) W = p.nbk >= 12 ? 4 : p.nbk >= 7 ? 2 : 0;
+    else if (p.total <= 512 && p.nbk >= 20) W = p.total <= 256 && p.nbk >= 32 ? 4 : 2;
+  } else if (p.total <= 256) {
+    W = p.total <= 128 && p.nbk >= 16 ? 4 : 2;
+  }
   const size_t smem = D == 64 ? split_lds<64>(p.nbk, W) : split_lds<128>(p.nbk, W);
   return smem <= 160 * 1024 ? W : 0;
 }

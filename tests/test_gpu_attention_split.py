@@ -44,6 +44,18 @@ def test_same_result_as_two_waves(dev, B, H, nb, D, dtype, causal, mode):
     assert torch.count_nonzero(a[:, 0, :64]) == 0   # the q-block without a kept block
 
 
+# around the lines of split_width: more than 256 q-blocks, and few key blocks
+@pytest.mark.parametrize("B,H,nb,D", [(1, 9, 32, 64), (1, 16, 32, 64), (2, 5, 20, 64), (1, 2, 12, 64), (1, 3, 7, 64), (1, 6, 31, 64),
+                                      (1, 3, 2, 128), (1, 8, 16, 128), (1, 9, 15, 128), (2, 2, 64, 128), (1, 5, 1, 128)])
+@pytest.mark.parametrize("causal,mode", [(False, "fast"), (True, "exact"), (True, "lse")])
+def test_same_result_as_two_waves_around_the_lines(dev, B, H, nb, D, causal, mode):
+    from paroatten_amd import _lib as L
+    N, lse = nb * 64 - 19, mode == "lse"
+    form = L.load().paro_attn_kernel_form(B, H, N, N, D, int(causal), int(lse), L.PARO_ATTN_EXACT_EXP if mode == "exact" else 0)
+    assert (form == L.PARO_ATTN_FORM_SPLIT) == (not lse or (nb >= 20 and B * H * nb <= 448))
+    test_same_result_as_two_waves(dev, B, H, nb, D, torch.bfloat16, causal, mode)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("H", [4, 8])
 @pytest.mark.parametrize("pattern,causal,density", [("ramp", False, 1.0), ("ramp", True, 1.0), ("ramp", False, 0.5), ("spike", False, 0.5)])

@@ -49,29 +49,29 @@ struct OpParams {
 template <int DT, int D>
 __global__ void __launch_bounds__(256) op_stats_kernel(const OpParams p) {
   // K and V of a head one after the other, in x: y and z keep the whole range of head and batch counts
-  const int h = blockIdx.y, b = blockIdx.z;
+  const int h = blockIdx.y, b = blockIdx.z, block = with_args(p, blockIdx.x);
   const int k_chunks = p.stats_k ? p.chunks : 0;
-  if ((int)blockIdx.x < k_chunks)
-    v_stats_body<DT, D, true>(p.k, p.k_partial, p.Nk, p.chunks, p.ks_b, p.ks_h, p.ks_n, blockIdx.x, h, b, p.Hkv);
+  if (block < k_chunks)
+    v_stats_body<DT, D, true>(p.k, p.k_partial, p.Nk, p.chunks, p.ks_b, p.ks_h, p.ks_n, block, h, b, p.Hkv);
   else
     v_stats_body<DT, D>(p.v, p.v_work + v_stats_offset((int64_t)p.B * p.Hkv, p.Nk, D), p.Nk, p.chunks, p.vs_b, p.vs_h,
-                        p.vs_n, (int)blockIdx.x - k_chunks, h, b, p.Hkv);
+                        p.vs_n, block - k_chunks, h, b, p.Hkv);
 }
 
 template <int DT, int D>
 __global__ void __launch_bounds__(1024) op_finalize_kernel(const OpParams p) {
-  const int BH = p.B * p.Hkv;
-  if ((int)blockIdx.x < BH * p.stats_k)
-    k_mean_finalize_body<DT, D, double>(p.k_partial, p.k_mean, p.Nk, p.chunks, (int64_t)p.Hkv * D, D, p.Hkv, blockIdx.x);
+  const int BH = p.B * p.Hkv, block = with_args(p, blockIdx.x);
+  if (block < BH * p.stats_k)
+    k_mean_finalize_body<DT, D, double>(p.k_partial, p.k_mean, p.Nk, p.chunks, (int64_t)p.Hkv * D, D, p.Hkv, block);
   else
-    v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.Nk, p.chunks, p.smooth_v, (int64_t)blockIdx.x - BH * p.stats_k, BH);
+    v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.Nk, p.chunks, p.smooth_v, (int64_t)block - BH * p.stats_k, BH);
 }
 
 // PT: per-thread scale granularity.  A workgroup takes one V tile, 256 tokens of K or 128 (PT: 256) tokens of Q.
 template <int DT, int D, bool PT, bool F16V>
 __global__ void __launch_bounds__(256) op_prep_kernel(const OpParams p) {
   const int wave = threadIdx.x >> 6;
-  int i = blockIdx.x;
+  int i = with_args(p, blockIdx.x);
   if (i < p.kv_blocks) {
     // K and V of a head one after the other, the heads in reverse: the last ones that the statistics have read are
     // still in the memory-side cache
@@ -134,8 +134,8 @@ __global__ void __launch_bounds__(1024) op_head_kernel(const OpParams p) {
   constexpr int LPR = D / 8;                // lanes per token row (K)
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int k_parts = p.k_parts, parts = k_parts + (F16V ? (p.nbk + 3) / 4 : D / 32);
-  const int bh = blockIdx.x / parts, b = bh / p.Hkv, h = bh % p.Hkv;
-  int part = blockIdx.x % parts;
+  const int block = with_args(p, blockIdx.x), bh = block / parts, b = bh / p.Hkv, h = bh % p.Hkv;
+  int part = block % parts;
   const int N = p.Nk;
   constexpr int V_BYTES = F16V ? 4 * 64 * (D + 8) * 2 : OP_HEAD_TOKENS * 64 + 32 * 3 * 32 * 4 + 2 * 32 * 4;
   constexpr int K_BYTES = 16 * D * 4 + D * 2 + 2 * 16 * 4;
@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(256) op_prep_short_kernel(const OpParams p) {
   constexpr int LPR = D / 8, ROWS = 256 / LPR, SL = 256 / D, PITCH = D + 8;
   const int t = threadIdx.x, wave = t >> 6;
   const int per_k = (p.nbk + 3) / 4, per = p.nbk + per_k;
-  const int bh = blockIdx.x / per, j = blockIdx.x % per;
+  const int block = with_args(p, blockIdx.x), bh = block / per, j = block % per;
   const int b = bh / p.Hkv, h = bh % p.Hkv, N = p.Nk;
   const int ch = t % D, sl = t / D;
   __shared__ double red_s[SL][D];

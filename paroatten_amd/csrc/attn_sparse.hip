@@ -696,7 +696,8 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
 __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_kernel(const AttnParams p) {
   // hardware deals workgroup ids round-robin to the 8 XCDs
-  const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
+  const int block = with_args(p, blockIdx.x);
+  const int vid = qblock_of<CAUSAL>(p, block & 7, block >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
   attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false, Q16>(p, vid);
 }

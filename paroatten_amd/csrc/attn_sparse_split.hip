@@ -49,7 +49,8 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
   uint8_t* flags = smem + Lds::FLAG_OFF;
 
   const int per = gridDim.x >> 3;   // each XCD walks a contiguous range of (batch, head, q-block, half)
-  const int vid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  const int block = with_args(p, blockIdx.x);
+  const int vid = (block & 7) * per + (block >> 3);
   if (vid >= 2 * p.total) return;
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int l32 = lane & 31, lh = lane >> 5;

@@ -592,7 +592,8 @@ __device__ __forceinline__ void attn_qblock_w64(const AttnParams& p, const int v
 template <int OUT_DT, bool CAUSAL, bool EXACT, bool LSE, bool Q16>
 __global__ void __launch_bounds__(64, 2) attn_sparse_w64_kernel(const AttnParams p) {
   // hardware deals workgroup ids round-robin to the 8 XCDs
-  const int vid = qblock_of<CAUSAL>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
+  const int block = with_args(p, blockIdx.x);
+  const int vid = qblock_of<CAUSAL>(p, block & 7, block >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
   attn_qblock_w64<OUT_DT, CAUSAL, EXACT, LSE, Q16>(p, vid);
 }

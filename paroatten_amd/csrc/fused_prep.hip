@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(256) rope_permute_quant_kernel(const PrepParam
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int kb = blockIdx.x;
+  const int kb = with_args(p, blockIdx.x);
   const int order = blockIdx.y % 6, split = blockIdx.y / 6;
   const bool rope = p.cos_t != nullptr;
 
@@ -373,11 +373,12 @@ struct KvStatsParams {
 
 template <int DT, int D, int KB>
 __global__ void __launch_bounds__(256) kv_stats_kernel(const KvStatsParams p) {
-  if ((int)blockIdx.x < p.k_blocks) {
+  const int block = with_args(p, blockIdx.x);
+  if (block < p.k_blocks) {
     rope_k_sum_body<DT, D, KB>(p.k, p.cos_t, p.sin_t, p.k_partial, p.B * p.H, p.H, p.N, p.n_text, p.k_chunks, p.ks_b,
-                               p.ks_h, p.ks_n, blockIdx.x);
+                               p.ks_h, p.ks_n, block);
   } else {
-    const int i = blockIdx.x - p.k_blocks;
+    const int i = block - p.k_blocks;
     const int chunk = i % p.v_chunks, bh = i / p.v_chunks;
     v_stats_body<DT, D>(p.v, p.v_work + v_stats_offset((int64_t)p.B * p.H, p.N, D), p.N, p.v_chunks, p.vs_b, p.vs_h, p.vs_n, chunk, bh % p.H, bh / p.H, p.H);
   }
@@ -385,11 +386,11 @@ __global__ void __launch_bounds__(256) kv_stats_kernel(const KvStatsParams p) {
 
 template <int DT, int D>
 __global__ void __launch_bounds__(1024) kv_finalize_kernel(const KvStatsParams p) {
-  const int BH = p.B * p.H;
-  if ((int)blockIdx.x < BH)
-    k_mean_finalize_body<DT, D>(p.k_partial, p.k_mean, p.N, p.k_chunks, p.ms_b, p.ms_h, p.H, blockIdx.x);
+  const int BH = p.B * p.H, block = with_args(p, blockIdx.x);
+  if (block < BH)
+    k_mean_finalize_body<DT, D>(p.k_partial, p.k_mean, p.N, p.k_chunks, p.ms_b, p.ms_h, p.H, block);
   else
-    v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.N, p.v_chunks, p.smooth_v, (int64_t)blockIdx.x - BH, BH);
+    v_finalize_body<D>(p.v_work, p.v_scale, p.v_mean, p.N, p.v_chunks, p.smooth_v, (int64_t)block - BH, BH);
 }
 
 template <int DT, int D>

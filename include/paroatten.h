@@ -296,6 +296,13 @@ int paro_permute_inv(const void* in, void* out, int dtype, const int32_t* orders
                      int64_t in_stride_b, int64_t in_stride_h, int64_t in_stride_n,
                      int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_n,
                      void* stream);
+/* LayerNorm over the D channels of each of `rows` contiguous rows of q and of k (any leading dimensions; 64 or 128 channels):
+ * out = (x - mean) / sqrt(var + eps) * weight + bias, statistics in fp32, rounded to `dtype`.  weight, bias: D values
+ * of `dtype`, or NULL (1, 0).  What CogVideoX's attention does to q and k between its projections and the rotation
+ * (paroattention/cogvideox.py:157-160), in one launch. */
+int paro_head_norm(const void* q, const void* k, void* q_out, void* k_out, int dtype,
+                   const void* q_weight, const void* q_bias, const void* k_weight, const void* k_bias,
+                   float q_eps, float k_eps, int64_t rows, int D, void* stream);
 /* new_of_old index map of every head: idx int32 [H, F*Hh*W] (parity of the integer index law). */
 int paro_permute_index_map(int32_t* idx, const int32_t* orders, int H, int F, int Hh, int W, void* stream);
 

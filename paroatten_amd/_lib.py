@@ -72,6 +72,7 @@ SIGNATURES = {
     "paro_rope_permute_fwd": (c_int, [_P, _P, _P, _P, _P, _P, _I, _P, _P, _P,
                                       _I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _P]),
     "paro_permute_inv": (c_int, [_P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _L, _P]),
+    "paro_head_norm": (c_int, [_P, _P, _P, _P, _I, _P, _P, _P, _P, _F, _F, _L, _I, _P]),
     "paro_permute_index_map": (c_int, [_P, _P, _I, _I, _I, _I, _P]),
     "paro_prep_workspace_bytes": (c_int64, [_I, _I, _I, _I]),
     "paro_rope_permute_quant_fwd": (c_int, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L,

@@ -179,3 +179,20 @@ def permute_inverse(o, orders, F, Hh, W, n_text, out):
     _lib.on(o).paro_permute_inv(ptr(o), ptr(out), _lib.DTYPE_CODE[o.dtype], ptr(orders), B, H, N, D, n_text, F, Hh, W,
                                 *o.stride()[:3], *out.stride()[:3], stream_of(o))
     return out
+
+
+def head_norm(q, k, q_weight, q_bias, q_eps, k_weight, k_bias, k_eps):
+    params = [w for w in (q_weight, q_bias, k_weight, k_bias) if w is not None]
+    if (any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.device != q.device or t.dtype != q.dtype
+            or torch.is_grad_enabled() and t.requires_grad or t.data_ptr() % 16 for t in (q, k, *params))
+            or q.dtype not in _lib.DTYPE_CODE or q.dim() != 4 or q.size(-1) not in (64, 128) or q.numel() == 0 or k.shape != q.shape
+            or any(w.dim() != 1 or w.numel() != q.size(-1) or not w.is_contiguous() for w in params)
+            or not q.transpose(1, 2).is_contiguous() or not k.transpose(1, 2).is_contiguous()
+            or torch.is_autocast_enabled() or torch.jit.is_tracing()
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()):
+        return []
+    B, H, N, D = q.shape
+    qo, ko = (torch.empty((B, N, H, D), dtype=q.dtype, device=q.device) for _ in range(2))
+    _lib.on(q).paro_head_norm(ptr(q), ptr(k), ptr(qo), ptr(ko), _lib.DTYPE_CODE[q.dtype], ptr(q_weight), ptr(q_bias),
+                              ptr(k_weight), ptr(k_bias), q_eps, k_eps, B * N * H, D, stream_of(q))
+    return [qo.transpose(1, 2), ko.transpose(1, 2)]

@@ -23,6 +23,7 @@ import torch
 import torch.nn.functional as F
 from torch.nn.modules.module import _has_any_global_hook
 
+from . import _lib
 from . import _qattn_sm80 as qattn
 from . import permute as PM
 from .permute import permute_attn_out, permute_qk  # noqa: F401  (same module-level names as the reference)
@@ -217,6 +218,18 @@ def _head_norm(norm, x: torch.Tensor) -> torch.Tensor:
     return norm(x)
 
 
+def _head_norms(norm_q, norm_k, q: torch.Tensor, k: torch.Tensor):
+    """(norm_q(q), norm_k(k)) for the [B,H,N,D] views of token-major projections: in one launch of the library's own where both
+    are plain LayerNorms over the channels and the tensors fit (csrc/torch_binding.cpp, head_norm)."""
+    if norm_q is not None and norm_k is not None and _is_plain_layer_norm(norm_q) and _is_plain_layer_norm(norm_k):
+        pq, pk, width = norm_q.__dict__["_parameters"], norm_k.__dict__["_parameters"], (q.shape[-1],)
+        if norm_q.normalized_shape == width and norm_k.normalized_shape == width and len(pq) == 2 and len(pk) == 2:
+            both = _lib.ops().head_norm(q, k, pq.get("weight"), pq.get("bias"), norm_q.eps, pk.get("weight"), pk.get("bias"), norm_k.eps)
+            if both:
+                return both
+    return (q if norm_q is None else _head_norm(norm_q, q)), (k if norm_k is None else _head_norm(norm_k, k))
+
+
 class PARO_CogVideoXAttnProcessor2_0(_ParoProcessorBase):
     r"""Joint text+video self-attention of CogVideoX with PAROAttention in place of dense SDPA
     (paroattention/cogvideox.py:112-250).  `i_timestep < 0` selects dense SDPA, as there (:215-221)."""
@@ -240,10 +253,7 @@ class PARO_CogVideoXAttnProcessor2_0(_ParoProcessorBase):
         query = query.view(batch_size, -1, attn.heads, head_dim).transpose(1, 2)
         key = key.view(batch_size, -1, attn.heads, head_dim).transpose(1, 2)
         value = value.view(batch_size, -1, attn.heads, head_dim).transpose(1, 2)
-        if attn.norm_q is not None:
-            query = _head_norm(attn.norm_q, query)
-        if attn.norm_k is not None:
-            key = _head_norm(attn.norm_k, key)
+        query, key = _head_norms(attn.norm_q, attn.norm_k, query, key)
 
         grid = self._grid_for(sequence_length - text_seq_length, {COG_GRID[0] * COG_GRID[1] * COG_GRID[2]: COG_GRID})
         cos = sin = None

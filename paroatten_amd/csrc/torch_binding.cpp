@@ -15,8 +15,12 @@
 // guard: paroattention/core.py:168-174 works around it) every call runs under a guard for the tensors'
 // device and on torch's current stream of that device.
 #include <torch/extension.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <atomic>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <stdexcept>
@@ -496,6 +500,37 @@ std::vector<OptTensor> rope_permute_quant(const torch::Tensor& q, const torch::T
   return {q8, q_scale, k8, k_scale, v8, v_scale, smooth_v ? OptTensor(v_mean) : c10::nullopt, compute_km ? km : c10::nullopt};
 }
 
+// cogvideox._head_norms: the LayerNorms over the channels of q and k, [B,H,N,D] views of token-major projections, in one launch;
+// nothing where the library's own modules have to do it (another type, size or order of rows, a subclass, or something that
+// records or rewrites the operation: autograd, autocast, a tracer, a mode).
+std::vector<torch::Tensor> head_norm(const torch::Tensor& q, const torch::Tensor& k, const OptTensor& q_weight,
+                                     const OptTensor& q_bias, double q_eps, const OptTensor& k_weight, const OptTensor& k_bias,
+                                     double k_eps) {
+  const bool grad = at::GradMode::is_enabled();
+  auto plain = [&](const torch::Tensor& x) {
+    return x.is_cuda() && x.device() == q.device() && x.scalar_type() == q.scalar_type() && !(grad && x.requires_grad()) &&
+           !x.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                                     c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize}));
+  };
+  if ((q.scalar_type() != at::kHalf && q.scalar_type() != at::kBFloat16) || q.dim() != 4 || !plain(q) || !plain(k)) return {};
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
+  if ((D != 64 && D != 128) || q.numel() == 0 || k.sizes() != q.sizes()) return {};
+  for (const OptTensor* w : {&q_weight, &q_bias, &k_weight, &k_bias})
+    if (*w && (!plain(**w) || (*w)->dim() != 1 || (*w)->size(0) != D || !(*w)->is_contiguous() || (uintptr_t)(*w)->data_ptr() % 16 != 0))
+      return {};
+  const torch::Tensor q_rows = q.transpose(1, 2), k_rows = k.transpose(1, 2);
+  if (!q_rows.is_contiguous() || !k_rows.is_contiguous() || ((uintptr_t)q.data_ptr() | (uintptr_t)k.data_ptr()) % 16 != 0 ||
+      at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing() ||
+      c10::impl::TorchDispatchModeTLS::stack_len() > 0 || at::impl::PythonTorchFunctionTLS::stack_len() > 0)
+    return {};
+  const c10::DeviceGuard guard(q.device());
+  torch::Tensor qo = torch::empty({B, N, H, D}, q.options()), ko = torch::empty({B, N, H, D}, q.options());
+  auto at_ = [](const OptTensor& w) -> const void* { return w ? w->data_ptr() : nullptr; };
+  check_rc(paro_head_norm(q.data_ptr(), k.data_ptr(), qo.data_ptr(), ko.data_ptr(), code_of(q), at_(q_weight), at_(q_bias),
+                          at_(k_weight), at_(k_bias), (float)q_eps, (float)k_eps, B * N * H, (int)D, stream_of(q)));
+  return {qo.transpose(1, 2), ko.transpose(1, 2)};
+}
+
 // _qattn_sm80.attn_sparse_prepacked; unpermute: orders with (F, Hh, W) and n_text, or none
 torch::Tensor attn_sparse_prepacked(const torch::Tensor& q8, const torch::Tensor& k8, const torch::Tensor& v8,
                                     const OptTensor& v_scale, const OptTensor& v_mean, const torch::Tensor& output,
@@ -598,5 +633,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   ops.def("rope_permute", &rope_permute, unlocked);
   ops.def("rope_permute_quant", &rope_permute_quant, unlocked);
   ops.def("permute_inverse", &permute_inverse, unlocked);
+  ops.def("head_norm", &head_norm, unlocked);
   rope.def("rope_permutation", &rope_permutation, "RoPE op with permutation.");
 }

@@ -342,14 +342,36 @@ __global__ void __launch_bounds__(256) rope_permute_quant_kernel(const PrepParam
 // K mean over tokens AFTER the rotation (the permutation does not change a mean) and the V statistics: the bodies
 // live in stats_device.hpp.  Alone (paro_rope_k_mean), or both in ONE launch when the preparation smooths K
 // itself: a workgroup takes a K chunk of a head group or a V chunk of a head, and one more launch finishes both.
-template <int DT, int D, int KB>
+// Which chunk and heads a workgroup of the K sums takes.  Workgroup ids are dealt round-robin to the 8 XCDs: XCD x takes the
+// token chunks 8*i + x, and for each of them all head groups one after the other, so that a chunk of the rotary tables
+// (twice the bytes of the K rows of one head) crosses the fabric once per launch and is served to the other head groups by
+// that XCD's L2.
+template <int GROUP>
+struct KSumPart {
+  int chunk, bh0;
+  __device__ KSumPart(int block, int n_chunks, int BH) {
+    const int n_hg = (BH + GROUP - 1) / GROUP;
+    if constexpr (GROUP == KM_GROUP) {
+      const int j = block >> 3;
+      chunk = (j / n_hg) * 8 + (block & 7);
+      bh0 = (j % n_hg) * GROUP;
+    } else {
+      chunk = block % n_chunks;
+      bh0 = block / n_chunks * GROUP;
+    }
+  }
+};
+
+template <int DT, int D, int KB, int GROUP>
 __global__ void __launch_bounds__(256) rope_k_sum_kernel(const unsigned short* __restrict__ k,
                                                          const float* __restrict__ cos_t,
                                                          const float* __restrict__ sin_t,
                                                          float* __restrict__ partial, int BH, int H, int N,
                                                          int n_text, int n_chunks, int64_t ks_b, int64_t ks_h,
                                                          int64_t ks_n) {
-  rope_k_sum_body<DT, D, KB>(k, cos_t, sin_t, partial, BH, H, N, n_text, n_chunks, ks_b, ks_h, ks_n, blockIdx.x);
+  const KSumPart<GROUP> part(blockIdx.x, n_chunks, BH);
+  if (part.chunk < n_chunks)
+    rope_k_sum_body<DT, D, KB, GROUP>(k, cos_t, sin_t, partial, BH, H, N, n_text, n_chunks, ks_b, ks_h, ks_n, part.chunk, part.bh0);
 }
 
 template <int DT, int D>
@@ -359,8 +381,20 @@ __global__ void __launch_bounds__(1024) k_mean_finalize_kernel(const float* __re
   k_mean_finalize_body<DT, D>(partial, k_mean, N, n_chunks, ms_b, ms_h, H, blockIdx.x);
 }
 
-// workgroups of the K sums: XCD x takes the chunks 8*i + x, and for each of them all head groups
-static inline int k_sum_blocks(int n_chunks, int BH) { return ceil_div(n_chunks, 8) * 8 * ceil_div(BH, KM_GROUP); }
+// Whether the K sums take one head at a time, four tokens per thread in flight.  Four heads at a time read the tables once for all
+// of them, but with few workgroups a launch lasts as long as one, which at D = 128 takes its 256 tokens in 16 trips to memory
+// one after the other.  The preparation with the K mean, four heads at a time / one, us:
+//   D = 128   N = 1008   8 heads 25.9 / 20.0   40 heads 39.9 / 32.6     D = 64   N = 1008  40 heads 22.6 / 20.4
+//             N = 4352   1 head 26.9 / 19.5    20 heads 61.2 / 57.2              N = 4352   8 heads 23.6 / 21.1   20 heads 34.1 / 33.5
+//             N = 8112   8 heads 56.2 / 47.8   20 heads 89.0 / 89.5              N = 8112   8 heads 30.9 / 27.7   20 heads 48.5 / 50.2
+//             N = 20787  1 head 40.8 / 33.1     3 heads 55.5 / 55.6              N = 20787  3 heads 31.9 / 32.7
+static bool k_sum_one_head(int n_chunks, int BH) {
+  const int64_t blocks = (int64_t)n_chunks * BH;
+  return blocks <= (n_chunks <= 64 ? 360 : 128);
+}
+static inline int k_sum_blocks(int n_chunks, int BH, bool one_head) {
+  return one_head ? n_chunks * BH : ceil_div(n_chunks, 8) * 8 * ceil_div(BH, KM_GROUP);
+}
 
 struct KvStatsParams {
   const unsigned short* k; const unsigned short* v;
@@ -371,12 +405,14 @@ struct KvStatsParams {
   int64_t ks_b, ks_h, ks_n, vs_b, vs_h, vs_n, ms_b, ms_h;
 };
 
-template <int DT, int D, int KB>
+template <int DT, int D, int KB, int GROUP>
 __global__ void __launch_bounds__(256) kv_stats_kernel(const KvStatsParams p) {
   const int block = with_args(p, blockIdx.x);
   if (block < p.k_blocks) {
-    rope_k_sum_body<DT, D, KB>(p.k, p.cos_t, p.sin_t, p.k_partial, p.B * p.H, p.H, p.N, p.n_text, p.k_chunks, p.ks_b,
-                               p.ks_h, p.ks_n, block);
+    const KSumPart<GROUP> part(block, p.k_chunks, p.B * p.H);
+    if (part.chunk < p.k_chunks)
+      rope_k_sum_body<DT, D, KB, GROUP>(p.k, p.cos_t, p.sin_t, p.k_partial, p.B * p.H, p.H, p.N, p.n_text, p.k_chunks, p.ks_b,
+                                        p.ks_h, p.ks_n, part.chunk, part.bh0);
   } else {
     const int i = block - p.k_blocks;
     const int chunk = i % p.v_chunks, bh = i / p.v_chunks;
@@ -446,11 +482,13 @@ extern "C" int paro_rope_k_mean(const void* k, int dtype, const float* cos, cons
   hipStream_t st = (hipStream_t)stream;
   float* partial = (float*)workspace;
   // tokens per thread whose loads are requested together: 2 at D = 64, 1 at D = 128 (measured)
+  const bool one_head = k_sum_one_head(n_chunks, B * H);
+  const dim3 grid(k_sum_blocks(n_chunks, B * H, one_head));
 #define PARO_KM(DTV, DV)                                                                                        \
   do {                                                                                                          \
-    hipLaunchKernelGGL((rope_k_sum_kernel<DTV, DV, (DV == 64 ? 2 : 1)>), dim3(k_sum_blocks(n_chunks, B * H)), dim3(256), 0, \
-                       st, (const unsigned short*)k, cos, sin, partial, B * H, H, N, n_text, n_chunks,          \
-                       k_stride_b, k_stride_h, k_stride_n);                                                     \
+    auto kern = one_head ? rope_k_sum_kernel<DTV, DV, 4, 1> : rope_k_sum_kernel<DTV, DV, (DV == 64 ? 2 : 1), KM_GROUP>; \
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const unsigned short*)k, cos, sin, partial, B * H, H, N,  \
+                       n_text, n_chunks, k_stride_b, k_stride_h, k_stride_n);                                   \
     hipLaunchKernelGGL((k_mean_finalize_kernel<DTV, DV>), dim3(B * H), dim3(1024), 0, st, (const float*)partial, \
                        (unsigned short*)k_mean, N, n_chunks, mean_stride_b, mean_stride_h, H);                  \
   } while (0)
@@ -539,13 +577,15 @@ static int prep_impl(bool compute_k_mean, const void* q, const void* k, const vo
     sp.k_partial = (float*)workspace + paro_v_fp8_partial_floats(B, H, N, D);   // behind the V partials
     sp.k_mean = (unsigned short*)k_mean; sp.v_scale = v_scale; sp.v_mean = v_mean;
     sp.B = B; sp.H = H; sp.N = N; sp.n_text = n_text; sp.k_chunks = ceil_div(N, K_CHUNK); sp.v_chunks = ceil_div(N, v_chunk(N));
-    sp.k_blocks = k_sum_blocks(sp.k_chunks, B * H); sp.smooth_v = smooth_v;
+    const bool one_head = k_sum_one_head(sp.k_chunks, B * H);
+    sp.k_blocks = k_sum_blocks(sp.k_chunks, B * H, one_head); sp.smooth_v = smooth_v;
     sp.ks_b = k_stride_b; sp.ks_h = k_stride_h; sp.ks_n = k_stride_n;
     sp.vs_b = v_stride_b; sp.vs_h = v_stride_h; sp.vs_n = v_stride_n; sp.ms_b = mean_stride_b; sp.ms_h = mean_stride_h;
     const int n_blocks = sp.k_blocks + sp.v_chunks * B * H;
 #define PARO_KV(DTV, DV)                                                                                          \
   do {                                                                                                            \
-    hipLaunchKernelGGL((kv_stats_kernel<DTV, DV, (DV == 64 ? 2 : 1)>), dim3(n_blocks), dim3(256), 0, st, sp);      \
+    auto kern = one_head ? kv_stats_kernel<DTV, DV, 4, 1> : kv_stats_kernel<DTV, DV, (DV == 64 ? 2 : 1), KM_GROUP>; \
+    hipLaunchKernelGGL(kern, dim3(n_blocks), dim3(256), 0, st, sp);                                               \
     hipLaunchKernelGGL((kv_finalize_kernel<DTV, DV>), dim3(2 * B * H), dim3(1024), 0, st, sp);                    \
   } while (0)
     if (dtype == PARO_DTYPE_F16) {

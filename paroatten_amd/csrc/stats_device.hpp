@@ -174,31 +174,22 @@ __device__ __forceinline__ void v_finalize_body(float* work, float* __restrict__
 // K_CHUNK-token chunk, then one workgroup per (batch, head) adds them in a fixed order.  A thread keeps
 // the table entries of its token piece while it walks over a group of (batch, head) pairs.
 constexpr int KM_GROUP = 4;   // measured: 4 beats 8 (too few workgroups at 40 heads) and 2 (tables re-read twice as often)
-template <int DT, int D, int KB>
+template <int DT, int D, int KB, int GROUP>
 __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict__ k, const float* __restrict__ cos_t,
                                                 const float* __restrict__ sin_t, float* __restrict__ partial, int BH,
                                                 int H, int N, int n_text, int n_chunks, int64_t ks_b, int64_t ks_h,
-                                                int64_t ks_n, int block) {
+                                                int64_t ks_n, int chunk, int bh0) {
   constexpr int LPR = D / 8;
   constexpr int ROWS = 256 / LPR;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  // Workgroup ids are dealt round-robin to the 8 XCDs: XCD x takes the token chunks 8*i + x, and for each of
-  // them all head groups one after the other, so that a chunk of the rotary tables (twice the bytes of the
-  // K rows of one head) crosses the fabric once per launch and is served to the other head groups by that
-  // XCD's L2.
-  const int n_hg = (BH + KM_GROUP - 1) / KM_GROUP;
-  const int xcd = block & 7, j = block >> 3;
-  const int chunk = (j / n_hg) * 8 + xcd;
-  if (chunk >= n_chunks) return;
-  const int bh0 = (j % n_hg) * KM_GROUP;
   const int col = (t % LPR) * 8;
-  float s[KM_GROUP][8];
+  float s[GROUP][8];
 #pragma unroll
-  for (int g = 0; g < KM_GROUP; g++)
+  for (int g = 0; g < GROUP; g++)
 #pragma unroll
     for (int j = 0; j < 8; j++) s[g][j] = 0.f;
   // one step: the rows of one token of the group's heads (table entries first: they are shared by the heads)
-  auto add_rows = [&](const v4i (&raw)[KM_GROUP], bool rot, const v4f& c0, const v4f& c1, const v4f& s0, const v4f& s1) {
+  auto add_rows = [&](const v4i (&raw)[GROUP], bool rot, const v4f& c0, const v4f& c1, const v4f& s0, const v4f& s1) {
     float cs[8], sn[8];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -206,7 +197,7 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
       sn[j] = s0[j]; sn[4 + j] = s1[j];
     }
 #pragma unroll
-    for (int g = 0; g < KM_GROUP; g++) {
+    for (int g = 0; g < GROUP; g++) {
       const v4i x = rot ? rotate8<DT>(raw[g], cs, sn) : raw[g];
 #pragma unroll
       for (int j = 0; j < 8; j++) s[g][j] += elem16_to_f32<DT>(x, j);
@@ -218,9 +209,9 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
   // `whole`: every row and head is there and every row rotated alike; otherwise rows and heads past the end re-read
   // the last one, such rows are not added and such heads not stored, and a row says for itself whether it is rotated
   const bool tables = cos_t != nullptr;
-  const unsigned short* kp[KM_GROUP];
+  const unsigned short* kp[GROUP];
 #pragma unroll
-  for (int g = 0; g < KM_GROUP; g++) {
+  for (int g = 0; g < GROUP; g++) {
     const int bh = min(bh0 + g, BH - 1), b = bh / H, h = bh - b * H;
     kp[g] = k + b * ks_b + h * ks_h + col;
   }
@@ -229,7 +220,7 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
     for (int r = t / LPR; r < K_CHUNK; r += ROWS * KB) {
       if (!whole && tok_first + (r - t / LPR) >= N) break;
       v4f c0[KB], c1[KB], s0[KB], s1[KB];
-      v4i raw[KB][KM_GROUP];
+      v4i raw[KB][GROUP];
 #pragma unroll
       for (int u = 0; u < KB; u++) {
         const int tok = whole ? tok_first + r + u * ROWS : min(tok_first + r + u * ROWS, N - 1);
@@ -239,7 +230,7 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
           s0[u] = *reinterpret_cast<const v4f*>(sin_t + o); s1[u] = *reinterpret_cast<const v4f*>(sin_t + o + 4);
         }
 #pragma unroll
-        for (int g = 0; g < KM_GROUP; g++) raw[u][g] = *reinterpret_cast<const v4i*>(kp[g] + (int64_t)tok * ks_n);
+        for (int g = 0; g < GROUP; g++) raw[u][g] = *reinterpret_cast<const v4i*>(kp[g] + (int64_t)tok * ks_n);
       }
 #pragma unroll
       for (int u = 0; u < KB; u++) {
@@ -248,11 +239,11 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
       }
     }
   };
-  if (tok_first + K_CHUNK <= N && bh0 + KM_GROUP <= BH && (!tables || tok_first >= n_text)) walk(std::true_type{});
+  if (tok_first + K_CHUNK <= N && bh0 + GROUP <= BH && (!tables || tok_first >= n_text)) walk(std::true_type{});
   else walk(std::false_type{});
-  __shared__ float red[4][KM_GROUP][D];
+  __shared__ float red[4][GROUP][D];
 #pragma unroll
-  for (int g = 0; g < KM_GROUP; g++) {
+  for (int g = 0; g < GROUP; g++) {
     // lanes that share a column sit LPR apart
 #pragma unroll
     for (int j = 0; j < 8; j++) {
@@ -269,7 +260,7 @@ __device__ __forceinline__ void rope_k_sum_body(const unsigned short* __restrict
     }
   }
   __syncthreads();
-  for (int i = t; i < KM_GROUP * D; i += 256) {
+  for (int i = t; i < GROUP * D; i += 256) {
     const int g = i / D, ch = i % D;
     if (bh0 + g < BH)
       partial[((int64_t)(bh0 + g) * n_chunks + chunk) * D + ch] =

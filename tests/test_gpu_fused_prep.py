@@ -237,3 +237,28 @@ def test_k_mean_inside_the_preparation_call(dev, B, H, D, grid, n_text, dtype, r
         a, b = getattr(one, name), getattr(two, name)
         assert torch.equal(a.view(torch.uint8) if a.dtype != torch.float32 else a, b.view(torch.uint8) if b.dtype != torch.float32 else b), name
     assert float(km.float().abs().mean()) > 0.5
+
+
+@pytest.mark.parametrize("D,heads,grid,n_text,dtype", [
+    (64, 91, (4, 15, 17), 0, torch.float16),      # 4 chunks, the last one short of 4 tokens; heads that four do not divide
+    (128, 121, (5, 9, 15), 30, torch.bfloat16),   # 3 chunks, text in the first
+    (128, 2, (21, 30, 27), 0, torch.float16),     # 67 chunks
+])
+def test_k_mean_of_many_heads_is_that_of_a_few(dev, D, heads, grid, n_text, dtype):
+    """The K sums take four heads at a time, or one where there are few workgroups: the same sums in the same order, hence the
+    same bits; and the mean of the rotated K to half a unit in the last place and fp32 sums of N terms."""
+    from paroatten_amd import permute as PM
+    N = n_text + grid[0] * grid[1] * grid[2]
+    g = torch.Generator(device=dev).manual_seed(heads)
+    k = (torch.randn(1, heads, N, D, generator=g, device=dev) + 3).to(dtype)
+    angle = torch.rand(N - n_text, D // 2, generator=g, device=dev).repeat_interleave(2, dim=1) * 6
+    cos, sin = angle.cos().contiguous(), angle.sin().contiguous()
+    km = PM.rope_k_mean(k, grid, n_text, cos, sin)
+    few = 1 if heads == 2 else 7
+    assert torch.equal(PM.rope_k_mean(k[:, :few], grid, n_text, cos, sin), km[:, :few])
+    x = k.float()
+    rot = torch.stack((x[..., 0::2] * cos[:, 0::2] - x[..., 1::2] * sin[:, 0::2], x[..., 1::2] * cos[:, 1::2] + x[..., 0::2] * sin[:, 1::2]),
+                      dim=-1).flatten(-2) if n_text == 0 else None
+    if rot is not None:
+        want = rot.to(dtype).double().mean(dim=2, keepdim=True)
+        assert ((km.double() - want).abs() <= want.abs() * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) + 2.0 ** -18).all()

@@ -209,8 +209,27 @@ int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8, const uin
                                    const int32_t* orders, int n_text, int F, int Hh, int W,
                                    void* stream);
 
+/* (2b) or, with orders, (2b') with device scratch of paro_attn_scratch_bytes() bytes (4-byte aligned, contents arbitrary, this
+ * call's until it has run; NULL: none).  With it, head size 128 and enough work, heads in which neighbouring q-blocks keep
+ * the same key blocks are found on the device and taken by a kernel in which two q-blocks share their tiles; outputs are the
+ * same bits.  paro_attn_scratch_bytes: 0 for calls that have no use for it. */
+int64_t paro_attn_scratch_bytes(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags);
+int paro_attn_sparse_scratch_fwd(const int8_t* q8, const int8_t* k8, const uint8_t* v8,
+                                 const float* q_scale, const float* k_scale,
+                                 const float* v_scale, const float* v_mean,
+                                 const uint8_t* sparse, int64_t sparse_batch_stride,
+                                 void* out, int out_dtype, float* lse,
+                                 int B, int H, int Hkv, int Nq, int Nk, int D,
+                                 int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                                 int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                                 int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
+                                 float sm_scale, int is_causal, int flags,
+                                 const int32_t* orders, int n_text, int F, int Hh, int W,
+                                 void* scratch, void* stream);
+
 /* The form of the attention kernel that a call of these sizes and flags gets: one of PARO_ATTN_FORM_* (host only, no GPU is
  * needed), or a negative error code.  A measurement names the kernel it timed by this, a test the one it means to run.
+ * (Heads that a call with scratch finds to share their tiles, (2b) above, leave it for the kernel made for them.)
  * PARO_ATTN_FORM_PACED: a launch of a single generation of workgroups is the plain one all the same. */
 #define PARO_ATTN_FORM_TWO_WAVES 0 /* two waves per q-block, plain launch */
 #define PARO_ATTN_FORM_PACED 1     /* the same kernel, paced launch */

@@ -57,6 +57,11 @@ SIGNATURES = {
                                                _I, _I, _I, _I, _I, _I,
                                                _L, _L, _L, _L, _L, _L, _L, _L, _L, _F, _I, _I,
                                                _P, _I, _I, _I, _I, _P]),
+    "paro_attn_scratch_bytes": (c_int64, [_I, _I, _I, _I, _I, _I, _I, _I]),
+    "paro_attn_sparse_scratch_fwd": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _L, _P, _I, _P,
+                                             _I, _I, _I, _I, _I, _I,
+                                             _L, _L, _L, _L, _L, _L, _L, _L, _L, _F, _I, _I,
+                                             _P, _I, _I, _I, _I, _P, _P]),
     "paro_attn_kernel_form": (c_int, [_I, _I, _I, _I, _I, _I, _I, _I]),
     "paro_attn_workspace_bytes": (c_int64, [_I, _I, _I, _I]),
     "paro_attn_workspace_bytes_for": (c_int64, [_I, _I, _I, _I, _I]),

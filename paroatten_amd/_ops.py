@@ -87,12 +87,12 @@ def attn_sparse_prepacked(q8, k8, v8, v_scale, v_mean, output, q_scale, k_scale,
     head = (ptr(q8), ptr(k8), ptr(v8), ptr(q_scale), ptr(k_scale), ptr(v_scale), ptr(v_mean), ptr(sparse), sparse_bs, ptr(output),
             _lib.DTYPE_CODE[output.dtype], ptr(lse) if return_lse else None)
     tail = (B, H, Hkv, Nq, Nk, D, *q8.stride()[:3], *k8.stride()[:3], *output.stride()[:3], float(sm_scale), int(is_causal), flags)
-    if orders is None:
-        _lib.on(q8).paro_attn_sparse_fwd(*head, None, *tail, stream_of(q8))
-    else:
+    n_scratch = load().paro_attn_scratch_bytes(B, H, Nq, Nk, D, int(is_causal), int(return_lse), flags)
+    scratch = torch.empty(n_scratch, dtype=torch.uint8, device=q8.device) if n_scratch else None
+    if orders is not None:
         _need(orders.is_cuda and orders.dtype == torch.int32 and orders.dim() == 1 and orders.numel() == H
               and orders.is_contiguous(), f"orders must be a contiguous int32 GPU tensor of {H} entries")
-        _lib.on(q8).paro_attn_sparse_unpermute_fwd(*head, *tail, ptr(orders), n_text, F, Hh, W, stream_of(q8))
+    _lib.on(q8).paro_attn_sparse_scratch_fwd(*head, *tail, ptr(orders), n_text, F, Hh, W, ptr(scratch), stream_of(q8))
     return lse
 
 

@@ -4,6 +4,7 @@
 // softmax-weight arithmetic and small device helpers.  gfx950 only.
 #pragma once
 #include "paro_device.hpp"
+#include "share_device.hpp"
 #include <type_traits>
 
 namespace paro {
@@ -43,7 +44,12 @@ struct AttnParams {
   const unsigned short* q16;
   const unsigned short* k_mean;
   float lse_dot_scale;
+  // Scratch of the call (null: none given), one word per head of the mask: whether the pair kernel takes it (attn_share_kernel)
+  int* share;
+  int share_ready;   // it holds that already
 };
+
+__device__ __forceinline__ bool tiles_shared(const AttnParams& p, int bh) { return p.share[p.sparse_bs != 0 ? bh : bh % p.H] != 0; }
 
 // P~ = 2^(S*c - m + P_EXP_OFFSET).  m is the running row maximum, refreshed lazily: only when a
 // weight leaves the range of e4m3 are m, O and the row sums rescaled.  Fast exponentials: a weight that would round to
@@ -66,13 +72,18 @@ constexpr float FAST_FIELD_SCALE = 256.0f / 32767.0f;
 // fill the card at the end, and heads that do not come out even are dealt out q-block by q-block, since the two halves of
 // a head are 1 : 3 in work.  B = 2, H = 32, N = 8192, D = 128, every block below the diagonal, kernel alone: 609 -> 592 us;
 // B = 1, H = 48, D = 64: 273 -> 257 us.
-template <bool CAUSAL>
+// PAIR: the same over pairs of neighbouring q-blocks of a head, qblock_units of them.
+template <bool PAIR> __device__ __forceinline__ int qblock_units(const AttnParams& p) {
+  return PAIR ? p.B * p.H * ((p.nbq + 1) >> 1) : p.total;
+}
+template <bool CAUSAL, bool PAIR = false>
 __device__ __forceinline__ int qblock_of(const AttnParams& p, int xcd, int slot, int per) {
   if constexpr (!CAUSAL) return xcd * per + slot;
-  const int heads = p.total / p.nbq, own = (heads >> 3) * p.nbq;   // q-blocks of the heads that an XCD has to itself
+  const int n = PAIR ? (p.nbq + 1) >> 1 : p.nbq, total = qblock_units<PAIR>(p);
+  const int heads = total / n, own = (heads >> 3) * n;   // q-blocks of the heads that an XCD has to itself
   const int i = slot < own ? xcd * own + slot : 8 * own + (slot - own) * 8 + xcd;
-  const int head = i / p.nbq;
-  return head < heads ? head * p.nbq + (p.nbq - 1 - (i - head * p.nbq)) : p.total;
+  const int head = i / n;
+  return head < heads ? head * n + (n - 1 - (i - head * n)) : total;
 }
 
 __device__ __forceinline__ void store_lse(const AttnParams& p, int64_t row, float lse2) {
@@ -227,7 +238,12 @@ struct AttnExtra {
   const unsigned short* q16 = nullptr;
   const unsigned short* k_mean = nullptr;
   float lse_dot_scale = 0.f;
+  int* share = nullptr;   // B * H words, or null
+  bool share_ready = false;
 };
+
+// Whether a call of these sizes and flags has a use for AttnExtra::share
+bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags);
 
 // paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip).  extra.q16: q8 and q_scale are not read, the q strides are those of
 // the 16-bit tensor, which is of the type out_dtype.

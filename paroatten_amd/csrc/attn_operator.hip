@@ -648,9 +648,16 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   else
     rc = D == 64 ? launch_op_prep<PARO_DTYPE_BF16, 64>(p, per_thread, f16v, st) : launch_op_prep<PARO_DTYPE_BF16, 128>(p, per_thread, f16v, st);
   if (rc) return rc;
-  if (p.v_resid && !p.one_launch)
-    if ((rc = v_fp8_add_residual(p.v_resid, p.v_scale, p.v_mean, B, Hkv, Nk, D, st))) return rc;
   AttnExtra extra;
+  // (of v_work, what lies in front of the residual sums is nobody's any more)
+  if (v_resid_offset((int64_t)B * Hkv, Nk, D) >= (int64_t)B * H &&
+      attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, lse != nullptr, flags | (per_thread ? PARO_ATTN_QK_PER_THREAD : 0)))
+    extra.share = (int*)p.v_work;
+  if (p.v_resid && !p.one_launch) {
+    const ShareLook look = {sparse, sparse_batch_stride != 0 ? B * H : H, p.nbq, p.nbk, is_causal, extra.share};
+    if ((rc = v_fp8_add_residual(p.v_resid, p.v_scale, p.v_mean, B, Hkv, Nk, D, st, extra.share ? &look : nullptr))) return rc;
+    extra.share_ready = extra.share != nullptr;
+  }
   extra.lse_scale = 0.6931471805599453f;
   extra.lse_add = p.lse_add != nullptr;
   if (!p.q_pass) {

@@ -74,31 +74,43 @@ template <int D> struct AttnLds {
 // the odd pair 2 lh + 1: two affine maps from score to exponent per block instead of one.
 //
 // Q16: Q as 16-bit rows (AttnParams::q16).
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED, bool Q16>
+//
+// PAIR: two q-blocks, the vid-th pair, by four waves (attn_sparse_pair_kernel).  A block that the other q-block alone keeps runs
+// through the loop with all its columns out of the softmax and V as zero, which leaves the state as it was; as a branch round
+// the products it cost 22 to 90 spilled registers.
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED, bool Q16, bool PAIR = false>
 __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) {
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
   static_assert(!Q16 || (!PT && !DUMP), "16-bit queries: neither per-thread scales nor the score dump");
+  static_assert(!PAIR || (D == 128 && !PT && !DUMP && !LSE && !EXACT), "shared tiles: the fast path at D = 128");
   using Lds = AttnLds<D>;
   constexpr int CW = PT ? 4 : 1;    // k scales per key block
   constexpr int KS = D / 32;        // k-steps of the QK MFMA (32 channels each)
   constexpr int DT_TILES = D / 32;  // 32-channel tiles of O^T
-  constexpr int NLD = D / 32;       // 16-byte pieces per thread per K (or V) tile
+  constexpr int NLD = D / (PAIR ? 64 : 32);   // 16-byte pieces per thread per K (or V) tile
   constexpr int CPR = D / 16;       // 16-byte chunks per K row
 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* clist = reinterpret_cast<float*>(smem + Lds::LIST_OFF);  // [nbk + LIST_PAD + 1] k_scale of kept blocks
-  unsigned short* klist = reinterpret_cast<unsigned short*>(clist + (p.nbk + Lds::LIST_PAD + 1) * CW);  // their indices
+  // their indices (PAIR: and in bits 16 and 17 which of the two q-blocks keeps them)
+  using KIdx = std::conditional_t<PAIR, unsigned, unsigned short>;
+  KIdx* klist = reinterpret_cast<KIdx*>(clist + (p.nbk + Lds::LIST_PAD + 1) * CW);
+  auto kidx = [](int entry) { return PAIR ? entry & 0xffff : entry; };
 
   // (D = 64: opaque to the compiler.  In the paced kernel, which calls this in a loop, everything derived from
   // the lane number alone is otherwise computed once in front of that loop and kept in registers, 35 more than
   // the 168 that three waves per SIMD allow; at D = 128, with registers to spare, hoisting measured 2 % faster)
   int t = threadIdx.x;
   if constexpr (D == 64) asm volatile("" : "+v"(t));
-  const int lane = t & 63, wave = t >> 6;
+  const int lane = t & 63, part = t >> 6;   // part: what the wave moves of a tile
+  const int wave = PAIR ? part & 1 : part;  // its half of the q-block
   const int l32 = lane & 31, lh = lane >> 5;
 
-  const int qb = vid % p.nbq;
-  const int bh = vid / p.nbq;
+  const int sub = PAIR ? __builtin_amdgcn_readfirstlane(part >> 1) : 0;
+  const int units = PAIR ? (p.nbq + 1) >> 1 : p.nbq;
+  const int unit = vid % units;
+  const int qb = PAIR ? 2 * unit + sub : unit;   // (an odd number of q-blocks: the last pair's second one does not exist)
+  const int bh = vid / units;
   const int h = bh % p.H, b = bh / p.H;
   const int hk = h / (p.H / p.Hkv);
   const int64_t bhk = (int64_t)b * p.Hkv + hk;
@@ -111,10 +123,13 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   // entries that are not kept go to a spare slot instead of being skipped.
   const int order_h = p.orders != nullptr ? p.orders[h] : 0;
   const float* ksc_base = p.k_scale + bhk * p.nbk * CW;
-  const int kmax = CAUSAL ? min(p.nbk, qb + 1) : p.nbk;
-  const uint8_t* mrow = p.sparse + b * p.sparse_bs + ((int64_t)h * p.nbq + qb) * p.nbk;
+  const int kmax = CAUSAL ? min(p.nbk, PAIR ? 2 * unit + 2 : qb + 1) : p.nbk;
+  const uint8_t* mrow = p.sparse + b * p.sparse_bs + ((int64_t)h * p.nbq + (PAIR ? 2 * unit : qb)) * p.nbk;
+  const bool second = PAIR && 2 * unit + 1 < p.nbq;
+  const uint8_t* mrow2 = mrow + (second ? p.nbk : 0);
   constexpr int MU = 8;   // 64 x MU blocks per pass: one pass up to 512 blocks
   uint8_t m[MU];
+  uint8_t m2[PAIR ? MU : 1];
   float msc[MU];
   v4f msc4[PT ? MU : 1];
   auto list_load = [&](int base) {
@@ -122,20 +137,29 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     for (int u = 0; u < MU; u++) {
       const int j = min(base + u * 64 + lane, kmax - 1);   // past the end: the last entry again
       m[u] = mrow[j];
+      if constexpr (PAIR) m2[u] = mrow2[j];
       if constexpr (PT) msc4[u] = *reinterpret_cast<const v4f*>(ksc_base + 4 * j);
       else msc[u] = ksc_base[j];
     }
   };
   const int trash = p.nbk + Lds::LIST_PAD;   // the spare slot
   int cnt = 0;
+  [[maybe_unused]] int own = 0;   // PAIR: blocks that this wave's q-block keeps
   auto list_take = [&](int base) {
 #pragma unroll
     for (int u = 0; u < MU; u++) {
       const int j = base + u * 64 + lane;
-      const bool keep = m[u] != 0 && j < kmax;
+      bool keep = m[u] != 0 && j < kmax;
+      unsigned bits = 0;
+      if constexpr (PAIR) {
+        const bool keep1 = keep && !(CAUSAL && j > 2 * unit), keep2 = second && m2[u] != 0 && j < kmax;
+        bits = (keep1 ? 1u << 16 : 0u) | (keep2 ? 1u << 17 : 0u);
+        keep = keep1 || keep2;
+        own += __popcll(__ballot(sub == 0 ? keep1 : keep2));
+      }
       const unsigned long long bal = __ballot(keep);
       const int pos = keep ? cnt + __popcll(bal & ((1ull << lane) - 1ull)) : trash;
-      klist[pos] = (unsigned short)j;
+      klist[pos] = (KIdx)((unsigned)j | bits);
       if constexpr (PT) *reinterpret_cast<v4f*>(clist + 4 * pos) = msc4[u];
       else clist[pos] = msc[u];
       cnt += __popcll(bal);
@@ -154,7 +178,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     if constexpr (Q16) {
       q16.load(p.q16 + qoff);
     } else {
-      const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + qb * 2 + wave;
+      const int64_t qs_group = ((int64_t)b * p.H + h) * (p.nbq * 2) + (PAIR ? min(qb, p.nbq - 1) : qb) * 2 + wave;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const v4i*>(p.q8 + qoff + 32 * ks);
       qsc = PT ? p.q_scale[qs_group * 8 + (l32 & 7)] : p.q_scale[qs_group];
@@ -197,13 +221,16 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     return reinterpret_cast<unsigned short*>(p.out) + b * p.os_b + h * p.os_h + (int64_t)drow * p.os_n;
   };
 
-  if (cnt == 0) {  // no kept block: the row outputs 0 (reference: m = -5e6, d = 1, O = 0)
+  auto store_nothing_kept = [&]() {  // the row outputs 0 (reference: m = -5e6, d = 1, O = 0)
     if (qrow < p.Nq) {
       unsigned short* outp = out_row_ptr();
 #pragma unroll
       for (int c = 0; c < D / 16; c++) *reinterpret_cast<v4i*>(outp + (lh * (D / 16) + c) * 8) = v4i{0, 0, 0, 0};
       if (p.lse && lh == 0) p.lse[((int64_t)b * p.H + h) * p.Nq + qrow] = -INFINITY;
     }
+  };
+  if (cnt == 0) {
+    store_nothing_kept();
     return;
   }
 
@@ -214,11 +241,11 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       uniform_ptr(p.k8 + b * p.ks_b + hk * p.ks_h), 0, (int)((int64_t)(p.Nk - 1) * p.ks_n + D), 0x00020000);
   const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(p.v8 + bhk * p.nbk * (int64_t)Lds::VTILE), 0, p.nbk * Lds::VTILE, 0x00020000);
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int part_u = __builtin_amdgcn_readfirstlane(part);
   int k_goff[NLD], v_goff[NLD];
 #pragma unroll
   for (int i = 0; i < NLD; i++) {
-    const int pos = (wave_u * NLD + i) * 1024 + lane * 16;  // byte position inside the LDS tile
+    const int pos = (part_u * NLD + i) * 1024 + lane * 16;  // byte position inside the LDS tile
     const int row = pos / D, cpos = (pos % D) / 16;
     // (less the immediate offset i * 1024 that the instruction adds on both sides; row * ks_n >= i * 1024)
     k_goff[i] = row * (int)p.ks_n + ((cpos ^ Lds::swz(row)) * 16) - i * 1024;
@@ -226,7 +253,8 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   }
   const int k_blk_stride = 64 * (int)p.ks_n;
   auto load_k = [&](int kb, int ST) {  // rows >= Nk read as 0
-    uint8_t* base = smem + ST * Lds::KTILE + wave_u * NLD * 1024;
+    uint8_t* base = smem + ST * Lds::KTILE + part_u * NLD * 1024;
+    kb = kidx(kb);
     buffer_load16_lds<0>(k_rsrc, base, k_goff[0], kb * k_blk_stride);
     buffer_load16_lds<1024>(k_rsrc, base, k_goff[1], kb * k_blk_stride);
     if constexpr (NLD == 4) {
@@ -235,7 +263,8 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     }
   };
   auto load_v = [&](int kb, int ST) {
-    uint8_t* base = smem + Lds::V_OFF + ST * Lds::VTILE + wave_u * NLD * 1024;
+    uint8_t* base = smem + Lds::V_OFF + ST * Lds::VTILE + part_u * NLD * 1024;
+    kb = kidx(kb);
     buffer_load16_lds<0>(v_rsrc, base, v_goff[0], kb * Lds::VTILE);
     buffer_load16_lds<1024>(v_rsrc, base, v_goff[1], kb * Lds::VTILE);
     if constexpr (NLD == 4) {
@@ -398,7 +427,10 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     float cb_next = 0.f;
     if constexpr (PT) cb_next = qsc * clist[(it + 1) * CW + 2 * lh + 1];
     // scale of this block and what follows from it and from the current maximum alone
-    const float c = c_cur;
+    // PAIR: a block that the other q-block alone keeps leaves the softmax as one does that lies past the end, whatever its k
+    // scale and its V hold
+    const bool mine = !PAIR || ((kb_c >> (16 + sub)) & 1) != 0;
+    const float c = mine ? c_cur : 1.f;
     const float cb = cb_cur;
     const float nmc = -S_MAGIC_F * c;
     const float c8 = (8.0f * FAST_FIELD_SCALE) * c;
@@ -417,16 +449,17 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       for (int i = 0; i < 16; i++) s[mt][i] = __int_as_float(acc[mt][i]);
 
     // columns past the end of K (last block) or above the diagonal (causal) leave the softmax
-    const bool edge = (kb_c == p.nbk - 1 && (p.Nk & 63) != 0) || (CAUSAL && kb_c == qb);
+    const bool edge = (kidx(kb_c) == p.nbk - 1 && (p.Nk & 63) != 0) || (CAUSAL && kidx(kb_c) == qb) || !mine;
     if (edge) {
       // One threshold per lane: the element of row tile mt, register i is column
       // kb*64 + 4*lh + cidx, cidx = 32*mt + 8*(i/4) + i%4, and it is dead from the first column past the end
       // of K (or above the diagonal) on.  (The block index is made opaque: from loop invariants the compiler
       // would evaluate the 32 lane masks in front of the loop and hold them in 64 scalar registers.)
-      int kb_e = kb_c;
+      int kb_e = kidx(kb_c);
       asm volatile("" : "+s"(kb_e));
       int thr = p.Nk - kb_e * 64 - 4 * lh;
       if constexpr (CAUSAL) thr = min(thr, qrow + 1 - kb_e * 64 - 4 * lh);
+      if (!mine) thr = -1;
 #pragma unroll
       for (int mt = 0; mt < 2; mt++)
 #pragma unroll
@@ -614,6 +647,10 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
           vfrag[ks][mt] = *reinterpret_cast<const v4i*>(smem + sv * Lds::VTILE + vr_base + (ks * 2 + mt) * 1024);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (!mine) {
+#pragma unroll
+        for (int i = 0; i < 2 * DT_TILES; i++) vfrag[i >> 1][i & 1] = v4i{0, 0, 0, 0};
+      }
     } else {
       qk_mfma();
       __builtin_amdgcn_sched_barrier(0);
@@ -656,6 +693,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // DMA of the padded tail blocks: nobody reads it
 
+  if constexpr (PAIR) {
+    if (own == 0) {
+      store_nothing_kept();
+      return;
+    }
+  }
   // ---- epilogue: O = O~/d * v_scale + v_mean ------------------------------------------------
   const float d_lo = __shfl(d_acc[0], l32 & 15, 64), d_hi = __shfl(d_acc[1], l32 & 15, 64);
   const float d_tot = l32 < 16 ? d_lo : d_hi;
@@ -699,7 +742,25 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
   const int block = with_args(p, blockIdx.x);
   const int vid = qblock_of<CAUSAL>(p, block & 7, block >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
+  if (p.share != nullptr && tiles_shared(p, vid / p.nbq)) return;
   attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false, Q16>(p, vid);
+}
+
+// Two neighbouring q-blocks of a head on the same tiles, four waves.  A wave's own instructions are those of the plain kernel,
+// but it moves a quarter of a tile and not half of one: the DMA instructions and the LDS writes behind them are a fifth of
+// that kernel's time.  Both walk the union of their lists, and each gives the weight zero to a block that only the other one
+// keeps, so that it pays where neighbours keep the same blocks: rows of one contiguous run, dense masks (share_look).  Outputs are
+// those of the plain kernel to the bit.  Attention, us, plain (paced where that is the rule) / pair: B = 2, H = 32, Hkv = 8,
+// N = 8192, causal, every block 616 / 573, half of them in one run per row 376 / 359; H = 32, N = 8192, every block 564 / 512,
+// runs of density 0.3 201 / 186; H = 40, N = 32760, runs of density 0.3 3339 / 2964; H = 40, N = 75600, runs of density 0.2
+// 11530 / 10405; H = 8, N = 75600, every block 11203 / 10022.  On scattered blocks of density 0.3 it is 3385 / 5726.
+// A paced form of it was slower than the plain launch at every one of these sizes.
+template <int OUT_DT, bool CAUSAL, bool Q16>
+__global__ void __launch_bounds__(256, 2) attn_sparse_pair_kernel(const AttnParams p) {
+  int vid = qblock_of<CAUSAL, true>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
+  if (vid >= qblock_units<true>(p) || !tiles_shared(p, vid / ((p.nbq + 1) >> 1))) return;
+  vid = with_args(p, vid);
+  attn_qblock<128, OUT_DT, CAUSAL, false, false, false, false, false, Q16, true>(p, vid);
 }
 
 // The same work with a resident set of workgroups per XCD that take the XCD's q-blocks generation by
@@ -729,9 +790,24 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, G = gridDim.x >> 3;
   unsigned arrivals = 0;
   bool waiting = true;   // a workgroup that has once waited in vain goes on without waiting for the rest of the launch
+  // (looked at once: at every generation it was 2 us of each, 40 us at N = 32760, H = 40)
+  bool some = false;     // whether the pair kernel has heads of this launch
+  if (p.share != nullptr) {
+    for (int i = threadIdx.x; i < (p.sparse_bs != 0 ? p.B * p.H : p.H); i += 128) some |= p.share[i] != 0;
+    some = __syncthreads_or(some);
+  }
   for (int base = 0; base < per; base += G) {
     const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
-    if (vid < p.total) attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true, Q16>(p, vid);
+    if (some) {
+      // a generation all of whose heads are attn_sparse_pair_kernel's does not meet (its heads are those from its first
+      // slot's to its last one's, and every workgroup of the XCD comes to the same answer)
+      const int last = qblock_of<CAUSAL>(p, xcd, min(base + G, per) - 1, per) / p.nbq;
+      bool any = false;
+      for (int bh = qblock_of<CAUSAL>(p, xcd, base, per) / p.nbq; bh <= last && bh < p.B * p.H; bh++) any |= !tiles_shared(p, bh);
+      if (!any) continue;
+    }
+    if (vid < p.total && !(some && tiles_shared(p, vid / p.nbq)))
+      attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true, Q16>(p, vid);
     if (base + G >= per) break;
     // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
     __syncthreads();   // also: both waves are done with this q-block's lists in LDS
@@ -755,6 +831,13 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
 }
 
 __global__ void attn_pace_reset_kernel(unsigned* counters) { counters[threadIdx.x] = 0u; }
+
+// share_look on its own (the operator has it done beside its last preparation step), and the paced launch's counters.
+__global__ void __launch_bounds__(SHARE_THREADS) attn_share_kernel(const ShareLook look, unsigned* __restrict__ counters) {
+  static_assert(SHARE_THREADS == 8 * PACE_PAD, "one counter word per thread");
+  if (counters != nullptr && blockIdx.x == 0) counters[threadIdx.x] = 0u;
+  share_look(look, blockIdx.x);
+}
 
 // Counters of the paced kernel: library-owned (looked up once per device), PACE_SETS sets of one counter per XCD.
 // Consecutive paced launches of the process take the sets in turn, so that launches which overlap on one GPU
@@ -828,6 +911,24 @@ static size_t attn_smem(int nbk, bool per_thread) {
   return AttnLds<D>::LIST_OFF + attn_list_bytes(nbk, AttnLds<D>::LIST_PAD, per_thread);
 }
 
+// The pair kernel's list has eight bytes per key block.
+static size_t pair_smem(int nbk) { return AttnLds<128>::LIST_OFF + (((size_t)(nbk + AttnLds<128>::LIST_PAD + 1) * 8 + 15) & ~(size_t)15); }
+
+// Whether the heads are looked at (share_look).  Where they turn out to be scattered, that and a launch that finds nothing to do
+// cost 3 to 15 us, where they are not the gain grows with the work.  Operator, D = 128, scattered blocks of density 0.3 / rows of one
+// run of density 0.3 / every block, us, not looked at -> looked at: B = 2, H = 32, N = 4096 181 -> 185 / 181 -> 183 / 360 -> 326;
+// H = 16, N = 8192 153 -> 156 / 154 -> 137 / 356 -> 288; H = 40, N = 12000 574 -> 577 / 563 -> 546; H = 24, N = 16384 596 -> 601 /
+// 596 -> 553; H = 48, N = 20000 1700 -> 1705 / 1615 -> 1548; attention, H = 40, N = 32760 3400 -> 3415 / 3350 -> 3030.  From 16384
+// keys on that is 1 % at most against 5 to 10.  Causal calls are those of dense masks as a rule, and gain that early: B = 2,
+// H = 32, Hkv = 8, N = 8192 278 -> 281 / 280 -> 284 / 611 -> 580, half of the blocks 369 -> 371 / 374 -> 371.
+// (Beyond 6135 key blocks the list leaves a compute unit one workgroup.)
+static bool pairs_pay(int64_t q_blocks, int nbk, bool causal) {
+  return nbk >= (causal ? 128 : 256) && q_blocks * nbk >= (int64_t)1 << 20 && pair_smem(nbk) <= 80 * 1024;
+}
+
+// Calls that have a pair kernel; a caller who names a kernel form or a launch gets that one.
+static bool pair_call(int D, int flags) { return D == 128 && flags == 0 && getenv("PARO_ATTN_PACING") == nullptr; }
+
 // Per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup, Wan 720p, the
 // paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms.  The lists that fit, up to 446 key
 // blocks at D = 128 and 872 at 64, end where the lines above begin, so only PARO_ATTN_PACED paces such a call.  Below, the plain
@@ -838,8 +939,25 @@ static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
   return !per_thread || (D == 64 ? attn_smem<64>(p.nbk, true) : attn_smem<128>(p.nbk, true)) <= 40 * 1024;
 }
 
+// The two launches in front of one on p, whose heads they divide between the pair kernel and that one.
+template <int OUT_DT, bool CAUSAL, bool Q16>
+static int launch_attn_pairs(const AttnParams& p, unsigned* counters, hipStream_t st) {
+  const ShareLook look = {p.sparse, p.sparse_bs != 0 ? p.B * p.H : p.H, p.nbq, p.nbk, CAUSAL, p.share};
+  if (!p.share_ready) hipLaunchKernelGGL(attn_share_kernel, dim3(look.heads), dim3(SHARE_THREADS), 0, st, look, counters);
+  const size_t smem = pair_smem(p.nbk);
+  auto kern = attn_sparse_pair_kernel<OUT_DT, CAUSAL, Q16>;
+  if (smem > 48 * 1024)
+    PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  const int units = p.B * p.H * ((p.nbq + 1) / 2);
+  hipLaunchKernelGGL(kern, dim3((units + 7) / 8 * 8), dim3(256), smem, st, p);
+  PARO_HIP(hipGetLastError());
+  return PARO_OK;
+}
+
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
-static int launch_attn(const AttnParams& p, hipStream_t st) {
+static int launch_attn(AttnParams p, hipStream_t st) {
+  constexpr bool PAIRS = D == 128 && !DUMP && !LSE && !EXACT && !PT;
+  if (!PAIRS || !pairs_pay(p.total, p.nbk, CAUSAL)) p.share = nullptr;
   const size_t smem = attn_smem<D>(p.nbk, PT);
   if (!DUMP && want_pacing(p, D, CAUSAL, EXACT) && pace_list_fits(p, D, PT)) {
     auto kern = attn_sparse_paced_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, Q16>;
@@ -863,12 +981,17 @@ static int launch_attn(const AttnParams& p, hipStream_t st) {
       int slack = (int)min((int64_t)G / 4, (int64_t)G * ((int64_t)2 << 20) / head_bytes);
       if (const char* e = getenv("PARO_ATTN_PACE_SLACK")) slack = max(0, min(G - 1, atoi(e)));
       unsigned* counters = pd.counters + (g_pace_launches.fetch_add(1u) % PACE_SETS) * (8 * PACE_PAD);
-      hipLaunchKernelGGL(attn_pace_reset_kernel, dim3(1), dim3(8 * PACE_PAD), 0, st, counters);
+      if (p.share == nullptr || p.share_ready) hipLaunchKernelGGL(attn_pace_reset_kernel, dim3(1), dim3(8 * PACE_PAD), 0, st, counters);
+      if constexpr (PAIRS)
+        if (int rc = p.share == nullptr ? PARO_OK : launch_attn_pairs<OUT_DT, CAUSAL, Q16>(p, counters, st)) return rc;
       hipLaunchKernelGGL(kern, dim3(8 * G), dim3(128), smem, st, p, counters, per, spins, slack);
       PARO_HIP(hipGetLastError());
       return PARO_OK;
     }
   }
+  if constexpr (PAIRS)
+    if (p.share != nullptr)
+      if (int rc = launch_attn_pairs<OUT_DT, CAUSAL, Q16>(p, nullptr, st)) return rc;
   const int grid = ((p.total + 7) / 8) * 8;
   auto kern = attn_sparse_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, Q16>;
   if (smem > 48 * 1024)
@@ -952,6 +1075,10 @@ static int attn_form(const AttnParams& p, int D, bool causal, bool exact, bool d
 }  // namespace paro
 
 namespace paro {
+bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags) {
+  return !with_lse && pair_call(D, flags) && pairs_pay((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), causal);
+}
+
 int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
                      const float* v_scale, const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
                      void* out, int out_dtype, float* lse, const AttnExtra& extra, int32_t* s_dump, int B,
@@ -1007,6 +1134,8 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   p.q8 = q8; p.k8 = k8; p.v8 = v8; p.q_scale = q_scale; p.k_scale = k_scale; p.v_scale = v_scale; p.v_mean = v_mean;
   p.sparse = sparse; p.out = out; p.lse = lse; p.s_dump = s_dump; p.sparse_bs = sparse_batch_stride;
   p.lse_scale = extra.lse_scale; p.k_mean = lse ? extra.k_mean : nullptr; p.lse_add = extra.lse_add || p.k_mean != nullptr;
+  p.share = pair_call(D, flags) ? extra.share : nullptr;
+  p.share_ready = extra.share_ready;
   p.q16 = extra.q16; p.lse_dot_scale = extra.lse_dot_scale;
   p.qs_b = q_stride_b; p.qs_h = q_stride_h; p.qs_n = q_stride_n;
   p.ks_b = k_stride_b; p.ks_h = k_stride_h; p.ks_n = k_stride_n;
@@ -1078,13 +1207,36 @@ extern "C" int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8
                                               void* stream) {
   using namespace paro;
   PARO_CHECK(orders, PARO_ERR_RUNTIME, "paro_attn_sparse_unpermute_fwd: null orders");
-  PARO_CHECK(n_text >= 0 && F > 0 && Hh > 0 && W > 0 && (int64_t)n_text + (int64_t)F * Hh * W == Nq, PARO_ERR_RUNTIME,
-             "paro_attn_sparse_unpermute_fwd: n_text + F*H*W = %d + %d*%d*%d does not equal the token count %d",
+  return paro_attn_sparse_scratch_fwd(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out, out_dtype,
+                                      lse, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b, k_stride_h,
+                                      k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale, is_causal, flags, orders, n_text,
+                                      F, Hh, W, nullptr, stream);
+}
+
+extern "C" int64_t paro_attn_scratch_bytes(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags) {
+  if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0) return 0;
+  return paro::attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, with_lse != 0, flags) ? (int64_t)B * H * 4 : 0;
+}
+
+extern "C" int paro_attn_sparse_scratch_fwd(const int8_t* q8, const int8_t* k8, const uint8_t* v8,
+                                            const float* q_scale, const float* k_scale, const float* v_scale,
+                                            const float* v_mean, const uint8_t* sparse, int64_t sparse_batch_stride,
+                                            void* out, int out_dtype, float* lse, int B, int H, int Hkv, int Nq, int Nk, int D,
+                                            int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n, int64_t k_stride_b,
+                                            int64_t k_stride_h, int64_t k_stride_n, int64_t o_stride_b, int64_t o_stride_h,
+                                            int64_t o_stride_n, float sm_scale, int is_causal, int flags,
+                                            const int32_t* orders, int n_text, int F, int Hh, int W, void* scratch, void* stream) {
+  using namespace paro;
+  PARO_CHECK(!orders || (n_text >= 0 && F > 0 && Hh > 0 && W > 0 && (int64_t)n_text + (int64_t)F * Hh * W == Nq),
+             PARO_ERR_RUNTIME, "paro_attn_sparse_unpermute_fwd: n_text + F*H*W = %d + %d*%d*%d does not equal the token count %d",
              n_text, F, Hh, W, Nq);
+  PARO_CHECK(((uintptr_t)scratch % 4) == 0, PARO_ERR_RUNTIME, "paro_attn_sparse_scratch_fwd: scratch must be 4-byte aligned");
+  AttnExtra extra;
+  extra.share = static_cast<int*>(scratch);
   return attn_sparse_impl(q8, k8, v8, q_scale, k_scale, v_scale, v_mean, sparse, sparse_batch_stride, out, out_dtype,
-                          lse, AttnExtra(), nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n, k_stride_b,
-                          k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale, is_causal, flags,
-                          orders, n_text, F, Hh, W, stream);
+                          lse, extra, nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h, q_stride_n,
+                          k_stride_b, k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n, sm_scale, is_causal, flags,
+                          orders, orders ? n_text : 0, orders ? F : 0, orders ? Hh : 0, orders ? W : 0, stream);
 }
 
 extern "C" int64_t paro_attn_workspace_bytes(int B, int Hkv, int Nk, int D) {
@@ -1141,8 +1293,9 @@ extern "C" int paro_qk_int8_sv_f16_attn(const int8_t* q8, const int8_t* k8, cons
   int rc = paro_v_fp8_pack(v, v_dtype, v8, v_scale, v_mean, partial, B, Hkv, Nk, D, v_stride_b, v_stride_h,
                            v_stride_n, smooth_v, stream);
   if (rc) return rc;
-  return paro_attn_sparse_fwd(q8, k8, v8, q_scale, k_scale, v_scale, smooth_v ? v_mean : nullptr, sparse,
-                              sparse_batch_stride, out, out_dtype, lse, nullptr, B, H, Hkv, Nq, Nk, D, q_stride_b,
-                              q_stride_h, q_stride_n, k_stride_b, k_stride_h, k_stride_n, o_stride_b, o_stride_h,
-                              o_stride_n, sm_scale, is_causal, flags, stream);
+  int* scratch = paro_v_fp8_partial_floats(B, Hkv, Nk, D) >= (int64_t)B * H ? (int*)partial : nullptr;   // (nobody's any more)
+  return paro_attn_sparse_scratch_fwd(q8, k8, v8, q_scale, k_scale, v_scale, smooth_v ? v_mean : nullptr, sparse,
+                                      sparse_batch_stride, out, out_dtype, lse, B, H, Hkv, Nq, Nk, D, q_stride_b, q_stride_h,
+                                      q_stride_n, k_stride_b, k_stride_h, k_stride_n, o_stride_b, o_stride_h, o_stride_n,
+                                      sm_scale, is_causal, flags, nullptr, 0, 0, 0, 0, scratch, stream);
 }

@@ -188,7 +188,9 @@ __host__ __device__ inline int64_t v_recp_offset(int64_t bh, int N, int D) { ret
 int v_fp8_stats(const void* v, int dtype, float* v_scale, float* v_mean, float* partial, int B, int Hkv, int N,
                 int D, int64_t vs_b, int64_t vs_h, int64_t vs_n, int smooth, hipStream_t st);
 // v_mean[b,h,ch] += v_scale[b,h,ch] * (sum of the channel's residual sums) / N, in a fixed order (one launch)
+// look (may be null): share_look of its heads in the same launch
+struct ShareLook;
 int v_fp8_add_residual(const float* resid, const float* v_scale, float* v_mean, int B, int Hkv, int N, int D,
-                       hipStream_t st);
+                       hipStream_t st, const ShareLook* look = nullptr);
 
 }  // namespace paro

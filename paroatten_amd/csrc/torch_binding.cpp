@@ -576,23 +576,21 @@ torch::Tensor attn_sparse_prepacked(const torch::Tensor& q8, const torch::Tensor
   const float* vsp = v_scale ? v_scale->data_ptr<float>() : nullptr;
   const float* vmp = v_mean ? v_mean->data_ptr<float>() : nullptr;
   const uint8_t* mask = static_cast<const uint8_t*>(sparse.data_ptr());
-  if (orders) {
+  if (orders)
     TORCH_CHECK(orders->is_cuda() && orders->scalar_type() == at::kInt && orders->dim() == 1 && orders->numel() == H &&
                     orders->is_contiguous(),
                 "orders must be a contiguous int32 GPU tensor of ", H, " entries");
-    check_rc(paro_attn_sparse_unpermute_fwd(
-        q8.data_ptr<int8_t>(), k8.data_ptr<int8_t>(), static_cast<const uint8_t*>(v8.data_ptr()), q_scale.data_ptr<float>(),
-        k_scale.data_ptr<float>(), vsp, vmp, mask, sparse_bs, output.data_ptr(), code_of(output), lse_p, (int)B, (int)H, (int)Hkv,
-        (int)Nq, (int)Nk, (int)D, q8.stride(0), q8.stride(1), q8.stride(2), k8.stride(0), k8.stride(1), k8.stride(2),
-        output.stride(0), output.stride(1), output.stride(2), (float)sm_scale, is_causal, flags, orders->data_ptr<int32_t>(),
-        n_text, F, Hh, W, stream_of(q8)));
-  } else {
-    check_rc(paro_attn_sparse_fwd(
-        q8.data_ptr<int8_t>(), k8.data_ptr<int8_t>(), static_cast<const uint8_t*>(v8.data_ptr()), q_scale.data_ptr<float>(),
-        k_scale.data_ptr<float>(), vsp, vmp, mask, sparse_bs, output.data_ptr(), code_of(output), lse_p, nullptr, (int)B, (int)H,
-        (int)Hkv, (int)Nq, (int)Nk, (int)D, q8.stride(0), q8.stride(1), q8.stride(2), k8.stride(0), k8.stride(1), k8.stride(2),
-        output.stride(0), output.stride(1), output.stride(2), (float)sm_scale, is_causal, flags, stream_of(q8)));
-  }
+  const int64_t n_scratch =
+      paro_attn_scratch_bytes((int)B, (int)H, (int)Nq, (int)Nk, (int)D, is_causal, return_lse, flags);
+  torch::Tensor scratch;
+  if (n_scratch > 0) scratch = torch::empty({n_scratch}, q8.options().dtype(at::kByte));
+  check_rc(paro_attn_sparse_scratch_fwd(
+      q8.data_ptr<int8_t>(), k8.data_ptr<int8_t>(), static_cast<const uint8_t*>(v8.data_ptr()), q_scale.data_ptr<float>(),
+      k_scale.data_ptr<float>(), vsp, vmp, mask, sparse_bs, output.data_ptr(), code_of(output), lse_p, (int)B, (int)H, (int)Hkv,
+      (int)Nq, (int)Nk, (int)D, q8.stride(0), q8.stride(1), q8.stride(2), k8.stride(0), k8.stride(1), k8.stride(2),
+      output.stride(0), output.stride(1), output.stride(2), (float)sm_scale, is_causal, flags,
+      orders ? orders->data_ptr<int32_t>() : nullptr, n_text, F, Hh, W, n_scratch > 0 ? scratch.data_ptr() : nullptr,
+      stream_of(q8)));
   return lse;
 }
 

@@ -17,6 +17,7 @@
 // monotonic, so no second reduction pass is needed.
 // Arithmetic follows MeanScaleKernel of the reference (csrc/fused/fused.cu:316-427) except that the
 // mean divides by the true token count.
+#include "share_device.hpp"
 #include "stats_device.hpp"
 #include "v_pack_device.hpp"
 
@@ -51,7 +52,12 @@ __global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __res
 template <int D>
 __global__ void __launch_bounds__(1024) v_residual_kernel(const float* __restrict__ resid,
                                                           const float* __restrict__ v_scale,
-                                                          float* __restrict__ v_mean, int N, int n_rows) {
+                                                          float* __restrict__ v_mean, int N, int n_rows, int heads,
+                                                          const ShareLook look) {
+  if ((int)blockIdx.x >= heads) {
+    share_look(look, blockIdx.x - heads);
+    return;
+  }
   constexpr int C4 = D / 4;          // threads per row
   constexpr int SL = 1024 / C4;      // rows in flight per pass
   __shared__ v4f red[SL][C4];
@@ -72,12 +78,14 @@ __global__ void __launch_bounds__(1024) v_residual_kernel(const float* __restric
 }
 
 int v_fp8_add_residual(const float* resid, const float* v_scale, float* v_mean, int B, int Hkv, int N, int D,
-                       hipStream_t st) {
-  const int n_rows = ceil_div(N, 64) * 2;
+                       hipStream_t st, const ShareLook* look) {
+  const int n_rows = ceil_div(N, 64) * 2, heads = B * Hkv;
+  const ShareLook l = look ? *look : ShareLook{};
+  const dim3 grid(heads + l.heads);
   if (D == 64)
-    hipLaunchKernelGGL((v_residual_kernel<64>), dim3(B * Hkv), dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows);
+    hipLaunchKernelGGL((v_residual_kernel<64>), grid, dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
   else
-    hipLaunchKernelGGL((v_residual_kernel<128>), dim3(B * Hkv), dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows);
+    hipLaunchKernelGGL((v_residual_kernel<128>), grid, dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
   PARO_HIP(hipGetLastError());
   return PARO_OK;
 }

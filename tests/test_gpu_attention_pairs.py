@@ -1,0 +1,123 @@
+"""The attention kernel in which two q-blocks share their tiles: the bits of the two-wave kernel (which the oracle tests cover)
+over the masks that divide a launch between the two, and the look at the mask that divides it."""
+import pytest
+import torch
+
+import paroatten_amd as P
+from paroatten_amd import _lib, synth
+from paroatten_amd._lib import ptr, stream_of
+
+pytestmark = pytest.mark.gpu
+
+# what a head's mask is, and whether its neighbouring rows keep the same blocks
+HEADS = (("window", 1), ("scattered", 0), ("dense", 1), ("empty", 0), ("window, rows missing", 1), ("half", 0))
+
+
+def _masks(H, nbq, nbk, causal, seed):
+    g = torch.Generator().manual_seed(seed)
+    m = torch.zeros(H, nbq, nbk, dtype=torch.bool)
+    want = []
+    for h in range(H):
+        kind, shared = HEADS[h % len(HEADS)]
+        if kind.startswith("window"):
+            for r in range(nbq):
+                lo = max(0, r * nbk // nbq - 40)
+                m[h, r, lo:lo + 41] = True
+            if "missing" in kind:   # one q-block of a pair, both, the last row, a block that one row alone has lost
+                m[h, [0, 5, 20, 21, nbq - 1]] = False
+                m[h, 30, :28] = False
+        elif kind == "dense":
+            m[h] = True
+        elif kind != "empty":
+            m[h] = torch.rand(nbq, nbk, generator=g) < (0.5 if kind == "half" else 0.1)
+        want.append(shared)
+    return m.cuda(), want
+
+
+def _operands(B, H, Hkv, Nq, Nk, seed, dtype=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    make = lambda h, n: torch.randn(B, h, n, 128, generator=g, device="cuda").to(dtype)
+    return make(H, Nq), make(Hkv, Nk), make(Hkv, Nk)
+
+
+@pytest.mark.parametrize("Nq,Nk,H,Hkv,causal", [
+    (16384, 16384, 18, 18, False),
+    (16321, 16400, 18, 6, False),    # odd and ragged: the last pair has one q-block of one row
+    (11200, 32768, 12, 12, False),   # 512 key blocks: 8 MB a head, beside the paced launch
+    (8129, 8129, 72, 24, True),
+    (16447, 16447, 24, 24, True),    # 257 q-blocks
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_same_bits_as_two_waves(Nq, Nk, H, Hkv, causal, dtype):
+    nbq, nbk = (Nq + 63) // 64, (Nk + 63) // 64
+    assert _lib.load().paro_attn_scratch_bytes(1, H, Nq, Nk, 128, int(causal), 0, 0) == 4 * H
+    q, k, v = _operands(1, H, Hkv, Nq, Nk, Nq, dtype)
+    m, _ = _masks(H, nbq, nbk, causal, 3)
+    # a block whose V is NaN, kept by one q-block of a pair in a head that is shared: the other one must not see it
+    m[0, 10, 5], m[0, 11, 5] = True, False
+    v[0, 0, 5 * 64 + 3, 7] = float("nan")
+    v[0, 0, 5 * 64 + 4, 9] = float("inf")
+    run = lambda **kw: P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, m, is_causal=causal, smooth_v=False, **kw)
+    got, ref = run(), run(two_waves=True)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    got, ref = (P.paroattn_qk_int8_pv_fp16_cuda(q, k, v.nan_to_num(1.0, 1.0, 1.0), m, is_causal=causal, smooth_k=True, two_waves=w)
+                for w in (False, True))
+    assert torch.isfinite(ref).all() and torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("B,per_batch,unpermute", [(1, False, True), (2, True, True), (2, False, False)])
+def test_heads_are_told_apart(B, per_batch, unpermute):
+    """INT8 operands through the C entry, with its scratch looked at afterwards; the unpermuting store."""
+    H, N, D = 12 if B > 1 else 18, 8 * 45 * 46 if unpermute else 16384, 128
+    nb = (N + 63) // 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q8, k8 = (torch.randint(-127, 128, (B, H, N, D), generator=g, device="cuda", dtype=torch.int8) for _ in range(2))
+    v8 = torch.randint(0, 100, (B * H * nb * 64 * D,), generator=g, device="cuda", dtype=torch.uint8)
+    qs, ks = torch.rand(B, H, 2 * nb, generator=g, device="cuda") * 1e-2, torch.rand(B, H, nb, generator=g, device="cuda") * 1e-2
+    vs, vm = torch.rand(B, H, D, generator=g, device="cuda"), torch.randn(B, H, D, generator=g, device="cuda")
+    if per_batch:
+        parts = [_masks(H, nb, nb, False, 1), _masks(H + 1, nb, nb, False, 2)]
+        m = torch.stack([parts[0][0], parts[1][0][1:]])
+        want = parts[0][1] + parts[1][1][1:]
+    else:
+        m, want = _masks(H, nb, nb, False, 1)
+    orders = torch.arange(H, device="cuda", dtype=torch.int32) % 6
+    grid = (0, 8, 45, 46) if unpermute else (0, 0, 0, 0)
+    outs = []
+    for flags in (0, _lib.PARO_ATTN_TWO_WAVES):
+        out = torch.full((B, H, N, D), 9.0, dtype=torch.bfloat16, device="cuda")
+        scratch = torch.full((B * H,), -1, dtype=torch.int32, device="cuda")
+        _lib.on(q8).paro_attn_sparse_scratch_fwd(
+            ptr(q8), ptr(k8), ptr(v8), ptr(qs), ptr(ks), ptr(vs), ptr(vm), ptr(m), m.stride(0) if per_batch else 0, ptr(out),
+            _lib.DTYPE_CODE[out.dtype], None, B, H, H, N, N, D, *q8.stride()[:3], *k8.stride()[:3], *out.stride()[:3], 0.05, 0, flags,
+            ptr(orders) if unpermute else None, *grid, ptr(scratch), stream_of(q8))
+        outs.append(out)
+        if flags == 0:
+            assert scratch[:len(want)].tolist() == want
+        else:
+            assert (scratch == -1).all()   # a named kernel form: nothing is looked at
+    assert torch.equal(*outs)
+
+
+def test_replayed_graph():
+    q, k, v = _operands(1, 16, 16, 16384, 16384, 8)
+    m, _ = _masks(16, 256, 256, False, 4)
+    ref = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, m, two_waves=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, m)
+    for i in range(3):
+        if i == 2:   # another mask: the heads are looked up again
+            m.copy_(m.flip(0))
+            ref = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, m, two_waves=True)
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, ref)
+
+
+def test_calls_without_the_kernel():
+    L = _lib.load()
+    for args in ((1, 48, 16384, 16384, 64, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 1, 0), (1, 48, 16320, 16320, 128, 0, 0, 0),
+                 (1, 15, 16384, 16384, 128, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 0, _lib.PARO_ATTN_EXACT_EXP),
+                 (1, 48, 64 * 6136, 64 * 6136, 128, 0, 0, 0), (0, 1, 1, 1, 128, 0, 0, 0)):
+        assert L.paro_attn_scratch_bytes(*args) == 0

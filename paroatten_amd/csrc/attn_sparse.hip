@@ -34,11 +34,12 @@
 
 namespace paro {
 
-template <int D> struct AttnLds {
+template <int D, bool PAIR = false> struct AttnLds {
   // LDS ring stages per operand.  D = 64: three, tiles are requested two iterations ahead.  D = 128:
   // two, requested one iteration ahead (an iteration is twice as long there), which keeps a workgroup
   // at 32 KB + lists so that four of them, the register-limited number, fit a CU's 160 KB.
-  static constexpr int NST = D == 128 ? 2 : 3;
+  // Pairs of q-blocks: four, so that their four waves meet at every second block.
+  static constexpr int NST = PAIR ? 4 : D == 128 ? 2 : 3;
   static constexpr int KTILE = 64 * D;   // bytes of one K8 tile: 64 rows of D bytes, 16-byte chunks XOR-swizzled
   static constexpr int VTILE = 64 * D;   // bytes of one V8 tile (fragment order, as in HBM)
   static constexpr int V_OFF = NST * KTILE;
@@ -83,7 +84,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
   static_assert(!Q16 || (!PT && !DUMP), "16-bit queries: neither per-thread scales nor the score dump");
   static_assert(!PAIR || (D == 128 && !PT && !DUMP && !LSE && !EXACT), "shared tiles: the fast path at D = 128");
-  using Lds = AttnLds<D>;
+  using Lds = AttnLds<D, PAIR>;
   constexpr int CW = PT ? 4 : 1;    // k scales per key block
   constexpr int KS = D / 32;        // k-steps of the QK MFMA (32 channels each)
   constexpr int DT_TILES = D / 32;  // 32-channel tiles of O^T
@@ -97,11 +98,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   KIdx* klist = reinterpret_cast<KIdx*>(clist + (p.nbk + Lds::LIST_PAD + 1) * CW);
   auto kidx = [](int entry) { return PAIR ? entry & 0xffff : entry; };
 
-  // (D = 64: opaque to the compiler.  In the paced kernel, which calls this in a loop, everything derived from
-  // the lane number alone is otherwise computed once in front of that loop and kept in registers, 35 more than
-  // the 168 that three waves per SIMD allow; at D = 128, with registers to spare, hoisting measured 2 % faster)
+  // (opaque to the compiler.  In the paced kernel, which calls this in a loop, everything derived from the lane number
+  // alone is otherwise computed once in front of that loop and kept in registers: at D = 64 35 more than the 168 that
+  // three waves per SIMD allow, at D = 128 all 256 and two to eight spilled, which took N = 32760, H = 40, density 0.3 from
+  // 3684 to 3710 us)
   int t = threadIdx.x;
-  if constexpr (D == 64) asm volatile("" : "+v"(t));
+  if constexpr (D == 64 || PACED) asm volatile("" : "+v"(t));
   const int lane = t & 63, part = t >> 6;   // part: what the wave moves of a tile
   const int wave = PAIR ? part & 1 : part;  // its half of the q-block
   const int l32 = lane & 31, lh = lane >> 5;
@@ -413,7 +415,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 
   // One block.  `acc` holds its S^T on entry and that of the next block on exit.  sk1: K stage of block
   // it+1; sv: V stage of block it; skn / svn: the stages this iteration's DMA refills.
-  auto step = [&](int it, int sk1, int sv, int skn, int svn) {
+  auto step = [&](int it, int sk1, int sv, int skn, int svn, bool meet = true) {
     // -- memory traffic of this iteration, issued up front
     if constexpr (RING2) {
       load_k(kb_2, skn);   // K(it+2) into the stage K(it) has left
@@ -664,8 +666,10 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     // -- what the ring needs next has to have landed before the barrier publishes it
     const int kb_4 = __builtin_amdgcn_readfirstlane(kidx_v);
     // (a bare s_barrier: __syncthreads() would add a fence that waits for ALL outstanding loads)
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(RING2 ? 0 : LOADS_PER_IT) : "memory");
-    __builtin_amdgcn_s_barrier();
+    if (meet) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(RING2 || PAIR ? 0 : LOADS_PER_IT) : "memory");
+      __builtin_amdgcn_s_barrier();
+    }
     kb_c = kb_1; kb_1 = kb_2; kb_2 = kb_3; kb_3 = kb_4;
     c_cur = c_next;
     if constexpr (PT) cb_cur = cb_next;
@@ -678,6 +682,19 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       step(it, 1, 0, 0, 1);
       if (it + 1 >= cnt) break;
       step(it + 1, 0, 1, 1, 0);
+    }
+  } else if constexpr (PAIR) {
+    // stage of block j is j % 4: iteration `it` reads K stage it+1 and V stage it and refills K stage it+3 and V stage it+2, which
+    // the two iterations in front of the last meeting have left; what an odd iteration and the one before it have requested is
+    // waited for at the odd one's end
+    for (int it = 0; it < cnt; it += 4) {
+      step(it, 1, 0, 3, 2, false);
+      if (it + 1 >= cnt) break;
+      step(it + 1, 2, 1, 0, 3);
+      if (it + 2 >= cnt) break;
+      step(it + 2, 3, 2, 1, 0, false);
+      if (it + 3 >= cnt) break;
+      step(it + 3, 0, 3, 2, 1);
     }
   } else {
     // stage of block j is j % 3: with i = it % 3, iteration `it` reads K stage i+1 and V stage i, refills
@@ -754,7 +771,9 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
 // N = 8192, causal, every block 616 / 573, half of them in one run per row 376 / 359; H = 32, N = 8192, every block 564 / 512,
 // runs of density 0.3 201 / 186; H = 40, N = 32760, runs of density 0.3 3339 / 2964; H = 40, N = 75600, runs of density 0.2
 // 11530 / 10405; H = 8, N = 75600, every block 11203 / 10022.  On scattered blocks of density 0.3 it is 3385 / 5726.
-// A paced form of it was slower than the plain launch at every one of these sizes.
+// A paced form of it was slower than the plain launch at every one of these sizes.  (These with two ring stages, one meeting of
+// the four waves per block.  The 80 KB of LDS that each of a compute unit's two workgroups has hold four, and a meeting at every
+// second block: the operator and the layer, start to end, 593 -> 584 and 11460 -> 11381.)
 template <int OUT_DT, bool CAUSAL, bool Q16>
 __global__ void __launch_bounds__(256, 2) attn_sparse_pair_kernel(const AttnParams p) {
   int vid = qblock_of<CAUSAL, true>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
@@ -912,7 +931,10 @@ static size_t attn_smem(int nbk, bool per_thread) {
 }
 
 // The pair kernel's list has eight bytes per key block.
-static size_t pair_smem(int nbk) { return AttnLds<128>::LIST_OFF + (((size_t)(nbk + AttnLds<128>::LIST_PAD + 1) * 8 + 15) & ~(size_t)15); }
+static size_t pair_smem(int nbk) {
+  using Lds = AttnLds<128, true>;
+  return Lds::LIST_OFF + (((size_t)(nbk + Lds::LIST_PAD + 1) * 8 + 15) & ~(size_t)15);
+}
 
 // Whether the heads are looked at (share_look).  Where they turn out to be scattered, that and a launch that finds nothing to do
 // cost 3 to 15 us, where they are not the gain grows with the work.  Operator, D = 128, scattered blocks of density 0.3 / rows of one
@@ -921,7 +943,7 @@ static size_t pair_smem(int nbk) { return AttnLds<128>::LIST_OFF + (((size_t)(nb
 // 596 -> 553; H = 48, N = 20000 1700 -> 1705 / 1615 -> 1548; attention, H = 40, N = 32760 3400 -> 3415 / 3350 -> 3030.  From 16384
 // keys on that is 1 % at most against 5 to 10.  Causal calls are those of dense masks as a rule, and gain that early: B = 2,
 // H = 32, Hkv = 8, N = 8192 278 -> 281 / 280 -> 284 / 611 -> 580, half of the blocks 369 -> 371 / 374 -> 371.
-// (Beyond 6135 key blocks the list leaves a compute unit one workgroup.)
+// (Beyond 2039 key blocks the list leaves a compute unit one workgroup.)
 static bool pairs_pay(int64_t q_blocks, int nbk, bool causal) {
   return nbk >= (causal ? 128 : 256) && q_blocks * nbk >= (int64_t)1 << 20 && pair_smem(nbk) <= 80 * 1024;
 }

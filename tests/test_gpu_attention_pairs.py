@@ -119,5 +119,5 @@ def test_calls_without_the_kernel():
     L = _lib.load()
     for args in ((1, 48, 16384, 16384, 64, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 1, 0), (1, 48, 16320, 16320, 128, 0, 0, 0),
                  (1, 15, 16384, 16384, 128, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 0, _lib.PARO_ATTN_EXACT_EXP),
-                 (1, 48, 64 * 6136, 64 * 6136, 128, 0, 0, 0), (0, 1, 1, 1, 128, 0, 0, 0)):
+                 (1, 48, 64 * 2040, 64 * 2040, 128, 0, 0, 0), (0, 1, 1, 1, 128, 0, 0, 0)):
         assert L.paro_attn_scratch_bytes(*args) == 0

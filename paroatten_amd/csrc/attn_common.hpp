@@ -47,6 +47,10 @@ struct AttnParams {
   // Scratch of the call (null: none given), one word per head of the mask: whether the pair kernel takes it (attn_share_kernel)
   int* share;
   int share_ready;   // it holds that already
+  // The residual sums of the V tiles, [B,Hkv][resid_rows][D], that v_mean still lacks (null: it is complete).  attn_sparse_split.hip
+  // alone takes them (attn_takes_residual).
+  const float* v_resid;
+  int resid_rows;
 };
 
 __device__ __forceinline__ bool tiles_shared(const AttnParams& p, int bh) { return p.share[p.sparse_bs != 0 ? bh : bh % p.H] != 0; }
@@ -229,6 +233,7 @@ int launch_attn_pv16(const AttnParams& p, int D, int out_dtype, bool causal, hip
 // The kernel that takes several kept blocks of a q-block at a time (attn_sparse_split.hip): either head size, with or
 // without lse, plain launch.  split_width: how many, or 0 where another kernel is the faster one.
 int split_width(const AttnParams& p, int D);
+bool split_takes_residual(int64_t q_blocks, int nbk, int D);   // AttnParams::v_resid
 int launch_attn_split(const AttnParams& p, int D, int out_dtype, bool causal, bool exact, hipStream_t st);
 
 // Q from 16 bits, and what goes into a stored log-sum-exp (AttnParams says what they are)
@@ -240,7 +245,12 @@ struct AttnExtra {
   float lse_dot_scale = 0.f;
   int* share = nullptr;   // B * H words, or null
   bool share_ready = false;
+  const float* v_resid = nullptr;
+  int resid_rows = 0;
 };
+
+// Whether a call of these sizes and flags, on FP8 tiles, adds the residual sums up by itself
+bool attn_takes_residual(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags);
 
 // Whether a call of these sizes and flags has a use for AttnExtra::share
 bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags);

@@ -653,7 +653,10 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   if (v_resid_offset((int64_t)B * Hkv, Nk, D) >= (int64_t)B * H &&
       attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, lse != nullptr, flags | (per_thread ? PARO_ATTN_QK_PER_THREAD : 0)))
     extra.share = (int*)p.v_work;
-  if (p.v_resid && !p.one_launch) {
+  if (p.v_resid && !p.one_launch && !per_thread && attn_takes_residual(B, H, Nq, Nk, D, is_causal != 0, lse != nullptr, flags)) {
+    extra.v_resid = p.v_resid;
+    extra.resid_rows = 2 * p.nbk;
+  } else if (p.v_resid && !p.one_launch) {
     const ShareLook look = {sparse, sparse_batch_stride != 0 ? B * H : H, p.nbq, p.nbk, is_causal, extra.share};
     if ((rc = v_fp8_add_residual(p.v_resid, p.v_scale, p.v_mean, B, Hkv, Nk, D, st, extra.share ? &look : nullptr))) return rc;
     extra.share_ready = extra.share != nullptr;

@@ -1097,6 +1097,11 @@ static int attn_form(const AttnParams& p, int D, bool causal, bool exact, bool d
 }  // namespace paro
 
 namespace paro {
+bool attn_takes_residual(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags) {
+  return paro_attn_kernel_form(B, H, Nq, Nk, D, causal, with_lse, flags) == PARO_ATTN_FORM_SPLIT &&
+         split_takes_residual((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), D);
+}
+
 bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags) {
   return !with_lse && pair_call(D, flags) && pairs_pay((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), causal);
 }
@@ -1158,6 +1163,7 @@ int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, cons
   p.lse_scale = extra.lse_scale; p.k_mean = lse ? extra.k_mean : nullptr; p.lse_add = extra.lse_add || p.k_mean != nullptr;
   p.share = pair_call(D, flags) ? extra.share : nullptr;
   p.share_ready = extra.share_ready;
+  p.v_resid = extra.v_resid; p.resid_rows = extra.resid_rows;
   p.q16 = extra.q16; p.lse_dot_scale = extra.lse_dot_scale;
   p.qs_b = q_stride_b; p.qs_h = q_stride_h; p.qs_n = q_stride_n;
   p.ks_b = k_stride_b; p.ks_h = k_stride_h; p.ks_n = k_stride_n;

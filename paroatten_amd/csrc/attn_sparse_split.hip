@@ -33,7 +33,11 @@ template <int D, int W> struct SplitLds {
   static constexpr int EPI_OFF = W * RING > SHARES ? W * RING : SHARES;   // v_scale and v_mean of the head
   static constexpr int M_OFF = EPI_OFF + 2 * D * 4;              // the settled maximum of the 32 rows
   static constexpr int FLAG_OFF = M_OFF + 32 * 4;                // [round parity][8] bytes, one per wave
-  static constexpr int LIST_OFF = FLAG_OFF + 16;
+  // Partial sums of the residual sums, 1024 x 16 bytes: at D = 64 where the shares come at the end.
+  static constexpr bool RESID = D == 64 || W == 4;
+  static constexpr int RED_OFF = D == 64 ? 0 : FLAG_OFF + 16;
+  static_assert(D == 128 || SHARES >= 1024 * 16, "the partial sums fit where the shares go");
+  static constexpr int LIST_OFF = FLAG_OFF + 16 + (D == 128 && RESID ? 1024 * 16 : 0);
   static constexpr int LIST_PAD = 4 * W;                         // a wave looks up to 4 rounds ahead
 };
 
@@ -108,6 +112,25 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
   const int epi_ch = t % D;   // (W * 64 >= D; every wave writes the same values)
   epi_sc = p.v_scale[bhk * D + epi_ch];
   if (p.v_mean) epi_mn = p.v_mean[bhk * D + epi_ch];
+  // What v_mean still lacks, in the order of v_residual_kernel, to the bit: SL partial sums per channel, added up below
+  constexpr int C4 = D / 4, SL = 1024 / C4, SIDE = 64 * W / C4, PASSES = SL / SIDE;
+  v4f* red = reinterpret_cast<v4f*>(smem + Lds::RED_OFF);
+  if (Lds::RESID && p.v_resid != nullptr) {
+    const v4f* src = reinterpret_cast<const v4f*>(p.v_resid + bhk * p.resid_rows * D) + t % C4;
+    v4f x[PASSES];
+#pragma unroll
+    for (int u = 0; u < PASSES; u++) x[u] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int r = t / C4; r < p.resid_rows; r += SL)
+#pragma unroll
+      for (int u = 0; u < PASSES; u++) {
+        const v4f y = src[(int64_t)min(r + u * SIDE, p.resid_rows - 1) * C4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[u][q] += r + u * SIDE < p.resid_rows ? y[q] : 0.f;
+      }
+#pragma unroll
+    for (int u = 0; u < PASSES; u++) red[(t / C4 + u * SIDE) * C4 + t % C4] = x[u];
+  }
   list_take(0);
   for (int base = 64 * MU; base < kmax; base += 64 * MU) {
     list_load(base);
@@ -339,6 +362,11 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
     load_v(kb_c, vfrag[0]);
     quantise_q();
   }
+  if (Lds::RESID && p.v_resid != nullptr && t < D) {   // (while the tiles are on their way; read behind the barriers of the rounds)
+    float s = 0.f;
+    for (int i = 0; i < SL; i++) s += red[i * C4 + (t >> 2)][t & 3];
+    epi[D + t] = epi_mn + epi_sc * (s / (float)p.Nk);
+  }
   v16i acc[2][2];   // [round parity][row tile of the 64 keys]: the next round's products are issued before the barrier
   qk(acc[0], kfrag[0]);
   // columns past the end of K or above the diagonal leave the softmax
@@ -523,6 +551,15 @@ int split_width(const AttnParams& p, int D) {
   }
   const size_t smem = D == 64 ? split_lds<64>(p.nbk, W) : split_lds<128>(p.nbk, W);
   return smem <= 160 * 1024 ? W : 0;
+}
+
+// A launch of their own for the residual sums of V is worth 1 to 1.4 us; here every workgroup reads all of its head's, beside its
+// mask row.  Operator, device time, us, a launch of their own / here: D = 64, two heads N = 1200 16.9 / 15.8, N = 2048 17.6 / 16.5,
+// N = 4096 20.9 / 19.7 (four heads 23.6 / 22.2, eight 29.5 / 28.4), N = 8192 one head 25.3 / 25.4, two 29.1 / 28.7; one head, N = 30000
+// 81.8 / 85.9.  D = 128, W = 4, N = 1200 23.4 / 22.3, N = 2048 25.2 / 23.8, N = 4096 30.7 / 30.0, N = 8192 38.9 / 38.9; W = 2, where
+// the partial sums take the LDS of another workgroup, N = 2048, eight heads 30.9 / 32.8, N = 4096, four heads 37.5 / 43.0.
+bool split_takes_residual(int64_t q_blocks, int nbk, int D) {
+  return nbk <= 64 && (D == 64 || (q_blocks <= 128 && nbk >= 16));   // (D = 128: W = 4)
 }
 
 int launch_attn_split(const AttnParams& p, int D, int out_dtype, bool causal, bool exact, hipStream_t st) {

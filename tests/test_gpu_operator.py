@@ -233,3 +233,28 @@ def test_queries_in_a_pass_of_their_own(dev, H, Hkv, Nq, Nk, D, mode, smooth_k):
         scale = scale + terms.abs().sum(-1) * D ** -0.5
     # one product and one sum in fp32, and an fp32 dot product of D terms
     assert ((lse.double() - want).abs() <= (D + 4) * 2.0 ** -24 * scale + 1e-30).all()
+
+
+@pytest.mark.parametrize("N,D,H,dtype", [
+    (1025, 64, 1, torch.float16), (1473, 64, 2, torch.bfloat16), (2049, 64, 12, torch.float16), (4033, 64, 8, torch.float16),
+    (4096, 64, 2, torch.bfloat16), (4097, 64, 2, torch.float16),
+    (1025, 128, 1, torch.float16), (2047, 128, 4, torch.bfloat16), (4096, 128, 2, torch.bfloat16), (4096, 128, 3, torch.float16),
+])
+@pytest.mark.parametrize("with_lse", [False, True])
+def test_residual_sums_in_the_attention_launch(dev, N, D, H, dtype, with_lse):
+    """Both sides of the rule by which the kernel of few q-blocks adds up what v_mean lacks: a V with a mean beside a wide channel, so
+    that the sums matter, against the extension entry point, which has a launch of their own for them.  The same bits."""
+    import paroatten_amd as P
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    g = torch.Generator().manual_seed(N + D)
+    q, k, v = ((torch.randint(-63, 64, (1, H, N, D), generator=g) / 8).to(dtype).to(dev) for _ in range(3))
+    v[..., ::3] += 5
+    nb = (N + 63) // 64
+    mask = synth.make_block_mask(H, nb, 0.6, seed=N, device=dev)
+    mask[0, 1] = False
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, None, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="HND")
+    ref = torch.empty_like(q)
+    qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, ref, qs, ks, 1, 0, 2, D ** -0.5, int(with_lse), mask)
+    got = P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, mask, return_lse=with_lse)
+    assert torch.equal(got[0] if with_lse else got, ref)

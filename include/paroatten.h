@@ -54,7 +54,7 @@ extern "C" {
 #define PARO_ATTN_TWO_WAVES 8 /* kernel form: two waves per 64-row q-block (32 q-rows each) also where the
                                  library would pick one wave per q-block (head size 64, plain launch, more than
                                  1024 q-blocks; bit-identical results) or several key blocks of a q-block at a
-                                 time (without any of the form flags, up to 256 q-blocks and at least 20 key blocks;
+                                 time (without any of the form flags, up to 512 q-blocks (head size 128: 256);
                                  the same weights, summed in another order) */
 #define PARO_ATTN_PV_F16 16   /* accuracy mode: the P.V product in float16 with fp32 accumulation, as the reference's
                                  qk_int8_sv_f16_accum_f16_attn computes it (csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:263-391),

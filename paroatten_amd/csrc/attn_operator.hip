@@ -3,7 +3,7 @@
 //   op_stats     K sums (smooth_k) and V statistics (FP8 product), side by side
 //   op_finalize  their second steps
 //   op_prep      quantised K and the V tiles, side by side (op_q_pass: quantised Q too)
-//   v_residual   (FP8 product with smooth_v)
+//   v_residual   (FP8 product with smooth_v; up to 4096 keys and with few q-blocks the attention launch does it: split_takes_residual)
 //   attention    on 16-bit Q, which the q-block's own waves quantise (QRows; op_q_pass: on INT8 Q); the
 //                log-sum-exp leaves as the natural one of the scores of q and k as given
 // Short sequences take one launch for the first four (op_head: up to 1024 tokens, as many heads as op_head_plan says) or one for

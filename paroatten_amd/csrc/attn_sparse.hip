@@ -812,8 +812,14 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
   // (looked at once: at every generation it was 2 us of each, 40 us at N = 32760, H = 40)
   bool some = false;     // whether the pair kernel has heads of this launch
   if (p.share != nullptr) {
-    for (int i = threadIdx.x; i < (p.sparse_bs != 0 ? p.B * p.H : p.H); i += 128) some |= p.share[i] != 0;
+    bool all = true;
+    for (int i = threadIdx.x; i < (p.sparse_bs != 0 ? p.B * p.H : p.H); i += 128) {
+      const bool shared = p.share[i] != 0;
+      some |= shared;
+      all &= shared;
+    }
     some = __syncthreads_or(some);
+    if (__syncthreads_and(all)) return;
   }
   for (int base = 0; base < per; base += G) {
     const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;

@@ -46,34 +46,39 @@ __global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __res
   v_pack_body<DT, D>(v + b * vs_b + h * vs_h, v8, work, v_mean, resid, N, nb, vs_n, blockIdx.x, (int64_t)b * gridDim.y + h);
 }
 
-// v_mean += v_scale * (sum over tiles and row tiles of the residual sums) / N.  A thread takes four
-// channels of every SL-th row (16-byte loads, all independent), the SL partial sums per channel are
-// combined through LDS in a fixed order.
+// v_mean += v_scale * (sum over tiles and row tiles of the residual sums) / N.  A workgroup has 32 channels of a head; a thread
+// takes four of them of every SL-th row (16-byte loads, all independent), the SL partial sums per channel are
+// combined through LDS in a fixed order.  What bounds it is the trips to memory one after the other, behind a launch of 4 to
+// 5 us in a kernel trace; with one workgroup to a head and four loads in flight per thread instead of eight, 40 heads, D = 128:
+// N = 75600 15.0 -> 10.4 us, N = 32760 8.0 -> 6.3 (D = 64, N = 17776, 96 heads: 5.3 and 5.6).
+template <int D> constexpr int V_RESIDUAL_THREADS = 1024 / D * 4 * 8;
 template <int D>
-__global__ void __launch_bounds__(1024) v_residual_kernel(const float* __restrict__ resid,
+__global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const float* __restrict__ resid,
                                                           const float* __restrict__ v_scale,
                                                           float* __restrict__ v_mean, int N, int n_rows, int heads,
                                                           const ShareLook look) {
-  if ((int)blockIdx.x >= heads) {
-    share_look(look, blockIdx.x - heads);
+  constexpr int PARTS = D / 32;
+  if ((int)blockIdx.x >= heads * PARTS) {
+    share_look(look, blockIdx.x - heads * PARTS);
     return;
   }
   constexpr int C4 = D / 4;          // threads per row
   constexpr int SL = 1024 / C4;      // rows in flight per pass
-  __shared__ v4f red[SL][C4];
-  const int c4 = threadIdx.x % C4, sl = threadIdx.x / C4;
-  const int64_t bh = blockIdx.x;
-  const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + c4;
+  __shared__ v4f red[SL][8];
+  const int c4 = threadIdx.x % 8, sl = threadIdx.x / 8, part = blockIdx.x % PARTS;
+  const int64_t bh = blockIdx.x / PARTS;
+  const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + part * 8 + c4;
   v4f s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
+#pragma unroll 8
   for (int r = sl; r < n_rows; r += SL) s += p[(int64_t)r * C4];
   red[sl][c4] = s;
   __syncthreads();
-  if (threadIdx.x < D) {
-    const int ch = threadIdx.x;
+  if (threadIdx.x < 32) {
+    const int64_t ch = bh * D + part * 32 + threadIdx.x;
     float t = 0.f;
-    for (int i = 0; i < SL; i++) t += red[i][ch >> 2][ch & 3];
-    v_mean[bh * D + ch] += v_scale[bh * D + ch] * (t / (float)N);
+#pragma unroll 8
+    for (int i = 0; i < SL; i++) t += red[i][threadIdx.x >> 2][threadIdx.x & 3];
+    v_mean[ch] += v_scale[ch] * (t / (float)N);
   }
 }
 
@@ -81,11 +86,11 @@ int v_fp8_add_residual(const float* resid, const float* v_scale, float* v_mean, 
                        hipStream_t st, const ShareLook* look) {
   const int n_rows = ceil_div(N, 64) * 2, heads = B * Hkv;
   const ShareLook l = look ? *look : ShareLook{};
-  const dim3 grid(heads + l.heads);
+  const dim3 grid(heads * (D / 32) + l.heads);
   if (D == 64)
-    hipLaunchKernelGGL((v_residual_kernel<64>), grid, dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
+    hipLaunchKernelGGL((v_residual_kernel<64>), grid, dim3(V_RESIDUAL_THREADS<64>), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
   else
-    hipLaunchKernelGGL((v_residual_kernel<128>), grid, dim3(1024), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
+    hipLaunchKernelGGL((v_residual_kernel<128>), grid, dim3(V_RESIDUAL_THREADS<128>), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
   PARO_HIP(hipGetLastError());
   return PARO_OK;
 }

@@ -210,7 +210,8 @@ int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8, const uin
                                    void* stream);
 
 /* (2b) or, with orders, (2b') with device scratch of paro_attn_scratch_bytes() bytes (4-byte aligned, contents arbitrary, this
- * call's until it has run; NULL: none).  With it, head size 128 and enough work, heads in which neighbouring q-blocks keep
+ * call's until it has run; NULL: none).  With it, head size 128, enough work and no flag but
+ * PARO_ATTN_EXACT_EXP, heads in which neighbouring q-blocks keep
  * the same key blocks are found on the device and taken by a kernel in which two q-blocks share their tiles; outputs are the
  * same bits.  paro_attn_scratch_bytes: 0 for calls that have no use for it. */
 int64_t paro_attn_scratch_bytes(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags);

@@ -253,7 +253,7 @@ struct AttnExtra {
 bool attn_takes_residual(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags);
 
 // Whether a call of these sizes and flags has a use for AttnExtra::share
-bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags);
+bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, int flags);
 
 // paro_attn_sparse_fwd / _unpermute_fwd (attn_sparse.hip).  extra.q16: q8 and q_scale are not read, the q strides are those of
 // the 16-bit tensor, which is of the type out_dtype.

@@ -651,7 +651,7 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
   AttnExtra extra;
   // (of v_work, what lies in front of the residual sums is nobody's any more)
   if (v_resid_offset((int64_t)B * Hkv, Nk, D) >= (int64_t)B * H &&
-      attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, lse != nullptr, flags | (per_thread ? PARO_ATTN_QK_PER_THREAD : 0)))
+      attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, flags | (per_thread ? PARO_ATTN_QK_PER_THREAD : 0)))
     extra.share = (int*)p.v_work;
   if (p.v_resid && !p.one_launch && !per_thread && attn_takes_residual(B, H, Nq, Nk, D, is_causal != 0, lse != nullptr, flags)) {
     extra.v_resid = p.v_resid;

@@ -83,7 +83,7 @@ template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool 
 __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) {
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
   static_assert(!Q16 || (!PT && !DUMP), "16-bit queries: neither per-thread scales nor the score dump");
-  static_assert(!PAIR || (D == 128 && !PT && !DUMP && !LSE && !EXACT), "shared tiles: the fast path at D = 128");
+  static_assert(!PAIR || (D == 128 && !PT && !DUMP), "shared tiles: D = 128, neither per-thread scales nor the score dump");
   using Lds = AttnLds<D, PAIR>;
   constexpr int CW = PT ? 4 : 1;    // k scales per key block
   constexpr int KS = D / 32;        // k-steps of the QK MFMA (32 channels each)
@@ -345,6 +345,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
   v8i ones = {sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word, sel_word};
   asm volatile("" : "+v"(ones));  // same: resident constant operand
   float m_i = -1e30f;
+  [[maybe_unused]] bool begun = false;   // PAIR: a block of this q-block's has been
   float m_off = 0.f, m_off8 = 0.f;  // the m-dependent offsets (see step)
   float d_exact = 0.f;  // LSE only: sum of the unrounded P~ of this lane's 32 kv-columns per block
 
@@ -610,8 +611,10 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     __builtin_amdgcn_sched_barrier(0);
     // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
     // and d_new[1]; a NaN byte of either row makes its own sum NaN whatever the hardware makes of 0 x NaN)
+    const bool first = PAIR ? !begun : it == 0;
+    if constexpr (PAIR) begun = begun || mine;
     if constexpr (EXACT) {
-      if (it == 0 || headroom_suspect(d_new)) {
+      if (first || headroom_suspect(d_new)) {
         const float m_blk = block_max();
         if (__ballot(m_blk > m_i + P_HEADROOM) != 0ull) {
           apply_refresh(m_blk);
@@ -619,7 +622,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
         }
       }
       d_new = row_sums();
-    } else if (it == 0 || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
+    } else if (first || __ballot(__builtin_isunordered(d_new[0], d_new[1])) != 0ull) {
       apply_refresh(block_max());
       words();
       d_new = row_sums();
@@ -771,15 +774,18 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
 // N = 8192, causal, every block 616 / 573, half of them in one run per row 376 / 359; H = 32, N = 8192, every block 564 / 512,
 // runs of density 0.3 201 / 186; H = 40, N = 32760, runs of density 0.3 3339 / 2964; H = 40, N = 75600, runs of density 0.2
 // 11530 / 10405; H = 8, N = 75600, every block 11203 / 10022.  On scattered blocks of density 0.3 it is 3385 / 5726.
+// With true exponentials, operator, start to end, rows of one run of density 0.3: H = 16, N = 30000 1491 / 1317, with the log-sum-exp
+// 1556 / 1395, H = 32, N = 17000 958 / 921; causal as above, every block 768 / 740 (scattered blocks with the look at them: N = 30000
+// 1486 / 1497 and 1548 / 1557, N = 17000 991 / 995, causal half of the blocks 448 / 452).
 // A paced form of it was slower than the plain launch at every one of these sizes.  (These with two ring stages, one meeting of
 // the four waves per block.  The 80 KB of LDS that each of a compute unit's two workgroups has hold four, and a meeting at every
 // second block: the operator and the layer, start to end, 593 -> 584 and 11460 -> 11381.)
-template <int OUT_DT, bool CAUSAL, bool Q16>
+template <int OUT_DT, bool CAUSAL, bool LSE, bool EXACT, bool Q16>
 __global__ void __launch_bounds__(256, 2) attn_sparse_pair_kernel(const AttnParams p) {
   int vid = qblock_of<CAUSAL, true>(p, blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3);
   if (vid >= qblock_units<true>(p) || !tiles_shared(p, vid / ((p.nbq + 1) >> 1))) return;
   vid = with_args(p, vid);
-  attn_qblock<128, OUT_DT, CAUSAL, false, false, false, false, false, Q16, true>(p, vid);
+  attn_qblock<128, OUT_DT, CAUSAL, false, LSE, EXACT, false, false, Q16, true>(p, vid);
 }
 
 // The same work with a resident set of workgroups per XCD that take the XCD's q-blocks generation by
@@ -955,7 +961,9 @@ static bool pairs_pay(int64_t q_blocks, int nbk, bool causal) {
 }
 
 // Calls that have a pair kernel; a caller who names a kernel form or a launch gets that one.
-static bool pair_call(int D, int flags) { return D == 128 && flags == 0 && getenv("PARO_ATTN_PACING") == nullptr; }
+static bool pair_call(int D, int flags) {
+  return D == 128 && (flags & ~PARO_ATTN_EXACT_EXP) == 0 && getenv("PARO_ATTN_PACING") == nullptr;
+}
 
 // Per-thread scales make the list three times as long: where that costs a compute unit its fourth workgroup, Wan 720p, the
 // paced form with half the waves measured slower than the plain launch, 21.8 against 17.3 ms.  The lists that fit, up to 446 key
@@ -968,12 +976,12 @@ static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
 }
 
 // The two launches in front of one on p, whose heads they divide between the pair kernel and that one.
-template <int OUT_DT, bool CAUSAL, bool Q16>
+template <int OUT_DT, bool CAUSAL, bool LSE, bool EXACT, bool Q16>
 static int launch_attn_pairs(const AttnParams& p, unsigned* counters, hipStream_t st) {
   const ShareLook look = {p.sparse, p.sparse_bs != 0 ? p.B * p.H : p.H, p.nbq, p.nbk, CAUSAL, p.share};
   if (!p.share_ready) hipLaunchKernelGGL(attn_share_kernel, dim3(look.heads), dim3(SHARE_THREADS), 0, st, look, counters);
   const size_t smem = pair_smem(p.nbk);
-  auto kern = attn_sparse_pair_kernel<OUT_DT, CAUSAL, Q16>;
+  auto kern = attn_sparse_pair_kernel<OUT_DT, CAUSAL, LSE, EXACT, Q16>;
   if (smem > 48 * 1024)
     PARO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   const int units = p.B * p.H * ((p.nbq + 1) / 2);
@@ -984,7 +992,7 @@ static int launch_attn_pairs(const AttnParams& p, unsigned* counters, hipStream_
 
 template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool Q16>
 static int launch_attn(AttnParams p, hipStream_t st) {
-  constexpr bool PAIRS = D == 128 && !DUMP && !LSE && !EXACT && !PT;
+  constexpr bool PAIRS = D == 128 && !DUMP && !PT;
   if (!PAIRS || !pairs_pay(p.total, p.nbk, CAUSAL)) p.share = nullptr;
   const size_t smem = attn_smem<D>(p.nbk, PT);
   if (!DUMP && want_pacing(p, D, CAUSAL, EXACT) && pace_list_fits(p, D, PT)) {
@@ -1011,7 +1019,7 @@ static int launch_attn(AttnParams p, hipStream_t st) {
       unsigned* counters = pd.counters + (g_pace_launches.fetch_add(1u) % PACE_SETS) * (8 * PACE_PAD);
       if (p.share == nullptr || p.share_ready) hipLaunchKernelGGL(attn_pace_reset_kernel, dim3(1), dim3(8 * PACE_PAD), 0, st, counters);
       if constexpr (PAIRS)
-        if (int rc = p.share == nullptr ? PARO_OK : launch_attn_pairs<OUT_DT, CAUSAL, Q16>(p, counters, st)) return rc;
+        if (int rc = p.share == nullptr ? PARO_OK : launch_attn_pairs<OUT_DT, CAUSAL, LSE, EXACT, Q16>(p, counters, st)) return rc;
       hipLaunchKernelGGL(kern, dim3(8 * G), dim3(128), smem, st, p, counters, per, spins, slack);
       PARO_HIP(hipGetLastError());
       return PARO_OK;
@@ -1019,7 +1027,7 @@ static int launch_attn(AttnParams p, hipStream_t st) {
   }
   if constexpr (PAIRS)
     if (p.share != nullptr)
-      if (int rc = launch_attn_pairs<OUT_DT, CAUSAL, Q16>(p, nullptr, st)) return rc;
+      if (int rc = launch_attn_pairs<OUT_DT, CAUSAL, LSE, EXACT, Q16>(p, nullptr, st)) return rc;
   const int grid = ((p.total + 7) / 8) * 8;
   auto kern = attn_sparse_kernel<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, Q16>;
   if (smem > 48 * 1024)
@@ -1108,8 +1116,8 @@ bool attn_takes_residual(int B, int H, int Nq, int Nk, int D, bool causal, bool 
          split_takes_residual((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), D);
 }
 
-bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, bool with_lse, int flags) {
-  return !with_lse && pair_call(D, flags) && pairs_pay((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), causal);
+bool attn_wants_share(int B, int H, int Nq, int Nk, int D, bool causal, int flags) {
+  return pair_call(D, flags) && pairs_pay((int64_t)B * H * ceil_div(Nq, 64), ceil_div(Nk, 64), causal);
 }
 
 int attn_sparse_impl(const int8_t* q8, const int8_t* k8, const uint8_t* v8, const float* q_scale, const float* k_scale,
@@ -1249,7 +1257,8 @@ extern "C" int paro_attn_sparse_unpermute_fwd(const int8_t* q8, const int8_t* k8
 
 extern "C" int64_t paro_attn_scratch_bytes(int B, int H, int Nq, int Nk, int D, int is_causal, int with_lse, int flags) {
   if (B <= 0 || H <= 0 || Nq <= 0 || Nk <= 0) return 0;
-  return paro::attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, with_lse != 0, flags) ? (int64_t)B * H * 4 : 0;
+  (void)with_lse;
+  return paro::attn_wants_share(B, H, Nq, Nk, D, is_causal != 0, flags) ? (int64_t)B * H * 4 : 0;
 }
 
 extern "C" int paro_attn_sparse_scratch_fwd(const int8_t* q8, const int8_t* k8, const uint8_t* v8,

@@ -60,6 +60,12 @@ def test_same_bits_as_two_waves(Nq, Nk, H, Hkv, causal, dtype):
     run = lambda **kw: P.paroattn_qk_int8_pv_fp16_cuda(q, k, v, m, is_causal=causal, smooth_v=False, **kw)
     got, ref = run(), run(two_waves=True)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    # true exponentials, and the log-sum-exp of rows with and without a kept block, with and without the K mean
+    got, ref = run(exact_exp=True), run(exact_exp=True, two_waves=True)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    for smooth_k in (False, True):
+        got, ref = run(return_lse=True, smooth_k=smooth_k), run(return_lse=True, smooth_k=smooth_k, two_waves=True)
+        assert torch.equal(got[0].view(torch.int16), ref[0].view(torch.int16)) and torch.equal(got[1], ref[1])
     got, ref = (P.paroattn_qk_int8_pv_fp16_cuda(q, k, v.nan_to_num(1.0, 1.0, 1.0), m, is_causal=causal, smooth_k=True, two_waves=w)
                 for w in (False, True))
     assert torch.isfinite(ref).all() and torch.equal(got, ref)
@@ -117,7 +123,7 @@ def test_replayed_graph():
 
 def test_calls_without_the_kernel():
     L = _lib.load()
-    for args in ((1, 48, 16384, 16384, 64, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 1, 0), (1, 48, 16320, 16320, 128, 0, 0, 0),
-                 (1, 15, 16384, 16384, 128, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 0, _lib.PARO_ATTN_EXACT_EXP),
+    for args in ((1, 48, 16384, 16384, 64, 0, 0, 0), (1, 48, 16320, 16320, 128, 0, 0, 0),
+                 (1, 15, 16384, 16384, 128, 0, 0, 0), (1, 48, 16384, 16384, 128, 0, 0, _lib.PARO_ATTN_UNPACED),
                  (1, 48, 64 * 2040, 64 * 2040, 128, 0, 0, 0), (0, 1, 1, 1, 128, 0, 0, 0)):
         assert L.paro_attn_scratch_bytes(*args) == 0

@@ -69,8 +69,15 @@ __global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const
   const int64_t bh = blockIdx.x / PARTS;
   const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + part * 8 + c4;
   v4f s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int r = sl; r < n_rows; r += SL) s += p[(int64_t)r * C4];
+  // (eight at a time also where there are fewer: a loop unrolled by eight takes the remainder one by one)
+  for (int r = sl; r < n_rows; r += 8 * SL) {
+    v4f x[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = p[(int64_t)min(r + u * SL, n_rows - 1) * C4];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (r + u * SL < n_rows) s += x[u];
+  }
   red[sl][c4] = s;
   __syncthreads();
   if (threadIdx.x < 32) {

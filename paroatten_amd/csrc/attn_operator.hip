@@ -657,7 +657,7 @@ extern "C" int paro_attn_operator(const void* q, const void* k, const void* v, i
     extra.v_resid = p.v_resid;
     extra.resid_rows = 2 * p.nbk;
   } else if (p.v_resid && !p.one_launch) {
-    const ShareLook look = {sparse, sparse_batch_stride != 0 ? B * H : H, p.nbq, p.nbk, is_causal, extra.share};
+    const ShareLook look = {sparse, sparse_batch_stride, H, sparse_batch_stride != 0 ? B * H : H, p.nbq, p.nbk, is_causal, extra.share};
     if ((rc = v_fp8_add_residual(p.v_resid, p.v_scale, p.v_mean, B, Hkv, Nk, D, st, extra.share ? &look : nullptr))) return rc;
     extra.share_ready = extra.share != nullptr;
   }

@@ -20,6 +20,9 @@
 // blocks are in flight; then the MFMAs of S^T(i+1) and P.V(i) are issued back to back and run on under
 // the VALU phase of block i+1.  One barrier per block.
 //
+// D = 128: heads whose neighbouring q-blocks keep the same blocks are taken two q-blocks to a workgroup of four waves, on one set
+// of tiles (attn_sparse_pair_kernel).
+//
 // Workgroups are renumbered so that each of the 8 XCDs walks a contiguous range of (batch, head,
 // q-block): the K8/V8 of the one or two heads an XCD is working on stay resident in its own L2.
 //
@@ -978,7 +981,7 @@ static bool pace_list_fits(const AttnParams& p, int D, bool per_thread) {
 // The two launches in front of one on p, whose heads they divide between the pair kernel and that one.
 template <int OUT_DT, bool CAUSAL, bool LSE, bool EXACT, bool Q16>
 static int launch_attn_pairs(const AttnParams& p, unsigned* counters, hipStream_t st) {
-  const ShareLook look = {p.sparse, p.sparse_bs != 0 ? p.B * p.H : p.H, p.nbq, p.nbk, CAUSAL, p.share};
+  const ShareLook look = {p.sparse, p.sparse_bs, p.H, p.sparse_bs != 0 ? p.B * p.H : p.H, p.nbq, p.nbk, CAUSAL, p.share};
   if (!p.share_ready) hipLaunchKernelGGL(attn_share_kernel, dim3(look.heads), dim3(SHARE_THREADS), 0, st, look, counters);
   const size_t smem = pair_smem(p.nbk);
   auto kern = attn_sparse_pair_kernel<OUT_DT, CAUSAL, LSE, EXACT, Q16>;

@@ -6,8 +6,9 @@
 namespace paro {
 
 struct ShareLook {
-  const uint8_t* mask;     // [heads][nbq][nbk] bytes
-  int heads;               // of the mask: B * H, or H where one mask serves every batch entry
+  const uint8_t* mask;     // [batch][H][nbq][nbk] bytes
+  int64_t batch_stride;
+  int H, heads;            // heads of the mask: B * H, or H where one mask serves every batch entry
   int nbq, nbk, causal;
   int* share;              // [heads], 1 or 0
 };
@@ -25,7 +26,7 @@ __device__ __forceinline__ void share_look(const ShareLook& p, int head) {
     const int pair = t * pairs / SHARE_THREADS;
     const int cols = p.causal ? min(p.nbk, 2 * pair + 2) : p.nbk;
     if (cols >= 8) {
-      const uint8_t* a = p.mask + ((int64_t)head * p.nbq + 2 * pair) * p.nbk;
+      const uint8_t* a = p.mask + head / p.H * p.batch_stride + ((int64_t)(head % p.H) * p.nbq + 2 * pair) * p.nbk;
       unsigned seed = (unsigned)t * 2654435761u + 12345u;
       uint64_t xa[4], xb[4];
 #pragma unroll

@@ -83,7 +83,9 @@ def test_heads_are_told_apart(B, per_batch, unpermute):
     vs, vm = torch.rand(B, H, D, generator=g, device="cuda"), torch.randn(B, H, D, generator=g, device="cuda")
     if per_batch:
         parts = [_masks(H, nb, nb, False, 1), _masks(H + 1, nb, nb, False, 2)]
-        m = torch.stack([parts[0][0], parts[1][0][1:]])
+        room = torch.ones(2, H + 3, nb, nb, dtype=torch.bool, device="cuda")   # (the C entry's batch stride, three heads more than the mask has)
+        m = room[:, :H]
+        m.copy_(torch.stack([parts[0][0], parts[1][0][1:]]))
         want = parts[0][1] + parts[1][1][1:]
     else:
         m, want = _masks(H, nb, nb, False, 1)

@@ -344,11 +344,13 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
   const int kb_first = __builtin_amdgcn_readfirstlane((int)klist[0]);
   v4i k_first[2 * KS];
   if constexpr (K_LDS) {
-    // (issued in this order: the count below leaves in flight what comes after the first tile)
+    // (issued in this order: the count below leaves in flight what comes after the first tile, and that of round 0 what comes
+    // after the second: V alone)
     load_k(kb_first, k_first);
     dma_k(kb_c, 0);
     __builtin_amdgcn_sched_barrier(0);
     dma_k(kb_1, 1);
+    __builtin_amdgcn_sched_barrier(0);
     load_v(kb_c, vfrag[0]);
     __builtin_amdgcn_sched_barrier(0);
     quantise_q();
@@ -398,7 +400,7 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
     const bool active = j < cnt;
     const float c = c_cur, c_next = qsc * clist[j + W];
     const int kidx = (int)klist[j + 3 * W];
-    if constexpr (K_LDS) {   // K(r + 1) has landed: everything older than V(r)
+    if constexpr (K_LDS) {   // K(r + 1) has landed: everything older than V(r), whose requests are the last ones
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DT) : "memory");
       read_k(par ^ 1);
     }
@@ -414,8 +416,12 @@ __global__ void __launch_bounds__(64 * W, D == 64 ? 2 : 1) attn_sparse_split_ker
     const bool left = active && left_range(cur, c);
     if (lane == 0) flag[wave] = left;
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (K_LDS) dma_k(kb_2, par);       // K(r + 2): K(r) has been used
-    else load_k(kb_2, kfrag[par]);
+    if constexpr (K_LDS) {
+      dma_k(kb_2, par);                          // K(r + 2): K(r) has been used
+      __builtin_amdgcn_sched_barrier(0);         // (in front of V: the next round's count leaves in flight the last 2 * DT)
+    } else {
+      load_k(kb_2, kfrag[par]);
+    }
     load_v(kb_1, vfrag[par ^ 1]);                // V(r + 1)
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

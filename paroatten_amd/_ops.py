@@ -4,6 +4,7 @@ some tens of microseconds more on the host."""
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import load, ptr, require_gpu, stream_of
@@ -181,10 +182,15 @@ def permute_inverse(o, orders, F, Hh, W, n_text, out):
     return out
 
 
+def _has_tangent(t):
+    return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
+
+
 def head_norm(q, k, q_weight, q_bias, q_eps, k_weight, k_bias, k_eps):
     params = [w for w in (q_weight, q_bias, k_weight, k_bias) if w is not None]
     if (any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.device != q.device or t.dtype != q.dtype
-            or torch.is_grad_enabled() and t.requires_grad or t.data_ptr() % 16 for t in (q, k, *params))
+            or torch._C._functorch.is_functorch_wrapped_tensor(t) or t.is_neg() or t._is_zerotensor()
+            or torch.is_grad_enabled() and t.requires_grad or _has_tangent(t) or t.data_ptr() % 16 for t in (q, k, *params))
             or q.dtype not in _lib.DTYPE_CODE or q.dim() != 4 or q.size(-1) not in (64, 128) or q.numel() == 0 or k.shape != q.shape
             or any(w.dim() != 1 or w.numel() != q.size(-1) or not w.is_contiguous() for w in params)
             or not q.transpose(1, 2).is_contiguous() or not k.transpose(1, 2).is_contiguous()

@@ -218,13 +218,19 @@ def _head_norm(norm, x: torch.Tensor) -> torch.Tensor:
     return norm(x)
 
 
+_PLAIN_PARAMETERS = frozenset((torch.nn.Parameter, torch.Tensor, type(None)))
+
+
 def _head_norms(norm_q, norm_k, q: torch.Tensor, k: torch.Tensor):
     """(norm_q(q), norm_k(k)) for the [B,H,N,D] views of token-major projections: in one launch of the library's own where both
     are plain LayerNorms over the channels and the tensors fit (csrc/torch_binding.cpp, head_norm)."""
     if norm_q is not None and norm_k is not None and _is_plain_layer_norm(norm_q) and _is_plain_layer_norm(norm_k):
         pq, pk, width = norm_q.__dict__["_parameters"], norm_k.__dict__["_parameters"], (q.shape[-1],)
-        if norm_q.normalized_shape == width and norm_k.normalized_shape == width and len(pq) == 2 and len(pk) == 2:
-            both = _lib.ops().head_norm(q, k, pq.get("weight"), pq.get("bias"), norm_q.eps, pk.get("weight"), pk.get("bias"), norm_k.eps)
+        params = (pq.get("weight"), pq.get("bias"), pk.get("weight"), pk.get("bias"))
+        # (a subclass of tensors may have a LayerNorm of its own)
+        if (norm_q.normalized_shape == width and norm_k.normalized_shape == width and len(pq) == 2 and len(pk) == 2
+                and type(q) is torch.Tensor and type(k) is torch.Tensor and _PLAIN_PARAMETERS.issuperset(map(type, params))):
+            both = _lib.ops().head_norm(q, k, params[0], params[1], norm_q.eps, params[2], params[3], norm_k.eps)
             if both:
                 return both
     return (q if norm_q is None else _head_norm(norm_q, q)), (k if norm_k is None else _head_norm(norm_k, k))

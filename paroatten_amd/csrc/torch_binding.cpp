@@ -501,8 +501,9 @@ std::vector<OptTensor> rope_permute_quant(const torch::Tensor& q, const torch::T
 }
 
 // cogvideox._head_norms: the LayerNorms over the channels of q and k, [B,H,N,D] views of token-major projections, in one launch;
-// nothing where the library's own modules have to do it (another type, size or order of rows, a subclass, or something that
-// records or rewrites the operation: autograd, autocast, a tracer, a mode).
+// nothing where the library's own modules have to do it (another type, size or order of rows, or something that
+// records or rewrites the operation: autograd in either direction, autocast, a tracer, a mode, a dispatching subclass; the
+// subclasses that a tensor's Python type alone tells stay with the caller).
 std::vector<torch::Tensor> head_norm(const torch::Tensor& q, const torch::Tensor& k, const OptTensor& q_weight,
                                      const OptTensor& q_bias, double q_eps, const OptTensor& k_weight, const OptTensor& k_bias,
                                      double k_eps) {
@@ -510,7 +511,9 @@ std::vector<torch::Tensor> head_norm(const torch::Tensor& q, const torch::Tensor
   auto plain = [&](const torch::Tensor& x) {
     return x.is_cuda() && x.device() == q.device() && x.scalar_type() == q.scalar_type() && !(grad && x.requires_grad()) &&
            !x.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
-                                                     c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize}));
+                                                     c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
+                                                     c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor})) &&
+           !x._fw_grad(0).defined();   // (a tangent rides on the tensor, with gradients off too)
   };
   if ((q.scalar_type() != at::kHalf && q.scalar_type() != at::kBFloat16) || q.dim() != 4 || !plain(q) || !plain(k)) return {};
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);

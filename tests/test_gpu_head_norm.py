@@ -105,3 +105,57 @@ def test_where_the_modules_keep_the_work(dev, kind, ctypes, monkeypatch):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
     assert got[0].requires_grad == (kind == "grad_of_the_input") and got[1].requires_grad == (kind == "grad_of_the_weight")
     assert bool(seen) == (kind in ("hook", "mode"))
+
+
+@pytest.mark.parametrize("ctypes", [False, True])
+@pytest.mark.parametrize("kind", ["tangent_of_the_input", "tangent_of_the_weight", "subclass", "subclass_of_the_weight", "negated_view",
+                                  "vmap"])
+def test_what_rides_on_a_tensor_is_kept(dev, kind, ctypes, monkeypatch):
+    """With gradients off: forward-mode tangents, subclasses of tensors that know no dispatch, lazily negated views and batched tensors
+    come out of the modules as they always did."""
+    import torch.autograd.forward_ad as fw
+
+    from paroatten_amd import _lib
+    from paroatten_amd import _ops as mirror
+    from paroatten_amd import cogvideox as C
+    if ctypes:
+        monkeypatch.setattr(_lib, "ops", lambda: mirror)
+    D = 64
+    x = torch.randn(2, 9, 3, D, device=dev, dtype=torch.float16)
+    dx = torch.randn_like(x)
+    nq, nk, seen = _norm(D, torch.float16, dev, True, 1), _norm(D, torch.float16, dev, True, 2), []
+
+    class Sub(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    with torch.no_grad(), fw.dual_level():
+        q, k = x.transpose(1, 2), (x * 2).transpose(1, 2)
+        if kind == "tangent_of_the_input":
+            k = fw.make_dual(x * 2, dx).transpose(1, 2)
+        elif kind == "tangent_of_the_weight":
+            del nq.weight
+            nq.register_parameter("weight", None)
+            nq.__dict__["_parameters"]["weight"] = fw.make_dual(torch.ones(D, device=dev, dtype=torch.float16), dx[0, 0, 0])
+        elif kind == "subclass":
+            q = q.as_subclass(Sub)
+        elif kind == "subclass_of_the_weight":
+            nk.__dict__["_parameters"]["weight"] = nk.weight.data.as_subclass(Sub)
+        elif kind == "negated_view":
+            q = torch._neg_view(x).transpose(1, 2)
+        seen.clear()
+        if kind == "vmap":
+            got = torch.vmap(lambda a, b: C._head_norms(nq, nk, a, b))(q[None].repeat(2, 1, 1, 1, 1), k[None].repeat(2, 1, 1, 1, 1))
+            got = [g[1] for g in got]
+        else:
+            got = C._head_norms(nq, nk, q, k)
+        called = len(seen)
+        want = [n(t.transpose(1, 2)).transpose(1, 2) for n, t in ((nq, q), (nk, k))]
+        for g, w in zip(got, want):
+            assert type(g) is type(w) and torch.allclose(g.as_subclass(torch.Tensor).float(), w.as_subclass(torch.Tensor).float(), atol=2e-3, rtol=2e-3)
+            gt, wt = fw.unpack_dual(g.as_subclass(torch.Tensor)).tangent, fw.unpack_dual(w.as_subclass(torch.Tensor)).tangent
+            assert (gt is None) == (wt is None) and (gt is None or torch.allclose(gt.float(), wt.float(), atol=2e-3, rtol=2e-3))
+        assert any(fw.unpack_dual(w.as_subclass(torch.Tensor)).tangent is not None for w in want) == kind.startswith("tangent")
+    assert (called > 0) == kind.startswith("subclass")

@@ -157,7 +157,10 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
       bool keep = m[u] != 0 && j < kmax;
       unsigned bits = 0;
       if constexpr (PAIR) {
-        const bool keep1 = keep && !(CAUSAL && j > 2 * unit), keep2 = second && m2[u] != 0 && j < kmax;
+        // (a second q-block that does not exist keeps what the first one does: results nobody stores, but a block that is not its
+        // own costs a wave a third more, and here every block would be.  Eight heads of 375 q-blocks, every block: 1290 us, with the
+        // maximum left alone until a block of the wave's own has come 1202, so 1068; of 376: 1070)
+        const bool keep1 = keep && !(CAUSAL && j > 2 * unit), keep2 = second ? m2[u] != 0 && j < kmax : keep1;
         bits = (keep1 ? 1u << 16 : 0u) | (keep2 ? 1u << 17 : 0u);
         keep = keep1 || keep2;
         own += __popcll(__ballot(sub == 0 ? keep1 : keep2));
@@ -614,7 +617,7 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
     __builtin_amdgcn_sched_barrier(0);
     // (the first block has no maximum yet.  Lane j < 16 holds the sums of q-rows j and j + 16 in d_new[0]
     // and d_new[1]; a NaN byte of either row makes its own sum NaN whatever the hardware makes of 0 x NaN)
-    const bool first = PAIR ? !begun : it == 0;
+    const bool first = PAIR ? mine && !begun : it == 0;
     if constexpr (PAIR) begun = begun || mine;
     if constexpr (EXACT) {
       if (first || headroom_suspect(d_new)) {

@@ -67,7 +67,7 @@ template <int D, bool PAIR = false> struct AttnLds {
 
 // One 64-row q-block `vid` (numbered over batch, head, q-block) by one workgroup of two waves.
 //
-// PACED: called from the paced launch, once per generation.
+// PACED: called from the paced launch, once per generation; 2: whose heads the pair kernel has a part of.
 //
 // PT: the scales have the reference's per-thread granularity (qk_quant_gran 3, csrc/qattn/
 // qk_int_sv_f16_cuda_sm80.cu:112-116 and :129-133): eight q scales per 32-row group, scale g for the rows
@@ -82,7 +82,7 @@ template <int D, bool PAIR = false> struct AttnLds {
 // PAIR: two q-blocks, the vid-th pair, by four waves (attn_sparse_pair_kernel).  A block that the other q-block alone keeps runs
 // through the loop with all its columns out of the softmax and V as zero, which leaves the state as it was; as a branch round
 // the products it cost 22 to 90 spilled registers.
-template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, bool PACED, bool Q16, bool PAIR = false>
+template <int D, int OUT_DT, bool CAUSAL, bool DUMP, bool LSE, bool EXACT, bool PT, int PACED, bool Q16, bool PAIR = false>
 __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) {
   static_assert(!PT || !DUMP, "per-thread scales: no score dump");
   static_assert(!Q16 || (!PT && !DUMP), "16-bit queries: neither per-thread scales nor the score dump");
@@ -103,10 +103,12 @@ __device__ __forceinline__ void attn_qblock(const AttnParams& p, const int vid) 
 
   // (opaque to the compiler.  In the paced kernel, which calls this in a loop, everything derived from the lane number
   // alone is otherwise computed once in front of that loop and kept in registers: at D = 64 35 more than the 168 that
-  // three waves per SIMD allow, at D = 128 all 256 and two to eight spilled, which took N = 32760, H = 40, density 0.3 from
-  // 3684 to 3710 us)
+  // three waves per SIMD allow; at D = 128 beside the look at the heads, or with per-thread scales, all 256 and 2 to 30
+  // spilled, and with 16-bit queries nothing is gained, N = 30000, 12 and 20 heads 971 and 1611 us, opaque 956 and 1589.  On INT8
+  // queries the registers are there: a layer of N = 32760, H = 40, scattered blocks of density 0.3, 3757 us, opaque 3822)
+  constexpr bool HOIST = D == 128 && PACED == 1 && !PT && !Q16;
   int t = threadIdx.x;
-  if constexpr (D == 64 || PACED) asm volatile("" : "+v"(t));
+  if constexpr (!HOIST && (D == 64 || PACED)) asm volatile("" : "+v"(t));
   const int lane = t & 63, part = t >> 6;   // part: what the wave moves of a tile
   const int wave = PAIR ? part & 1 : part;  // its half of the q-block
   const int l32 = lane & 31, lh = lane >> 5;
@@ -823,7 +825,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
   bool waiting = true;   // a workgroup that has once waited in vain goes on without waiting for the rest of the launch
   // (looked at once: at every generation it was 2 us of each, 40 us at N = 32760, H = 40)
   bool some = false;     // whether the pair kernel has heads of this launch
-  if (p.share != nullptr) {
+  if (D == 128 && !DUMP && !PT && p.share != nullptr) {
     bool all = true;
     for (int i = threadIdx.x; i < (p.sparse_bs != 0 ? p.B * p.H : p.H); i += 128) {
       const bool shared = p.share[i] != 0;
@@ -833,38 +835,49 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD)
     some = __syncthreads_or(some);
     if (__syncthreads_and(all)) return;
   }
-  for (int base = 0; base < per; base += G) {
-    const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
-    if (some) {
-      // a generation all of whose heads are attn_sparse_pair_kernel's does not meet (its heads are those from its first
-      // slot's to its last one's, and every workgroup of the XCD comes to the same answer)
-      const int last = qblock_of<CAUSAL>(p, xcd, min(base + G, per) - 1, per) / p.nbq;
-      bool any = false;
-      for (int bh = qblock_of<CAUSAL>(p, xcd, base, per) / p.nbq; bh <= last && bh < p.B * p.H; bh++) any |= !tiles_shared(p, bh);
-      if (!any) continue;
-    }
-    if (vid < p.total && !(some && tiles_shared(p, vid / p.nbq)))
-      attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, true, Q16>(p, vid);
-    if (base + G >= per) break;
-    // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
-    __syncthreads();   // also: both waves are done with this q-block's lists in LDS
-    if (threadIdx.x == 0) {
-      arrivals += (unsigned)G;
-      unsigned* c = counters + xcd * PACE_PAD;
-      __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (waiting) {
-        int spin = 0;
-        for (; spin < spin_limit; spin++) {
-          if (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + (unsigned)slack >= arrivals) break;
-          __builtin_amdgcn_s_sleep(32);
-        }
-        // its generation is not co-resident (another kernel holds compute units, or the counters are not this
-        // launch's alone): waiting again at every generation would cost the spin limit each time
-        if (spin >= spin_limit && spin_limit > 0) waiting = false;
+  auto generations = [&](auto mixed) __attribute__((always_inline)) {
+    constexpr bool MIXED = decltype(mixed)::value;
+    for (int base = 0; base < per; base += G) {
+      const int vid = base + slot < per ? qblock_of<CAUSAL>(p, xcd, base + slot, per) : p.total;
+      if constexpr (MIXED) {
+        // a generation all of whose heads are attn_sparse_pair_kernel's does not meet (its heads are those from its first
+        // slot's to its last one's, and every workgroup of the XCD comes to the same answer)
+        const int last = qblock_of<CAUSAL>(p, xcd, min(base + G, per) - 1, per) / p.nbq;
+        bool any = false;
+        for (int bh = qblock_of<CAUSAL>(p, xcd, base, per) / p.nbq; bh <= last && bh < p.B * p.H; bh++) any |= !tiles_shared(p, bh);
+        if (!any) continue;
       }
+      if (vid < p.total && !(MIXED && tiles_shared(p, vid / p.nbq)))
+        attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, MIXED ? 2 : 1, Q16>(p, vid);
+      if (base + G >= per) break;
+      // every workgroup of the XCD arrives once per generation, with or without a q-block of its own
+      __syncthreads();   // also: both waves are done with this q-block's lists in LDS
+      if (threadIdx.x == 0) {
+        arrivals += (unsigned)G;
+        unsigned* c = counters + xcd * PACE_PAD;
+        __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (waiting) {
+          int spin = 0;
+          for (; spin < spin_limit; spin++) {
+            if (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + (unsigned)slack >= arrivals) break;
+            __builtin_amdgcn_s_sleep(32);
+          }
+          // its generation is not co-resident (another kernel holds compute units, or the counters are not this
+          // launch's alone): waiting again at every generation would cost the spin limit each time
+          if (spin >= spin_limit && spin_limit > 0) waiting = false;
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
+  };
+  // (two loops: a launch that has all heads to itself runs the code that it ran before there was a pair kernel)
+  if constexpr (D == 128 && !DUMP && !PT) {
+    if (some) {
+      generations(std::true_type{});
+      return;
+    }
   }
+  generations(std::false_type{});
 }
 
 __global__ void attn_pace_reset_kernel(unsigned* counters) { counters[threadIdx.x] = 0u; }

@@ -69,6 +69,12 @@ __global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const
   const int64_t bh = blockIdx.x / PARTS;
   const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + part * 8 + c4;
   v4f s = {0.f, 0.f, 0.f, 0.f};
+  // (what the sum goes into is asked for here: behind it, it was one more trip)
+  const int64_t ch = bh * D + part * 32 + (threadIdx.x & 31);
+  const float mean = v_mean[ch], scale = v_scale[ch];
+  if (n_rows <= SL) {
+    if (sl < n_rows) s = p[(int64_t)sl * C4];
+  } else
   // (eight at a time also where there are fewer: a loop unrolled by eight takes the remainder one by one)
   for (int r = sl; r < n_rows; r += 8 * SL) {
     v4f x[8];
@@ -81,11 +87,10 @@ __global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const
   red[sl][c4] = s;
   __syncthreads();
   if (threadIdx.x < 32) {
-    const int64_t ch = bh * D + part * 32 + threadIdx.x;
     float t = 0.f;
 #pragma unroll 8
     for (int i = 0; i < SL; i++) t += red[i][threadIdx.x >> 2][threadIdx.x & 3];
-    v_mean[ch] += v_scale[ch] * (t / (float)N);
+    v_mean[ch] = mean + scale * (t / (float)N);
   }
 }
 

@@ -88,7 +88,8 @@ __global__ void __launch_bounds__(128, (D == 64 ? 3 : 2)) attn_sparse_pv16_kerne
   float* clist = reinterpret_cast<float*>(smem + Lds::LIST_OFF);
   unsigned short* klist = reinterpret_cast<unsigned short*>(clist + p.nbk + Lds::LIST_PAD + 1);
 
-  const int block = with_args(p, blockIdx.x), xcd = block & 7, slot = block >> 3, per = gridDim.x >> 3;
+  // (arguments as they come to be needed: all of them asked for at once, 8 heads of 4000 tokens, D = 64 took 40.1 us instead of 38.2)
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, per = gridDim.x >> 3;
   const int vid = causal ? qblock_of<true>(p, xcd, slot, per) : qblock_of<false>(p, xcd, slot, per);
   if (vid >= p.total) return;
 

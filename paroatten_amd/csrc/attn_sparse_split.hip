@@ -545,11 +545,30 @@ static int launch_split(const AttnParams& p, bool causal, bool exact, hipStream_
 // A SIMD holds two of these waves at D = 64 and one at D = 128, so W is what fills the card with one round of workgroups.
 // (Beyond: D = 64, 520 q-blocks, W = 2 0.82; D = 128, 260 q-blocks, W = 2 0.87.)  Longer lists gain more, up to 1.9 times at 77
 // blocks of 128; of the lists the host knows only the bound, the number of key blocks.  With less than one block in eight
-// kept (lists of one to four) the lines below lose up to 6 %, at 12 to 20 key blocks.  Calls with the log-sum-exp below 20 key
-// blocks or above 448 q-blocks stay with two waves: their bits are those of the per-thread kernels, which callers may compare.
+// kept (lists of one to four) the lines below lose up to 6 %, at 12 to 20 key blocks.
+// (Those are of the attention alone, on operands that it has just read.  Behind the launches that write them, which is how it is
+// called, each workgroup's first tiles come from further away, the waves of this kernel wait for them all together, and it gains
+// less.  Replayed graphs, faster than two waves by, in per cent, runs of 0.25 / scattered blocks of 0.3 / every block:
+//   D = 64   q-blocks                 110 to 120         180 to 256               320             400            500
+//   operator       7 key blocks   1 / 2 / 3
+//                 27              16 / 25 / 35   (W = 4) 6 / 16 / 21   (W = 2) 4 / 4 / 9      2 / 3 / 4
+//                 64                             (W = 4) 16 / 29 / 34          8 / 11 / 13    8 / 15 / 10    4 / 10 / 5
+//   layer          7             -0 / -1 / -3
+//                 12 (W = 4)     -2 / -2 / 3
+//                 27              -2 / 2 / 8     (W = 2) -5 / -5 / -4  (W = 2) -2 / -3 / -0   -5 / -4 / -2
+//                 36               1 / 11 / 19   (W = 4) -3 / 3 / 6            -1 / -3 / 2    -4 / -2 / -0   -5 / -3 / -1
+//                 64                             (W = 4) 2 / 8 / 21            -1 / 0 / 4     0 / 2 / 5      -3 / 0 / 1
+//                100                             (W = 4) 4 / 19 / 34           1 / 5 / 8      0 / 1 / 7      -2 / 1 / 4
+//   D = 128: 3 to 25 ahead in both.
+// An operator call saves the launch of the residual sums besides, a layer, which stores through the inverse permutation, does
+// not: there two waves keep the calls of more than 256 q-blocks below 100 key blocks and those of fewer than 12.)
+// The lines of the log-sum-exp, 20 key blocks and 448 q-blocks, are not where this kernel stops paying (operator, D = 64, 400
+// q-blocks, W = 2: 12 to 20 % ahead): the answers of paro_attn_kernel_form for calls of 512 q-blocks, and the bits of short calls,
+// which are the per-thread kernel's, are older than it and kept.
 int split_width(const AttnParams& p, int D) {
   int W = 0;
   if (p.lse != nullptr && (p.nbk < 20 || p.total > 448)) return 0;
+  if (p.orders != nullptr && D == 64 && (p.nbk < 12 || (p.total > 256 && p.nbk < 100))) return 0;
   if (D == 64) {
     if (p.total <= 128) W = p.nbk >= 12 ? 4 : p.nbk >= 7 ? 2 : 0;
     else if (p.total <= 512 && p.nbk >= 20) W = p.total <= 256 && p.nbk >= 32 ? 4 : 2;

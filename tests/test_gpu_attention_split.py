@@ -94,3 +94,22 @@ def test_grouped_heads_and_unpermuting_store(dev):
                                     two_waves=two)
         outs.append(o)
     _close(outs[0], outs[1], v)
+
+
+@pytest.mark.parametrize("H,grid,n_text", [(9, (8, 16, 16), 0), (16, (8, 16, 15), 100), (3, (7, 8, 7), 40), (12, (9, 8, 8), 0),
+                                           (5, (16, 15, 17), 7)])
+def test_layers_stay_with_two_waves_where_those_are_faster(dev, H, grid, n_text):
+    """Stores through the inverse permutation: with more than 256 q-blocks below 100 key blocks, and with fewer than 12 key blocks,
+    the bits of two waves, which the other order of sums does not give."""
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import permute as PM
+    N, D = n_text + grid[0] * grid[1] * grid[2], 64
+    q, k, v = (t.to(dev) for t in synth.make_qkv(1, H, N, D, torch.float16, seed=N))
+    mask = synth.make_block_mask(H, (N + 63) // 64, 0.7, seed=N, device=dev)
+    orders = PM.head_orders(synth.make_permute_plan(1, H, seed=3), 0, dev)
+    ops = PM.rope_permute_quant(q, k, v, orders, grid, n_text)
+    outs = [torch.empty_like(q) for _ in range(2)]
+    for two, o in enumerate(outs):
+        qattn.attn_sparse_prepacked(ops.q8, ops.k8, ops.v8, ops.v_scale, ops.v_mean, o, ops.q_scale, ops.k_scale, D ** -0.5, mask,
+                                    unpermute=(orders, grid, n_text), two_waves=bool(two))
+    assert torch.equal(*outs)

@@ -968,15 +968,31 @@ static size_t pair_smem(int nbk) {
 }
 
 // Whether the heads are looked at (share_look).  Where they turn out to be scattered, that and a launch that finds nothing to do
-// cost 3 to 15 us, where they are not the gain grows with the work.  Operator, D = 128, scattered blocks of density 0.3 / rows of one
-// run of density 0.3 / every block, us, not looked at -> looked at: B = 2, H = 32, N = 4096 181 -> 185 / 181 -> 183 / 360 -> 326;
-// H = 16, N = 8192 153 -> 156 / 154 -> 137 / 356 -> 288; H = 40, N = 12000 574 -> 577 / 563 -> 546; H = 24, N = 16384 596 -> 601 /
-// 596 -> 553; H = 48, N = 20000 1700 -> 1705 / 1615 -> 1548; attention, H = 40, N = 32760 3400 -> 3415 / 3350 -> 3030.  From 16384
-// keys on that is 1 % at most against 5 to 10.  Causal calls are those of dense masks as a rule, and gain that early: B = 2,
-// H = 32, Hkv = 8, N = 8192 278 -> 281 / 280 -> 284 / 611 -> 580, half of the blocks 369 -> 371 / 374 -> 371.
+// cost 3 to 15 us, where they are not the gain grows with the work.  Operator, D = 128, replayed graphs, looked at against not, per
+// cent faster, and the mean of the five kinds of masks; products are q-blocks times key blocks:
+//            key blocks  products   every block   runs of 0.5   0.25   scattered 0.4   0.2     mean
+//   causal       64      2^17..19    4 / 5 / 3     -1 / 0 / 1   -2 / -4 / -3   -3       -3     -0.9 / -1.0 / -0.8
+//                96      2^18, 2^19  4 / 4          0 / 1       -3 / -3     -3 / -2   -3 / -2  -0.8 / -0.5
+//               128      2^18        2.9           2.8         1.1          -2.4     -3.1     0.3
+//                        2^19        5.5           3.3        -0.5          -1.8     -2.3     0.8
+//                        2^20        6.3           3.5        -0.1          -1.2     -2.2     1.2    (688 -> 647 us, 305 -> 312)
+//               192      2^19, 2^20  6.4 / 5.1     4.5 / 4.0   4.9 / 1.9  -1.4 / -0.9  -2.7 / -1.9   2.3 / 1.7
+//               256      2^19, 2^20  4.0 / 6.1     3.8 / 5.4   2.1 / 2.6  -1.9 / -1.3  -2.3 / -2.6   1.1 / 2.0
+//               375      2^20        6.2           5.1         3.2          -1.2     -1.4     2.4
+//   full        128      2^19, 2^20  13 / 8        10 / 7      5 / 2      -1.2 / -0.7  -2.0 / -1.8   5.0 / 3.0
+//               192      2^19, 2^20  4.4 / 7.0     2.8 / 5.2   0 / 2.2    -1.4 / -0.9  -1.5 / -1.3   0.8 / 2.4
+//               256      2^19, 2^20  25 / 15       22 / 13     17 / 9     -1.2 / -1.1  -2.4 / -1.5   12 / 7
+//               438      2^20, 2^21  3.7 / 6.8     3.8 / 5.9   2.2 / 5.1  -0.9 / -0.4  -1.2 / 0.2    1.5 / 3.5
+//   layer       320      2^19, 2^20  2.2 / 4.5    -0.6 / 2.4  -2.6 / -0.1 -2.0 / -1.2  -3.2 / -2.2  -1.2 / 0.7
+//               434      2^20, 2^21.5  2.6 / 6.6   1.3 / 5.2  -0.5 / 2.6  -1.6 / -2.2  -1.8 / -0.8   0.0 / 2.3
+//               512      2^20, 2^22  8.7 / 9.7     8.1 / 10    8.1 / 13   -0.3 / 1.3   -1.5 / 1.9    4.6 / 7.2
+// So causal calls are ahead on the mean from somewhere between 96 and 128 key blocks on, and lose less than 2 % on scattered masks
+// from 2^19 to 2^20 products on.  Full ones and layers are ahead from 2^20; those below 256 key blocks are left as they are, since what
+// they would gain on runs is 2 to 7 % and what scattered masks would lose 0.5 to 1.9.
 // (Beyond 2039 key blocks the list leaves a compute unit one workgroup.)
 static bool pairs_pay(int64_t q_blocks, int nbk, bool causal) {
-  return nbk >= (causal ? 128 : 256) && q_blocks * nbk >= (int64_t)1 << 20 && pair_smem(nbk) <= 80 * 1024;
+  const int64_t products = q_blocks * nbk;
+  return (causal ? nbk >= 112 && products >= (int64_t)3 << 18 : nbk >= 256 && products >= (int64_t)1 << 20) && pair_smem(nbk) <= 80 * 1024;
 }
 
 // Calls that have a pair kernel; a caller who names a kernel form or a launch gets that one.

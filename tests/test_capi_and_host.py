@@ -99,6 +99,18 @@ def test_kernel_form_query_needs_no_gpu(monkeypatch):
     assert form(1, 1, 64, 64, 64, 0, 0, L.PARO_ATTN_PACED | L.PARO_ATTN_UNPACED) == L.PARO_ERR_INVALID_VALUE
 
 
+def test_calls_that_look_for_shared_tiles_need_no_gpu(monkeypatch):
+    """both sides of the lines: key blocks, and q-blocks times key blocks (the smallest causal sizes on them have 112 key blocks)"""
+    import paroatten_amd._lib as L
+    monkeypatch.delenv("PARO_ATTN_PACING", raising=False)
+    words = lambda B, H, nbq, nbk, causal: L.load().paro_attn_scratch_bytes(B, H, 64 * nbq, 64 * nbk, 128, causal, 0, 0) // (4 * B * H)
+    assert words(1, 63, 112, 112, 1) == 1 and words(1, 62, 112, 112, 1) == 0    # 3 * 2^18 / 112^2 = 62.7
+    assert words(2, 48, 111, 111, 1) == 0 and words(2, 48, 112, 112, 1) == 1
+    assert words(1, 24, 256, 128, 1) == 1 and words(1, 23, 256, 128, 1) == 0
+    assert words(1, 16, 256, 256, 0) == 1 and words(1, 15, 256, 256, 0) == 0 and words(4, 48, 255, 255, 0) == 0
+    assert words(1, 8, 2039, 2039, 0) == 1 and words(1, 8, 2040, 2040, 1) == 0
+
+
 def test_c_abi_argument_errors_without_gpu():
     """argument validation happens before any launch: codes and messages come back on CPU"""
     import paroatten_amd._lib as L

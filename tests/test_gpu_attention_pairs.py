@@ -151,3 +151,43 @@ def test_an_odd_number_of_q_blocks_costs_no_more():
             end.synchronize()
             best[N] = min(best.get(N, 1e9), start.elapsed_time(end))
     assert best[24000] < 1.05 * best[24064], best
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+def test_token_major_codes(causal):
+    """INT8 codes of q and k and the output in [B,N,H,D] memory, through the extension entry point."""
+    from paroatten_amd import _qattn_sm80 as qattn
+    from paroatten_amd import quant as Q
+    H, N, D = 16, 16321, 128
+    nb = (N + 63) // 64
+    q, k, v = (t.transpose(1, 2).contiguous() for t in _operands(1, H, H, N, N, 11))
+    m, _ = _masks(H, nb, nb, bool(causal), 12)
+    q8, qs, k8, ks = Q.per_warp_int8(q, k, None, BLKQ=64, WARPQ=32, BLKK=64, tensor_layout="NHD")
+    assert q8.shape == (1, N, H, D) and q8.is_contiguous()
+    outs = [torch.empty_like(q) for _ in range(2)]
+    for two, o in enumerate(outs):
+        qattn.qk_int8_sv_f16_accum_f16_attn(q8, k8, v, o, qs, ks, 0, causal, 2, D ** -0.5, 0, m, two_waves=bool(two))
+    assert torch.equal(*outs)
+
+
+def test_two_streams_at_once():
+    """Calls that overlap on the card, one on runs and one on scattered blocks, and the same the other way round: each looks at its own
+    heads."""
+    H, N = 16, 16384
+    ops = [_operands(1, H, H, N, N, s) for s in (21, 22)]
+    runs, scattered = torch.zeros(H, 256, 256, dtype=torch.bool, device="cuda"), torch.rand(H, 256, 256, device="cuda") < 0.2
+    for r in range(256):
+        runs[:, r, max(0, r - 50):r + 1] = True
+    masks = [runs, scattered]
+    call = lambda i, m, **kw: P.paroattn_qk_int8_pv_fp16_cuda(*ops[i], m, **kw)
+    ref = {(i, j): call(i, masks[j], two_waves=True) for i in (0, 1) for j in (0, 1)}
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for turn in range(4):
+        outs = []
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs.append([call(i, masks[(i + turn) % 2]) for _ in range(3)])
+        torch.cuda.synchronize()
+        for i in (0, 1):
+            assert all(torch.equal(o, ref[i, (i + turn) % 2]) for o in outs[i])

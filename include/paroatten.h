@@ -54,8 +54,8 @@ extern "C" {
 #define PARO_ATTN_TWO_WAVES 8 /* kernel form: two waves per 64-row q-block (32 q-rows each) also where the
                                  library would pick one wave per q-block (head size 64, plain launch, more than
                                  1024 q-blocks; bit-identical results) or several key blocks of a q-block at a
-                                 time (without any of the form flags, up to 512 q-blocks (head size 128: 256);
-                                 the same weights, summed in another order) */
+                                 time (calls of few q-blocks without any of the form flags: paro_attn_kernel_form
+                                 says which; the same weights, summed in another order) */
 #define PARO_ATTN_PV_F16 16   /* accuracy mode: the P.V product in float16 with fp32 accumulation, as the reference's
                                  qk_int8_sv_f16_accum_f16_attn computes it (csrc/qattn/qk_int_sv_f16_cuda_sm80.cu:263-391),
                                  instead of FP8 e4m3 P and V.  True exponentials; V as given (no per-channel scale, no
@@ -231,7 +231,9 @@ int paro_attn_sparse_scratch_fwd(const int8_t* q8, const int8_t* k8, const uint8
 /* The form of the attention kernel that a call of these sizes and flags gets: one of PARO_ATTN_FORM_* (host only, no GPU is
  * needed), or a negative error code.  A measurement names the kernel it timed by this, a test the one it means to run.
  * (Heads that a call with scratch finds to share their tiles, (2b) above, leave it for the kernel made for them.)
- * PARO_ATTN_FORM_PACED: a launch of a single generation of workgroups is the plain one all the same. */
+ * PARO_ATTN_FORM_PACED: a launch of a single generation of workgroups is the plain one all the same.
+ * PARO_ATTN_FORM_SPLIT: calls with orders, (2b'), at head size 64 are PARO_ATTN_FORM_TWO_WAVES all the same below 12 key blocks of 64
+ * and, with more than 256 q-blocks of 64 rows in all heads, below 100 key blocks. */
 #define PARO_ATTN_FORM_TWO_WAVES 0 /* two waves per q-block, plain launch */
 #define PARO_ATTN_FORM_PACED 1     /* the same kernel, paced launch */
 #define PARO_ATTN_FORM_ONE_WAVE 2  /* head size 64: one wave per q-block */

@@ -19,7 +19,8 @@
 // wave for all of them, 0.6 us), the next round's products in front of the look at the row sums and all waves adding up
 // (instead of the first): 12.6 -> 11.8 us.  With the registers of two waves per SIMD at D = 64: 256 q-blocks 17.4 -> 14.3 us,
 // 384 21.9 -> 18.4.  (Tried: eight blocks a round, no faster at 64 q-blocks; K through LDS at D = 64, 12.3; D = 128 in the
-// registers of two waves per SIMD spills 70 of them, three times the time.)
+// registers of two waves per SIMD spills 70 of them, three times the time.)  The log-sum-exp at D = 64 spills two to four there, and
+// is 12 to 24 % ahead of two waves per q-block all the same (split_width).
 #include "attn_common.hpp"
 
 namespace paro {

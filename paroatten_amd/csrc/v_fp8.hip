@@ -72,18 +72,23 @@ __global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const
   // (what the sum goes into is asked for here: behind it, it was one more trip)
   const int64_t ch = bh * D + part * 32 + (threadIdx.x & 31);
   const float mean = v_mean[ch], scale = v_scale[ch];
-  if (n_rows <= SL) {
-    if (sl < n_rows) s = p[(int64_t)sl * C4];
-  } else
-  // (eight at a time also where there are fewer: a loop unrolled by eight takes the remainder one by one)
-  for (int r = sl; r < n_rows; r += 8 * SL) {
-    v4f x[8];
+  // (a batch at a time also where less of it is left, since a loop unrolled by eight takes the remainder one by one; but no more than
+  // a thread has rows: eight throughout, a layer of 20 heads, N = 2192, D = 64 39.4 us, so 38.4)
+  auto add = [&](auto batch) __attribute__((always_inline)) {
+    constexpr int U = decltype(batch)::value;
+    for (int r = sl; r < n_rows; r += U * SL) {
+      v4f x[U];
 #pragma unroll
-    for (int u = 0; u < 8; u++) x[u] = p[(int64_t)min(r + u * SL, n_rows - 1) * C4];
+      for (int u = 0; u < U; u++) x[u] = p[(int64_t)min(r + u * SL, n_rows - 1) * C4];
 #pragma unroll
-    for (int u = 0; u < 8; u++)
-      if (r + u * SL < n_rows) s += x[u];
-  }
+      for (int u = 0; u < U; u++)
+        if (r + u * SL < n_rows) s += x[u];
+    }
+  };
+  if (n_rows <= SL) add(std::integral_constant<int, 1>{});
+  else if (n_rows <= 2 * SL) add(std::integral_constant<int, 2>{});
+  else if (n_rows <= 4 * SL) add(std::integral_constant<int, 4>{});
+  else add(std::integral_constant<int, 8>{});
   red[sl][c4] = s;
   __syncthreads();
   if (threadIdx.x < 32) {

@@ -233,7 +233,7 @@ int paro_attn_sparse_scratch_fwd(const int8_t* q8, const int8_t* k8, const uint8
  * (Heads that a call with scratch finds to share their tiles, (2b) above, leave it for the kernel made for them.)
  * PARO_ATTN_FORM_PACED: a launch of a single generation of workgroups is the plain one all the same.
  * PARO_ATTN_FORM_SPLIT: calls with orders, (2b'), at head size 64 are PARO_ATTN_FORM_TWO_WAVES all the same below 12 key blocks of 64
- * and, with more than 256 q-blocks of 64 rows in all heads, below 100 key blocks. */
+ * and, with more than 256 q-blocks of 64 rows in all heads, below 76 key blocks. */
 #define PARO_ATTN_FORM_TWO_WAVES 0 /* two waves per q-block, plain launch */
 #define PARO_ATTN_FORM_PACED 1     /* the same kernel, paced launch */
 #define PARO_ATTN_FORM_ONE_WAVE 2  /* head size 64: one wave per q-block */

@@ -562,14 +562,16 @@ static int launch_split(const AttnParams& p, bool causal, bool exact, hipStream_
 //                100                             (W = 4) 4 / 19 / 34           1 / 5 / 8      0 / 1 / 7      -2 / 1 / 4
 //   D = 128: 3 to 25 ahead in both.
 // An operator call saves the launch of the residual sums besides, a layer, which stores through the inverse permutation, does
-// not: there two waves keep the calls of more than 256 q-blocks below 100 key blocks and those of fewer than 12.)
+// not: there two waves keep the calls of more than 256 q-blocks below 76 key blocks and those of fewer than 12.  Around that line,
+// on the mean of runs of 0.15 and 0.3, scattered blocks of 0.2 and 0.4 and every block: 48 key blocks -2.6 to 0.1, 56 -2.3 to 0.2, 64
+// -0.9 to 0.4, 72 (288, 360, 432 and 504 q-blocks) 0.4, 1.0, 0.0 and -1.4, 80 (320, 400, 480) 2.0, 0.5 and 0.4, 91 0.6 to 3.4.)
 // The lines of the log-sum-exp, 20 key blocks and 448 q-blocks, are not where this kernel stops paying (operator, D = 64, 400
 // q-blocks, W = 2: 12 to 20 % ahead): the answers of paro_attn_kernel_form for calls of 512 q-blocks, and the bits of short calls,
 // which are the per-thread kernel's, are older than it and kept.
 int split_width(const AttnParams& p, int D) {
   int W = 0;
   if (p.lse != nullptr && (p.nbk < 20 || p.total > 448)) return 0;
-  if (p.orders != nullptr && D == 64 && (p.nbk < 12 || (p.total > 256 && p.nbk < 100))) return 0;
+  if (p.orders != nullptr && D == 64 && (p.nbk < 12 || (p.total > 256 && p.nbk < 76))) return 0;
   if (D == 64) {
     if (p.total <= 128) W = p.nbk >= 12 ? 4 : p.nbk >= 7 ? 2 : 0;
     else if (p.total <= 512 && p.nbk >= 20) W = p.total <= 256 && p.nbk >= 32 ? 4 : 2;

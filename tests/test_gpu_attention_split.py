@@ -99,7 +99,7 @@ def test_grouped_heads_and_unpermuting_store(dev):
 @pytest.mark.parametrize("H,grid,n_text", [(9, (8, 16, 16), 0), (16, (8, 16, 15), 100), (3, (7, 8, 7), 40), (12, (9, 8, 8), 0),
                                            (5, (16, 15, 17), 7)])
 def test_layers_stay_with_two_waves_where_those_are_faster(dev, H, grid, n_text):
-    """Stores through the inverse permutation: with more than 256 q-blocks below 100 key blocks, and with fewer than 12 key blocks,
+    """Stores through the inverse permutation: with more than 256 q-blocks below 76 key blocks, and with fewer than 12 key blocks,
     the bits of two waves, which the other order of sums does not give."""
     from paroatten_amd import _qattn_sm80 as qattn
     from paroatten_amd import permute as PM

@@ -770,9 +770,7 @@ __global__ void __launch_bounds__(128, PARO_ATTN_WAVES_PER_SIMD) attn_sparse_ker
   const int block = with_args(p, blockIdx.x);
   const int vid = qblock_of<CAUSAL>(p, block & 7, block >> 3, gridDim.x >> 3);
   if (vid >= p.total) return;
-  if constexpr (D == 128 && !DUMP && !PT) {   // (the others have no pair kernel)
-    if (p.share != nullptr && tiles_shared(p, vid / p.nbq)) return;
-  }
+  if (p.share != nullptr && tiles_shared(p, vid / p.nbq)) return;
   attn_qblock<D, OUT_DT, CAUSAL, DUMP, LSE, EXACT, PT, false, Q16>(p, vid);
 }
 

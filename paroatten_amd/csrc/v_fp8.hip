@@ -46,31 +46,30 @@ __global__ void __launch_bounds__(256) v_pack_kernel(const unsigned short* __res
   v_pack_body<DT, D>(v + b * vs_b + h * vs_h, v8, work, v_mean, resid, N, nb, vs_n, blockIdx.x, (int64_t)b * gridDim.y + h);
 }
 
-// v_mean += v_scale * (sum over tiles and row tiles of the residual sums) / N.  A workgroup has 32 channels of a head; a thread
-// takes four of them of every SL-th row (16-byte loads, all independent), the SL partial sums per channel are
-// combined through LDS in a fixed order.  What bounds it is the trips to memory one after the other, behind a launch of 4 to
+// v_mean += v_scale * (sum over tiles and row tiles of the residual sums) / N.  A workgroup has one of PARTS parts of a head's channels;
+// a thread takes four of them of every SL-th row (16-byte loads, all independent), the SL partial sums per channel are
+// combined through LDS in a fixed order, the same for any PARTS.  What bounds it is the trips to memory one after the other, behind a launch of 4 to
 // 5 us in a kernel trace; with one workgroup to a head and four loads in flight per thread instead of eight, 40 heads, D = 128:
-// N = 75600 15.0 -> 10.4 us, N = 32760 8.0 -> 6.3 (D = 64, N = 17776, 96 heads: 5.3 and 5.6).
-template <int D> constexpr int V_RESIDUAL_THREADS = 1024 / D * 4 * 8;
-template <int D>
-__global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const float* __restrict__ resid,
+// four parts N = 75600 15.0 -> 10.4 us, N = 32760 8.0 -> 6.3 (D = 64, two parts, N = 17776, 96 heads: 5.3 and 5.6).
+template <int D, int PARTS>
+__global__ void __launch_bounds__(1024 / PARTS) v_residual_kernel(const float* __restrict__ resid,
                                                           const float* __restrict__ v_scale,
                                                           float* __restrict__ v_mean, int N, int n_rows, int heads,
                                                           const ShareLook look) {
-  constexpr int PARTS = D / 32;
+  constexpr int CH = D / PARTS, CW = CH / 4;   // a workgroup's channels, and threads per row
   if ((int)blockIdx.x >= heads * PARTS) {
     share_look(look, blockIdx.x - heads * PARTS);
     return;
   }
-  constexpr int C4 = D / 4;          // threads per row
+  constexpr int C4 = D / 4;
   constexpr int SL = 1024 / C4;      // rows in flight per pass
-  __shared__ v4f red[SL][8];
-  const int c4 = threadIdx.x % 8, sl = threadIdx.x / 8, part = blockIdx.x % PARTS;
+  __shared__ v4f red[SL][CW];
+  const int c4 = threadIdx.x % CW, sl = threadIdx.x / CW, part = blockIdx.x % PARTS;
   const int64_t bh = blockIdx.x / PARTS;
-  const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + part * 8 + c4;
+  const v4f* p = reinterpret_cast<const v4f*>(resid + bh * n_rows * D) + part * CW + c4;
   v4f s = {0.f, 0.f, 0.f, 0.f};
   // (what the sum goes into is asked for here: behind it, it was one more trip)
-  const int64_t ch = bh * D + part * 32 + (threadIdx.x & 31);
+  const int64_t ch = bh * D + part * CH + (threadIdx.x & (CH - 1));
   const float mean = v_mean[ch], scale = v_scale[ch];
   // (a batch at a time also where less of it is left, since a loop unrolled by eight takes the remainder one by one; but no more than
   // a thread has rows: eight throughout, a layer of 20 heads, N = 2192, D = 64 39.4 us, so 38.4)
@@ -91,7 +90,7 @@ __global__ void __launch_bounds__(V_RESIDUAL_THREADS<D>) v_residual_kernel(const
   else add(std::integral_constant<int, 8>{});
   red[sl][c4] = s;
   __syncthreads();
-  if (threadIdx.x < 32) {
+  if (threadIdx.x < CH) {
     float t = 0.f;
 #pragma unroll 8
     for (int i = 0; i < SL; i++) t += red[i][threadIdx.x >> 2][threadIdx.x & 3];
@@ -103,13 +102,15 @@ int v_fp8_add_residual(const float* resid, const float* v_scale, float* v_mean, 
                        hipStream_t st, const ShareLook* look) {
   const int n_rows = ceil_div(N, 64) * 2, heads = B * Hkv;
   const ShareLook l = look ? *look : ShareLook{};
-  const dim3 grid(heads * (D / 32) + l.heads);
-  if (D == 64)
-    hipLaunchKernelGGL((v_residual_kernel<64>), grid, dim3(V_RESIDUAL_THREADS<64>), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
-  else
-    hipLaunchKernelGGL((v_residual_kernel<128>), grid, dim3(V_RESIDUAL_THREADS<128>), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
-  PARO_HIP(hipGetLastError());
-  return PARO_OK;
+  auto launch = [&](auto kern, int parts) {
+    hipLaunchKernelGGL(kern, dim3(heads * parts + l.heads), dim3(1024 / parts), 0, st, resid, v_scale, v_mean, N, n_rows, heads, l);
+    PARO_HIP(hipGetLastError());
+    return PARO_OK;
+  };
+  if (D == 128) return launch(v_residual_kernel<128, 4>, 4);
+  // (a workgroup per head / two, layer, replayed graphs, us: 14 heads, N = 630 22.60 / 22.78, 1024 24.42 / 24.57, 2048 30.79 / 30.90, 3 heads,
+  // 4096 29.36 / 29.49; from 8192 tokens on two are ahead, 3 heads 43.77 / 43.58, 48 188.3 / 188.1)
+  return n_rows <= 128 ? launch(v_residual_kernel<64, 1>, 1) : launch(v_residual_kernel<64, 2>, 2);
 }
 
 template <int DT, int D>

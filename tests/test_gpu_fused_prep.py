@@ -262,3 +262,17 @@ def test_k_mean_of_many_heads_is_that_of_a_few(dev, D, heads, grid, n_text, dtyp
     if rot is not None:
         want = rot.to(dtype).double().mean(dim=2, keepdim=True)
         assert ((km.double() - want).abs() <= want.abs() * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) + 2.0 ** -18).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("N", [1, 63, 2048, 2049, 4096, 4097, 8193])
+def test_residual_sums_of_v_by_length(dev, N, D):
+    """One, two, four or eight rows per thread at a time, and at D = 64 one workgroup per head up to 4096 tokens, two above: the offset
+    is the one that the codes call for, in float64."""
+    from paroatten_amd import permute as PM
+    B, H = 2, 3
+    v = synth.make_qkv(B, H, N, D, torch.float16, seed=N)[2]
+    orders = torch.zeros(H, dtype=torch.int32, device=dev)
+    got = PM.rope_permute_quant(v.to(dev), v.to(dev), v.to(dev), orders, (1, 1, N), 0)
+    want = v8_offset_expected(v, untile_v8(got.v8, B, H, N, D), got.v_scale)
+    assert torch.allclose(got.v_mean.cpu().double(), want, atol=1e-5, rtol=1e-5)
